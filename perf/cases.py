@@ -153,6 +153,10 @@ def _ptr(a, kind=ctypes.c_int32):
     return ctypes.cast(ctypes.c_void_p(at), ctypes.POINTER(kind))
 
 
+def _view(at, shape):
+    return torch.from_numpy(np.ctypeslib.as_array(at, shape=shape))
+
+
 class Session:
     """A program's context."""
 
@@ -196,7 +200,7 @@ class Session:
         r = g.Result()
         self.ok(self.lib.g4d_triangulate(self.ctx, _ptr(xyz, ctypes.c_double), xyz.shape[0], ctypes.byref(r)))
         self.take(r, tets, opp)
-        np.copyto(perm, np.ctypeslib.as_array(r.perm, shape=perm.shape))
+        perm.copy_(_view(r.perm, tuple(perm.shape)))
         return r.num_tets, tets, opp, perm
 
     def batch(self, xyz, offsets, tets, opp, tet_offsets):
@@ -204,15 +208,15 @@ class Session:
         self.ok(self.lib.g4d_triangulate_batch(self.ctx, _ptr(xyz, ctypes.c_double), _ptr(offsets, ctypes.c_int64),
                                                offsets.shape[0] - 1, None, ctypes.byref(r)))
         self.take(r, tets, opp)
-        np.copyto(tet_offsets, np.ctypeslib.as_array(r.tet_offsets, shape=tet_offsets.shape))
+        tet_offsets.copy_(_view(r.tet_offsets, tuple(tet_offsets.shape)))
         return r.num_tets, tets, opp, tet_offsets
 
     def take(self, r, tets, opp):
         """The result out of the context's memory, which its next call reuses."""
         nt = self.room(r.num_tets, tets)
-        np.copyto(tets[:nt], np.ctypeslib.as_array(r.tets, shape=(nt, 4)))
+        tets[:nt].copy_(_view(r.tets, (nt, 4)))
         if opp is not None:
-            np.copyto(opp[:nt], np.ctypeslib.as_array(r.opp, shape=(nt, 4)))
+            opp[:nt].copy_(_view(r.opp, (nt, 4)))
 
     def __del__(self):
         if self.ctx:
@@ -245,13 +249,12 @@ def prepare(case, seed):
     room = 7 * n + 1024
     if call in ("host", "batch"):
         xyz = xyz.cpu().numpy()
-        tets = np.full((room, 4), -1, np.int32)
-        opp = np.full((room, 4), -1, np.int32) if case["adjacency"] else None
-        last = np.zeros(n, np.int32) if call == "host" else np.zeros(case["sets"] + 1, np.int64)
+    where = dict(device="cuda") if call == "serve" else dict(pin_memory=True) if call == "device" else {}
+    tets = torch.empty((room, 4), dtype=torch.int32, **where).fill_(-1)
+    opp = torch.empty((room, 4), dtype=torch.int32, **where).fill_(-1) if case["adjacency"] else None
+    if call == "batch":
+        last = torch.zeros(case["sets"] + 1, dtype=torch.int64)
     else:
-        where = dict(device="cuda") if call == "serve" else dict(pin_memory=True)
-        tets = torch.empty((room, 4), dtype=torch.int32, **where).fill_(-1)
-        opp = torch.empty((room, 4), dtype=torch.int32, **where).fill_(-1) if case["adjacency"] else None
         last = torch.empty(n, dtype=torch.int32, **where).fill_(-1)
     return dict(call=getattr(_session(case), call), args=[xyz] + args + [tets, opp, last])
 
