@@ -360,13 +360,14 @@ static int setup_sets(g4d_ctx *ctx, const SetSpec &spec, int n, g4d::GridSets &G
     int64_t *h_pt = tab.data(), *h_vox = h_pt + (S + 1), *h_blk = h_vox + (S + 1), *h_spill = h_blk + (S + 1),
             *h_thr = h_spill + (S + 1);
     h_pt[0] = h_vox[0] = h_blk[0] = h_spill[0] = h_thr[0] = 0;
+    GS.pair_zc = g4d::grid_pair_chunk(spec.g.data(), S);
     for (int k = 0; k < S; k++) {
         const int64_t G = spec.g[k];
         h_pt[k + 1] = spec.pt_off[k + 1];
         h_vox[k + 1] = h_vox[k] + G * G * G;
         h_blk[k + 1] = h_blk[k] + g4d::pba_blocks((int)G);
         h_spill[k + 1] = h_spill[k] + g4d::pba_spill_ints((int)G);
-        h_thr[k + 1] = h_thr[k] + g4d::grid_pair_threads((int)G, g4d::grid_pair_chunk((int)G));
+        h_thr[k + 1] = h_thr[k] + g4d::grid_pair_threads((int)G, GS.pair_zc);
     }
     tot.voxels = h_vox[S];
     tot.pba_blocks = h_blk[S];
@@ -689,17 +690,17 @@ static int run_device(g4d_ctx *ctx, const double *d_xyz, int n, const SetSpec &s
     // ---- D: missing points, grid pairs, worksets, pumping (GD/GDelaunay/GDelHost.cu:259-529) ----
     // Pairs are extracted once per unordered pair (min<<32 | max), deduplicated, then
     // reciprocated into directed workset keys (star<<32 | vertex) and grouped by star.
-    // Raw pairs are counted per thread; each 256-thread tile then writes its pairs, deduplicated
-    // on chip, into its raw region at pr[ucap...], and the tiles are packed into pr[0...).
-    const int64_t nthr = tot.pair_threads, ntiles = nthr / 256;
-    HCK(ctx->pcount.ensure(sizeof(int64_t) * (size_t)(nthr + 1 + 2 * ntiles + 1)));
+    // Raw pairs are counted per 256-thread tile; each tile then writes its pairs, deduplicated on
+    // chip, into its raw region at pr[ucap...], and the tiles are packed into pr[0...).
+    const int64_t ntiles = tot.pair_threads / 256;
+    HCK(ctx->pcount.ensure(sizeof(int64_t) * (size_t)(3 * ntiles + 2)));
     int64_t *pcnt = buf<int64_t>(ctx->pcount);
-    int64_t *ttot = pcnt + nthr + 1;
+    int64_t *ttot = pcnt + ntiles + 1;
     uint2 *tcnt = reinterpret_cast<uint2 *>(ttot + ntiles + 1);
-    HCK(g4d::launch_grid_pairs(idg, GS, nthr, pcnt, nullptr, false, s));
-    HCK(g4d::scan_excl_i64(P, pcnt, pcnt, nthr, pcnt + nthr, s));
+    HCK(g4d::launch_grid_pair_count(idg, GS, ntiles, pcnt, s));
+    HCK(g4d::scan_excl_i64(P, pcnt, pcnt, ntiles, pcnt + ntiles, s));
     int64_t ngp_f = 0, *ngp_h = hslot(ctx, 0, &ngp_f);
-    HCK(hipMemcpyAsync(ngp_h, pcnt + nthr, 8, hipMemcpyDeviceToHost, s));
+    HCK(hipMemcpyAsync(ngp_h, pcnt + ntiles, 8, hipMemcpyDeviceToHost, s));
     HCK(hipStreamSynchronize(s));
     const int64_t ngp = *ngp_h;
     CK(guard_keys(ctx, 2 * (ngp + (int64_t)n), "grid pairs"));
@@ -707,8 +708,7 @@ static int run_device(g4d_ctx *ctx, const double *d_xyz, int n, const SetSpec &s
     const int64_t prop_room = ctx->prop_on ? 2 * (int64_t)g4d::PROP_SLOTS * n : 0;
     HCK(ctx->pairs.ensure(sizeof(uint64_t) * (size_t)(2 * ucap + prop_room + 2 * (int64_t)n * min_ws + 64)));
     uint64_t *pr = buf<uint64_t>(ctx->pairs);
-    HCK(g4d::launch_grid_pairs_dedup(idg, GS, nthr, pcnt, pr + ucap, tcnt, s));
-    HCK(g4d::launch_tile_totals(tcnt, ntiles, ttot, s));
+    HCK(g4d::launch_grid_pairs_dedup(idg, GS, ntiles, pcnt, pr + ucap, tcnt, ttot, s));
     HCK(g4d::scan_excl_i64(P, ttot, ttot, ntiles, ttot + ntiles, s));
     HCK(g4d::launch_gather_tiles(pr + ucap, pcnt, tcnt, ntiles, ttot, pr, s));
     HCK(hipMemsetAsync(cnt + G4D_CNT_APPEND0, 0, 8, s));
@@ -2092,17 +2092,22 @@ int g4d_diag_grid_pairs(g4d_ctx *ctx, const int32_t *id_grid, int32_t grid, uint
     g4d::GridSets GS;
     SetTotals tot;
     CK(setup_sets(ctx, single_set(1, grid), 1, GS, tot));
-    const int64_t nthr = tot.pair_threads;
-    HCK(ctx->pcount.ensure(sizeof(int64_t) * (size_t)(nthr + 1)));
-    int64_t *pcnt = buf<int64_t>(ctx->pcount);
-    HCK(g4d::launch_grid_pairs(buf<int>(ctx->gtmp), GS, nthr, pcnt, nullptr, false, s));
-    HCK(g4d::scan_excl_i64(ctx->P, pcnt, pcnt, nthr, pcnt + nthr, s));
-    int64_t m = 0;
-    HCK(hipMemcpyAsync(&m, pcnt + nthr, 8, hipMemcpyDeviceToHost, s));
+    const int64_t ntiles = tot.pair_threads / 256;
+    HCK(ctx->pcount.ensure(sizeof(int64_t) * (size_t)(3 * ntiles + 2)));
+    int64_t *pcnt = buf<int64_t>(ctx->pcount), *ttot = pcnt + ntiles + 1;
+    uint2 *tcnt = reinterpret_cast<uint2 *>(ttot + ntiles + 1);
+    HCK(g4d::launch_grid_pair_count(buf<int>(ctx->gtmp), GS, ntiles, pcnt, s));
+    HCK(g4d::scan_excl_i64(ctx->P, pcnt, pcnt, ntiles, pcnt + ntiles, s));
+    int64_t raw = 0, m = 0;
+    HCK(hipMemcpyAsync(&raw, pcnt + ntiles, 8, hipMemcpyDeviceToHost, s));
     HCK(hipStreamSynchronize(s));
-    HCK(ctx->pairs.ensure(sizeof(uint64_t) * (size_t)std::max<int64_t>(m, 1)));
+    HCK(ctx->pairs.ensure(sizeof(uint64_t) * (size_t)std::max<int64_t>(2 * raw, 1)));
     uint64_t *pr = buf<uint64_t>(ctx->pairs);
-    HCK(g4d::launch_grid_pairs(buf<int>(ctx->gtmp), GS, nthr, pcnt, pr, true, s));
+    HCK(g4d::launch_grid_pairs_dedup(buf<int>(ctx->gtmp), GS, ntiles, pcnt, pr + raw, tcnt, ttot, s));
+    HCK(g4d::scan_excl_i64(ctx->P, ttot, ttot, ntiles, ttot + ntiles, s));
+    HCK(g4d::launch_gather_tiles(pr + raw, pcnt, tcnt, ntiles, ttot, pr, s));
+    HCK(hipMemcpyAsync(&m, ttot + ntiles, 8, hipMemcpyDeviceToHost, s));
+    HCK(hipStreamSynchronize(s));
     int maxid = 0;
     for (int64_t i = 0; i < G3; i++) maxid = std::max(maxid, id_grid[i]);
     const int nb = bits_for((int64_t)maxid + 1);

@@ -19,6 +19,7 @@ struct GridSets {
     const int64_t *pba_blk; // nsets + 1: PBA work-groups
     const int64_t *spill;   // nsets + 1: PBA spill ints
     const int64_t *pair_thr;// nsets + 1: grid-pair threads
+    int pair_zc;            // cubes along z of a grid-pair tile
     int key_shift;          // one set: Morton keys are code << key_shift | index
 };
 // Batched Morton keys: set (16 bits) | code (24 bits, G <= 256) | index within the set (24 bits).
@@ -63,18 +64,17 @@ hipError_t pba_pass_banded(int axis, const GridSets &S, int64_t nblocks, int ban
 // Ordered pairs (min<<32 | max) of each non-leader point with its voxel's leader.
 hipError_t launch_missing(const uint64_t *vox, int n, const GridSets &S, const int *grid, uint64_t *out,
                           unsigned long long *counter, int64_t cap, hipStream_t s);
-// Voronoi-neighbour pairs (min<<32 | max): pass write=false fills count[thread], the caller
-// scans it to offsets (in place), pass write=true writes the pairs.  nthreads = pair_thr[nsets].
-int grid_pair_chunk(int g);
+// Voronoi-neighbour pairs (min<<32 | max) by tiles of 256 threads, 16 x 16 columns by
+// grid_pair_chunk cubes (for the sets' grids g together); pair_thr[nsets] / 256 tiles in all.
+int grid_pair_chunk(const int *g, int nsets);
 int64_t grid_pair_threads(int g, int zc);
-hipError_t launch_grid_pairs(const int *grid, const GridSets &S, int64_t nthreads, int64_t *count, uint64_t *out,
-                             bool write, hipStream_t s);
-// Pass 1 with each 256-thread tile's pairs deduplicated on chip: tile b writes into its raw
-// region [off[256 b], off[256 (b + 1)]) and reports (distinct, overflow) counts in cnt[b];
-// launch_tile_totals + an exclusive scan give the dense offsets for launch_gather_tiles.
-hipError_t launch_grid_pairs_dedup(const int *grid, const GridSets &S, int64_t nthreads, const int64_t *off,
-                                   uint64_t *out, uint2 *cnt, hipStream_t s);
-hipError_t launch_tile_totals(const uint2 *cnt, int64_t ntiles, int64_t *tot, hipStream_t s);
+// Raw pairs of each tile; scanned in place (with the total behind) they are the tiles' regions.
+hipError_t launch_grid_pair_count(const int *grid, const GridSets &S, int64_t ntiles, int64_t *count, hipStream_t s);
+// Every tile's pairs, deduplicated on chip: tile b writes into its raw region [off[b], off[b + 1])
+// and reports (distinct, overflow) counts in cnt[b] and their sum in tot[b], whose exclusive scan
+// gives the dense offsets for launch_gather_tiles.
+hipError_t launch_grid_pairs_dedup(const int *grid, const GridSets &S, int64_t ntiles, const int64_t *off,
+                                   uint64_t *out, uint2 *cnt, int64_t *tot, hipStream_t s);
 hipError_t launch_gather_tiles(const uint64_t *src, const int64_t *off, const uint2 *cnt, int64_t ntiles,
                                const int64_t *doff, uint64_t *dst, hipStream_t s);
 hipError_t launch_csr_offsets(const uint64_t *keys, int64_t m, int n, int64_t *off, hipStream_t s);

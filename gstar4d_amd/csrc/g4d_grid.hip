@@ -849,40 +849,57 @@ __device__ __forceinline__ int grid_at(const int *grid, int g, int x, int y, int
 }
 
 // Voronoi-neighbour pairs of one 2x2x2 cube (GD/GDelaunay/GDelKernels.cu:181-290): corner
-// c = ix + 2 iy + 4 iz, root = corner 0, opp = corner 7, link cycle 6,2,3,1,5,4.  Slot
-// 5i+{0..4} holds the pairs of link edge i (root-a, opp-a, root-b, opp-b, a-b); slot 30 is
-// root-opp.  Returns the bit mask of emitted slots.
-__device__ __forceinline__ uint32_t cube_pairs(const int *v, uint64_t *pr)
+// c = ix + 2 iy + 4 iz, root = corner 0, opp = corner 7, link cycle 6,2,3,1,5,4.  A link edge is
+// active when its two corners, root and opp are four different sites; it gives the pairs of root
+// and of opp with both corners (grabPair skips a Marker first value, :155-176) and the corners'
+// own, and any active edge gives root-opp (unless one is the Marker).  Neighbouring active edges
+// share a corner, whose pairs are emitted once.
+static constexpr int GP_LINK[6] = {6, 2, 3, 1, 5, 4};
+static constexpr int GP_SLOTS = 19; // 6 root-corner, 6 opp-corner, 6 corner-corner, root-opp
+
+// Bit i: link edge (i, i + 1 mod 6) is active.
+__device__ __forceinline__ uint32_t cube_edges(const int *v)
 {
     const int root = v[0], opp = v[7];
-    if (root == opp) return 0u;
-    const bool has_marker = (root == G4D_MARKER) || (opp == G4D_MARKER);
-    const int link[7] = {v[6], v[2], v[3], v[1], v[5], v[4], v[6]};
-    uint32_t mask = 0;
+    bool ok[6];
+#pragma unroll
+    for (int i = 0; i < 6; i++) ok[i] = v[GP_LINK[i]] != root && v[GP_LINK[i]] != opp;
+    uint32_t e = 0;
+#pragma unroll
+    for (int i = 0; i < 6; i++)
+        if (ok[i] && ok[(i + 1) % 6] && v[GP_LINK[i]] != v[GP_LINK[(i + 1) % 6]]) e |= 1u << i;
+    return root == opp ? 0u : e;
+}
+
+// Corners of the active edges.
+__device__ __forceinline__ uint32_t cube_corners(uint32_t e) { return (e | (e << 1) | (e >> 5)) & 63u; }
+
+__device__ __forceinline__ int cube_pair_count(const int *v, uint32_t e)
+{
+    const int r = v[0] != G4D_MARKER, o = v[7] != G4D_MARKER;
+    return (r + o) * __popc(cube_corners(e)) + __popc(e) + (e != 0 && r && o ? 1 : 0);
+}
+
+// The pairs of the active edges e; returns the bit mask of the emitted slots.
+__device__ __forceinline__ uint32_t cube_pairs(const int *v, uint32_t e, uint64_t *pr)
+{
+    const int root = v[0], opp = v[7];
+    const uint32_t c = cube_corners(e);
+    uint32_t mask = (root != G4D_MARKER ? c : 0u) | (opp != G4D_MARKER ? c << 6 : 0u) | (e << 12);
+    if (e && root != G4D_MARKER && opp != G4D_MARKER) mask |= 1u << 18;
 #pragma unroll
     for (int i = 0; i < 6; i++) {
-        const int a = link[i], b = link[i + 1];
-        if (a != b && a != root && a != opp && b != root && b != opp) {
-            // grabPair skips a pair whose first value is the Marker (:155-176)
-            if (root != G4D_MARKER) { mask |= 1u << (5 * i + 0); pr[5 * i + 0] = upair(root, a); }
-            if (opp != G4D_MARKER) { mask |= 1u << (5 * i + 1); pr[5 * i + 1] = upair(opp, a); }
-            if (root != G4D_MARKER) { mask |= 1u << (5 * i + 2); pr[5 * i + 2] = upair(root, b); }
-            if (opp != G4D_MARKER) { mask |= 1u << (5 * i + 3); pr[5 * i + 3] = upair(opp, b); }
-            mask |= 1u << (5 * i + 4);
-            pr[5 * i + 4] = upair(a, b);
-        }
+        const int a = v[GP_LINK[i]];
+        pr[i] = upair(root, a);
+        pr[6 + i] = upair(opp, a);
+        pr[12 + i] = upair(a, v[GP_LINK[(i + 1) % 6]]);
     }
-    if (mask && !has_marker) {
-        mask |= 1u << 30;
-        pr[30] = upair(root, opp);
-    }
+    pr[18] = upair(root, opp);
     return mask;
 }
 
-__host__ __device__ inline int grid_pair_chunk_dev(int g) { return g > 512 ? 32 : 16; }
-
 // Threads are laid out in tiles of GP_TILE x GP_TILE (x, y) columns of cubes (x, y from -1,
-// the outer Marker layer) and a chunk of zc cubes along z; a set's thread count is a whole
+// the outer Marker layer) and a chunk of zc = S.pair_zc cubes along z; a set's thread count is a whole
 // number of tiles, so a 256-thread work-group never spans two sets.
 static constexpr int GP_TILE = 16;
 static constexpr int GP_THREADS = GP_TILE * GP_TILE;
@@ -901,61 +918,60 @@ __device__ __forceinline__ bool gp_coords(int64_t lt, int g, int zc, int *x, int
     return *x < g && *y < g;
 }
 
-// Pass 0 counts each thread's raw pairs, pass 1 writes them at the scanned offset
-// (deterministic order, no atomics).
-template <bool WRITE>
-__global__ void __launch_bounds__(256) k_grid_pairs(const int *grid_all, GridSets S, int64_t nthr, int64_t *count,
-                                                    uint64_t *out)
+// Raw pairs of each tile (one 256-thread work-group a tile).
+__global__ void __launch_bounds__(GP_THREADS) k_grid_pair_count(const int *grid_all, GridSets S, int64_t *count)
 {
-    for (int64_t tid = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; tid < nthr; tid += (int64_t)gridDim.x * blockDim.x) {
-        const int st = S.nsets == 1 ? 0 : set_of_work(S.pair_thr, S.nsets, tid);
-        const int64_t lt = tid - S.pair_thr[st];
-        const int g = S.g[st];
-        const int *grid = grid_all + S.vox_off[st];
-        int x, y, z0, z1;
-        if (!gp_coords(lt, g, grid_pair_chunk_dev(g), &x, &y, &z0, &z1)) {
-            if (!WRITE) count[tid] = 0;
-            continue;
-        }
+    __shared__ int wsum[GP_THREADS / 64];
+    const int64_t tid = (int64_t)blockIdx.x * GP_THREADS + threadIdx.x;
+    const int st = S.nsets == 1 ? 0 : set_of_work(S.pair_thr, S.nsets, tid);
+    const int g = S.g[st];
+    const int *grid = grid_all + S.vox_off[st];
+    int x, y, z0, z1, k = 0;
+    if (gp_coords(tid - S.pair_thr[st], g, S.pair_zc, &x, &y, &z0, &z1)) {
         int v[8];
         v[0] = grid_at(grid, g, x, y, z0);
         v[1] = grid_at(grid, g, x + 1, y, z0);
         v[2] = grid_at(grid, g, x, y + 1, z0);
         v[3] = grid_at(grid, g, x + 1, y + 1, z0);
-        int64_t k = WRITE ? count[tid] : 0;
-        uint64_t pr[31];
         for (int z = z0; z < z1; z++) {
             v[4] = grid_at(grid, g, x, y, z + 1);
             v[5] = grid_at(grid, g, x + 1, y, z + 1);
             v[6] = grid_at(grid, g, x, y + 1, z + 1);
             v[7] = grid_at(grid, g, x + 1, y + 1, z + 1);
-            const uint32_t mask = cube_pairs(v, pr);
-            if (WRITE) {
-#pragma unroll
-                for (int j = 0; j < 31; j++)
-                    if (mask & (1u << j)) out[k++] = pr[j];
-            } else {
-                k += __popc(mask);
-            }
+            k += cube_pair_count(v, cube_edges(v));
             v[0] = v[4];
             v[1] = v[5];
             v[2] = v[6];
             v[3] = v[7];
         }
-        if (!WRITE) count[tid] = k;
+    }
+    const int inc = g4d_wave_incl_sum(k);
+    if ((threadIdx.x & 63) == 63) wsum[threadIdx.x >> 6] = inc;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        int64_t t = 0;
+        for (int w = 0; w < GP_THREADS / 64; w++) t += wsum[w];
+        count[blockIdx.x] = t;
     }
 }
 
-// Pass 1 with the work-group's pairs deduplicated in an LDS hash set: one work-group per tile,
-// whose raw pairs have the region [off[first thread], off[first thread of the next tile]) of
-// `out`.  Distinct pairs go to the bottom of the region in table order; a pair that finds no
-// free slot within GP_PROBES probes is written as is from the top of the region down.  Either
-// way the region holds at most the tile's raw count.  cnt[tile] = (table count, overflow count).
+// Each tile's pairs, deduplicated in an LDS hash set: one work-group per tile, whose raw pairs
+// have the region [off[tile], off[tile + 1]) of `out`.  Distinct pairs go to the bottom of the
+// region in table order; a pair that finds no free slot is written as is from the top of the
+// region down.  Either way the region holds at most the tile's raw count.  cnt[tile] = (table
+// count, overflow count), tot[tile] their sum.
 // Adjacent columns see the same Voronoi faces, so a 16 x 16 x zc tile keeps roughly one pair in
 // four; the global sort and unique that follow remove what remains duplicated across tiles.
+//
+// Bound by vector instructions (pair construction), not by the 4 bytes a voxel: with every cube
+// of the walk constructing its pairs 4,194,304 uniform points at G = 512 took 2.40 ms, with only
+// the queued ones 1.45 ms; 64 sets of 1,000-200,000 points 4.28 -> 1.12 ms, 4,000,000 clustered
+// points 5.75 -> 1.52 ms.  The sizes below keep four work-groups on a CU (40 KB of LDS each; a
+// stage of 512 pairs leaves three, 1.64 ms; 2,048 slots send more pairs to the sort, same total).
+static constexpr int GP_WAYS = 4; // slots of a bucket, read together
 static constexpr int GP_HASH = 4096;
-static constexpr int GP_PROBES = 32;
-static constexpr int GP_STAGE = 256;
+static constexpr int GP_STAGE = 192;
+static constexpr int GP_QUEUE = 128;
 static constexpr uint64_t GP_EMPTY = ~0ull;
 
 __device__ __forceinline__ void gp_wave_sync()
@@ -965,27 +981,39 @@ __device__ __forceinline__ void gp_wave_sync()
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// Inserts a pair into the tile's hash set (a plain read settles a repeat without an atomic);
-// a pair that finds no free slot within GP_PROBES probes goes straight to the top of the region.
+// Inserts a pair into the tile's hash set: its bucket, then the next one; the bucket's slots are
+// read together and a plain read settles a repeat without an atomic.  A pair that finds both
+// buckets full goes straight to the top of the region.  Two reads bound the cost where a tile has
+// more distinct pairs than slots (one point per voxel, as in the middle of a Gaussian): single
+// slots with 32 probes took 1.49 ms for such a set of 16,384 points (G = 64), this takes 0.08 ms.
 __device__ __forceinline__ void gp_insert(unsigned long long *tab, uint64_t key, uint64_t *out, int64_t rend,
                                           unsigned int *nover)
 {
-    uint32_t h = (uint32_t)((key * 0x9E3779B97F4A7C15ull) >> 52);
+    uint32_t h = (uint32_t)((key * 0x9E3779B97F4A7C15ull) >> 52) & ~(uint32_t)(GP_WAYS - 1);
     bool done = false;
-    for (int p = 0; p < GP_PROBES && !done; p++) {
-        unsigned long long cur = ((volatile unsigned long long *)tab)[h];
-        if (cur == GP_EMPTY) cur = atomicCAS(&tab[h], GP_EMPTY, (unsigned long long)key);
-        done = cur == GP_EMPTY || cur == key;
-        h = (h + 1) & (GP_HASH - 1);
+    for (int p = 0; p < 2 && !done; p++) {
+        unsigned long long cur[GP_WAYS];
+#pragma unroll
+        for (int i = 0; i < GP_WAYS; i++) cur[i] = ((volatile unsigned long long *)tab)[h + i];
+#pragma unroll
+        for (int i = 0; i < GP_WAYS; i++) done = done || cur[i] == key;
+#pragma unroll
+        for (int i = 0; i < GP_WAYS; i++)
+            if (!done && cur[i] == GP_EMPTY) {
+                const unsigned long long was = atomicCAS(&tab[h + i], GP_EMPTY, (unsigned long long)key);
+                done = was == GP_EMPTY || was == key;
+            }
+        h = (h + GP_WAYS) & (GP_HASH - 1);
     }
     if (!done) out[rend - 1 - atomicAdd(nover, 1u)] = key;
 }
 
 __global__ void __launch_bounds__(GP_THREADS) k_grid_pairs_dedup(const int *grid_all, GridSets S, const int64_t *off,
-                                                                 uint64_t *out, uint2 *cnt)
+                                                                 uint64_t *out, uint2 *cnt, int64_t *tot)
 {
     __shared__ unsigned long long tab[GP_HASH];
     __shared__ unsigned long long stage[GP_THREADS / 64][GP_STAGE];
+    __shared__ uint16_t queue[GP_THREADS / 64][GP_QUEUE];
     __shared__ unsigned int nover;
     __shared__ unsigned int wsum[GP_THREADS / 64];
     for (int i = threadIdx.x; i < GP_HASH; i += GP_THREADS) tab[i] = GP_EMPTY;
@@ -996,50 +1024,73 @@ __global__ void __launch_bounds__(GP_THREADS) k_grid_pairs_dedup(const int *grid
     const int64_t lt = tid - S.pair_thr[st];
     const int g = S.g[st];
     const int *grid = grid_all + S.vox_off[st];
-    const int64_t rbeg = off[(int64_t)blockIdx.x * GP_THREADS];
-    const int64_t rend = off[(int64_t)(blockIdx.x + 1) * GP_THREADS];
+    const int64_t rbeg = off[blockIdx.x], rend = off[blockIdx.x + 1];
     // Every lane walks its column (a lane outside the grid sees only Marker cubes, which emit
-    // nothing), so the wave steps through its cubes in lockstep: a step's pairs are first
-    // packed into the wave's LDS stage (exclusive scan of the lanes' counts) and then inserted
-    // by all 64 lanes together, instead of one pass per pair slot that any lane uses.  A step
-    // with more pairs than the stage holds inserts slot by slot.
+    // nothing), so the wave steps through its cubes in lockstep.  Most cubes lie inside one cell
+    // or on a face between two and emit nothing, so the walk only queues the cubes that do, and
+    // the wave takes them 64 at a time (the corners read again, from cache): their pairs are
+    // packed into the wave's LDS stage, a stage's worth at a time, and inserted by all 64 lanes.
     int x, y, z0, z1;
-    (void)gp_coords(lt, g, grid_pair_chunk_dev(g), &x, &y, &z0, &z1);
+    (void)gp_coords(lt, g, S.pair_zc, &x, &y, &z0, &z1);
     const int lane = __lane_id(), wid = threadIdx.x >> 6;
+    const int xt = x - (int)threadIdx.x % GP_TILE, yt = y - (int)threadIdx.x / GP_TILE;
     unsigned long long *stg = stage[wid];
-    int v[8];
+    uint16_t *que = queue[wid];
+    auto take = [&](int from, int n) { // queued cubes [from, from + n), n <= 64
+        int w[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+        uint32_t e = 0;
+        if (lane < n) {
+            const int q = que[from + lane], t = wid * 64 + (q & 63);
+            const int cx = xt + t % GP_TILE, cy = yt + t / GP_TILE, cz = z0 + (q >> 6);
+#pragma unroll
+            for (int i = 0; i < 8; i++) w[i] = grid_at(grid, g, cx + (i & 1), cy + ((i >> 1) & 1), cz + (i >> 2));
+            e = cube_edges(w);
+        }
+        uint64_t pr[GP_SLOTS];
+        const uint32_t mask = cube_pairs(w, e, pr);
+        const uint32_t c = (uint32_t)__popc(mask);
+        const uint32_t inc = (uint32_t)g4d_wave_incl_sum((int)c);
+        const uint32_t all = (uint32_t)__builtin_amdgcn_readlane((int)inc, 63);
+        for (uint32_t w0 = 0; w0 < all; w0 += GP_STAGE) {
+            uint32_t pos = inc - c - w0; // lanes and slots before the window wrap beyond it
+#pragma unroll
+            for (int j = 0; j < GP_SLOTS; j++)
+                if (mask & (1u << j)) {
+                    if (pos < GP_STAGE) stg[pos] = pr[j];
+                    pos++;
+                }
+            gp_wave_sync();
+            const uint32_t nw = min(all - w0, (uint32_t)GP_STAGE);
+            for (uint32_t k = lane; k < nw; k += 64) gp_insert(tab, stg[k], out, rend, &nover);
+            gp_wave_sync();
+        }
+    };
+    int v[8], nq = 0;
     v[0] = grid_at(grid, g, x, y, z0);
     v[1] = grid_at(grid, g, x + 1, y, z0);
     v[2] = grid_at(grid, g, x, y + 1, z0);
     v[3] = grid_at(grid, g, x + 1, y + 1, z0);
-    uint64_t pr[31];
     for (int z = z0; z < z1; z++) {
         v[4] = grid_at(grid, g, x, y, z + 1);
         v[5] = grid_at(grid, g, x + 1, y, z + 1);
         v[6] = grid_at(grid, g, x, y + 1, z + 1);
         v[7] = grid_at(grid, g, x + 1, y + 1, z + 1);
-        const uint32_t mask = cube_pairs(v, pr);
-        const uint32_t c = (uint32_t)__popc(mask);
-        const uint32_t inc = (uint32_t)g4d_wave_incl_sum((int)c);
-        const uint32_t tot = (uint32_t)__builtin_amdgcn_readlane((int)inc, 63);
-        if (tot <= GP_STAGE) {
-            uint32_t pos = inc - c;
-#pragma unroll
-            for (int j = 0; j < 31; j++)
-                if (mask & (1u << j)) stg[pos++] = pr[j];
-            gp_wave_sync();
-            for (uint32_t k = lane; k < tot; k += 64) gp_insert(tab, stg[k], out, rend, &nover);
-            gp_wave_sync();
-        } else {
-#pragma unroll
-            for (int j = 0; j < 31; j++)
-                if (mask & (1u << j)) gp_insert(tab, pr[j], out, rend, &nover);
+        const bool act = cube_edges(v) != 0;
+        int tot;
+        const int at = nq + g4d_wave_excl_count(act, &tot);
+        if (act) que[at] = (uint16_t)(((z - z0) << 6) | lane);
+        nq += tot;
+        gp_wave_sync();
+        if (nq >= 64) {
+            nq -= 64;
+            take(nq, 64);
         }
         v[0] = v[4];
         v[1] = v[5];
         v[2] = v[6];
         v[3] = v[7];
     }
+    take(0, nq);
     __syncthreads();
     // compact the table: GP_HASH / GP_THREADS slots per thread, block-wide exclusive scan
     constexpr int PER = GP_HASH / GP_THREADS;
@@ -1063,7 +1114,10 @@ __global__ void __launch_bounds__(GP_THREADS) k_grid_pairs_dedup(const int *grid
 #pragma unroll
     for (int i = 0; i < PER; i++)
         if (e[i] != GP_EMPTY) *dst++ = e[i];
-    if (threadIdx.x == 0) cnt[blockIdx.x] = make_uint2(total, nover);
+    if (threadIdx.x == 0) {
+        cnt[blockIdx.x] = make_uint2(total, nover);
+        tot[blockIdx.x] = (int64_t)total + nover;
+    }
 }
 
 // Packs every tile's table pairs and overflow pairs densely: tile b's pairs go to
@@ -1072,17 +1126,11 @@ __global__ void __launch_bounds__(256) k_gather_tiles(const uint64_t *src, const
                                                       const int64_t *doff, uint64_t *dst)
 {
     const int64_t b = blockIdx.x;
-    const int64_t rbeg = off[b * GP_THREADS], rend = off[(b + 1) * GP_THREADS];
+    const int64_t rbeg = off[b], rend = off[b + 1];
     const uint2 c = cnt[b];
     uint64_t *d = dst + doff[b];
     for (uint32_t i = threadIdx.x; i < c.x; i += blockDim.x) d[i] = src[rbeg + i];
     for (uint32_t i = threadIdx.x; i < c.y; i += blockDim.x) d[c.x + i] = src[rend - c.y + i];
-}
-
-__global__ void k_tile_totals(const uint2 *cnt, int64_t nb, int64_t *tot)
-{
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < nb; i += (int64_t)gridDim.x * blockDim.x)
-        tot[i] = (int64_t)cnt[i].x + cnt[i].y;
 }
 
 // CSR offsets of sorted directed keys: off[s] = first index with star >= s (off has n+1).
@@ -1215,7 +1263,18 @@ hipError_t launch_missing(const uint64_t *vox, int n, const GridSets &S, const i
     return hipGetLastError();
 }
 
-int grid_pair_chunk(int g) { return grid_pair_chunk_dev(g); }
+int grid_pair_chunk(const int *g, int nsets)
+{
+    // 16 cubes a tile (32 above G = 512) unless that leaves most of the chip without a tile; a
+    // quarter of the depth then gives four times the tiles, each with a quarter of the serial walk.
+    int zc = 16;
+    int64_t tiles = 0;
+    for (int k = 0; k < nsets; k++) {
+        if (g[k] > 512) zc = 32;
+        tiles += grid_pair_threads(g[k], 16) / GP_THREADS;
+    }
+    return tiles < 512 ? 4 : zc;
+}
 
 int64_t grid_pair_threads(int g, int zc)
 {
@@ -1223,19 +1282,20 @@ int64_t grid_pair_threads(int g, int zc)
     return ntx * ntx * ((w + zc - 1) / zc) * GP_THREADS;
 }
 
-hipError_t launch_grid_pairs_dedup(const int *grid, const GridSets &S, int64_t nthr, const int64_t *off, uint64_t *out,
-                                   uint2 *cnt, hipStream_t s)
+hipError_t launch_grid_pair_count(const int *grid, const GridSets &S, int64_t ntiles, int64_t *count, hipStream_t s)
 {
-    if (nthr <= 0) return hipSuccess;
-    if (nthr % GP_THREADS || nthr / GP_THREADS > INT32_MAX) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(k_grid_pairs_dedup, dim3((unsigned)(nthr / GP_THREADS)), dim3(GP_THREADS), 0, s, grid, S, off, out,
-                       cnt);
+    if (ntiles <= 0) return hipSuccess;
+    if (ntiles > INT32_MAX) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(k_grid_pair_count, dim3((unsigned)ntiles), dim3(GP_THREADS), 0, s, grid, S, count);
     return hipGetLastError();
 }
 
-hipError_t launch_tile_totals(const uint2 *cnt, int64_t ntiles, int64_t *tot, hipStream_t s)
+hipError_t launch_grid_pairs_dedup(const int *grid, const GridSets &S, int64_t ntiles, const int64_t *off,
+                                   uint64_t *out, uint2 *cnt, int64_t *tot, hipStream_t s)
 {
-    hipLaunchKernelGGL(k_tile_totals, dim3(g4d_blocks(ntiles, 256, 65536)), dim3(256), 0, s, cnt, ntiles, tot);
+    if (ntiles <= 0) return hipSuccess;
+    if (ntiles > INT32_MAX) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(k_grid_pairs_dedup, dim3((unsigned)ntiles), dim3(GP_THREADS), 0, s, grid, S, off, out, cnt, tot);
     return hipGetLastError();
 }
 
@@ -1245,19 +1305,6 @@ hipError_t launch_gather_tiles(const uint64_t *src, const int64_t *off, const ui
     if (ntiles <= 0) return hipSuccess;
     if (ntiles > INT32_MAX) return hipErrorInvalidValue;
     hipLaunchKernelGGL(k_gather_tiles, dim3((unsigned)ntiles), dim3(256), 0, s, src, off, cnt, doff, dst);
-    return hipGetLastError();
-}
-
-hipError_t launch_grid_pairs(const int *grid, const GridSets &S, int64_t nthr, int64_t *count, uint64_t *out,
-                             bool write, hipStream_t s)
-{
-    if (nthr <= 0) return hipSuccess;
-    if (write)
-        hipLaunchKernelGGL(k_grid_pairs<true>, dim3(g4d_blocks(nthr, 256, 65536)), dim3(256), 0, s, grid, S, nthr, count,
-                           out);
-    else
-        hipLaunchKernelGGL(k_grid_pairs<false>, dim3(g4d_blocks(nthr, 256, 65536)), dim3(256), 0, s, grid, S, nthr, count,
-                           out);
     return hipGetLastError();
 }
 

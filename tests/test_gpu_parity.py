@@ -128,6 +128,15 @@ def test_morton_matches_oracle(tri, orc, g_, n):
     assert (pg == po).all() and (vg == vo).all()
 
 
+@pytest.mark.parametrize("g_,cells", [(4, 64), (15, 2), (33, 33 ** 3), (64, 5000), (160, 160 ** 3)])
+def test_grid_pairs_of_crowded_tiles(tri, orc, g_, cells):
+    """Id grids from two sites to one site a voxel: a tile then has more distinct pairs than its
+    hash set holds.  64 wide and below take the shallow tiles, 160 the deep ones."""
+    ids = (np.random.default_rng(g_).permutation(g_ ** 3).astype(np.int32) % cells).reshape(g_, g_, g_)
+    got, want = tri.diag_grid_pairs(ids), orc.grid_pairs(ids)
+    assert got.shape == want.shape and (got == want).all()
+
+
 @pytest.mark.parametrize("g_,n", [(16, 40), (64, 3000), (96, 20000), (128, 8000)])
 @pytest.mark.parametrize("bands", [1, 2, 3, 4])
 def test_pba_matches_oracle(tri, orc, g_, n, bands):
