@@ -15,15 +15,13 @@ __global__ void k_diag_orient4(const double *pts5, const int *idx5, int64_t T, i
             idx[i] = idx5[5 * t + i];
         }
         int s = 0, d = 0;
-        if (mode == 0) {
-            s = filter_insphere(p);
+        if (mode == 0 || mode == 1) {
+            if (mode == 0) s = filter_insphere(p);
             if (s == 0) {
-                s = exact_insphere(p, cnt);
-                if (s == 0) s = sos_orient4(p, idx, &d, cnt);
+                const int r = orient4_exact(p[0], p[1], p[2], p[3], p[4], idx[0], idx[1], idx[2], idx[3], idx[4], cnt);
+                s = r > 0 ? 1 : -1;
+                d = (r > 0 ? r : -r) - 1;
             }
-        } else if (mode == 1) {
-            s = exact_insphere(p, cnt);
-            if (s == 0) s = sos_orient4(p, idx, &d, cnt);
         } else if (mode == 2) {
             // the star kernel's cached-cofactor filter for orient4(a, b, c, s, v)
             const double sx = p[3][0], sy = p[3][1], sz = p[3][2];

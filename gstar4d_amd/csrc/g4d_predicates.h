@@ -658,6 +658,401 @@ __device__ __noinline__ int sos_orient4(const double *const *pin, const int *idx
     return sign;
 }
 
+// ------------------------------------------------------------------------------------
+// orient4 without the filter, in FP64 registers.
+//
+// The functions above keep the points' integer form in private arrays indexed at run time, so
+// nearly every operand goes through scratch memory, and 64-bit integer products cost four
+// quarter-rate instructions and carry chains: one evaluation takes a wave about 40 us, and the
+// exact star kernels wait for one or more of them per insertion.  The same integers in base 2^21
+// with signed digits held in doubles multiply by plain fused multiply-adds (digit products stay
+// below 2^42, sums of them below 2^53, so every operation is exact) at four times the rate, and
+// carries wait until a factor has to be short again.
+//
+// The common scale is the power of two that takes the largest coordinate below 2^61; a coordinate
+// fits it when its scaled value is a whole number, which one rounding instruction tells.  Where
+// the coordinates span more bits, their differences to the last point, when FP64 forms them
+// without rounding, often do not, which settles the determinant.  What is left goes to the
+// functions above.  SoS ends within depth 13 for distinct points: minors of differences and of
+// one lift each.
+//
+// Bound by the latency of one wave's dependent FP64 operations (few lanes have work).  30,000
+// points, half of them on a sphere and a lattice (1.8 M evaluations, 1.5 M of them zero): the
+// exact star kernels 125 -> 32 ms, the exact proofs 9.1 -> 4.0 ms.
+// ------------------------------------------------------------------------------------
+
+namespace lb {
+
+constexpr double BASE = 2097152.0, INV = 1.0 / 2097152.0;
+constexpr double SNAP = 1.5 * 4503599627370496.0 * BASE; // adding it rounds to multiples of BASE
+
+// Whole X, |X| < 2^62, to three digits of at most 2^20 (the top one of 2^20).
+__device__ __forceinline__ void split(double X, double (&v)[3])
+{
+    const double h2 = __builtin_rint(X * (INV * INV));
+    const double r = fma(-h2, BASE * BASE, X);
+    const double h1 = __builtin_rint(r * INV);
+    v[0] = fma(-h1, BASE, r);
+    v[1] = h1;
+    v[2] = h2;
+}
+
+// Carries: v[0..N) to digits of at most 2^20, the last carry in v[N].
+template <int N>
+__device__ __forceinline__ void carry(double (&v)[N + 1])
+{
+    v[N] = 0.0;
+#pragma unroll
+    for (int i = 0; i < N; i++) {
+        const double c = (v[i] + SNAP) - SNAP; // the multiple of 2^21 nearest to v[i], |v[i]| < 2^51
+        v[i] -= c;
+        v[i + 1] = fma(c, INV, v[i + 1]);
+    }
+}
+
+// r += f a b, f = 1 or -1.
+template <int NA, int NB, int NR>
+__device__ __forceinline__ void mac(double (&r)[NR], const double (&a)[NA], const double (&b)[NB], double f)
+{
+    static_assert(NR >= NA + NB - 1, "digits of a product");
+#pragma unroll
+    for (int i = 0; i < NA; i++) {
+        const double x = f * a[i];
+#pragma unroll
+        for (int j = 0; j < NB; j++) r[i + j] = fma(x, b[j], r[i + j]);
+    }
+}
+
+template <int N>
+__device__ __forceinline__ void zero(double (&r)[N])
+{
+#pragma unroll
+    for (int i = 0; i < N; i++) r[i] = 0.0;
+}
+
+// Sign of a number of carried digits: that of its highest nonzero one (the digits below it come
+// to less than one unit of it).
+template <int N>
+__device__ __forceinline__ int lead(const double (&v)[N])
+{
+    double t = v[N - 1];
+#pragma unroll
+    for (int i = N - 2; i >= 0; i--) t = t == 0.0 ? v[i] : t;
+    return t > 0.0 ? 1 : (t < 0.0 ? -1 : 0);
+}
+
+// The same of N uncarried digits.
+template <int N>
+__device__ __forceinline__ int sign(double (&v)[N + 1])
+{
+    carry<N>(v);
+    return lead(v);
+}
+
+struct Pt {
+    double c[3][3]; // digits of x, y, z
+};
+
+__device__ __forceinline__ Pt sub(const Pt &a, const Pt &b)
+{
+    Pt r;
+#pragma unroll
+    for (int c = 0; c < 3; c++)
+#pragma unroll
+        for (int i = 0; i < 3; i++) r.c[c][i] = a.c[c][i] - b.c[c][i];
+    return r;
+}
+
+// m = a[C0] b[C1] - b[C0] a[C1], carried.
+template <int C0, int C1>
+__device__ __forceinline__ void minor2(const Pt &a, const Pt &b, double (&m)[6])
+{
+    zero(m);
+    mac(m, a.c[C0], b.c[C1], 1.0);
+    mac(m, b.c[C0], a.c[C1], -1.0);
+    carry<5>(m);
+}
+
+// det of rows a, b, c (differences), uncarried in r[0..8).
+__device__ __forceinline__ void det3(const Pt &a, const Pt &b, const Pt &c, double (&r)[9])
+{
+    double m[6];
+    zero(r);
+    minor2<0, 1>(b, c, m);
+    mac(r, a.c[2], m, 1.0);
+    minor2<0, 1>(c, a, m);
+    mac(r, b.c[2], m, 1.0);
+    minor2<0, 1>(a, b, m);
+    mac(r, c.c[2], m, 1.0);
+}
+
+// x^2 + y^2 + z^2, uncarried in r[0..5).
+__device__ __forceinline__ void lift(const Pt &a, double (&r)[6])
+{
+    zero(r);
+#pragma unroll
+    for (int c = 0; c < 3; c++) mac(r, a.c[c], a.c[c], 1.0);
+}
+
+// acc += f lift(own) det(a, b, c): one term of the lifted 4x4 determinant, 14 uncarried digits.
+__device__ __forceinline__ void lifted_term(const Pt &a, const Pt &b, const Pt &c, const Pt &own, double f,
+                                            double (&acc)[15])
+{
+    double m[9], l[6];
+    det3(a, b, c, m);
+    carry<8>(m);
+    lift(own, l);
+    carry<5>(l);
+    mac(acc, l, m, f);
+}
+
+// Sign of the SoS minor of columns C0, C1 and the lift over rows a, b, c translated by the last
+// row, their translated lifts in la, lb, lc (carried).
+template <int C0, int C1>
+__device__ __forceinline__ int minor_lift(const Pt &a, const Pt &b, const Pt &c, const double (&la)[6],
+                                          const double (&l2)[6], const double (&lc)[6])
+{
+    double r[12], m[6];
+    zero(r);
+    minor2<C0, C1>(b, c, m);
+    mac(r, la, m, 1.0);
+    minor2<C0, C1>(c, a, m);
+    mac(r, l2, m, 1.0);
+    minor2<C0, C1>(a, b, m);
+    mac(r, lc, m, 1.0);
+    return sign<11>(r);
+}
+
+// The same with two rows b, c and columns C0 and the lift.
+template <int C0>
+__device__ __forceinline__ int minor_lift2(const Pt &b, const Pt &c, const double (&l2)[6], const double (&lc)[6])
+{
+    double r[9];
+    zero(r);
+    mac(r, b.c[C0], lc, 1.0);
+    mac(r, c.c[C0], l2, -1.0);
+    return sign<8>(r);
+}
+
+} // namespace lb
+
+// Largest frexp exponent so far; zero has none.
+__device__ __forceinline__ int frexp_top(double x, int top)
+{
+    const int e = __builtin_amdgcn_frexp_exp(x);
+    return x == 0.0 ? top : max(top, e);
+}
+
+// x 2^sh into *X; whether that is a whole number.
+__device__ __forceinline__ bool scaled_whole(double x, int sh, double *X)
+{
+    *X = __builtin_ldexp(x, sh);
+    return __builtin_rint(*X) == *X;
+}
+
+// fl(a - b) into *w; whether nothing was rounded.
+__device__ __forceinline__ bool exact_diff(double a, double b, double *w)
+{
+    const double d = a - b, bv = a - d, av = d + bv;
+    *w = d;
+    return (a - av) + (bv - b) == 0.0;
+}
+
+struct ScaledPt {
+    double c[3]; // whole numbers on the common scale
+};
+
+__device__ __forceinline__ lb::Pt digits(const ScaledPt &p)
+{
+    lb::Pt r;
+#pragma unroll
+    for (int c = 0; c < 3; c++) lb::split(p.c[c], r.c[c]);
+    return r;
+}
+
+__device__ __forceinline__ void sos_order(int &ia, ScaledPt &a, int &ib, ScaledPt &b, int &parity)
+{
+    const bool sw = ib < ia;
+    const int ti = ia;
+    ia = sw ? ib : ia;
+    ib = sw ? ti : ib;
+#pragma unroll
+    for (int c = 0; c < 3; c++) {
+        const double t = a.c[c];
+        a.c[c] = sw ? b.c[c] : a.c[c];
+        b.c[c] = sw ? t : b.c[c];
+    }
+    parity ^= sw ? 1 : 0;
+}
+
+// SoS sign through depth 13 of five whole points with ids i0..i4; 0 when all thirteen minors
+// vanish.
+__device__ __forceinline__ int sos_whole(ScaledPt x0, ScaledPt x1, ScaledPt x2, ScaledPt x3, ScaledPt x4, int i0, int i1,
+                                         int i2, int i3, int i4, int *depth)
+{
+    int par = 0; // a sorting network; each exchange flips the parity
+    sos_order(i0, x0, i1, x1, par);
+    sos_order(i3, x3, i4, x4, par);
+    sos_order(i2, x2, i4, x4, par);
+    sos_order(i2, x2, i3, x3, par);
+    sos_order(i1, x1, i4, x4, par);
+    sos_order(i0, x0, i3, x3, par);
+    sos_order(i0, x0, i2, x2, par);
+    sos_order(i1, x1, i3, x3, par);
+    sos_order(i1, x1, i2, x2, par);
+    const lb::Pt q4 = digits(x4);
+    const lb::Pt a = lb::sub(digits(x1), q4), b = lb::sub(digits(x2), q4), c = lb::sub(digits(x3), q4);
+    double r[9], m[6];
+    lb::det3(a, b, c, r);
+    int d = 1, s = -lb::sign<8>(r);
+    if (s == 0) {
+        // the lifts, translated by the last row's
+        double l4[6], l0[6], la[6], l2[6], lc[6];
+        lb::lift(q4, l4);
+        lb::lift(digits(x0), l0);
+        lb::lift(digits(x1), la);
+        lb::lift(digits(x2), l2);
+        lb::lift(digits(x3), lc);
+#pragma unroll
+        for (int i = 0; i < 5; i++) {
+            l0[i] -= l4[i];
+            la[i] -= l4[i];
+            l2[i] -= l4[i];
+            lc[i] -= l4[i];
+        }
+        lb::carry<5>(l0);
+        lb::carry<5>(la);
+        lb::carry<5>(l2);
+        lb::carry<5>(lc);
+        const lb::Pt e = lb::sub(digits(x0), q4);
+        d = 2;
+        s = lb::minor_lift<0, 1>(a, b, c, la, l2, lc);
+        if (s == 0) {
+            d = 3;
+            s = -lb::minor_lift<0, 2>(a, b, c, la, l2, lc);
+        }
+        if (s == 0) {
+            d = 4;
+            s = lb::minor_lift<1, 2>(a, b, c, la, l2, lc);
+        }
+        if (s == 0) {
+            d = 5;
+            lb::det3(e, b, c, r);
+            s = lb::sign<8>(r);
+        }
+        if (s == 0) {
+            d = 6;
+            lb::minor2<0, 1>(b, c, m);
+            s = lb::lead(m);
+        }
+        if (s == 0) {
+            d = 7;
+            lb::minor2<0, 2>(b, c, m);
+            s = -lb::lead(m);
+        }
+        if (s == 0) {
+            d = 8;
+            lb::minor2<1, 2>(b, c, m);
+            s = lb::lead(m);
+        }
+        if (s == 0) {
+            d = 9;
+            s = -lb::minor_lift<0, 1>(e, b, c, l0, l2, lc);
+        }
+        if (s == 0) {
+            d = 10;
+            s = lb::minor_lift2<0>(b, c, l2, lc);
+        }
+        if (s == 0) {
+            d = 11;
+            s = -lb::minor_lift2<1>(b, c, l2, lc);
+        }
+        if (s == 0) {
+            d = 12;
+            s = lb::minor_lift<0, 2>(e, b, c, l0, l2, lc);
+        }
+        if (s == 0) {
+            d = 13;
+            s = lb::minor_lift2<2>(b, c, l2, lc);
+        }
+    }
+    *depth = d;
+    return par ? -s : s;
+}
+
+// The exact sign of orient4(p0..p4) with ids i0..i4, SoS included: sign * (1 + SoS depth), the
+// depth 0 where the determinant decides.  Arguments travel in registers.
+__device__ __noinline__ int orient4_exact(const double *p0, const double *p1, const double *p2, const double *p3,
+                                          const double *p4, int i0, int i1, int i2, int i3, int i4,
+                                          unsigned long long *cnt)
+{
+    const double x[5][3] = {{p0[0], p0[1], p0[2]}, {p1[0], p1[1], p1[2]}, {p2[0], p2[1], p2[2]},
+                            {p3[0], p3[1], p3[2]}, {p4[0], p4[1], p4[2]}};
+    int top = -2000, bot = 2000;
+#pragma unroll
+    for (int i = 0; i < 5; i++)
+#pragma unroll
+        for (int c = 0; c < 3; c++) {
+            top = frexp_top(x[i][c], top);
+            bot = x[i][c] == 0.0 ? bot : min(bot, __builtin_amdgcn_frexp_exp(x[i][c]));
+        }
+    bool whole = true;
+    ScaledPt X[5];
+#pragma unroll
+    for (int i = 0; i < 5; i++)
+#pragma unroll
+        for (int c = 0; c < 3; c++) whole = scaled_whole(x[i][c], 61 - top, &X[i].c[c]) && whole;
+    bool diffs = whole;
+    lb::Pt d[4];
+    if (whole) {
+        const lb::Pt q4 = digits(X[4]);
+#pragma unroll
+        for (int i = 0; i < 4; i++) d[i] = lb::sub(digits(X[i]), q4);
+    } else if (top - bot <= 72) { // within the range of the general path (125 bits), which reports the rest
+        double w[4][3];
+        int dtop = -2000;
+        diffs = true;
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+#pragma unroll
+            for (int c = 0; c < 3; c++) {
+                diffs = exact_diff(x[i][c], x[4][c], &w[i][c]) && diffs;
+                dtop = frexp_top(w[i][c], dtop);
+            }
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            ScaledPt W;
+#pragma unroll
+            for (int c = 0; c < 3; c++) diffs = scaled_whole(w[i][c], 61 - dtop, &W.c[c]) && diffs;
+            d[i] = digits(W);
+        }
+    }
+    int s = 0;
+    if (diffs) {
+        double acc[15];
+        lb::zero(acc);
+        lb::lifted_term(d[1], d[2], d[3], d[0], -1.0, acc);
+        lb::lifted_term(d[0], d[2], d[3], d[1], 1.0, acc);
+        lb::lifted_term(d[0], d[1], d[3], d[2], -1.0, acc);
+        lb::lifted_term(d[0], d[1], d[2], d[3], 1.0, acc);
+        s = lb::sign<14>(acc);
+    } else {
+        const double *p[5] = {p0, p1, p2, p3, p4};
+        s = exact_insphere(p, cnt);
+    }
+    if (s != 0) return s;
+    if (cnt) atomicAdd(&cnt[G4D_CNT_SOS], 1ull);
+    int depth = 0;
+    if (whole) {
+        s = sos_whole(X[0], X[1], X[2], X[3], X[4], i0, i1, i2, i3, i4, &depth);
+        if (s != 0) return s * (1 + depth);
+    }
+    const double *p[5] = {p0, p1, p2, p3, p4};
+    const int idx[5] = {i0, i1, i2, i3, i4};
+    s = sos_orient4(p, idx, &depth, cnt);
+    return s * (1 + depth);
+}
+
 // Filtered lifted determinant sign of (p0..p4) with the 4x4 form translated by p4.
 // Returns 0 when the forward-error bound cannot certify the sign.  Every monomial carries
 // at most 17 roundings (inputs 1+1+1+5 via the lift, minors 5, final sum 4), so the error
@@ -743,10 +1138,7 @@ __device__ __forceinline__ int orient4_full(const double *const *p, const int *i
     int s = filter_insphere(p);
     if (s != 0) return s;
     if (cnt) atomicAdd(&cnt[G4D_CNT_EXACT], 1ull);
-    s = exact_insphere(p, cnt);
-    if (s != 0) return s;
-    if (cnt) atomicAdd(&cnt[G4D_CNT_SOS], 1ull);
-    return sos_orient4(p, idx, nullptr, cnt);
+    return orient4_exact(p[0], p[1], p[2], p[3], p[4], idx[0], idx[1], idx[2], idx[3], idx[4], cnt) > 0 ? 1 : -1;
 }
 
 __device__ __forceinline__ int orient3d_full(const double *const *p, unsigned long long *cnt)

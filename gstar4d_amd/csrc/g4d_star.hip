@@ -369,7 +369,7 @@ __device__ __forceinline__ void star_body(const StarParams &p, int nitems)
                 const double r[4] = {L.vc[Vn][0], L.vc[Vn][1], L.vc[Vn][2], L.vc[Vn][3]};
                 int nv = 0;
                 unsigned vm = 0; // bit k: slot lane + 64 k sees the vertex
-                bool unc = false;
+                unsigned um = 0; // bit k: its filter is inconclusive
 #pragma unroll 1
                 for (int k = 0; k < KPL; k++) {
                     const int slot = lane + 64 * k;
@@ -380,19 +380,8 @@ __device__ __forceinline__ void star_body(const StarParams &p, int nitems)
                             double c[8];
 #pragma unroll
                             for (int j = 0; j < 8; j++) c[j] = L.cof[j][slot];
-                            int sg = cofactor_filter_sign(r, c, c + 4);
-                            if (sg == 0) {
-                                if (EXACT) {
-                                    const int a = L.vid[tvert(t, 0)], b = L.vid[tvert(t, 1)], c = L.vid[tvert(t, 2)];
-                                    const double *pp[5] = {p.pts + 3 * (int64_t)a, p.pts + 3 * (int64_t)b,
-                                                           p.pts + 3 * (int64_t)c, p.pts + 3 * (int64_t)s,
-                                                           p.pts + 3 * (int64_t)gv};
-                                    const int idx[5] = {a, b, c, s, gv};
-                                    sg = orient4_full(pp, idx, cnt);
-                                } else {
-                                    unc = true;
-                                }
-                            }
+                            const int sg = cofactor_filter_sign(r, c, c + 4);
+                            if (sg == 0) um |= 1u << k;
                             if (sg < 0) {
                                 L.tv[slot] = t | TF_VIS;
                                 vm |= 1u << k;
@@ -401,9 +390,38 @@ __device__ __forceinline__ void star_body(const StarParams &p, int nitems)
                         }
                     }
                 }
-                if (!EXACT && __ballot(unc)) {
-                    unsure = true;
-                    break;
+                if (__ballot(um != 0)) {
+                    if (!EXACT) {
+                        unsure = true;
+                        break;
+                    }
+                    // The inconclusive slots of the whole wave in one list (be_slot is free until the
+                    // new triangles), decided 64 at a time: slot by slot in their owners' lanes a
+                    // 256-vertex star paid up to eight exact evaluations per insertion, each with
+                    // a few lanes active.
+                    const int nu = __popc(um);
+                    const int uinc = g4d_wave_incl_sum(nu), nutot = __builtin_amdgcn_readlane(uinc, 63);
+                    int upos = uinc - nu;
+#pragma unroll 1
+                    for (int k = 0; k < KPL; k++)
+                        if ((um >> k) & 1) L.be_slot[upos++] = (uint16_t)(lane + 64 * k);
+                    wave_sync();
+                    for (int x = lane; x < nutot; x += 64) {
+                        const int slot = L.be_slot[x];
+                        const uint32_t t = L.tv[slot];
+                        const int a = L.vid[tvert(t, 0)], b = L.vid[tvert(t, 1)], c = L.vid[tvert(t, 2)];
+                        const double *pp[5] = {p.pts + 3 * (int64_t)a, p.pts + 3 * (int64_t)b, p.pts + 3 * (int64_t)c,
+                                               p.pts + 3 * (int64_t)s, p.pts + 3 * (int64_t)gv};
+                        const int idx[5] = {a, b, c, s, gv};
+                        if (orient4_full(pp, idx, cnt) < 0) L.tv[slot] = t | TF_VIS;
+                    }
+                    wave_sync();
+#pragma unroll 1
+                    for (int k = 0; k < KPL; k++)
+                        if (((um >> k) & 1) && (L.tv[lane + 64 * k] & TF_VIS)) {
+                            vm |= 1u << k;
+                            nv++;
+                        }
                 }
                 const int vinc = g4d_wave_incl_sum(nv);
                 const int vbase = vinc - nv, nvis = __builtin_amdgcn_readlane(vinc, 63);
@@ -1518,7 +1536,8 @@ __global__ void __launch_bounds__(GSTAR_NT) k_star_global(StarParams p, const in
                 ub = block_excl(nunc, &nunc_tot, red);
                 vbase = block_excl(nv, &nvis, red);
             }
-            if (nunc_tot > 0) {
+            // rare: the registers that the call takes are saved here and not around the loop
+            if (__builtin_expect(nunc_tot > 0, 0)) {
                 for (int slot = tid; slot < T && nunc > 0; slot += GSTAR_NT)
                     if (L.tfl[slot] & TF_UNSURE) {
                         L.be_slot[ub++] = slot;

@@ -61,6 +61,40 @@ def test_orient4_sos_matches_oracle(tri, orc):
     assert (depth > 0).sum() > 100
 
 
+def _span_bits(points):
+    """Bits from the highest to the lowest set one over all coordinates."""
+    r = [v.as_integer_ratio() for v in points.ravel().tolist() if v != 0.0]
+    low = min((abs(a) & -abs(a)).bit_length() - 1 - (b.bit_length() - 1) for a, b in r)
+    return max(abs(a).bit_length() - (b.bit_length() - 1) for a, b in r) - low
+
+
+@pytest.mark.parametrize("low", [0, 3, 4, 7, 8, 9, 12, 19, 20, 40, 71, 72, 73])
+def test_orient4_across_coordinate_spans(tri, orc, low):
+    """Coordinates from 1 down to 2^-low in one tuple: up to 61 bits together they are whole
+    numbers on one scale, beyond that their differences may be, and else the general path runs.
+    Lattice tuples (zero determinants, SoS) and general ones, each scaled per point, per axis or
+    by a common offset.  Tuples beyond 125 bits are refused."""
+    rng = np.random.default_rng(100 + low)
+    n, t = 60, []
+    for base in (rng.random((n, 5, 3)), rng.integers(0, 3, size=(n, 5, 3)) / 20.0 + 0.3,
+                 rng.integers(0, 3, size=(n, 5, 3)) / 4.0):
+        point, axis = np.ones((n, 5, 1)), np.ones((n, 1, 3))
+        point[:, rng.integers(5)] = axis[:, :, rng.integers(3)] = 2.0 ** -low
+        t += [base * point, base * axis, base * 2.0 ** -low + [0.0, 0.5, 0.0]]
+    t = np.concatenate(t)
+    t = t[[len({tuple(r) for r in q}) == 5 for q in t]]
+    idx = np.array([rng.permutation(10 ** 6)[:5] for _ in range(t.shape[0])], np.int32)
+    ok = np.array([_span_bits(q) <= 125 for q in t])
+    if not ok.all():
+        with pytest.raises(g.G4DError, match="PREDICATE_RANGE"):
+            tri.diag_orient4(t[~ok].reshape(-1, 15), idx[~ok], mode=1)
+        t, idx = t[ok], idx[ok]
+    sign, depth = tri.diag_orient4(t.reshape(-1, 15), idx, mode=1)
+    ref = [orc.orient4_sos(t[j], idx[j]) for j in range(t.shape[0])]
+    assert (sign == np.array([r[0] for r in ref])).all()
+    assert (depth == np.array([r[1] for r in ref])).all()
+
+
 @pytest.mark.parametrize("mode", [0, 1])
 def test_sos_every_depth_matches_oracle(tri, orc, mode):
     """Tuples built to stop SoS at each depth 1..13 (all reachable depths): the GPU's exact +
