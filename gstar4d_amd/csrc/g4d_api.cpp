@@ -911,12 +911,12 @@ static int run_device(g4d_ctx *ctx, const double *d_xyz, int n, const SetSpec &s
         sp.exact_cap = n;
         sp.exact_counter = G4D_CNT_APPEND4;
         sp.t0_variant = ctx->star_t0_variant;
-        // list counters, filter counts and the six work-queue heads of this pass, in one launch
+        // list counters, filter counts and the work-queue heads of this pass, in one launch
         {
             uint32_t zmask = (1u << G4D_CNT_APPEND2) | (1u << G4D_CNT_APPEND3) | (1u << G4D_CNT_APPEND4) |
                              (1u << G4D_CNT_APPEND6) | (1u << G4D_CNT_XMID) | (1u << G4D_CNT_XBIG) |
-                             (1u << G4D_CNT_ORIENT4) | (1u << G4D_CNT_COFACTOR);
-            for (int q = 0; q < 6; q++) zmask |= 1u << (G4D_CNT_QUEUE0 + q);
+                             (1u << G4D_CNT_XL) | (1u << G4D_CNT_ORIENT4) | (1u << G4D_CNT_COFACTOR);
+            for (int q = 0; q < 7; q++) zmask |= 1u << (G4D_CNT_QUEUE0 + q);
             HCK(g4d::launch_zero_counters(cnt, zmask, s));
         }
         int queue = G4D_CNT_QUEUE0;
@@ -924,11 +924,10 @@ static int run_device(g4d_ctx *ctx, const double *d_xyz, int n, const SetSpec &s
         sp.star_list = list;
         sp.nlist = nitems;
         sp.nlist_dev = nullptr;
-        // Filter-only LDS kernels by size tier (32 -> 64 -> 256 link vertices); each passes the
-        // stars it cannot hold to the next tier's list and the ones its filters cannot decide
-        // to the exact list.  Then the exact-capable kernels of the same tiers over the exact
-        // list.  Every later launch reads its list length on the device, so the chain runs
-        // without host round trips; lists and counters are reused in stream order.
+        // Filter-only LDS kernels by size tier (32 -> 64 -> 128 -> 256 link vertices); each passes
+        // the stars it cannot hold to the next tier's list and the ones its filters cannot decide
+        // to the exact list.  Every later launch reads its list length on the device, so the chain
+        // runs without host round trips; lists and counters are reused in stream order.
         if (ctx->ev_ok) (void)hipEventRecord(ctx->ev_t0[0], s);
         HCK(g4d::launch_star_kernel(sp, g4d::STAR_VMAX_T0, false, nblk_star, s));
         if (ctx->ev_ok) (void)hipEventRecord(ctx->ev_t0[1], s);
@@ -941,21 +940,30 @@ static int run_device(g4d_ctx *ctx, const double *d_xyz, int n, const SetSpec &s
             sp.work_counter = queue++;
             // a tier's list is a subset of the pass's stars: late rounds with a few thousand stars
             // dispatch a few hundred work-groups instead of thousands that would leave at once
-            const int full = vmax == g4d::STAR_VMAX_T1 && !exact ? 4096 : 1024;
+            // as many as the tier has resident waves
+            const int full = exact ? 1024 : vmax == g4d::STAR_VMAX_T1 ? 4096 : vmax == g4d::STAR_VMAX_TM ? 3072 : 1536;
             const int nblk = std::max(64, std::min(full, (nitems + 7) / 8));
             HCK(g4d::launch_star_kernel(sp, vmax, exact, nblk, s));
             return G4D_OK;
         };
-        // filter tiers: mid list (A6) -> 64, big list (A2) -> 256, beyond -> huge (A3)
+        // filter tiers: mid list (A6) -> 64, big list (A2) -> 128, mid list again (XL) -> 256, beyond
+        // -> huge (A3)
         CK(chain(buf<int>(ctx->mid), G4D_CNT_APPEND6, buf<int>(ctx->big), G4D_CNT_APPEND2, g4d::STAR_VMAX_T1, false));
-        CK(chain(buf<int>(ctx->big), G4D_CNT_APPEND2, buf<int>(ctx->huge), G4D_CNT_APPEND3, g4d::STAR_VMAX_T2, false));
-        // the exact chain reuses the mid/big lists (the filter chain is done with them in stream
-        // order) under counters of its own, so the filter tiers' counts stay for the statistics
-        CK(chain(buf<int>(ctx->xstars), G4D_CNT_APPEND4, buf<int>(ctx->mid), G4D_CNT_XMID, g4d::STAR_VMAX_T0, true));
-        CK(chain(buf<int>(ctx->mid), G4D_CNT_XMID, buf<int>(ctx->big), G4D_CNT_XBIG, g4d::STAR_VMAX_T1, true));
-        CK(chain(buf<int>(ctx->big), G4D_CNT_XBIG, buf<int>(ctx->huge), G4D_CNT_APPEND3, g4d::STAR_VMAX_T2, true));
-        sp.nlist_dev = nullptr;
+        CK(chain(buf<int>(ctx->big), G4D_CNT_APPEND2, buf<int>(ctx->mid), G4D_CNT_XL, g4d::STAR_VMAX_TM, false));
+        CK(chain(buf<int>(ctx->mid), G4D_CNT_XL, buf<int>(ctx->huge), G4D_CNT_APPEND3, g4d::STAR_VMAX_T2, false));
         CK(read_counters(ctx, hc));
+        const int64_t nmid = (int64_t)hc[G4D_CNT_APPEND6], nbig = (int64_t)hc[G4D_CNT_APPEND2];
+        const int64_t nexact = (int64_t)hc[G4D_CNT_APPEND4];
+        if (nexact > 0) {
+            // The exact-capable kernels of tiers 32, 64 and 256 over the exact list.  They reuse the
+            // mid and big lists (the filter chain is done with them) under counters of their own, so
+            // the filter tiers' counts stay for the statistics.
+            CK(chain(buf<int>(ctx->xstars), G4D_CNT_APPEND4, buf<int>(ctx->mid), G4D_CNT_XMID, g4d::STAR_VMAX_T0, true));
+            CK(chain(buf<int>(ctx->mid), G4D_CNT_XMID, buf<int>(ctx->big), G4D_CNT_XBIG, g4d::STAR_VMAX_T1, true));
+            CK(chain(buf<int>(ctx->big), G4D_CNT_XBIG, buf<int>(ctx->huge), G4D_CNT_APPEND3, g4d::STAR_VMAX_T2, true));
+            CK(read_counters(ctx, hc));
+        }
+        sp.nlist_dev = nullptr;
         {
             float ms = 0.f;
             if (ctx->ev_ok && hipEventElapsedTime(&ms, ctx->ev_t0[0], ctx->ev_t0[1]) == hipSuccess)
@@ -964,8 +972,6 @@ static int run_device(g4d_ctx *ctx, const double *d_xyz, int n, const SetSpec &s
             ctx->st.star_t0_cofactors += (int64_t)hc[G4D_CNT_COFACTOR];
             ctx->st.star_t0_launches++;
         }
-        const int64_t nmid = (int64_t)hc[G4D_CNT_APPEND6], nbig = (int64_t)hc[G4D_CNT_APPEND2];
-        const int64_t nexact = (int64_t)hc[G4D_CNT_APPEND4];
         ctx->st.big_stars += (int32_t)nbig;
         ctx->st.exact_stars += nexact;
         const int64_t nhuge = (int64_t)hc[G4D_CNT_APPEND3];

@@ -51,7 +51,7 @@ enum g4d_counter : int {
     G4D_CNT_SOS = 6,      // SoS resolutions
     G4D_CNT_ORIENT3 = 7,
     G4D_CNT_MISC = 8,
-    G4D_CNT_WORK = 9,     // spare
+    G4D_CNT_XL = 9,       // list length of the filter chain's 256-vertex tier
     G4D_CNT_APPEND3 = 10,
     G4D_CNT_APPEND4 = 11,
     G4D_CNT_APPEND5 = 12,
@@ -59,7 +59,7 @@ enum g4d_counter : int {
     G4D_CNT_COFACTOR = 14, // cached-cofactor computations in the LDS star kernels
     G4D_CNT_XMID = 15,     // list lengths of the exact chain's 64- and 256-vertex tiers
     G4D_CNT_XBIG = 16,
-    G4D_CNT_QUEUE0 = 17,   // work-queue heads of the six star-kernel launches of one pass (17..22)
+    G4D_CNT_QUEUE0 = 17,   // work-queue heads of the star-kernel launches of one pass (17..23)
     G4D_CNT_NUM = 24
 };
 

@@ -1203,4 +1203,15 @@ __device__ __forceinline__ int cofactor_filter_sign(const double *r, const doubl
     return val > bnd ? 1 : (-val > bnd ? -1 : 0);
 }
 
+// The same with two permanents per triangle, the largest of P_0..P_2 and P_3, and rsum = |r_0| +
+// |r_1| + |r_2|: at least the sum above, up to roundings that the margin of 32 u over 17.1 u covers.
+__device__ __forceinline__ int cofactor_filter_sign2(const double *r, double rsum, const double *C, double pxyz, double pl)
+{
+    const double val = fma(r[3], C[3], fma(r[2], C[2], fma(r[1], C[1], r[0] * C[0])));
+    const double per = fma(r[3], pl, rsum * pxyz);
+    const double bnd = 32.0 * 1.1102230246251565e-16 * per;
+    if (!(per > 1e-250)) return 0;
+    return val > bnd ? 1 : (-val > bnd ? -1 : 0);
+}
+
 } // namespace g4d

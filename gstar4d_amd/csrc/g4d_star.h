@@ -8,6 +8,7 @@ namespace g4d {
 // LDS star kernel tiers by link vertices (plus this pass's insertions).
 static constexpr int STAR_VMAX_T0 = 32;
 static constexpr int STAR_VMAX_T1 = 64;
+static constexpr int STAR_VMAX_TM = 128; // filter-only
 static constexpr int STAR_VMAX_T2 = 256;
 // Stars taken per work-queue atomic by the filter-only LDS kernels.
 static constexpr int STAR_CHUNK = 8;
@@ -89,7 +90,7 @@ enum {
     STAR_T0_NUM = 5
 };
 
-// LDS star kernel for stars of up to vmax (STAR_VMAX_T0, T1 or T2) link vertices plus
+// LDS star kernel for stars of up to vmax (STAR_VMAX_T0, T1, TM or T2) link vertices plus
 // insertions; larger ones go to p.defer_list.  exact = false: filters only (no multiprecision
 // code, no private scratch), a star with an inconclusive orientation goes to p.exact_list
 // untouched.  exact = true: exact predicates and SoS, for the stars of star_list.

@@ -79,12 +79,19 @@ __device__ __forceinline__ void star_tri_verts(const uint64_t *tpool, int64_t to
     }
 }
 
-template <int VMAX>
-struct StarLds {
-    static constexpr int TMAX = 2 * VMAX;
-    // per triangle slot: cofactors C[0..3] and permanents P[0..3], stored component-major so
-    // that the lanes of a wave, each reading its own slot, touch consecutive 8-byte words
+// Per triangle slot: cofactors C[0..3] and permanents P[0..3], stored component-major so that the
+// lanes of a wave, each reading its own slot, touch consecutive 8-byte words.
+template <int TMAX, bool CACHED>
+struct StarCof {
     double cof[8][TMAX];
+};
+template <int TMAX>
+struct StarCof<TMAX, false> {
+};
+
+template <int VMAX, bool CACHED>
+struct StarLds : StarCof<2 * VMAX, CACHED> {
+    static constexpr int TMAX = 2 * VMAX;
     int vid[VMAX];
     double vc[VMAX][4];
     uint32_t tv[TMAX];
@@ -233,13 +240,19 @@ __device__ __forceinline__ void star_commit(const StarParams &p, int s, int vcou
 
 // EXACT = false: filters only.  A star with an inconclusive orientation is handed to
 // p.exact_list untouched (its output is written only at the end), so the kernel carries no
-// multiprecision code and no private scratch.
+// multiprecision code and no private scratch.  Its registers then have room for the cofactors of
+// the lane's own slots, with two permanents each (the largest of the three coordinates', and the
+// lift's), which only that lane reads: without them in LDS a 256-vertex star takes 25 KB instead
+// of 57 and six waves share a CU instead of two.
 template <int VMAX, bool EXACT>
 __device__ __forceinline__ void star_body(const StarParams &p, int nitems)
 {
-    constexpr int TMAX = StarLds<VMAX>::TMAX;
+    constexpr bool REGC = !EXACT;
+    using Lds = StarLds<VMAX, !REGC>;
+    constexpr int TMAX = Lds::TMAX;
     constexpr int KPL = TMAX / 64;
-    __shared__ StarLds<VMAX> L;
+    __shared__ Lds L;
+    double rc[REGC ? KPL : 1][4], rp[REGC ? KPL : 1][2];
     const int lane = threadIdx.x;
     unsigned long long *cnt = p.cnt;
 
@@ -353,15 +366,43 @@ __device__ __forceinline__ void star_body(const StarParams &p, int nitems)
                 T = 4;
             }
             wave_sync();
+            // The cofactors of this lane's slots k of the mask: registers are filled by rounds, a slot
+            // of each lane per round, so that a few new triangles spread over the lanes cost a
+            // round or two and not one for every k that some lane needs.
+            auto cofactors = [&](unsigned km) {
+                if constexpr (REGC) {
+                    while (__ballot(km != 0)) {
+                        const int k = km ? __builtin_ctz(km) : KPL;
+                        double C[4], P[4];
+                        if (km) {
+                            const uint32_t t = L.tv[lane + 64 * k];
+                            tri_cofactors(L.vc[tvert(t, 0)], L.vc[tvert(t, 1)], L.vc[tvert(t, 2)], C, P);
+                            L.tv[lane + 64 * k] = t & ~TF_FRESH;
+                            ncof++;
+                        }
+#pragma unroll
+                        for (int i = 0; i < KPL; i++)
+                            if (i == k) {
+#pragma unroll
+                                for (int j = 0; j < 4; j++) rc[i][j] = C[j];
+                                rp[i][0] = fmax(P[0], fmax(P[1], P[2]));
+                                rp[i][1] = P[3];
+                            }
+                        km &= km - 1;
+                    }
+                } else {
 #pragma unroll 1
-            for (int k = 0; k < KPL; k++) {
-                const int slot = lane + 64 * k;
-                if (slot < T) {
-                    const uint32_t t = L.tv[slot];
-                    lds_cofactors<TMAX>(L.vc[tvert(t, 0)], L.vc[tvert(t, 1)], L.vc[tvert(t, 2)], L.cof, slot);
-                    ncof++;
+                    for (int k = 0; k < KPL; k++)
+                        if ((km >> k) & 1) {
+                            const int slot = lane + 64 * k;
+                            const uint32_t t = L.tv[slot];
+                            lds_cofactors<TMAX>(L.vc[tvert(t, 0)], L.vc[tvert(t, 1)], L.vc[tvert(t, 2)], L.cof, slot);
+                            L.tv[slot] = t & ~TF_FRESH;
+                            ncof++;
+                        }
                 }
-            }
+            };
+            cofactors(T > lane ? (unsigned)((1ull << ((T - lane + 63) / 64)) - 1ull) : 0u);
             bool failed = false, unsure = false;
             for (int q = q0; q < m; q++) {
                 const int gv = L.ins[q];
@@ -370,17 +411,23 @@ __device__ __forceinline__ void star_body(const StarParams &p, int nitems)
                 int nv = 0;
                 unsigned vm = 0; // bit k: slot lane + 64 k sees the vertex
                 unsigned um = 0; // bit k: its filter is inconclusive
-#pragma unroll 1
+                const double rsum = fabs(r[0]) + fabs(r[1]) + fabs(r[2]);
+#pragma unroll(REGC ? KPL : 1)
                 for (int k = 0; k < KPL; k++) {
                     const int slot = lane + 64 * k;
                     if (slot < T) {
                         const uint32_t t = L.tv[slot];
                         if ((t & (TF_ALIVE | TF_VIS)) == TF_ALIVE) {
                             nfilt++;
-                            double c[8];
+                            int sg;
+                            if constexpr (REGC) {
+                                sg = cofactor_filter_sign2(r, rsum, rc[k], rp[k][0], rp[k][1]);
+                            } else {
+                                double c[8];
 #pragma unroll
-                            for (int j = 0; j < 8; j++) c[j] = L.cof[j][slot];
-                            const int sg = cofactor_filter_sign(r, c, c + 4);
+                                for (int j = 0; j < 8; j++) c[j] = L.cof[j][slot];
+                                sg = cofactor_filter_sign(r, c, c + 4);
+                            }
                             if (sg == 0) um |= 1u << k;
                             if (sg < 0) {
                                 L.tv[slot] = t | TF_VIS;
@@ -504,19 +551,11 @@ __device__ __forceinline__ void star_body(const StarParams &p, int nitems)
                 // the link writes above touch only the new slots' neighbour rows: the cofactor
                 // pass below (triangle words, coordinates, this lane's cofactor columns) needs no
                 // barrier after them
-#pragma unroll 1
-                for (int k = 0; k < KPL; k++) {
-                    const int slot = lane + 64 * k;
-                    if (slot < T) {
-                        const uint32_t t = L.tv[slot];
-                        if (t & TF_FRESH) {
-                            lds_cofactors<TMAX>(L.vc[tvert(t, 0)], L.vc[tvert(t, 1)], L.vc[tvert(t, 2)], L.cof,
-                                                slot);
-                            ncof++;
-                            L.tv[slot] = t & ~TF_FRESH;
-                        }
-                    }
-                }
+                unsigned fm = 0;
+#pragma unroll(REGC ? KPL : 1)
+                for (int k = 0; k < KPL; k++)
+                    if (lane + 64 * k < T && (L.tv[lane + 64 * k] & TF_FRESH)) fm |= 1u << k;
+                cofactors(fm);
                 // No barrier before the next step: its filter reads and writes only this lane's
                 // own slots and cofactor columns and the listed coordinates, and its first barrier
                 // precedes any read of another lane's words.
@@ -636,10 +675,20 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(5, 8)))
     star_body<STAR_VMAX_T0, false>(p, nitems);
 }
 
-template <int VMAX, bool EXACT>
-__global__ void __launch_bounds__(64) k_star(StarParams p, int nitems)
+// The filter-only tiers above: the registers that each occupancy leaves, measured on 1,000,000
+// clustered points (12 passes): 64 vertices at 3, 4, 5 waves per SIMD 11.0, 9.9, 10.5 ms; 128 at
+// 2, 3 waves 9.5, 8.3 ms; 256 at 2 waves 8.5 ms.  With cofactors in LDS and no 128-vertex tier
+// the 64-vertex stars took 11.7 ms and all larger ones 38.8.
+template <int VMAX>
+__global__ void __launch_bounds__(64) k_star_exact(StarParams p, int nitems)
 {
-    star_body<VMAX, EXACT>(p, nitems);
+    star_body<VMAX, true>(p, nitems);
+}
+
+template <int VMAX, int WPE>
+__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WPE, 8))) k_star(StarParams p, int nitems)
+{
+    star_body<VMAX, false>(p, nitems);
 }
 
 // ------------------------------------------------------------------------------------
@@ -1293,11 +1342,11 @@ hipError_t launch_star_kernel(const StarParams &p, int vmax, bool exact, int nbl
     if (nblocks > nitems) nblocks = nitems;
     if (exact) {
         if (vmax == STAR_VMAX_T0)
-            hipLaunchKernelGGL(HIP_KERNEL_NAME(k_star<STAR_VMAX_T0, true>), dim3(nblocks), dim3(64), 0, s, p, nitems);
+            hipLaunchKernelGGL(HIP_KERNEL_NAME(k_star_exact<STAR_VMAX_T0>), dim3(nblocks), dim3(64), 0, s, p, nitems);
         else if (vmax == STAR_VMAX_T1)
-            hipLaunchKernelGGL(HIP_KERNEL_NAME(k_star<STAR_VMAX_T1, true>), dim3(nblocks), dim3(64), 0, s, p, nitems);
+            hipLaunchKernelGGL(HIP_KERNEL_NAME(k_star_exact<STAR_VMAX_T1>), dim3(nblocks), dim3(64), 0, s, p, nitems);
         else if (vmax == STAR_VMAX_T2)
-            hipLaunchKernelGGL(HIP_KERNEL_NAME(k_star<STAR_VMAX_T2, true>), dim3(nblocks), dim3(64), 0, s, p, nitems);
+            hipLaunchKernelGGL(HIP_KERNEL_NAME(k_star_exact<STAR_VMAX_T2>), dim3(nblocks), dim3(64), 0, s, p, nitems);
         else
             return hipErrorInvalidValue;
     } else if (vmax == STAR_VMAX_T0) {
@@ -1317,9 +1366,11 @@ hipError_t launch_star_kernel(const StarParams &p, int vmax, bool exact, int nbl
             else hipLaunchKernelGGL(k_star32g32f, dim3(nb), dim3(64), 0, s, p, nitems);
         }
     } else if (vmax == STAR_VMAX_T1) {
-        hipLaunchKernelGGL(HIP_KERNEL_NAME(k_star<STAR_VMAX_T1, false>), dim3(nblocks), dim3(64), 0, s, p, nitems);
+        hipLaunchKernelGGL(HIP_KERNEL_NAME(k_star<STAR_VMAX_T1, 4>), dim3(nblocks), dim3(64), 0, s, p, nitems);
+    } else if (vmax == STAR_VMAX_TM) {
+        hipLaunchKernelGGL(HIP_KERNEL_NAME(k_star<STAR_VMAX_TM, 3>), dim3(nblocks), dim3(64), 0, s, p, nitems);
     } else if (vmax == STAR_VMAX_T2) {
-        hipLaunchKernelGGL(HIP_KERNEL_NAME(k_star<STAR_VMAX_T2, false>), dim3(nblocks), dim3(64), 0, s, p, nitems);
+        hipLaunchKernelGGL(HIP_KERNEL_NAME(k_star<STAR_VMAX_T2, 2>), dim3(nblocks), dim3(64), 0, s, p, nitems);
     } else {
         return hipErrorInvalidValue;
     }

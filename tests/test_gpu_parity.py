@@ -252,6 +252,18 @@ def test_uniform_small(orc, n, grid):
     assert st["splay_rounds"] == rst["splay_rounds"]
 
 
+@pytest.mark.parametrize("k", [30, 31, 32, 33, 60, 63, 64, 65, 120, 127, 128, 129, 250, 255, 256, 257, 500, 511, 512,
+                               513, 900, 1023, 1024, 1025])
+def test_star_sizes_around_the_kernel_tiers(orc, k):
+    """A point inside a shell of k points: the star's link and the insertions of a pass come to about
+    k, from the smallest star kernel past the largest."""
+    rng = np.random.default_rng(k)
+    shell = rng.normal(size=(k, 3))
+    shell *= (0.3 + 0.01 * rng.random((k, 1))) / np.linalg.norm(shell, axis=1)[:, None]
+    x = np.concatenate([[[0.5, 0.5, 0.5]], 0.5 + shell, rng.random((200, 3)) * 0.1])
+    _parity(orc, x, 24)
+
+
 @pytest.mark.parametrize("bands", [1, 3, 5])
 def test_pba_bands_same_triangulation(orc, bands):
     x = datasets.uniform_cube(20000, seed=31)
