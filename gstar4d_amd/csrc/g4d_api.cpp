@@ -977,18 +977,47 @@ static int run_device(g4d_ctx *ctx, const double *d_xyz, int n, const SetSpec &s
         const int64_t nhuge = (int64_t)hc[G4D_CNT_APPEND3];
         if (nhuge > 0) {
             ctx->st.huge_stars += (int32_t)nhuge;
-            HCK(hipMemsetAsync(cnt + G4D_CNT_MISC, 0, 8, s));
-            HCK(g4d::launch_need_max(sp, buf<int>(ctx->huge), (int)nhuge, cnt + G4D_CNT_MISC, s));
-            CK(read_counters(ctx, hc));
-            const int vcap_g = (int)hc[G4D_CNT_MISC];
-            const int64_t stride = (g4d::star_global_bytes(vcap_g) + 4095) & ~(int64_t)4095;
-            // bounded workspace: at most 256 blocks and 1 GiB
-            const int nblk = (int)std::max<int64_t>(1, std::min<int64_t>({nhuge, 256, ((int64_t)1 << 30) / stride}));
-            HCK(ctx->gwork.ensure((size_t)(stride * nblk)));
-            HCK(g4d::launch_star_global(sp, buf<int>(ctx->huge), (int)nhuge, buf<char>(ctx->gwork), stride, vcap_g,
-                                        nblk, s));
-            CK(read_counters(ctx, hc));
-            trace("global-memory star kernel: %lld stars, largest link plus insertions %d", (long long)nhuge, vcap_g);
+            // Beyond the one-wave kernels: the wide LDS kernel's two tiers (huge list -> 512, big list
+            // -> 1024), then the global-memory kernel for larger stars and those that need exact
+            // predicates (mid list).  A lowered lds_star_limit sends every star to the latter.
+            int *glist = buf<int>(ctx->huge);
+            int64_t nglobal = nhuge;
+            if (lds_limit == g4d::STAR_LDS_LIMIT) {
+                const int q = G4D_CNT_QUEUE0;
+                HCK(g4d::launch_zero_counters(cnt, (1u << G4D_CNT_XMID) | (1u << G4D_CNT_XBIG) | (1u << q) | (2u << q), s));
+                glist = buf<int>(ctx->mid);
+                sp.exact_list = glist;
+                sp.exact_counter = G4D_CNT_XMID;
+                sp.nlist = n;
+                sp.star_list = buf<int>(ctx->huge);
+                sp.nlist_dev = cnt + G4D_CNT_APPEND3;
+                sp.defer_list = buf<int>(ctx->big);
+                sp.defer_counter = G4D_CNT_XBIG;
+                sp.work_counter = q;
+                HCK(g4d::launch_star_wide(sp, g4d::STAR_VMAX_W1, s));
+                sp.star_list = buf<int>(ctx->big);
+                sp.nlist_dev = cnt + G4D_CNT_XBIG;
+                sp.defer_list = glist;
+                sp.defer_counter = G4D_CNT_XMID;
+                sp.work_counter = q + 1;
+                HCK(g4d::launch_star_wide(sp, g4d::STAR_VMAX_W2, s));
+                sp.nlist_dev = nullptr;
+                CK(read_counters(ctx, hc));
+                nglobal = (int64_t)hc[G4D_CNT_XMID];
+            }
+            if (nglobal > 0) {
+                HCK(hipMemsetAsync(cnt + G4D_CNT_MISC, 0, 8, s));
+                HCK(g4d::launch_need_max(sp, glist, (int)nglobal, cnt + G4D_CNT_MISC, s));
+                CK(read_counters(ctx, hc));
+                const int vcap_g = (int)hc[G4D_CNT_MISC];
+                const int64_t stride = (g4d::star_global_bytes(vcap_g) + 4095) & ~(int64_t)4095;
+                // bounded workspace: at most 256 blocks and 1 GiB
+                const int nblk = (int)std::max<int64_t>(1, std::min<int64_t>({nglobal, 256, ((int64_t)1 << 30) / stride}));
+                HCK(ctx->gwork.ensure((size_t)(stride * nblk)));
+                HCK(g4d::launch_star_global(sp, glist, (int)nglobal, buf<char>(ctx->gwork), stride, vcap_g, nblk, s));
+                CK(read_counters(ctx, hc));
+                trace("global-memory star kernel: %lld stars, largest link plus insertions %d", (long long)nglobal, vcap_g);
+            }
         }
         CK(check_dev_error(ctx, hc[G4D_CNT_ERROR], mode ? "splaying" : "star creation"));
         // drowned insertions and triangle pairs, in star order (both counts read back together)

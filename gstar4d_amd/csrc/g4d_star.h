@@ -10,6 +10,9 @@ static constexpr int STAR_VMAX_T0 = 32;
 static constexpr int STAR_VMAX_T1 = 64;
 static constexpr int STAR_VMAX_TM = 128; // filter-only
 static constexpr int STAR_VMAX_T2 = 256;
+// Tiers of the wide LDS kernel (a work-group per star).
+static constexpr int STAR_VMAX_W1 = 512;
+static constexpr int STAR_VMAX_W2 = 1024;
 // Stars taken per work-queue atomic by the filter-only LDS kernels.
 static constexpr int STAR_CHUNK = 8;
 // Star triangles in HBM.  A star with fewer than STAR_WIDE_MIN link vertices stores each
@@ -17,8 +20,9 @@ static constexpr int STAR_CHUNK = 8;
 // checked flag (bit 57).  A larger star stores two words per triangle: local vertices
 // (21 bits each, checked flag in bit 63), then adjacency slots (21 bits each).
 static constexpr int STAR_WIDE_MIN = 512;
-// Stars whose link (plus this pass's insertions) exceeds the LDS kernels' limit run in the
-// global-memory star kernel, which has no fixed capacity.
+// Largest star (link plus this pass's insertions) of the one-wave LDS kernels; larger ones go to the
+// wide LDS kernel, and beyond STAR_VMAX_W2 to the global-memory star kernel, which has no fixed
+// capacity.
 static constexpr int STAR_LDS_LIMIT = STAR_WIDE_MIN - 1;
 
 // Triangle words reserved for a star of v link vertices (including this pass's insertions):
@@ -97,6 +101,9 @@ enum {
 // Zeroes the counter words whose bits are set in mask (one launch instead of one fill per word).
 hipError_t launch_zero_counters(unsigned long long *cnt, uint32_t mask, hipStream_t s);
 hipError_t launch_star_kernel(const StarParams &p, int vmax, bool exact, int nblocks, hipStream_t s);
+// Wide LDS kernel, vmax = STAR_VMAX_W1 or W2, over the star_list whose length is at nlist_dev:
+// larger stars go to p.defer_list, inconclusive ones untouched to p.exact_list.
+hipError_t launch_star_wide(const StarParams &p, int vmax, hipStream_t s);
 // Global-memory star kernel for the stars in `list` (any size up to vcap link vertices);
 // each block owns a workspace of star_global_bytes(vcap) bytes at ws + blockIdx * stride.
 int64_t star_global_bytes(int vcap);

@@ -1378,13 +1378,416 @@ hipError_t launch_star_kernel(const StarParams &p, int vmax, bool exact, int nbl
 }
 
 // ------------------------------------------------------------------------------------
+// Wide star kernel: stars of up to VMAX link vertices plus insertions in LDS, one work-group of NT
+// threads per star, filters only.  A thread owns the slots tid, tid + NT, ... and keeps their
+// cofactors in registers as the one-wave kernels do; the step is theirs too, with work-group
+// barriers (five a step, one per scan and one before each pass that reads what others wrote).
+// Slots are counted in the order of the global-memory kernel below, as if 512 threads owned them, so
+// a star leaves either kernel with the same triangles in the same order.
+//
+// That kernel keeps these arrays in HBM, 64 bytes of cofactors a slot among them, and reads them
+// through L2 once per insertion; it now takes the stars beyond 1,024 and those whose filters are
+// inconclusive.  On 1,000,000 clustered points (11,766 stars of 257-2,283 over six passes) it took
+// 35.4 ms; 512 vertices take 4.7 ms here, 1,024 6.8 ms, and the few larger ones 6.9 ms there, each a
+// chain of its insertions.  (512 vertices with 256 threads at 2 waves per SIMD 5.6 ms, with 512
+// threads 5.8 ms.)
+// ------------------------------------------------------------------------------------
+
+static constexpr int STAR_ORDER = 512; // threads whose slot order both kernels follow
+
+template <int VMAX, int NT>
+struct StarWideLds {
+    static constexpr int TMAX = 2 * VMAX;
+    double vc[VMAX][4];
+    union {
+        uint16_t tv[TMAX][4]; // local vertices 0-2, flags (TW_*)
+        uint64_t tv64[TMAX];
+    };
+    union {
+        uint16_t to[TMAX][4]; // neighbours across the edges opposite vertices 0-2 (fourth unused)
+        uint64_t to64[TMAX];
+    };
+    int vid[VMAX], ins[VMAX];
+    uint16_t vstart[VMAX], vend[VMAX], freel[TMAX];
+    union {
+        struct {
+            uint16_t a[TMAX], b[TMAX], u[TMAX], slot[TMAX];
+            uint8_t j[TMAX];
+        } be; // hole boundary
+        struct {
+            uint16_t remap[TMAX], vremap[VMAX];
+            uint8_t present[VMAX];
+        } fin; // finalisation
+    };
+    int16_t ins_local[VMAX];
+    int red[4][NT / 64]; // rows 0 and 1: the filters' counts by turns; 2 and 3: the other scans
+    int item;
+};
+
+static constexpr uint32_t TW_ALIVE = 1u, TW_CHECKED = 2u, TW_VIS = 4u, TW_FRESH = 8u;
+
+__device__ __forceinline__ uint64_t wtri(int a, int b, int c, uint32_t fl)
+{
+    return (uint64_t)(uint32_t)a | ((uint64_t)(uint32_t)b << 16) | ((uint64_t)(uint32_t)c << 32) | ((uint64_t)fl << 48);
+}
+__device__ __forceinline__ int wtv(uint64_t t, int i) { return (int)((t >> (16 * i)) & 0xffffu); }
+__device__ __forceinline__ uint32_t wfl(uint64_t t) { return (uint32_t)(t >> 48); }
+
+// Exclusive prefix over the work-group of packed counts and their total; `add` joins the wave's
+// total (wave-uniform).  One barrier, so no row of red may serve two calls without a barrier between
+// the first call's reads and the second's write: consecutive calls use different rows.
+template <int NT>
+__device__ __forceinline__ int wide_excl(int v, int add, int *red, int *tot)
+{
+    const int lane = __lane_id(), w = threadIdx.x >> 6;
+    const int inc = g4d_wave_incl_sum(v);
+    if (lane == 63) red[w] = inc + add;
+    __syncthreads();
+    int base = 0, all = 0;
+#pragma unroll
+    for (int i = 0; i < NT / 64; i++) {
+        const int x = red[i];
+        if (i < w) base += x;
+        all += x;
+    }
+    *tot = all;
+    return base + inc - v;
+}
+
+template <int VMAX, int NT, int WPE>
+__global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(WPE, 8))) k_star_wide(StarParams p, int nitems)
+{
+    using Lds = StarWideLds<VMAX, NT>;
+    constexpr int TMAX = Lds::TMAX, KPL = TMAX / NT, H = STAR_ORDER / NT;
+    static_assert(H * NT == STAR_ORDER && TMAX < 4096, "packed counts of 12 bits");
+    __shared__ Lds L;
+    const int tid = threadIdx.x;
+    unsigned long long *cnt = p.cnt;
+    double rc[KPL][4], rp[KPL][2];
+    const unsigned long long c = *p.nlist_dev;
+    nitems = c < (unsigned long long)nitems ? (int)c : nitems;
+    if ((int)blockIdx.x >= nitems) return;
+    int ncof = 0, nfilt = 0;
+    for (;;) {
+        __syncthreads(); // the previous star is done with L
+        if (tid == 0) L.item = (int)atomicAdd(&cnt[p.work_counter], 1ull);
+        __syncthreads();
+        if (L.item >= nitems) break;
+        const int s = p.star_list[L.item];
+        const int64_t ib = p.ins_off[s];
+        const int m = (int)(p.ins_off[s + 1] - ib);
+        const int vn = p.mode ? p.vnum[s] : 0;
+        const int need = vn + m;
+        if (need > VMAX || (p.mode == 0 && m < 4)) {
+            if (need > VMAX) {
+                if (tid < 64) star_list_push(p.defer_list, p.defer_cap, &cnt[p.defer_counter], s, cnt);
+            } else if (tid == 0) {
+                atomicOr(&cnt[G4D_CNT_ERROR], (unsigned long long)G4D_DEV_ERR_CONE);
+                p.vnum[s] = 0;
+                p.tnum[s] = 0;
+            }
+            continue;
+        }
+        if (p.mode == 1 && m == 0) continue; // untouched star: stays where it is
+        const bool in_wide = vn >= STAR_WIDE_MIN;
+        const double sx = p.pts[3 * (int64_t)s], sy = p.pts[3 * (int64_t)s + 1], sz = p.pts[3 * (int64_t)s + 2];
+        const int q0 = p.mode ? 0 : 4;
+        for (int q = tid; q < m; q += NT) {
+            const int g = (int)(uint32_t)p.ins_keys[ib + q];
+            L.ins[q] = g;
+            L.ins_local[q] = -1;
+            if (q >= q0) {
+                L.vid[vn + q] = g;
+                rel_coords(p.pts, g, sx, sy, sz, L.vc[vn + q]);
+            }
+        }
+        int T, nfree = 0;
+        bool unsure = false, failed = false;
+        if (p.mode == 1) {
+            const int tn = p.tnum[s];
+            const int64_t vi = p.voff[s], ti = p.toff[s];
+            for (int v = tid; v < vn; v += NT) {
+                const int g = p.vpool[vi + v];
+                L.vid[v] = g;
+                rel_coords(p.pts, g, sx, sy, sz, L.vc[v]);
+            }
+            for (int t = tid; t < tn; t += NT) {
+                if (in_wide) {
+                    const uint64_t w0 = p.tpool[ti + 2 * (int64_t)t], w1 = p.tpool[ti + 2 * (int64_t)t + 1];
+                    L.tv64[t] = wtri(wfield(w0, 0), wfield(w0, 1), wfield(w0, 2), TW_ALIVE | ((w0 >> 63) ? TW_CHECKED : 0u));
+                    L.to64[t] = wtri(wfield(w1, 0), wfield(w1, 1), wfield(w1, 2), 0u);
+                } else {
+                    const uint64_t h = p.tpool[ti + t];
+                    L.tv64[t] = wtri(hvert(h, 0), hvert(h, 1), hvert(h, 2), TW_ALIVE | (hchecked(h) ? TW_CHECKED : 0u));
+                    L.to64[t] = wtri(hopp(h, 0), hopp(h, 1), hopp(h, 2), 0u);
+                }
+            }
+            T = tn;
+        } else {
+            // initial 4-simplex (GD/GDelaunay/GDelPredKernels.cu:45-158)
+            int l[4];
+            for (int i = 0; i < 4; i++) l[i] = (int)(uint32_t)p.ins_keys[ib + i];
+            const double *pp[5] = {p.pts + 3 * (int64_t)l[0], p.pts + 3 * (int64_t)l[1], p.pts + 3 * (int64_t)l[2],
+                                   p.pts + 3 * (int64_t)l[3], p.pts + 3 * (int64_t)s};
+            const int o = filter_insphere(pp);
+            unsure = o == 0;
+            const bool sw = o < 0;
+            if (tid < 4) {
+                const int from = (tid < 2 && sw) ? 1 - tid : tid;
+                L.vid[tid] = l[from];
+                rel_coords(p.pts, l[from], sx, sy, sz, L.vc[tid]);
+                const int lt[4][3] = {{1, 2, 3}, {0, 3, 2}, {0, 1, 3}, {0, 2, 1}};
+                L.tv64[tid] = wtri(lt[tid][0], lt[tid][1], lt[tid][2], TW_ALIVE);
+                L.to64[tid] = wtri(lt[tid][0], lt[tid][1], lt[tid][2], 0u);
+                L.ins_local[tid] = (int16_t)from;
+            }
+            T = 4;
+        }
+        __syncthreads();
+        // the cofactors of this thread's slots k of the mask, by rounds (as in star_body)
+        auto cofactors = [&](unsigned km) {
+            while (__ballot(km != 0)) {
+                const int k = km ? __builtin_ctz(km) : KPL;
+                double C[4], P[4];
+                if (km) {
+                    const uint64_t t = L.tv64[tid + NT * k];
+                    tri_cofactors(L.vc[wtv(t, 0)], L.vc[wtv(t, 1)], L.vc[wtv(t, 2)], C, P);
+                    L.tv[tid + NT * k][3] = (uint16_t)(wfl(t) & ~TW_FRESH);
+                    ncof++;
+                }
+#pragma unroll
+                for (int i = 0; i < KPL; i++)
+                    if (i == k) {
+#pragma unroll
+                        for (int j = 0; j < 4; j++) rc[i][j] = C[j];
+                        rp[i][0] = fmax(P[0], fmax(P[1], P[2]));
+                        rp[i][1] = P[3];
+                    }
+                km &= km - 1;
+            }
+        };
+        cofactors(T > tid ? (1u << ((T - tid + NT - 1) / NT)) - 1u : 0u);
+        for (int q = q0; q < m && !unsure; q++) {
+            const int Vn = vn + q;
+            const double r[4] = {L.vc[Vn][0], L.vc[Vn][1], L.vc[Vn][2], L.vc[Vn][3]};
+            const double rsum = fabs(r[0]) + fabs(r[1]) + fabs(r[2]);
+            unsigned vm = 0;
+            bool unc = false;
+            int nv = 0; // per half of the slot order, 12 bits each
+#pragma unroll
+            for (int k = 0; k < KPL; k++) {
+                const int slot = tid + NT * k;
+                if (slot < T) {
+                    const uint32_t f = L.tv[slot][3];
+                    if ((f & (TW_ALIVE | TW_VIS)) == TW_ALIVE) {
+                        nfilt++;
+                        const int sg = cofactor_filter_sign2(r, rsum, rc[k], rp[k][0], rp[k][1]);
+                        unc = unc || sg == 0;
+                        if (sg < 0) {
+                            L.tv[slot][3] = (uint16_t)(f | TW_VIS);
+                            vm |= 1u << k;
+                            nv += (k % H) ? 1 << 12 : 1;
+                        }
+                    }
+                }
+            }
+            int all;
+            const int pre = wide_excl<NT>(nv, __ballot(unc) ? 1 << 24 : 0, L.red[q & 1], &all);
+            if (all >> 24) {
+                unsure = true;
+                break;
+            }
+            const int nvis = (all & 0xfff) + ((all >> 12) & 0xfff);
+            if (nvis == 0) continue; // drowned at insertion
+            if (tid == 0) L.ins_local[q] = (int16_t)Vn;
+            {
+                // only the part of `pre` below bit 24 counts; the flag bits of earlier waves are zero here
+                int f0 = nfree + (pre & 0xfff), f1 = nfree + (all & 0xfff) + ((pre >> 12) & 0xfff);
+#pragma unroll
+                for (int k = 0; k < KPL; k++)
+                    if ((vm >> k) & 1) L.freel[(k % H) ? f1++ : f0++] = (uint16_t)(tid + NT * k);
+            }
+            __syncthreads();
+            // hole boundary in the order of the visible list (see star_body)
+            int nbtot = 0;
+            for (int x0 = 0, row = 2; x0 < nvis; x0 += NT, row ^= 1) {
+                const int x = x0 + tid;
+                uint64_t t = 0ull, o = 0ull, tu[3];
+                bool edge[3] = {false, false, false};
+                if (x < nvis) {
+                    const int slot = L.freel[nfree + x];
+                    t = L.tv64[slot];
+                    o = L.to64[slot];
+#pragma unroll
+                    for (int i = 0; i < 3; i++) {
+                        tu[i] = L.tv64[wtv(o, i)];
+                        edge[i] = !(wfl(tu[i]) & TW_VIS);
+                    }
+                }
+                int tot;
+                int e = nbtot + wide_excl<NT>((int)edge[0] + (int)edge[1] + (int)edge[2], 0, L.red[row], &tot);
+#pragma unroll
+                for (int i = 0; i < 3; i++) {
+                    if (!edge[i]) continue;
+                    const int a = wtv(t, (i + 1) % 3), b = wtv(t, (i + 2) % 3);
+                    const int u0 = wtv(tu[i], 0), u1 = wtv(tu[i], 1);
+                    if (e < TMAX) {
+                        L.be.a[e] = (uint16_t)a;
+                        L.be.b[e] = (uint16_t)b;
+                        L.be.u[e] = (uint16_t)wtv(o, i);
+                        L.be.j[e] = (uint8_t)((u0 != a && u0 != b) ? 0 : ((u1 != a && u1 != b) ? 1 : 2));
+                    }
+                    e++;
+                }
+                nbtot += tot;
+            }
+            const int nfree_tot = nfree + nvis;
+            const int newT = T + (nbtot > nfree_tot ? nbtot - nfree_tot : 0);
+            if (nbtot > TMAX || nbtot < 3 || newT > TMAX || Vn + 1 > VMAX) {
+                failed = true;
+                break;
+            }
+            __syncthreads();
+            for (int k = tid; k < nbtot; k += NT) {
+                const int slot = k < nfree_tot ? L.freel[nfree_tot - 1 - k] : T + (k - nfree_tot);
+                const int a = L.be.a[k], b = L.be.b[k], u = L.be.u[k];
+                L.be.slot[k] = (uint16_t)slot;
+                L.tv64[slot] = wtri(a, b, Vn, TW_ALIVE | TW_FRESH);
+                L.to[slot][2] = (uint16_t)u;
+                L.to[u][L.be.j[k]] = (uint16_t)slot;
+                L.vstart[a] = (uint16_t)slot;
+                L.vend[b] = (uint16_t)slot;
+            }
+            __syncthreads();
+            for (int k = tid; k < nbtot; k += NT) {
+                const int slot = L.be.slot[k];
+                L.to[slot][0] = L.vstart[L.be.b[k]];
+                L.to[slot][1] = L.vend[L.be.a[k]];
+            }
+            nfree = nfree_tot - (nbtot < nfree_tot ? nbtot : nfree_tot);
+            T = newT;
+            unsigned fm = 0;
+#pragma unroll
+            for (int k = 0; k < KPL; k++)
+                if (tid + NT * k < T && (L.tv[tid + NT * k][3] & TW_FRESH)) fm |= 1u << k;
+            cofactors(fm);
+            // No barrier before the next step, as in star_body: its filter touches this thread's own
+            // slots and the listed coordinates, and its scan's barrier comes before the rest.
+        }
+        __syncthreads();
+        if (unsure) {
+            if (tid < 64) star_list_push(p.exact_list, p.exact_cap, &cnt[p.exact_counter], s, cnt);
+            continue;
+        }
+        // ---- finalize: link set, drowned insertions, compaction, pairs, history ----
+        for (int v = tid; v < need; v += NT) L.fin.present[v] = 0;
+        __syncthreads();
+        if (!failed)
+            for (int t = tid; t < T; t += NT) {
+                const uint64_t w = L.tv64[t];
+                if ((wfl(w) & (TW_ALIVE | TW_VIS)) == TW_ALIVE)
+                    for (int i = 0; i < 3; i++) L.fin.present[wtv(w, i)] = 1;
+            }
+        __syncthreads();
+        const int64_t vo = p.nvoff[s], to = p.ntoff[s];
+        int vcount = 0, tcount = 0, row = 2;
+        if (!failed) {
+            for (int q = tid; q < m; q += NT) {
+                const int lv = L.ins_local[q];
+                p.dflag[ib + q] = (lv < 0 || !L.fin.present[lv]) ? 1 : 0;
+            }
+            for (int base = 0; base < need; base += NT, row ^= 1) {
+                const int v = base + tid;
+                const bool pr = v < need && L.fin.present[v];
+                int tot;
+                const int at = vcount + wide_excl<NT>(pr ? 1 : 0, 0, L.red[row], &tot);
+                if (pr) {
+                    L.fin.vremap[v] = (uint16_t)at;
+                    p.vpool[vo + at] = L.vid[v];
+                }
+                vcount += tot;
+            }
+            for (int base = 0; base < T; base += NT, row ^= 1) {
+                const int t = base + tid;
+                const bool al = t < T && (L.tv[t][3] & (TW_ALIVE | TW_VIS)) == TW_ALIVE;
+                int tot;
+                const int at = tcount + wide_excl<NT>(al ? 1 : 0, 0, L.red[row], &tot);
+                if (al) L.fin.remap[t] = (uint16_t)at;
+                tcount += tot;
+            }
+        }
+        const bool wide = vcount >= STAR_WIDE_MIN;
+        const int64_t words = wide ? 2 * (int64_t)tcount : tcount;
+        if (failed || words > star_tcap_words(need) || tcount != 2 * vcount - 4) {
+            // not a triangulated 2-sphere: report instead of writing past the star's region
+            if (tid == 0) {
+                atomicOr(&cnt[G4D_CNT_ERROR], (unsigned long long)G4D_DEV_ERR_HOLE);
+                p.vnum[s] = 0;
+                p.tnum[s] = 0;
+            }
+            continue;
+        }
+        __syncthreads();
+        const int64_t pb = 2 * (to - p.tbase);
+        int npair = 0;
+        for (int base = 0; base < T; base += NT, row ^= 1) {
+            const int t = base + tid;
+            const uint64_t w = t < T ? L.tv64[t] : 0ull;
+            TriPairs pr{STAR_PAIR_NONE, STAR_PAIR_NONE};
+            if ((wfl(w) & (TW_ALIVE | TW_VIS)) == TW_ALIVE) {
+                const int a = wtv(w, 0), b = wtv(w, 1), cc = wtv(w, 2);
+                const int ra = L.fin.vremap[a], rb = L.fin.vremap[b], rcc = L.fin.vremap[cc];
+                const int o0 = L.fin.remap[L.to[t][0]], o1 = L.fin.remap[L.to[t][1]], o2 = L.fin.remap[L.to[t][2]];
+                const int64_t d = L.fin.remap[t];
+                if (wide) {
+                    p.tpool[to + 2 * d] = wpack3(ra, rb, rcc) | (1ull << 63);
+                    p.tpool[to + 2 * d + 1] = wpack3(o0, o1, o2);
+                } else {
+                    p.tpool[to + d] = hpack(ra, rb, rcc, o0, o1, o2, true);
+                }
+                pr = star_tri_pairs(L.vid[a], L.vid[b], L.vid[cc], !(wfl(w) & TW_CHECKED));
+            }
+            // the star's pairs, dense, in triangle order
+            const int np = (pr.x != STAR_PAIR_NONE ? 1 : 0) + (pr.y != STAR_PAIR_NONE ? 1 : 0);
+            int tot;
+            const int64_t at = npair + wide_excl<NT>(np, 0, L.red[row], &tot);
+            if (np > 0) p.pairbuf[pb + at] = pr.x;
+            if (np > 1) p.pairbuf[pb + at + 1] = pr.y;
+            npair += tot;
+        }
+        if (tid == 0) p.pcount[s] = npair;
+        const int hn = star_history_merge(p, s, L.ins, m, tid, NT);
+        __syncthreads(); // every read of the old record and regions before the switch
+        if (tid == 0) star_commit(p, s, vcount, vo, tcount, to, hn + m);
+    }
+    const int wf = g4d_wave_sum(nfilt), wc = g4d_wave_sum(ncof);
+    if ((tid & 63) == 0) {
+        atomicAdd(&cnt[G4D_CNT_ORIENT4], (unsigned long long)wf);
+        atomicAdd(&cnt[G4D_CNT_COFACTOR], (unsigned long long)wc);
+    }
+}
+
+hipError_t launch_star_wide(const StarParams &p, int vmax, hipStream_t s)
+{
+    if (!p.star_list || !p.nlist_dev || p.nlist <= 0) return hipErrorInvalidValue;
+    // one work-group per resident one: LDS takes 50 KB at 512 vertices, 100 KB at 1,024
+    if (vmax == STAR_VMAX_W1)
+        hipLaunchKernelGGL(HIP_KERNEL_NAME(k_star_wide<STAR_VMAX_W1, 256, 3>), dim3(768), dim3(256), 0, s, p, p.nlist);
+    else if (vmax == STAR_VMAX_W2)
+        hipLaunchKernelGGL(HIP_KERNEL_NAME(k_star_wide<STAR_VMAX_W2, 512, 2>), dim3(256), dim3(512), 0, s, p, p.nlist);
+    else
+        return hipErrorInvalidValue;
+    return hipGetLastError();
+}
+
+// ------------------------------------------------------------------------------------
 // Global-memory star kernel: the same insertion / finalisation as k_star for stars whose
 // link exceeds the LDS kernels' capacity.  One wave per star; the star's working arrays
 // (32-bit local indices, cached cofactors per triangle slot) live in a per-block HBM
 // workspace sized for the largest such star of the pass.
 // ------------------------------------------------------------------------------------
 
-static constexpr int GSTAR_NT = 512; // threads per star in the global-memory kernel
+static constexpr int GSTAR_NT = STAR_ORDER; // threads per star in the global-memory kernel
 
 // Exclusive prefix sum of v over the work-group's threads in thread order; total in *tot.
 // red: GSTAR_NT / 64 ints of LDS.  Every thread of the work-group must call it.

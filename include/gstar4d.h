@@ -75,8 +75,8 @@ typedef struct {
     int32_t grid_size;
     int32_t splay_rounds;      /* LogLoopNum in the reference */
     int32_t max_workset;
-    int32_t big_stars;         /* star passes routed to the large-star LDS kernel */
-    int32_t huge_stars;        /* star passes routed to the global-memory star kernel */
+    int32_t big_stars;         /* star passes over 64 link vertices and insertions */
+    int32_t huge_stars;        /* star passes beyond the one-wave star kernels */
     int64_t num_missing;
     int64_t num_grid_pairs;    /* sort-unique Voronoi-neighbour pairs (one direction) */
     int64_t num_workset;       /* workset entries, both directions, after pumping */
