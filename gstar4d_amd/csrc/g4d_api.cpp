@@ -101,7 +101,7 @@ struct g4d_ctx {
     DevBuf xyz_up, keys, pts, perm, vox, bounds, settab, ptset, grid, gtmp, idgrid, pbaspill, pbaenv, pbacnt, pcount, pairs,
         ws_off, cnt;
     Store store;
-    DevBuf settet, drown, dflag, pairbuf, spcount, hkeys, dkeys, tasks, cand, keep, ins, ins_off, vcap, tcap, hcap, aflags, apos, active, mid, big, huge, xstars,
+    DevBuf settet, dflag, pairbuf, spcount, dkeys, tasks, cand, ins, ins_off, vcap, tcap, hcap, active, mid, big, huge, xstars,
         xtasks, xtris, gwork, tetcnt, tetoff, tets, opp, table;
     // learned proposal: parameters, candidates, features, proposed pairs, capacity bins, labels
     DevBuf mlp_params, fkeys, ford, frank, pcand, pd2, pfeat, ppairs, pcap, plab, pvcap;
@@ -111,7 +111,7 @@ struct g4d_ctx {
     PinnedBuf h_tets, h_opp, h_perm; // results of g4d_triangulate / g4d_triangulate_batch
     // Page-locked staging of the small reads back to the host (counters and counts): a pageable
     // destination makes the runtime stage every such read itself, about 8 us more per read.
-    // Slots 0..23 the counters, 24..39 scalars, 40..41 the primitives' counts.
+    // The counters first, then 16 scalars, then the primitives' two counts.
     PinnedBuf hpin;
     int64_t *hstage = nullptr; // in hpin, or the calling context's for a temporary context
     std::vector<int32_t> h_set_grid;
@@ -326,6 +326,10 @@ static double ev_ms(g4d_ctx *ctx, int a, int b)
     if (hipEventElapsedTime(&ms, ctx->ev[a], ctx->ev[b]) != hipSuccess) return 0.0;
     return ms;
 }
+
+// Counters of a pass's plan.
+static const uint64_t PLAN_COUNTERS = (1ull << G4D_CNT_ACTIVE) | (1ull << G4D_CNT_NEED_V) | (1ull << G4D_CNT_NEED_T) |
+                                      (1ull << G4D_CNT_NEED_H);
 
 // The whole path on device-resident FP64 points.
 // Point sets of one call (host side): set k holds points [pt_off[k], pt_off[k+1]) with grid
@@ -797,61 +801,47 @@ static int run_device(g4d_ctx *ctx, const double *d_xyz, int n, const SetSpec &s
     store.top[0] = store.top[1] = store.top[2] = 0;
     store.repacks = 0;
 
-    // One pass over the stars with insertions (mode 0: every star, from its workset).  Each
-    // such star gets a fresh region at the arenas' tops; the others are not touched.
-    auto star_pass = [&](int mode, const uint64_t *ins_keys, const int64_t *ins_off, int64_t nins, int64_t *drown_n,
-                         int64_t *tp_n) -> int {
-        const int *list = nullptr;
-        int nitems = n;
-        // sparse passes: the active list's length is known on the device first; the capacities
-        // and their scans run over the bound nins, and the length comes back with the needs
-        const int64_t *dev_na = nullptr;
-        int64_t na_f = 0, *na_h = hslot(ctx, 9, &na_f);
-        if (mode == 1 && nins < n / 2) {
-            // few insertions: offsets and active list from the runs of the sorted keys, O(keys)
-            // instead of O(stars)
-            HCK(ctx->active.ensure(sizeof(int) * (size_t)n));
-            HCK(ctx->hkeys.ensure(sizeof(uint64_t) * (size_t)std::max<int64_t>(nins, 1)));
-            HCK(P.sort_tmp_keys.ensure(sizeof(uint64_t) * (size_t)std::max<int64_t>(nins, 1)));
-            uint64_t *hk = buf<uint64_t>(ctx->hkeys);
-            HCK(g4d::launch_sparse_runs(ins_keys, nins, const_cast<int64_t *>(ins_off), hk, s));
-            uint64_t *runs = P.sort_tmp_keys.as<uint64_t>();
-            HCK(g4d::compact_valid_u64_deferred(P, hk, runs, nins, g4d::STAR_TASK_NONE, na_h, &dev_na, s));
-            HCK(g4d::launch_u64_to_i32(runs, nins, dev_na, buf<int>(ctx->active), s));
-            nitems = (int)nins; // bound until the needs come back
-            list = buf<int>(ctx->active);
-        } else if (mode == 1) {
-            HCK(g4d::launch_csr_offsets(ins_keys, nins, n, const_cast<int64_t *>(ins_off), s));
-            HCK(ctx->aflags.ensure(sizeof(uint32_t) * (size_t)n));
-            HCK(ctx->apos.ensure(sizeof(uint32_t) * (size_t)n));
-            HCK(ctx->active.ensure(sizeof(int) * (size_t)n));
-            uint32_t *fl = buf<uint32_t>(ctx->aflags), *pos = buf<uint32_t>(ctx->apos);
-            HCK(g4d::launch_active_flags(ins_off, n, fl, s));
-            HCK(g4d::scan_excl_u32(P, fl, pos, n, s));
-            HCK(g4d::launch_active_scatter(fl, pos, n, buf<int>(ctx->active), s));
-            int64_t last_f = 0, *last_h = hslot(ctx, 2, &last_f);
-            uint32_t *last = reinterpret_cast<uint32_t *>(last_h);
-            HCK(hipMemcpyAsync(&last[0], pos + n - 1, 4, hipMemcpyDeviceToHost, s));
-            HCK(hipMemcpyAsync(&last[1], fl + n - 1, 4, hipMemcpyDeviceToHost, s));
-            HCK(hipStreamSynchronize(s));
-            nitems = (int)(last[0] + last[1]);
-            list = buf<int>(ctx->active);
-        }
-        HCK(ctx->spcount.ensure(sizeof(int) * (size_t)n));
-        int *spc = buf<int>(ctx->spcount);
-        HCK(g4d::launch_capacities(list, nitems, dev_na, mode ? buf<int>(store.vnum) : nullptr,
-                                   mode ? buf<int>(store.hnum) : nullptr, ins_off, vcap, tcap, hcap, spc, s));
-        int64_t need[3] = {0, 0, 0};
-        int64_t *caps[3] = {vcap, tcap, hcap};
-        int64_t *need_h = hslot(ctx, 3, need); // three slots
-        for (int k = 0; k < 3; k++) {
-            HCK(g4d::scan_excl_i64(P, caps[k], caps[k], nitems, caps[k] + nitems, s));
-            HCK(hipMemcpyAsync(&need_h[k], caps[k] + nitems, 8, hipMemcpyDeviceToHost, s));
-        }
-        HCK(hipStreamSynchronize(s));
-        for (int k = 0; k < 3; k++) need[k] = need_h[k];
-        if (dev_na) nitems = (int)*na_h;
+    HCK(ctx->spcount.ensure(sizeof(int) * (size_t)n));
+    int *spc = buf<int>(ctx->spcount);
+    HCK(ctx->active.ensure(sizeof(int) * (size_t)n));
+    int *active = buf<int>(ctx->active);
+    HCK(ctx->ins_off.ensure(sizeof(int64_t) * (size_t)(n + 1)));
+    // splaying: the next pass's plan (regions from the arenas' tops as they are when it is launched)
+    auto pass_plan = [&]() {
+        g4d::PassPlan pl;
+        for (int k = 0; k < 3; k++) pl.base[k] = store.top[k];
+        pl.vnum = buf<int>(store.vnum);
+        pl.hnum = buf<int>(store.hnum);
+        pl.ins_off = buf<int64_t>(ctx->ins_off);
+        pl.list = active;
+        pl.nvoff = buf<int64_t>(store.nvoff);
+        pl.ntoff = buf<int64_t>(store.ntoff);
+        pl.nhoff = buf<int64_t>(store.nhoff);
+        pl.pcount = spc;
+        pl.cnt = cnt;
+        return pl;
+    };
+    int64_t tbase_last = 0;
+
+    // One pass over the stars with insertions (mode 0: every star, from its workset; mode 1: the
+    // nitems stars of the active list, whose regions of need[] elements are planned).  Each such
+    // star gets a fresh region at the arenas' tops; the others are not touched.  Returns the
+    // drowned insertions and the insertion pairs of the pass.
+    auto star_pass = [&](int mode, const uint64_t *ins_keys, const int64_t *ins_off, int64_t nins, int nitems,
+                         int64_t *need, int64_t *drown_n, int64_t *tp_n) -> int {
+        const int *list = mode ? active : nullptr;
         if (mode == 0) {
+            HCK(g4d::launch_capacities(n, ins_off, vcap, tcap, hcap, spc, s));
+            int64_t *caps[3] = {vcap, tcap, hcap};
+            int64_t *need_h = hslot(ctx, 3, need); // three slots
+            for (int k = 0; k < 3; k++) {
+                HCK(g4d::scan_excl_i64(P, caps[k], caps[k], n, caps[k] + n, s));
+                HCK(hipMemcpyAsync(&need_h[k], caps[k] + n, 8, hipMemcpyDeviceToHost, s));
+            }
+            HCK(g4d::launch_assign_regions(n, vcap, tcap, hcap, buf<int64_t>(store.nvoff), buf<int64_t>(store.ntoff),
+                                           buf<int64_t>(store.nhoff), s));
+            HCK(hipStreamSynchronize(s));
+            for (int k = 0; k < 3; k++) need[k] = need_h[k];
             // room for the splaying rounds: their regions come to about twice the creation's;
             // with the proposal's predicted link sizes, room for that many rebuilt stars too
             int64_t want[3] = {3 * need[0], 3 * need[1], 3 * need[2]};
@@ -864,21 +854,19 @@ static int run_device(g4d_ctx *ctx, const double *d_xyz, int n, const SetSpec &s
                 HCK(store.arena[k].ensure(Store::esz[k] * (size_t)std::max<int64_t>(want[k], 1024)));
         } else if (store.top[0] + need[0] > store.capacity(0) || store.top[1] + need[1] > store.capacity(1) ||
                    store.top[2] + need[2] > store.capacity(2)) {
+            // new arenas, new tops: plan again from the same keys
             CK(repack_store(ctx, n, need));
+            HCK(g4d::launch_zero_counters(cnt, PLAN_COUNTERS, s));
+            HCK(g4d::launch_pass_plan(pass_plan(), ins_keys, nins, nullptr, s));
         }
-        HCK(g4d::launch_assign_regions(list, nitems, vcap, tcap, hcap, store.top[0], store.top[1], store.top[2],
-                                       buf<int64_t>(store.nvoff), buf<int64_t>(store.ntoff), buf<int64_t>(store.nhoff),
-                                       s));
         const int64_t tbase = store.top[1];
+        tbase_last = tbase;
         for (int k = 0; k < 3; k++) store.top[k] += need[k];
         const int64_t dcap = std::max<int64_t>(nins, 1);
         const int64_t npb = 2 * need[1];
         CK(guard_keys(ctx, std::max(npb, nins), "star pass outputs"));
-        const int64_t tpcap = npb + 4 * dcap + 64;
-        HCK(ctx->drown.ensure(sizeof(uint64_t) * (size_t)dcap));
-        HCK(ctx->dflag.ensure((size_t)dcap));
+        HCK(ctx->dflag.ensure(((size_t)dcap + 15) & ~(size_t)15)); // read 16 flags at a time
         HCK(ctx->pairbuf.ensure(sizeof(uint64_t) * (size_t)std::max<int64_t>(npb, 1)));
-        HCK(ctx->cand.ensure(sizeof(uint64_t) * (size_t)tpcap));
         g4d::StarParams sp;
         memset(&sp, 0, sizeof(sp));
         sp.pts = pts;
@@ -911,12 +899,14 @@ static int run_device(g4d_ctx *ctx, const double *d_xyz, int n, const SetSpec &s
         sp.exact_cap = n;
         sp.exact_counter = G4D_CNT_APPEND4;
         sp.t0_variant = ctx->star_t0_variant;
-        // list counters, filter counts and the work-queue heads of this pass, in one launch
+        // list counters, totals and work-queue heads of this pass, and the lists made after it
         {
-            uint32_t zmask = (1u << G4D_CNT_APPEND2) | (1u << G4D_CNT_APPEND3) | (1u << G4D_CNT_APPEND4) |
-                             (1u << G4D_CNT_APPEND6) | (1u << G4D_CNT_XMID) | (1u << G4D_CNT_XBIG) |
-                             (1u << G4D_CNT_XL) | (1u << G4D_CNT_ORIENT4) | (1u << G4D_CNT_COFACTOR);
-            for (int q = 0; q < 7; q++) zmask |= 1u << (G4D_CNT_QUEUE0 + q);
+            uint64_t zmask = PLAN_COUNTERS;
+            for (int c : {G4D_CNT_APPEND2, G4D_CNT_APPEND3, G4D_CNT_APPEND4, G4D_CNT_APPEND5, G4D_CNT_APPEND6, G4D_CNT_XMID,
+                          G4D_CNT_XBIG, G4D_CNT_XL, G4D_CNT_ORIENT4, G4D_CNT_COFACTOR, G4D_CNT_PAIRS, G4D_CNT_DROWNED,
+                          G4D_CNT_DROWN_KEYS, G4D_CNT_TASKS, G4D_CNT_NEW_PAIRS, G4D_CNT_INS})
+                zmask |= 1ull << c;
+            for (int q = 0; q < 7; q++) zmask |= 1ull << (G4D_CNT_QUEUE0 + q);
             HCK(g4d::launch_zero_counters(cnt, zmask, s));
         }
         int queue = G4D_CNT_QUEUE0;
@@ -984,7 +974,7 @@ static int run_device(g4d_ctx *ctx, const double *d_xyz, int n, const SetSpec &s
             int64_t nglobal = nhuge;
             if (lds_limit == g4d::STAR_LDS_LIMIT) {
                 const int q = G4D_CNT_QUEUE0;
-                HCK(g4d::launch_zero_counters(cnt, (1u << G4D_CNT_XMID) | (1u << G4D_CNT_XBIG) | (1u << q) | (2u << q), s));
+                HCK(g4d::launch_zero_counters(cnt, (1ull << G4D_CNT_XMID) | (1ull << G4D_CNT_XBIG) | (3ull << q), s));
                 glist = buf<int>(ctx->mid);
                 sp.exact_list = glist;
                 sp.exact_counter = G4D_CNT_XMID;
@@ -1020,50 +1010,49 @@ static int run_device(g4d_ctx *ctx, const double *d_xyz, int n, const SetSpec &s
             }
         }
         CK(check_dev_error(ctx, hc[G4D_CNT_ERROR], mode ? "splaying" : "star creation"));
-        // drowned insertions and triangle pairs, in star order (both counts read back together)
-        int64_t cnt_f[2] = {0, 0}, *cnt_h = hslot(ctx, 6, cnt_f); // two slots
-        HCK(g4d::compact_u64_deferred(P, ins_keys, buf<uint8_t>(ctx->dflag), buf<uint64_t>(ctx->drown), nins,
-                                      &cnt_h[0], s));
-        // each star wrote its pairs densely at the front of its region and their count: offsets
-        // in list order (the vertex capacities are done with), then one copy per star
-        HCK(g4d::launch_pair_counts(list, nitems, spc, vcap, s));
-        HCK(g4d::scan_excl_i64(P, vcap, vcap, nitems, vcap + nitems, s));
-        HCK(hipMemcpyAsync(&cnt_h[1], vcap + nitems, 8, hipMemcpyDeviceToHost, s));
-        HCK(hipStreamSynchronize(s));
-        *drown_n = cnt_h[0];
-        const int64_t npairs = cnt_h[1];
-        if (npairs > npb) return set_err(ctx, G4D_ERR_INTERNAL, "star pairs exceed their regions");
-        HCK(g4d::launch_pair_gather(list, nitems, spc, vcap, buf<int64_t>(store.ntoff), tbase,
-                                    buf<uint64_t>(ctx->pairbuf), buf<uint64_t>(ctx->cand), s));
-        *tp_n = npairs;
+        *drown_n = (int64_t)hc[G4D_CNT_DROWNED];
+        *tp_n = (int64_t)hc[G4D_CNT_PAIRS];
+        if (*tp_n > npb) return set_err(ctx, G4D_ERR_INTERNAL, "star pairs exceed their regions");
         trace("star pass mode %d: %lld insertions into %d stars, over 32: %lld, over 64: %lld, exact %lld, "
-              "global-memory %lld, drowned %lld, pairs %lld",
+              "beyond 256 %lld, drowned %lld, pairs %lld",
               mode, (long long)nins, nitems, (long long)nmid, (long long)nbig, (long long)nexact, (long long)nhuge,
               (long long)*drown_n, (long long)*tp_n);
         return G4D_OK;
     };
 
-    int64_t nd = 0, ntp = 0;
-    CK(star_pass(0, pr, ws_off, m, &nd, &ntp));
+    int64_t nd = 0, ntp = 0, need[3] = {0, 0, 0};
+    const uint64_t *pass_keys = pr; // the last pass's insertions, and its stars
+    int64_t pass_n = m;
+    const int *pass_list = nullptr;
+    int pass_items = n;
+    CK(star_pass(0, pr, ws_off, m, n, need, &nd, &ntp));
     ev_record(ctx, EV_STAR);
 
     // ---- F: splaying rounds (GD/GDelaunay/GDelHost.cu:1389-1470) ----
+    // Between two passes the host waits once where the round is small (k_small_round planned the next
+    // pass by then), twice where it sorts longer lists, and once more where the proofs' count
+    // sizes large buffers.
     int rounds = 0;
     bool converged = false;
     for (int it = 0; it < ctx->opt.max_rounds; it++) {
         // F1-F3: drowned insertions, mutual removal, containment proofs
-        int64_t ntask = 0;
+        int64_t ntask = 0; // bound
         if (nd > 0) {
             CK(guard_keys(ctx, nd, "drowned insertions"));
             HCK(ctx->dkeys.ensure(sizeof(uint64_t) * (size_t)nd));
             HCK(ctx->tasks.ensure(sizeof(uint64_t) * (size_t)nd));
             uint64_t *dk = buf<uint64_t>(ctx->dkeys);
-            HCK(g4d::launch_drown_keys(buf<uint64_t>(ctx->drown), nd, dk, s));
+            HCK(g4d::launch_drown_keys(pass_keys, buf<uint8_t>(ctx->dflag), pass_n, dk, cnt, s));
             HCK(g4d::sort_keys_ab(P, dk, nd, 33, nb, 1 + nb, n, false, s));
-            HCK(g4d::launch_nonmutual(dk, nd, buf<uint64_t>(ctx->tasks), s));
-            HCK(g4d::compact_valid_u64(P, buf<uint64_t>(ctx->tasks), buf<uint64_t>(ctx->tasks), nd,
-                                       g4d::STAR_TASK_NONE, &ntask, s));
+            HCK(g4d::launch_nonmutual(dk, nd, buf<uint64_t>(ctx->tasks), cnt, s));
+            ntask = nd;
+            if (nd > (1 << 16)) { // the proofs' and the insertions' buffers by the count itself
+                CK(read_counters(ctx, hc));
+                ntask = (int64_t)hc[G4D_CNT_TASKS];
+            }
             if (ntask > 0) {
+                HCK(ctx->xtasks.ensure(sizeof(int64_t) * (size_t)ntask));
+                HCK(ctx->cand.ensure(sizeof(uint64_t) * 4 * (size_t)ntask));
                 g4d::ProofParams pp;
                 pp.pts = pts;
                 pp.tasks = buf<uint64_t>(ctx->tasks);
@@ -1074,52 +1063,72 @@ static int run_device(g4d_ctx *ctx, const double *d_xyz, int n, const SetSpec &s
                 pp.tnum = buf<int>(store.tnum);
                 pp.toff = buf<int64_t>(store.toff);
                 pp.tpool = buf<uint64_t>(store.arena[1]);
-                pp.out = buf<uint64_t>(ctx->cand) + ntp;
+                pp.out = buf<uint64_t>(ctx->cand);
                 pp.cnt = cnt;
-                HCK(ctx->xtasks.ensure(sizeof(int64_t) * (size_t)ntask));
                 pp.xlist = buf<int64_t>(ctx->xtasks);
                 pp.xcap = ntask;
-                pp.nx = 0;
-                HCK(hipMemsetAsync(cnt + G4D_CNT_APPEND5, 0, 8, s));
                 HCK(g4d::launch_proofs(pp, false, s));
-                pp.nx = -1; // the exact pass reads the filter pass's count on the device
-                HCK(g4d::launch_proofs(pp, true, s));
+                HCK(g4d::launch_proofs(pp, true, s)); // reads the filter pass's count on the device
             }
         }
-        // F4-F5: candidates = triangle pairs + proofs, history filter, sort-unique
+        // F4-F9: candidates = triangle pairs + proofs; those new to the histories, both directions,
+        // sorted without repeats; offsets, stars and regions of the next pass
         const int64_t ncand = ntp + 4 * ntask;
-        int64_t nins = 0;
+        int64_t nrec = 0;
         if (ncand > 0) {
             CK(guard_keys(ctx, 2 * ncand, "splaying candidates"));
-            HCK(ctx->keep.ensure((size_t)ncand));
             HCK(ctx->ins.ensure(sizeof(uint64_t) * (size_t)(2 * ncand + 2)));
             uint64_t *ins = buf<uint64_t>(ctx->ins);
-            HCK(g4d::launch_hist_filter(buf<uint64_t>(ctx->cand), ncand, buf<int>(store.arena[2]),
-                                        buf<int64_t>(store.hoff), buf<int>(store.hnum), buf<uint8_t>(ctx->keep), s));
-            HCK(g4d::compact_u64(P, buf<uint64_t>(ctx->cand), buf<uint8_t>(ctx->keep), ins, ncand, &nins, s));
-            if (nins > 0) {
-                HCK(sort_unique_pairs(P, ins, &nins, nb, n, s));
-            }
-        }
-        trace("round %d: %lld drowned, %lld proofs, %lld candidates, %lld new pairs", rounds + 1, (long long)nd,
-              (long long)ntask, (long long)ncand, (long long)nins);
-        if (nins == 0) {
-            // the proofs' errors; otherwise the star pass below reads them with its own counters
+            g4d::NewPairs np;
+            np.list = pass_list;
+            np.nitems = pass_items;
+            np.pcount = spc;
+            np.ntoff = buf<int64_t>(store.ntoff);
+            np.tbase = tbase_last;
+            np.pairbuf = buf<uint64_t>(ctx->pairbuf);
+            np.proofs = buf<uint64_t>(ctx->cand);
+            np.ntasks = ntask;
+            np.hpool = buf<int>(store.arena[2]);
+            np.hoff = buf<int64_t>(store.hoff);
+            np.hnum = buf<int>(store.hnum);
+            np.keys = ins;
+            np.cnt = cnt;
+            HCK(g4d::launch_new_pairs(np, s));
+            HCK(g4d::launch_small_round(pass_plan(), ins, s));
             CK(read_counters(ctx, hc));
+            const int64_t mk = 2 * (int64_t)hc[G4D_CNT_NEW_PAIRS];
+            if (mk > g4d::STAR_ROUND_SMALL) {
+                int64_t nrec_f = 0, *nrec_h = hslot(ctx, 9, &nrec_f);
+                const int64_t *dev_m = nullptr;
+                HCK(g4d::sort_unique_pair_keys_deferred(P, ins, mk, nb, n, nrec_h, &dev_m, s));
+                HCK(g4d::launch_pass_plan(pass_plan(), ins, dev_m ? mk : *nrec_h, dev_m, s));
+                CK(read_counters(ctx, hc));
+                nrec = *nrec_h;
+            } else {
+                nrec = (int64_t)hc[G4D_CNT_INS];
+            }
+        } else {
+            CK(read_counters(ctx, hc));
+        }
+        trace("round %d: %lld drowned, %lld proofs, %lld pairs, %lld new with repeats, %lld insertions", rounds + 1,
+              (long long)nd, (long long)hc[G4D_CNT_TASKS], (long long)ntp, (long long)hc[G4D_CNT_NEW_PAIRS],
+              (long long)nrec);
+        if (nrec == 0) {
+            // the proofs' errors; otherwise the star pass below reads them with its own counters
             CK(check_dev_error(ctx, hc[G4D_CNT_ERROR], "proofs"));
             converged = true;
             break;
         }
         rounds++;
-        // F6-F9: reciprocate, group by star, insert
-        uint64_t *ins = buf<uint64_t>(ctx->ins);
-        HCK(g4d::launch_reciprocate(ins, nins, s));
-        const int64_t nrec = 2 * nins;
-        HCK(sort_pairs(P, ins, nrec, nb, n, s));
         ctx->st.splay_insertions += nrec;
-        HCK(ctx->ins_off.ensure(sizeof(int64_t) * (size_t)(n + 1)));
-        int64_t *ioff = buf<int64_t>(ctx->ins_off);
-        CK(star_pass(1, ins, ioff, nrec, &nd, &ntp)); // builds the offsets of the stars with insertions
+        pass_keys = buf<uint64_t>(ctx->ins);
+        pass_n = nrec;
+        pass_list = active;
+        pass_items = (int)hc[G4D_CNT_ACTIVE];
+        need[0] = (int64_t)hc[G4D_CNT_NEED_V];
+        need[1] = (int64_t)hc[G4D_CNT_NEED_T];
+        need[2] = (int64_t)hc[G4D_CNT_NEED_H];
+        CK(star_pass(1, pass_keys, buf<int64_t>(ctx->ins_off), nrec, pass_items, need, &nd, &ntp));
     }
     if (!converged) return set_err(ctx, G4D_ERR_NOT_CONVERGED, "splaying did not converge in %d rounds", rounds);
     ctx->st.splay_rounds = rounds;
@@ -1293,9 +1302,9 @@ void g4d_destroy(g4d_ctx *ctx)
     (void)hipSetDevice(ctx->opt.device);
     if (ctx->stream) (void)hipStreamSynchronize(ctx->stream);
     DevBuf *bufs[] = {&ctx->xyz_up, &ctx->keys, &ctx->pts, &ctx->perm, &ctx->vox, &ctx->bounds, &ctx->settab, &ctx->ptset, &ctx->grid,
-                      &ctx->gtmp, &ctx->idgrid, &ctx->pbaspill, &ctx->pbaenv, &ctx->pbacnt, &ctx->pcount, &ctx->pairs, &ctx->ws_off, &ctx->cnt, &ctx->settet, &ctx->drown, &ctx->dflag, &ctx->pairbuf, &ctx->spcount, &ctx->hkeys, &ctx->dkeys,
-                      &ctx->tasks, &ctx->cand, &ctx->keep, &ctx->ins, &ctx->ins_off, &ctx->vcap, &ctx->tcap,
-                      &ctx->hcap, &ctx->aflags, &ctx->apos, &ctx->active, &ctx->mid, &ctx->big, &ctx->huge, &ctx->xstars, &ctx->xtasks, &ctx->xtris, &ctx->gwork, &ctx->tetcnt, &ctx->tetoff, &ctx->tets, &ctx->opp, &ctx->table,
+                      &ctx->gtmp, &ctx->idgrid, &ctx->pbaspill, &ctx->pbaenv, &ctx->pbacnt, &ctx->pcount, &ctx->pairs, &ctx->ws_off, &ctx->cnt, &ctx->settet, &ctx->dflag, &ctx->pairbuf, &ctx->spcount, &ctx->dkeys,
+                      &ctx->tasks, &ctx->cand, &ctx->ins, &ctx->ins_off, &ctx->vcap, &ctx->tcap,
+                      &ctx->hcap, &ctx->active, &ctx->mid, &ctx->big, &ctx->huge, &ctx->xstars, &ctx->xtasks, &ctx->xtris, &ctx->gwork, &ctx->tetcnt, &ctx->tetoff, &ctx->tets, &ctx->opp, &ctx->table,
                       &ctx->mlp_params, &ctx->fkeys, &ctx->ford, &ctx->frank, &ctx->pcand, &ctx->pd2, &ctx->pfeat,
                       &ctx->ppairs, &ctx->pcap, &ctx->plab, &ctx->pvcap};
     destroy_graphs(ctx);

@@ -60,7 +60,18 @@ enum g4d_counter : int {
     G4D_CNT_XMID = 15,     // list lengths of the exact chain's 64- and 256-vertex tiers
     G4D_CNT_XBIG = 16,
     G4D_CNT_QUEUE0 = 17,   // work-queue heads of the star-kernel launches of one pass (17..23)
-    G4D_CNT_NUM = 24
+    // a star pass's totals (added by its kernels) and the splaying lists made of them
+    G4D_CNT_PAIRS = 24,    // insertion pairs the pass wrote
+    G4D_CNT_DROWNED = 25,  // insertions it drowned
+    G4D_CNT_DROWN_KEYS = 26,
+    G4D_CNT_TASKS = 27,    // containment proofs to find
+    G4D_CNT_NEW_PAIRS = 28, // pairs the histories do not hold, with repeats
+    G4D_CNT_INS = 29,      // distinct insertions (two per pair)
+    G4D_CNT_ACTIVE = 30,   // stars with insertions, and the region sizes they need
+    G4D_CNT_NEED_V = 31,
+    G4D_CNT_NEED_T = 32,
+    G4D_CNT_NEED_H = 33,
+    G4D_CNT_NUM = 34
 };
 
 #define HIP_CHECK_RET(expr)                                                                    \

@@ -115,6 +115,11 @@ hipError_t sort_pair_keys(Prims &P, uint64_t *keys, int64_t m, int nb, int64_t n
 // compacted from the sort's scratch buffer straight into keys.  keys must not be P.sort_tmp_keys.
 hipError_t sort_unique_pair_keys(Prims &P, uint64_t *keys, int64_t m, int nb, int64_t nids, int64_t *m_out,
                                  hipStream_t s);
+// sort_unique_pair_keys without the host synchronisation: the count at *dev_count on the device
+// (int64, valid until the next compaction) and, once the stream reaches it, at *host_count
+// (page-locked).  Lists the bucket sort does not take come back synchronised, *dev_count null.
+hipError_t sort_unique_pair_keys_deferred(Prims &P, uint64_t *keys, int64_t m, int nb, int64_t nids, int64_t *host_count,
+                                          const int64_t **dev_count, hipStream_t s);
 // Bucket shift sort_pair_keys uses for m keys (buckets of 2^shift ids), -1 for the LSD sort.
 int pair_sort_shift(int64_t m, int nb, int64_t nids);
 // The same sort for keys a << ash | b with a < 2^na, b < 2^nbb and zeros between (nbb <= ash):
@@ -131,19 +136,6 @@ hipError_t merge_u64(const uint64_t *a, int64_t na, const uint64_t *b, int64_t n
 hipError_t unique_u64(Prims &P, uint64_t *keys, int64_t n, int64_t *n_out, hipStream_t s);
 // The same from in to out (distinct buffers; in may be P.sort_tmp_keys).
 hipError_t unique_copy_u64(Prims &P, const uint64_t *in, uint64_t *out, int64_t n, int64_t *n_out, hipStream_t s);
-
-// Order-preserving compaction keep[i] != 0.  Count returned via host sync.
-// compact_u64 without the host synchronisation (in and out distinct): the count is copied to
-// *host_count (page-locked memory, or the copy blocks) once the stream reaches it.
-hipError_t compact_u64_deferred(Prims &P, const uint64_t *in, const uint8_t *keep, uint64_t *out, int64_t n,
-                                int64_t *host_count, hipStream_t s);
-// compact_valid_u64 from in to a distinct out without the host synchronisation (n > 0): the
-// count at *dev_count on the device (int64, valid until the next compaction) and, once the
-// stream reaches it, at *host_count (page-locked).
-hipError_t compact_valid_u64_deferred(Prims &P, const uint64_t *in, uint64_t *out, int64_t n, uint64_t none,
-                                      int64_t *host_count, const int64_t **dev_count, hipStream_t s);
-hipError_t compact_u64(Prims &P, const uint64_t *in, const uint8_t *keep, uint64_t *out, int64_t n,
-                       int64_t *n_out, hipStream_t s);
 
 // Order-preserving compaction of the entries different from `none`.  Count via host sync.
 hipError_t compact_valid_u64(Prims &P, const uint64_t *in, uint64_t *out, int64_t n, uint64_t none,

@@ -840,11 +840,11 @@ hipError_t merge_u64(const uint64_t *a, int64_t na, const uint64_t *b, int64_t n
 // Lists up to SMALL_COMPACT entries are compacted by one work-group in a single launch
 // (tiles of 1024 in order, ballot ranks, a running offset), which also works in place: an
 // entry kept from index j lands at a position <= j, and later tiles read beyond every
-// position written so far.  MODE 0: adjacent-unique, 1: keep[i] != 0, 2: in[i] != none.
+// position written so far.  MODE 0: adjacent-unique, 2: in[i] != none.
 static constexpr int64_t SMALL_COMPACT = 32768;
 
 template <int MODE>
-__global__ void __launch_bounds__(1024) k_compact_small(const uint64_t *in, const uint8_t *keep, uint64_t none,
+__global__ void __launch_bounds__(1024) k_compact_small(const uint64_t *in, uint64_t none,
                                                         uint64_t *out, int64_t n, uint32_t *count)
 {
     __shared__ uint32_t wsum[16];
@@ -858,7 +858,6 @@ __global__ void __launch_bounds__(1024) k_compact_small(const uint64_t *in, cons
         if (i < n) {
             v = in[i];
             if (MODE == 0) f = i == 0 || v != (threadIdx.x == 0 ? last : in[i - 1]);
-            else if (MODE == 1) f = keep[i] != 0;
             else f = v != none;
         }
         const uint64_t m = __ballot(f);
@@ -883,12 +882,12 @@ __global__ void __launch_bounds__(1024) k_compact_small(const uint64_t *in, cons
 }
 
 template <int MODE>
-static hipError_t compact_small(Prims &P, const uint64_t *in, const uint8_t *keep, uint64_t none, uint64_t *out,
+static hipError_t compact_small(Prims &P, const uint64_t *in, uint64_t none, uint64_t *out,
                                 int64_t n, int64_t *n_out, hipStream_t s)
 {
     HIP_CHECK_RET(P.pos.ensure(sizeof(uint32_t) * 4));
     uint32_t *dcount = P.pos.as<uint32_t>();
-    hipLaunchKernelGGL(k_compact_small<MODE>, dim3(1), dim3(1024), 0, s, in, keep, none, out, n, dcount);
+    hipLaunchKernelGGL(k_compact_small<MODE>, dim3(1), dim3(1024), 0, s, in, none, out, n, dcount);
     HIP_CHECK_RET(hipGetLastError());
     uint32_t c = 0;
     uint32_t *hc = P.hstage ? reinterpret_cast<uint32_t *>(P.hstage) : &c;
@@ -905,16 +904,15 @@ static constexpr int CMP_ROUNDS = 16;
 static constexpr int CMP_TILE = 256 * CMP_ROUNDS;
 
 template <int MODE>
-__device__ __forceinline__ bool cmp_keep(const uint64_t *in, const uint8_t *keep, uint64_t none, int64_t i,
+__device__ __forceinline__ bool cmp_keep(const uint64_t *in, uint64_t none, int64_t i,
                                          uint64_t v)
 {
     if (MODE == 0) return i == 0 || v != in[i - 1];
-    if (MODE == 1) return keep[i] != 0;
     return v != none;
 }
 
 template <int MODE>
-__global__ void __launch_bounds__(256) k_cmp_count(const uint64_t *in, const uint8_t *keep, uint64_t none, int64_t n,
+__global__ void __launch_bounds__(256) k_cmp_count(const uint64_t *in, uint64_t none, int64_t n,
                                                    int64_t *tile_cnt)
 {
     __shared__ uint32_t wsum[4];
@@ -923,7 +921,7 @@ __global__ void __launch_bounds__(256) k_cmp_count(const uint64_t *in, const uin
 #pragma unroll 4
     for (int r = 0; r < CMP_ROUNDS; r++) {
         const int64_t i = t0 + r * 256 + threadIdx.x;
-        if (i < n) c += cmp_keep<MODE>(in, keep, none, i, in[i]) ? 1u : 0u;
+        if (i < n) c += cmp_keep<MODE>(in, none, i, in[i]) ? 1u : 0u;
     }
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) c += __shfl_xor(c, o, 64);
@@ -933,7 +931,7 @@ __global__ void __launch_bounds__(256) k_cmp_count(const uint64_t *in, const uin
 }
 
 template <int MODE>
-__global__ void __launch_bounds__(256) k_cmp_write(const uint64_t *in, const uint8_t *keep, uint64_t none, int64_t n,
+__global__ void __launch_bounds__(256) k_cmp_write(const uint64_t *in, uint64_t none, int64_t n,
                                                    const int64_t *tile_off, uint64_t *out)
 {
     __shared__ uint32_t wsum[4];
@@ -946,7 +944,7 @@ __global__ void __launch_bounds__(256) k_cmp_write(const uint64_t *in, const uin
         bool f = false;
         if (i < n) {
             v = in[i];
-            f = cmp_keep<MODE>(in, keep, none, i, v);
+            f = cmp_keep<MODE>(in, none, i, v);
         }
         const uint64_t m = __ballot(f);
         if (lane == 0) wsum[wid] = (uint32_t)__popcll(m);
@@ -965,14 +963,14 @@ __global__ void __launch_bounds__(256) k_cmp_write(const uint64_t *in, const uin
 }
 
 template <int MODE>
-static hipError_t compact_big(Prims &P, const uint64_t *in, const uint8_t *keep, uint64_t none, uint64_t *out,
+static hipError_t compact_big(Prims &P, const uint64_t *in, uint64_t none, uint64_t *out,
                               int64_t n, int64_t *n_out, hipStream_t s)
 {
     const int64_t nt = (n + CMP_TILE - 1) / CMP_TILE;
     if (nt > INT32_MAX) return hipErrorInvalidValue;
     HIP_CHECK_RET(P.flags.ensure(sizeof(int64_t) * (size_t)(nt + 1)));
     int64_t *tc = P.flags.as<int64_t>();
-    hipLaunchKernelGGL(k_cmp_count<MODE>, dim3((unsigned)nt), dim3(256), 0, s, in, keep, none, n, tc);
+    hipLaunchKernelGGL(k_cmp_count<MODE>, dim3((unsigned)nt), dim3(256), 0, s, in, none, n, tc);
     HIP_CHECK_RET(hipGetLastError());
     HIP_CHECK_RET(scan_excl_i64(P, tc, tc, nt, tc + nt, s));
     uint64_t *dst = out;
@@ -981,7 +979,7 @@ static hipError_t compact_big(Prims &P, const uint64_t *in, const uint8_t *keep,
         HIP_CHECK_RET(P.sort_tmp_keys.ensure(sizeof(uint64_t) * (size_t)n));
         dst = P.sort_tmp_keys.as<uint64_t>();
     }
-    hipLaunchKernelGGL(k_cmp_write<MODE>, dim3((unsigned)nt), dim3(256), 0, s, in, keep, none, n, tc, dst);
+    hipLaunchKernelGGL(k_cmp_write<MODE>, dim3((unsigned)nt), dim3(256), 0, s, in, none, n, tc, dst);
     HIP_CHECK_RET(hipGetLastError());
     int64_t m = 0;
     int64_t *hm = P.hstage ? P.hstage : &m;
@@ -997,7 +995,7 @@ static hipError_t compact_big(Prims &P, const uint64_t *in, const uint8_t *keep,
 // on the device at *dev_count (int64; valid until the next compaction) and, once the stream
 // reaches it, at *host_count (page-locked memory, or the copy blocks).
 template <int MODE>
-static hipError_t compact_deferred(Prims &P, const uint64_t *in, const uint8_t *keep, uint64_t none, uint64_t *out,
+static hipError_t compact_deferred(Prims &P, const uint64_t *in, uint64_t none, uint64_t *out,
                                    int64_t n, int64_t *host_count, const int64_t **dev_count, hipStream_t s)
 {
     *host_count = 0;
@@ -1005,7 +1003,7 @@ static hipError_t compact_deferred(Prims &P, const uint64_t *in, const uint8_t *
     if (n <= SMALL_COMPACT) {
         HIP_CHECK_RET(P.pos.ensure(sizeof(uint32_t) * 4));
         uint32_t *dcount = P.pos.as<uint32_t>();
-        hipLaunchKernelGGL(k_compact_small<MODE>, dim3(1), dim3(1024), 0, s, in, keep, none, out, n, dcount);
+        hipLaunchKernelGGL(k_compact_small<MODE>, dim3(1), dim3(1024), 0, s, in, none, out, n, dcount);
         HIP_CHECK_RET(hipGetLastError());
         if (dev_count) *dev_count = reinterpret_cast<const int64_t *>(dcount);
         return hipMemcpyAsync(host_count, dcount, 8, hipMemcpyDeviceToHost, s);
@@ -1014,29 +1012,23 @@ static hipError_t compact_deferred(Prims &P, const uint64_t *in, const uint8_t *
     if (nt > INT32_MAX) return hipErrorInvalidValue;
     HIP_CHECK_RET(P.flags.ensure(sizeof(int64_t) * (size_t)(nt + 1)));
     int64_t *tc = P.flags.as<int64_t>();
-    hipLaunchKernelGGL(k_cmp_count<MODE>, dim3((unsigned)nt), dim3(256), 0, s, in, keep, none, n, tc);
+    hipLaunchKernelGGL(k_cmp_count<MODE>, dim3((unsigned)nt), dim3(256), 0, s, in, none, n, tc);
     HIP_CHECK_RET(hipGetLastError());
     HIP_CHECK_RET(scan_excl_i64(P, tc, tc, nt, tc + nt, s));
-    hipLaunchKernelGGL(k_cmp_write<MODE>, dim3((unsigned)nt), dim3(256), 0, s, in, keep, none, n, tc, out);
+    hipLaunchKernelGGL(k_cmp_write<MODE>, dim3((unsigned)nt), dim3(256), 0, s, in, none, n, tc, out);
     HIP_CHECK_RET(hipGetLastError());
     if (dev_count) *dev_count = tc + nt;
     return hipMemcpyAsync(host_count, tc + nt, 8, hipMemcpyDeviceToHost, s);
 }
 
-hipError_t compact_u64_deferred(Prims &P, const uint64_t *in, const uint8_t *keep, uint64_t *out, int64_t n,
-                                int64_t *host_count, hipStream_t s)
+hipError_t sort_unique_pair_keys_deferred(Prims &P, uint64_t *keys, int64_t m, int nb, int64_t nids, int64_t *host_count,
+                                          const int64_t **dev_count, hipStream_t s)
 {
-    if (n <= 0) {
-        *host_count = 0;
-        return hipSuccess;
-    }
-    return compact_deferred<1>(P, in, keep, 0, out, n, host_count, nullptr, s);
-}
-
-hipError_t compact_valid_u64_deferred(Prims &P, const uint64_t *in, uint64_t *out, int64_t n, uint64_t none,
-                                      int64_t *host_count, const int64_t **dev_count, hipStream_t s)
-{
-    return compact_deferred<2>(P, in, nullptr, none, out, n, host_count, dev_count, s);
+    *dev_count = nullptr;
+    const int sb = key_sort_shift(m, nb, nb, nids, false);
+    if (m <= 1 || sb < 0) return sort_unique_pair_keys(P, keys, m, nb, nids, host_count, s);
+    HIP_CHECK_RET(bucket_sort(P, keys, m, 32, nb, nb, sb, nids, true, s));
+    return compact_deferred<0>(P, P.sort_tmp_keys.as<uint64_t>(), 0, keys, m, host_count, dev_count, s);
 }
 
 hipError_t unique_u64(Prims &P, uint64_t *keys, int64_t n, int64_t *n_out, hipStream_t s)
@@ -1045,8 +1037,8 @@ hipError_t unique_u64(Prims &P, uint64_t *keys, int64_t n, int64_t *n_out, hipSt
         *n_out = n;
         return hipSuccess;
     }
-    if (n <= SMALL_COMPACT) return compact_small<0>(P, keys, nullptr, 0, keys, n, n_out, s);
-    return compact_big<0>(P, keys, nullptr, 0, keys, n, n_out, s);
+    if (n <= SMALL_COMPACT) return compact_small<0>(P, keys, 0, keys, n, n_out, s);
+    return compact_big<0>(P, keys, 0, keys, n, n_out, s);
 }
 
 hipError_t unique_copy_u64(Prims &P, const uint64_t *in, uint64_t *out, int64_t n, int64_t *n_out, hipStream_t s)
@@ -1056,19 +1048,8 @@ hipError_t unique_copy_u64(Prims &P, const uint64_t *in, uint64_t *out, int64_t 
         return hipSuccess;
     }
     if (in == out) return hipErrorInvalidValue;
-    if (n <= SMALL_COMPACT) return compact_small<0>(P, in, nullptr, 0, out, n, n_out, s);
-    return compact_big<0>(P, in, nullptr, 0, out, n, n_out, s);
-}
-
-hipError_t compact_u64(Prims &P, const uint64_t *in, const uint8_t *keep, uint64_t *out, int64_t n, int64_t *n_out,
-                       hipStream_t s)
-{
-    if (n <= 0) {
-        *n_out = 0;
-        return hipSuccess;
-    }
-    if (n <= SMALL_COMPACT) return compact_small<1>(P, in, keep, 0, out, n, n_out, s);
-    return compact_big<1>(P, in, keep, 0, out, n, n_out, s);
+    if (n <= SMALL_COMPACT) return compact_small<0>(P, in, 0, out, n, n_out, s);
+    return compact_big<0>(P, in, 0, out, n, n_out, s);
 }
 
 hipError_t compact_valid_u64(Prims &P, const uint64_t *in, uint64_t *out, int64_t n, uint64_t none, int64_t *n_out,
@@ -1078,8 +1059,8 @@ hipError_t compact_valid_u64(Prims &P, const uint64_t *in, uint64_t *out, int64_
         *n_out = 0;
         return hipSuccess;
     }
-    if (n <= SMALL_COMPACT) return compact_small<2>(P, in, nullptr, none, out, n, n_out, s);
-    return compact_big<2>(P, in, nullptr, none, out, n, n_out, s);
+    if (n <= SMALL_COMPACT) return compact_small<2>(P, in, none, out, n, n_out, s);
+    return compact_big<2>(P, in, none, out, n, n_out, s);
 }
 
 } // namespace g4d

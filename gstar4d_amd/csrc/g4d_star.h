@@ -62,7 +62,8 @@ struct StarParams {
     const int64_t *ntoff;
     const int64_t *nhoff;
     // outputs without atomics (compacted by the host code after the pass)
-    uint8_t *dflag;       // per insertion, indexed like ins_keys: 1 when the vertex drowned
+    uint8_t *dflag;       // per insertion, indexed like ins_keys: 1 when the vertex drowned (total:
+                          // G4D_CNT_DROWNED; the pairs' total: G4D_CNT_PAIRS)
     uint64_t *pairbuf;    // per star, from 2 * (ntoff[s] - tbase): its insertion pairs (a<<32 | b,
     int64_t tbase;        // a < b) of unchecked triangles, dense, in triangle order
     int *pcount;          // per star: the number of those pairs
@@ -99,7 +100,7 @@ enum {
 // code, no private scratch), a star with an inconclusive orientation goes to p.exact_list
 // untouched.  exact = true: exact predicates and SoS, for the stars of star_list.
 // Zeroes the counter words whose bits are set in mask (one launch instead of one fill per word).
-hipError_t launch_zero_counters(unsigned long long *cnt, uint32_t mask, hipStream_t s);
+hipError_t launch_zero_counters(unsigned long long *cnt, uint64_t mask, hipStream_t s);
 hipError_t launch_star_kernel(const StarParams &p, int vmax, bool exact, int nblocks, hipStream_t s);
 // Wide LDS kernel, vmax = STAR_VMAX_W1 or W2, over the star_list whose length is at nlist_dev:
 // larger stars go to p.defer_list, inconclusive ones untouched to p.exact_list.
@@ -115,10 +116,9 @@ hipError_t launch_need_max(const StarParams &p, const int *list, int nitems, uns
 struct ProofParams {
     const double *pts;
     const uint64_t *tasks; // (star<<32 | vertex) drowned, non-mutual
-    int64_t ntasks;
+    int64_t ntasks;        // bound of the task count G4D_CNT_TASKS
     int64_t *xlist;       // filter-only pass: tasks needing exact predicates, counter G4D_CNT_APPEND5;
-    int64_t nx;           // exact pass: the task indices to redo (< 0: their count from the counter)
-    int64_t xcap;
+    int64_t xcap;          // entries it holds; the exact pass reads its length from the counter
     const int *vnum;
     const int64_t *voff;
     const int *vpool;
@@ -128,45 +128,68 @@ struct ProofParams {
     uint64_t *out;        // 4 pairs per task (a<<32|b, a<b)
     unsigned long long *cnt;
 };
-// exact = false: filter-only pass over all tasks; exact = true: the tasks in xlist[0, nx).
+// exact = false: filter-only pass over all tasks; exact = true: the tasks in xlist.
 hipError_t launch_proofs(const ProofParams &p, bool exact, hipStream_t s);
 
-// Drowned pairs -> keys (min<<33 | max<<1 | dir) for the mutual test.
-hipError_t launch_drown_keys(const uint64_t *drown, int64_t m, uint64_t *keys, hipStream_t s);
-// Sorted drowned keys -> tasks[i] = proof task (star<<32 | vertex), or STAR_TASK_NONE for a
-// mutual pair; compact the NONE entries away afterwards.
-static constexpr uint64_t STAR_TASK_NONE = ~0ull;
-hipError_t launch_nonmutual(const uint64_t *keys, int64_t m, uint64_t *tasks, hipStream_t s);
-// keep[i] = pair (a<<32|b) with a < b and b not in the history of star a.
-hipError_t launch_hist_filter(const uint64_t *pairs, int64_t m, const int *hpool, const int64_t *hoff, const int *hnum,
-                              uint8_t *keep, hipStream_t s);
+// Splaying lists between two star passes.  Each is consumed sorted, so its entries are appended in
+// any order, a tile's at a time, through a device counter.
+//
+// Keys (min<<33 | max<<1 | dir) of the insertions whose flag is set, for the mutual test (flags are
+// read 16 at a time: dflag holds a multiple of 16 bytes); counter G4D_CNT_DROWN_KEYS.
+hipError_t launch_drown_keys(const uint64_t *ins_keys, const uint8_t *dflag, int64_t m, uint64_t *keys,
+                             unsigned long long *cnt, hipStream_t s);
+// Sorted drowned keys -> proof tasks (star<<32 | vertex), the mutual pairs left out; counter
+// G4D_CNT_TASKS.
+hipError_t launch_nonmutual(const uint64_t *keys, int64_t m, uint64_t *tasks, unsigned long long *cnt, hipStream_t s);
+// Both directed keys of every pair (a<<32 | b, a < b) with b not in the history of star a, of the
+// last pass's stars (list = nullptr: stars 0..nitems-1) and of the proofs (four per task, tasks
+// counted at G4D_CNT_TASKS, at most ntasks); counter G4D_CNT_NEW_PAIRS (pairs).
+struct NewPairs {
+    const int *list;
+    int nitems;
+    const int *pcount;
+    const int64_t *ntoff;
+    int64_t tbase;
+    const uint64_t *pairbuf;
+    const uint64_t *proofs;
+    int64_t ntasks;
+    const int *hpool;
+    const int64_t *hoff;
+    const int *hnum;
+    uint64_t *keys;
+    unsigned long long *cnt;
+};
+hipError_t launch_new_pairs(const NewPairs &p, hipStream_t s);
+// The next pass's work from its sorted distinct insertion keys: CSR offsets of the stars with
+// insertions, their list (G4D_CNT_ACTIVE), and fresh regions for them from the arenas' tops base[]
+// (sizes at G4D_CNT_NEED_V / _T / _H).  pcount[s] = 0 for these stars.
+struct PassPlan {
+    int64_t base[3];
+    const int *vnum;
+    const int *hnum;
+    int64_t *ins_off;
+    int *list;
+    int64_t *nvoff;
+    int64_t *ntoff;
+    int64_t *nhoff;
+    int *pcount;
+    unsigned long long *cnt;
+};
+// m keys, or *dev_m (at most m) when dev_m is given.
+hipError_t launch_pass_plan(const PassPlan &p, const uint64_t *keys, int64_t m, const int64_t *dev_m, hipStream_t s);
+// Everything from the appended keys (twice G4D_CNT_NEW_PAIRS of them) to the plan in one launch of
+// one work-group: sort, removal of repeats (the count at G4D_CNT_INS), offsets, list and regions.
+// Does nothing above STAR_ROUND_SMALL keys.
+static constexpr int STAR_ROUND_SMALL = 4096;
+hipError_t launch_small_round(const PassPlan &p, uint64_t *keys, hipStream_t s);
 // Reciprocate m ordered pairs in place into 2m directed keys.
 hipError_t launch_reciprocate(uint64_t *keys, int64_t m, hipStream_t s);
-// Stars with at least one insertion (ins_off[s+1] > ins_off[s]): flags[s] in {0,1}; after
-// an exclusive scan of flags into pos, list[pos[s]] = s for the flagged stars (ascending).
-hipError_t launch_active_flags(const int64_t *ins_off, int n, uint32_t *flags, hipStream_t s);
-// Sparse alternative for few sorted keys: offsets of the stars with insertions only, and hk[i] =
-// star at the start of each run (STAR_TASK_NONE elsewhere; compact it for the active list).
-hipError_t launch_sparse_runs(const uint64_t *keys, int64_t m, int64_t *off, uint64_t *hk, hipStream_t s);
-hipError_t launch_u64_to_i32(const uint64_t *in, int64_t m, const int64_t *dev_m, int *out, hipStream_t s);
-hipError_t launch_active_scatter(const uint32_t *flags, const uint32_t *pos, int n, int *list, hipStream_t s);
-// Region sizes of the stars of a pass (list = nullptr: stars 0..nitems-1), per item: link
-// vertices v = vn + m, triangle words 2v - 4 (twice that for stars that may need the wide
-// format), history hn + m.
-// pcount[s] = 0 for the pass's stars (their kernel writes the dense pair count).  dev_n (may be
-// null): the list's length on the device when nitems is only its bound; entries beyond get zero.
-hipError_t launch_capacities(const int *list, int nitems, const int64_t *dev_n, const int *vnum, const int *hnum,
-                             const int64_t *ins_off, int64_t *vcap, int64_t *tcap, int64_t *hcap, int *pcount,
+// Star creation's regions: sizes per star (link vertices v = m, triangle words 2v - 4 (twice that
+// for stars that may need the wide format), history m), pcount[s] = 0; after scans, nvoff[s] =
+// vscan[s] (same for t, h).
+hipError_t launch_capacities(int n, const int64_t *ins_off, int64_t *vcap, int64_t *tcap, int64_t *hcap, int *pcount,
                              hipStream_t s);
-// The pass's insertion pairs, star after star in list order (list = nullptr: stars 0..nitems-1):
-// cnt64[i] = pcount[list[i]] for the offsets scan, then the copy to out[off[i] ...].
-hipError_t launch_pair_counts(const int *list, int nitems, const int *pcount, int64_t *cnt64, hipStream_t s);
-hipError_t launch_pair_gather(const int *list, int nitems, const int *pcount, const int64_t *off,
-                              const int64_t *ntoff, int64_t tbase, const uint64_t *pairbuf, uint64_t *out,
-                              hipStream_t s);
-// nvoff[s] = vbase + vscan[i] (same for t, h) for s = list[i].
-hipError_t launch_assign_regions(const int *list, int nitems, const int64_t *vscan, const int64_t *tscan,
-                                 const int64_t *hscan, int64_t vbase, int64_t tbase, int64_t hbase, int64_t *nvoff,
+hipError_t launch_assign_regions(int n, const int64_t *vscan, const int64_t *tscan, const int64_t *hscan, int64_t *nvoff,
                                  int64_t *ntoff, int64_t *nhoff, hipStream_t s);
 // Live region sizes of every star (vertices, triangle words, history), for repacking.
 hipError_t launch_live_sizes(int n, const int *vnum, const int *tnum, const int *hnum, int64_t *vsz, int64_t *tsz,

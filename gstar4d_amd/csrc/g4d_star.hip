@@ -270,6 +270,7 @@ __device__ __forceinline__ void star_body(const StarParams &p, int nitems)
     if ((int)blockIdx.x >= nitems) return;
     bool first = true;
     int nfilt = 0, ncof = 0; // this lane's cofactor-filter evaluations and cofactor computations
+    unsigned long long npairs = 0, ndrown = 0; // the wave's
     for (;;) {
         int base = 0;
         if (one_each) {
@@ -592,9 +593,12 @@ __device__ __forceinline__ void star_body(const StarParams &p, int nitems)
                 }
             }
             wave_sync();
-            for (int q = lane; q < m; q += 64) {
-                const int lv = L.ins_local[q];
-                p.dflag[ib + q] = (lv < 0 || !L.present[lv]) ? 1 : 0;
+            int drowned = 0;
+            for (int b0 = 0; b0 < m; b0 += 64) {
+                const int q = b0 + lane, lv = q < m ? L.ins_local[q] : 0;
+                const bool dr = q < m && (lv < 0 || !L.present[lv]);
+                if (q < m) p.dflag[ib + q] = dr ? 1 : 0;
+                drowned += __popcll(__ballot(dr));
             }
             // vertex compaction
             const int64_t vo = p.nvoff[s], to = p.ntoff[s];
@@ -653,6 +657,8 @@ __device__ __forceinline__ void star_body(const StarParams &p, int nitems)
                 npair += tot;
             }
             if (lane == 0) p.pcount[s] = npair;
+            npairs += npair;
+            ndrown += drowned;
             const int hn = star_history_merge(p, s, L.ins, m, lane, 64);
             wave_sync();
             if (lane == 0) star_commit(p, s, vcount, vo, tcount, to, hn + m);
@@ -663,6 +669,8 @@ __device__ __forceinline__ void star_body(const StarParams &p, int nitems)
     if (lane == 0) {
         atomicAdd(&cnt[G4D_CNT_ORIENT4], (unsigned long long)wf);
         atomicAdd(&cnt[G4D_CNT_COFACTOR], (unsigned long long)wc);
+        if (npairs) atomicAdd(&cnt[G4D_CNT_PAIRS], npairs);
+        if (ndrown) atomicAdd(&cnt[G4D_CNT_DROWNED], ndrown);
     }
 }
 
@@ -847,6 +855,7 @@ __device__ __forceinline__ void star_body_grp(const StarParams &p, int nitems)
     if ((int)blockIdx.x >= nbatch) return;
     bool first = true;
     int nfilt = 0, ncof = 0;
+    unsigned long long npairs = 0, ndrown = 0; // the wave's
     double C[KPL][4];
     typename std::conditional<PF, float, double[4]>::type P[KPL];
     for (;;) {
@@ -1196,11 +1205,17 @@ __device__ __forceinline__ void star_body_grp(const StarParams &p, int nitems)
                     L.present[tvert(tf[k], 2)] = 1;
                 }
             wave_sync();
-            if (fin)
-                for (int q = gl; q < m; q += GL) {
+#pragma unroll
+            for (int b0 = 0; b0 < VMAX; b0 += GL) {
+                const int q = b0 + gl;
+                bool dr = false;
+                if (fin && q < m) {
                     const int lv = L.ins_local[q];
-                    p.dflag[ib + q] = (lv < 0 || !L.present[lv]) ? 1 : 0;
+                    dr = lv < 0 || !L.present[lv];
+                    p.dflag[ib + q] = dr ? 1 : 0;
                 }
+                ndrown += __popcll(__ballot(dr));
+            }
             const int64_t vo = fin ? p.nvoff[s] : 0, to = fin ? p.ntoff[s] : 0;
             int vcount = 0;
 #pragma unroll
@@ -1264,6 +1279,9 @@ __device__ __forceinline__ void star_body_grp(const StarParams &p, int nitems)
                 if (np > 1) p.pairbuf[pb + at + 1] = pr.y;
                 npair += tot;
             }
+            // groups not finalised count none
+#pragma unroll
+            for (int j = 0; j < NG; j++) npairs += __builtin_amdgcn_readlane(npair, j * GL);
             int hn = 0;
             if (fin) {
                 if (gl == 0) p.pcount[s] = npair;
@@ -1278,6 +1296,8 @@ __device__ __forceinline__ void star_body_grp(const StarParams &p, int nitems)
     if (lane == 0) {
         atomicAdd(&cnt[G4D_CNT_ORIENT4], (unsigned long long)wf);
         atomicAdd(&cnt[G4D_CNT_COFACTOR], (unsigned long long)wc);
+        if (npairs) atomicAdd(&cnt[G4D_CNT_PAIRS], npairs);
+        if (ndrown) atomicAdd(&cnt[G4D_CNT_DROWNED], ndrown);
     }
 }
 
@@ -1318,17 +1338,17 @@ static int star_t0_variant(int requested)
 }
 
 static_assert(G4D_CNT_QUEUE0 + 6 <= G4D_CNT_NUM, "six queue heads must fit the counter block");
-static_assert(G4D_CNT_NUM <= 32, "counter masks are 32 bits wide");
+static_assert(G4D_CNT_NUM < 64, "counter masks are 64 bits wide");
 
-__global__ void k_zero_counters(unsigned long long *cnt, uint32_t mask)
+__global__ void k_zero_counters(unsigned long long *cnt, uint64_t mask)
 {
     const int i = threadIdx.x;
     if (i < G4D_CNT_NUM && ((mask >> i) & 1u)) cnt[i] = 0ull;
 }
 
-hipError_t launch_zero_counters(unsigned long long *cnt, uint32_t mask, hipStream_t s)
+hipError_t launch_zero_counters(unsigned long long *cnt, uint64_t mask, hipStream_t s)
 {
-    if (G4D_CNT_NUM < 32 && (mask >> G4D_CNT_NUM) != 0u) return hipErrorInvalidValue; // beyond the block
+    if ((mask >> G4D_CNT_NUM) != 0u) return hipErrorInvalidValue; // beyond the block
     hipLaunchKernelGGL(k_zero_counters, dim3(1), dim3(64), 0, s, cnt, mask);
     return hipGetLastError();
 }
@@ -1468,6 +1488,7 @@ __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(WPE, 8)
     nitems = c < (unsigned long long)nitems ? (int)c : nitems;
     if ((int)blockIdx.x >= nitems) return;
     int ncof = 0, nfilt = 0;
+    unsigned long long npairs = 0, ndrown = 0; // of the work-group, and of the wave
     for (;;) {
         __syncthreads(); // the previous star is done with L
         if (tid == 0) L.item = (int)atomicAdd(&cnt[p.work_counter], 1ull);
@@ -1692,9 +1713,11 @@ __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(WPE, 8)
         const int64_t vo = p.nvoff[s], to = p.ntoff[s];
         int vcount = 0, tcount = 0, row = 2;
         if (!failed) {
-            for (int q = tid; q < m; q += NT) {
-                const int lv = L.ins_local[q];
-                p.dflag[ib + q] = (lv < 0 || !L.fin.present[lv]) ? 1 : 0;
+            for (int b0 = 0; b0 < m; b0 += NT) {
+                const int q = b0 + tid, lv = q < m ? L.ins_local[q] : 0;
+                const bool dr = q < m && (lv < 0 || !L.fin.present[lv]);
+                if (q < m) p.dflag[ib + q] = dr ? 1 : 0;
+                ndrown += __popcll(__ballot(dr));
             }
             for (int base = 0; base < need; base += NT, row ^= 1) {
                 const int v = base + tid;
@@ -1756,6 +1779,7 @@ __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(WPE, 8)
             npair += tot;
         }
         if (tid == 0) p.pcount[s] = npair;
+        npairs += npair;
         const int hn = star_history_merge(p, s, L.ins, m, tid, NT);
         __syncthreads(); // every read of the old record and regions before the switch
         if (tid == 0) star_commit(p, s, vcount, vo, tcount, to, hn + m);
@@ -1764,6 +1788,8 @@ __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(WPE, 8)
     if ((tid & 63) == 0) {
         atomicAdd(&cnt[G4D_CNT_ORIENT4], (unsigned long long)wf);
         atomicAdd(&cnt[G4D_CNT_COFACTOR], (unsigned long long)wc);
+        if (tid == 0 && npairs) atomicAdd(&cnt[G4D_CNT_PAIRS], npairs);
+        if (ndrown) atomicAdd(&cnt[G4D_CNT_DROWNED], ndrown);
     }
 }
 
@@ -2108,10 +2134,14 @@ __global__ void __launch_bounds__(GSTAR_NT) k_star_global(StarParams p, const in
             if (L.tfl[slot] & TF_ALIVE)
                 for (int i = 0; i < 3; i++) L.present[L.tva[3 * slot + i]] = 1;
         __syncthreads();
-        for (int q = tid; q < m; q += GSTAR_NT) {
-            const int lv = L.ins_local[q];
-            p.dflag[ib + q] = (lv < 0 || !L.present[lv]) ? 1 : 0;
+        int ndrown = 0; // the wave's
+        for (int b0 = 0; b0 < m; b0 += GSTAR_NT) {
+            const int q = b0 + tid, lv = q < m ? L.ins_local[q] : 0;
+            const bool dr = q < m && (lv < 0 || !L.present[lv]);
+            if (q < m) p.dflag[ib + q] = dr ? 1 : 0;
+            ndrown += __popcll(__ballot(dr));
         }
+        if ((tid & 63) == 0 && ndrown) atomicAdd(&cnt[G4D_CNT_DROWNED], (unsigned long long)ndrown);
         const int64_t vo = p.nvoff[s], to = p.ntoff[s];
         int vcount = 0;
         for (int base = 0; base < V; base += GSTAR_NT) {
@@ -2173,7 +2203,10 @@ __global__ void __launch_bounds__(GSTAR_NT) k_star_global(StarParams p, const in
             if (np > 1) p.pairbuf[pb + at + 1] = pr.y;
             npair += tot;
         }
-        if (tid == 0) p.pcount[s] = (int)npair;
+        if (tid == 0) {
+            p.pcount[s] = (int)npair;
+            atomicAdd(&cnt[G4D_CNT_PAIRS], (unsigned long long)npair);
+        }
         const int hn = star_history_merge(p, s, L.ins, m, tid, GSTAR_NT);
         __syncthreads();
         if (tid == 0) star_commit(p, s, vcount, vo, tcount, to, hn + m);
@@ -2240,16 +2273,9 @@ __global__ void __launch_bounds__(64) k_proofs(ProofParams p)
 {
     constexpr int NG = 64 / GL;
     const int lane = threadIdx.x, g = lane / GL, gl = lane % GL;
-    // the exact pass reads its list length from the counter the filter pass appended with
-    // (nx < 0), so that no host round trip separates the two launches
-    int64_t nt = p.ntasks;
-    if (EXACT) {
-        nt = p.nx;
-        if (nt < 0) {
-            const int64_t c = (int64_t)p.cnt[G4D_CNT_APPEND5];
-            nt = c < p.xcap ? c : p.xcap;
-        }
-    }
+    // the counts come from the device, so that no host round trip precedes either launch
+    const int64_t nc = (int64_t)p.cnt[EXACT ? G4D_CNT_APPEND5 : G4D_CNT_TASKS];
+    const int64_t nt = min(nc, EXACT ? p.xcap : p.ntasks);
     for (int64_t it = (int64_t)blockIdx.x * NG + g; it < nt; it += (int64_t)gridDim.x * NG) {
         const int64_t task = EXACT ? p.xlist[it] : it;
         const uint64_t tk = p.tasks[task];
@@ -2327,7 +2353,7 @@ __global__ void __launch_bounds__(64) k_proofs(ProofParams p)
 
 hipError_t launch_proofs(const ProofParams &p, bool exact, hipStream_t s)
 {
-    const int64_t nt = exact ? (p.nx < 0 ? p.xcap : p.nx) : p.ntasks;
+    const int64_t nt = exact ? p.xcap : p.ntasks;
     if (nt <= 0) return hipSuccess;
     if (exact) {
         const int nb = (int)(nt < 1024 ? nt : 1024);
@@ -2345,71 +2371,413 @@ hipError_t launch_proofs(const ProofParams &p, bool exact, hipStream_t s)
 // reciprocation, capacities
 // ------------------------------------------------------------------------------------
 
-__global__ void k_drown_keys(const uint64_t *drown, int64_t m, uint64_t *keys)
+// Exclusive prefix of v over the work-group's threads and the total (LA_THREADS threads); red holds
+// LA_THREADS / 64 ints and is free again when every thread has passed the next barrier.
+static constexpr int LA_THREADS = 256;
+__device__ __forceinline__ int la_excl(int v, int *red, int *tot)
 {
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < m; i += (int64_t)gridDim.x * blockDim.x) {
-        const uint32_t s = (uint32_t)(drown[i] >> 32), v = (uint32_t)drown[i];
-        const uint32_t mn = s < v ? s : v, mx = s < v ? v : s;
-        keys[i] = ((uint64_t)mn << 33) | ((uint64_t)mx << 1) | (uint64_t)(s == mn ? 0 : 1);
+    const int inc = g4d_wave_incl_sum(v), w = threadIdx.x >> 6;
+    if ((threadIdx.x & 63) == 63) red[w] = inc;
+    __syncthreads();
+    int base = 0, all = 0;
+#pragma unroll
+    for (int i = 0; i < LA_THREADS / 64; i++) {
+        const int x = red[i];
+        if (i < w) base += x;
+        all += x;
+    }
+    *tot = all;
+    return base + inc - v;
+}
+
+// A tile of 16 flags a thread; HBM bound (one byte an insertion, 16 more for a drowned one).
+__global__ void __launch_bounds__(LA_THREADS) k_drown_keys(const uint64_t *ins_keys, const uint8_t *dflag, int64_t m,
+                                                           uint64_t *keys, unsigned long long *cnt)
+{
+    __shared__ int red[LA_THREADS / 64];
+    __shared__ unsigned long long base;
+    const int64_t i0 = ((int64_t)blockIdx.x * LA_THREADS + threadIdx.x) * 16;
+    uint32_t bits = 0;
+    if (i0 < m) {
+        const uint4 f = *reinterpret_cast<const uint4 *>(dflag + i0);
+        const uint32_t w[4] = {f.x, f.y, f.z, f.w};
+#pragma unroll
+        for (int j = 0; j < 16; j++) bits |= ((w[j >> 2] >> (8 * (j & 3))) & 1u) << j;
+        if (m - i0 < 16) bits &= (1u << (m - i0)) - 1u;
+    }
+    int tot;
+    const int at = la_excl(__popc(bits), red, &tot);
+    if (threadIdx.x == 0 && tot) base = atomicAdd(&cnt[G4D_CNT_DROWN_KEYS], (unsigned long long)tot);
+    __syncthreads();
+    uint64_t *out = keys + base + at;
+    for (; bits; bits &= bits - 1) {
+        const uint64_t k = ins_keys[i0 + __builtin_ctz(bits)];
+        const uint32_t st = (uint32_t)(k >> 32), v = (uint32_t)k;
+        const uint32_t mn = st < v ? st : v, mx = st < v ? v : st;
+        *out++ = ((uint64_t)mn << 33) | ((uint64_t)mx << 1) | (uint64_t)(st == mn ? 0 : 1);
     }
 }
 
-hipError_t launch_drown_keys(const uint64_t *drown, int64_t m, uint64_t *keys, hipStream_t s)
+hipError_t launch_drown_keys(const uint64_t *ins_keys, const uint8_t *dflag, int64_t m, uint64_t *keys,
+                             unsigned long long *cnt, hipStream_t s)
 {
     if (m <= 0) return hipSuccess;
-    hipLaunchKernelGGL(k_drown_keys, dim3(g4d_blocks(m, 256, 65536)), dim3(256), 0, s, drown, m, keys);
+    const int64_t nb = (m + 16 * LA_THREADS - 1) / (16 * LA_THREADS);
+    if (nb > INT32_MAX) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(k_drown_keys, dim3((unsigned)nb), dim3(LA_THREADS), 0, s, ins_keys, dflag, m, keys, cnt);
     return hipGetLastError();
 }
 
-// tasks[i] = (star << 32 | vertex) of the drowned insertion i unless it is mutual, else
-// STAR_TASK_NONE; the caller compacts (order-preserving, no atomics).
-__global__ void k_nonmutual(const uint64_t *keys, int64_t m, uint64_t *tasks)
+static constexpr int NM_ITEMS = 8;
+__global__ void __launch_bounds__(LA_THREADS) k_nonmutual(const uint64_t *keys, int64_t m, uint64_t *tasks,
+                                                          unsigned long long *cnt)
 {
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < m; i += (int64_t)gridDim.x * blockDim.x) {
-        const uint64_t k = keys[i] >> 1;
+    __shared__ int red[LA_THREADS / 64];
+    __shared__ unsigned long long base;
+    const int64_t b0 = (int64_t)blockIdx.x * (LA_THREADS * NM_ITEMS) + threadIdx.x;
+    uint64_t task[NM_ITEMS];
+    int c = 0;
+#pragma unroll
+    for (int j = 0; j < NM_ITEMS; j++) {
+        const int64_t i = b0 + j * LA_THREADS;
+        task[j] = STAR_PAIR_NONE;
+        if (i >= m) continue;
+        const uint64_t ki = keys[i], k = ki >> 1;
         const bool mutual = (i > 0 && (keys[i - 1] >> 1) == k) || (i + 1 < m && (keys[i + 1] >> 1) == k);
-        const uint32_t mn = (uint32_t)(keys[i] >> 33), mx = (uint32_t)((keys[i] >> 1) & 0xffffffffu);
-        const bool dir = keys[i] & 1;
-        const uint32_t st = dir ? mx : mn, v = dir ? mn : mx;
-        tasks[i] = mutual ? STAR_TASK_NONE : (((uint64_t)st << 32) | v);
+        if (mutual) continue;
+        const uint32_t mn = (uint32_t)(ki >> 33), mx = (uint32_t)(k & 0xffffffffu);
+        task[j] = (ki & 1) ? (((uint64_t)mx << 32) | mn) : (((uint64_t)mn << 32) | mx);
+        c++;
     }
+    int tot;
+    int at = la_excl(c, red, &tot);
+    if (threadIdx.x == 0 && tot) base = atomicAdd(&cnt[G4D_CNT_TASKS], (unsigned long long)tot);
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < NM_ITEMS; j++)
+        if (task[j] != STAR_PAIR_NONE) tasks[base + at++] = task[j];
 }
 
-hipError_t launch_nonmutual(const uint64_t *keys, int64_t m, uint64_t *tasks, hipStream_t s)
+hipError_t launch_nonmutual(const uint64_t *keys, int64_t m, uint64_t *tasks, unsigned long long *cnt, hipStream_t s)
 {
     if (m <= 0) return hipSuccess;
-    hipLaunchKernelGGL(k_nonmutual, dim3(g4d_blocks(m, 256, 65536)), dim3(256), 0, s, keys, m, tasks);
+    const int64_t nb = (m + LA_THREADS * NM_ITEMS - 1) / (LA_THREADS * NM_ITEMS);
+    if (nb > INT32_MAX) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(k_nonmutual, dim3((unsigned)nb), dim3(LA_THREADS), 0, s, keys, m, tasks, cnt);
     return hipGetLastError();
 }
 
-__global__ void k_hist_filter(const uint64_t *pairs, int64_t m, const int *hpool, const int64_t *hoff, const int *hnum,
-                              uint8_t *keep)
+// One pass from the stars' pair regions and the proofs' pairs to the appended keys: sixteen stars a
+// work-group step, 16 lanes each (a star of more than NP_WIDE pairs is left to the whole group),
+// then the proofs.  Surviving pairs are collected in LDS and leave a stage at a time, with one
+// atomic.  Bound by the latency of the histories' binary searches (dependent reads, some six for
+// a star of 40).  The gather of the pairs into one list, the filter over it and the compaction of
+// what it kept, three passes over 8 bytes a pair and six launches, took 4.3 ms on 4,194,304
+// uniform points (12 rounds); this takes 3.7.
+static constexpr int NP_STAGE = 2048, NP_WIDE = 128;
+
+__global__ void __launch_bounds__(LA_THREADS) k_new_pairs(NewPairs p)
 {
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < m; i += (int64_t)gridDim.x * blockDim.x) {
-        const uint64_t k = pairs[i];
+    __shared__ uint64_t stage[NP_STAGE];
+    __shared__ int nst, nwide, wide[LA_THREADS / 16];
+    __shared__ unsigned long long base;
+    const int tid = threadIdx.x, sub = tid & 15, lane = __lane_id();
+    if (tid == 0) nst = 0;
+    __syncthreads();
+    // Whether pair k is new (a < b and b not in a's history).
+    auto is_new = [&](uint64_t k) {
         const uint32_t a = (uint32_t)(k >> 32), b = (uint32_t)k;
-        if (!(a < b)) {
-            keep[i] = 0;
-            continue;
-        }
-        const int *h = hpool + hoff[a];
-        const int hn = hnum[a];
+        if (!(a < b)) return false;
+        const int *h = p.hpool + p.hoff[a];
+        const int hn = p.hnum[a];
         int lo = 0, hi = hn;
         while (lo < hi) {
             const int mid = (lo + hi) >> 1;
             if ((uint32_t)h[mid] < b) lo = mid + 1;
             else hi = mid;
         }
-        keep[i] = (lo < hn && (uint32_t)h[lo] == b) ? 0 : 1;
+        return !(lo < hn && (uint32_t)h[lo] == b);
+    };
+    auto emit = [&](unsigned long long at, uint64_t k) {
+        p.keys[2 * at] = k;
+        p.keys[2 * at + 1] = (k << 32) | (k >> 32);
+    };
+    // Called by whole waves; pairs that find the stage full are appended at once.
+    auto put = [&](bool keep, uint64_t k) {
+        const uint64_t mk = __ballot(keep);
+        if (!mk) return;
+        int at = 0;
+        if (lane == 0) at = atomicAdd(&nst, __popcll(mk));
+        at = __builtin_amdgcn_readfirstlane(at) + __popcll(mk & ((1ull << lane) - 1ull));
+        const bool full = keep && at >= NP_STAGE;
+        if (keep && !full) stage[at] = k;
+        if (__ballot(full)) {
+            const long long g = g4d_wave_append(full, &p.cnt[G4D_CNT_NEW_PAIRS]);
+            if (full) emit((unsigned long long)g, k);
+        }
+    };
+    // Called by the whole work-group: empties the stage when it holds more than `above`.
+    auto flush = [&](int above) {
+        __syncthreads();
+        const int have = min(nst, NP_STAGE);
+        __syncthreads();
+        if (have <= above) return;
+        if (tid == 0) {
+            base = atomicAdd(&p.cnt[G4D_CNT_NEW_PAIRS], (unsigned long long)have);
+            nst = 0;
+        }
+        __syncthreads();
+        for (int i = tid; i < have; i += LA_THREADS) emit(base + i, stage[i]);
+        __syncthreads();
+    };
+    for (int64_t i0 = (int64_t)blockIdx.x * (LA_THREADS / 16); i0 < p.nitems;
+         i0 += (int64_t)gridDim.x * (LA_THREADS / 16)) {
+        const int64_t i = i0 + (tid >> 4);
+        const int s = i < p.nitems ? (p.list ? p.list[i] : (int)i) : -1;
+        int c = s >= 0 ? p.pcount[s] : 0;
+        const uint64_t *src = s >= 0 ? p.pairbuf + 2 * (p.ntoff[s] - p.tbase) : p.pairbuf;
+        if (tid == 0) nwide = 0;
+        __syncthreads();
+        if (c > NP_WIDE) {
+            if (sub == 0) wide[atomicAdd(&nwide, 1)] = s;
+            c = 0;
+        }
+        const int cmax = g4d_wave_max(c);
+        for (int k0 = 0; k0 < cmax; k0 += 16) {
+            const int k = k0 + sub;
+            const uint64_t pr = k < c ? src[k] : 0ull;
+            put(k < c && is_new(pr), pr);
+        }
+        __syncthreads();
+        for (int w = 0; w < nwide; w++) {
+            const int sw = wide[w], cw = p.pcount[sw];
+            const uint64_t *srcw = p.pairbuf + 2 * (p.ntoff[sw] - p.tbase);
+            for (int k0 = 0; k0 < cw; k0 += LA_THREADS) {
+                const int k = k0 + tid;
+                const uint64_t pr = k < cw ? srcw[k] : 0ull;
+                put(k < cw && is_new(pr), pr);
+            }
+        }
+        flush(NP_STAGE / 2);
+    }
+    const int64_t nc = (int64_t)p.cnt[G4D_CNT_TASKS];
+    const int64_t np = 4 * min(nc, p.ntasks);
+    for (int64_t k0 = (int64_t)blockIdx.x * LA_THREADS; k0 < np; k0 += (int64_t)gridDim.x * LA_THREADS) {
+        const int64_t k = k0 + tid;
+        const uint64_t pr = k < np ? p.proofs[k] : 0ull;
+        put(k < np && is_new(pr), pr);
+        flush(NP_STAGE - LA_THREADS);
+    }
+    flush(0);
+}
+
+hipError_t launch_new_pairs(const NewPairs &p, hipStream_t s)
+{
+    const int64_t work = std::max<int64_t>(16 * (int64_t)p.nitems, 4 * p.ntasks);
+    if (work <= 0) return hipSuccess;
+    hipLaunchKernelGGL(k_new_pairs, dim3(g4d_blocks(work, LA_THREADS, 2048)), dim3(LA_THREADS), 0, s, p);
+    return hipGetLastError();
+}
+
+// Region sizes of star s with m insertions.
+__device__ __forceinline__ void plan_sizes(const PassPlan &p, int s, int m, int *v, int *t, int *h)
+{
+    *v = p.vnum[s] + m;
+    *t = (int)star_tcap_words(*v);
+    *h = p.hnum[s] + m;
+}
+
+__device__ __forceinline__ void plan_star(const PassPlan &p, int s, int64_t first, int m, unsigned long long item,
+                                          int64_t v, int64_t t, int64_t h)
+{
+    p.ins_off[s] = first;
+    p.ins_off[s + 1] = first + m; // the following star's first, when that has insertions too
+    p.list[item] = s;
+    p.nvoff[s] = v;
+    p.ntoff[s] = t;
+    p.nhoff[s] = h;
+    p.pcount[s] = 0;
+}
+
+// The key that starts a star's run plans the star (the run's end found by doubling steps); a tile's
+// stars take list entries and regions with one atomic per counter, in key order within the tile.
+static constexpr int PP_ITEMS = 8, PP_TILE = LA_THREADS * PP_ITEMS;
+__global__ void __launch_bounds__(LA_THREADS) k_pass_plan(PassPlan p, const uint64_t *keys, int64_t m, const int64_t *dev_m)
+{
+    __shared__ int red[4][LA_THREADS / 64];
+    __shared__ unsigned long long base[4];
+    if (dev_m) m = min(m, *dev_m);
+    const int64_t t0 = (int64_t)blockIdx.x * PP_TILE;
+    if (t0 >= m) return;
+    int st[PP_ITEMS], len[PP_ITEMS];
+    int a = 0, v = 0, t = 0, h = 0;
+#pragma unroll
+    for (int j = 0; j < PP_ITEMS; j++) {
+        const int64_t i = t0 + (int64_t)threadIdx.x * PP_ITEMS + j;
+        st[j] = -1;
+        if (i >= m) continue;
+        const uint32_t s = (uint32_t)(keys[i] >> 32);
+        if (i > 0 && (uint32_t)(keys[i - 1] >> 32) == s) continue;
+        int64_t lo = i, step = 1; // keys[lo] is s; doubling, then bisection
+        while (lo + step < m && (uint32_t)(keys[lo + step] >> 32) == s) {
+            lo += step;
+            step *= 2;
+        }
+        int64_t hi = min(lo + step, m);
+        while (lo + 1 < hi) {
+            const int64_t mid = (lo + hi) >> 1;
+            if ((uint32_t)(keys[mid] >> 32) == s) lo = mid;
+            else hi = mid;
+        }
+        st[j] = (int)s;
+        len[j] = (int)(lo + 1 - i);
+        int dv, dt, dh;
+        plan_sizes(p, st[j], len[j], &dv, &dt, &dh);
+        a++;
+        v += dv;
+        t += dt;
+        h += dh;
+    }
+    int ta, tv, tt, th;
+    const int ea = la_excl(a, red[0], &ta), ev = la_excl(v, red[1], &tv), et = la_excl(t, red[2], &tt),
+              eh = la_excl(h, red[3], &th);
+    if (threadIdx.x < 4) {
+        const int add[4] = {ta, tv, tt, th};
+        const int at[4] = {G4D_CNT_ACTIVE, G4D_CNT_NEED_V, G4D_CNT_NEED_T, G4D_CNT_NEED_H};
+        const int c = threadIdx.x;
+        base[c] = ta ? atomicAdd(&p.cnt[at[c]], (unsigned long long)add[c]) : 0ull;
+    }
+    __syncthreads();
+    unsigned long long item = base[0] + ea;
+    int64_t vo = p.base[0] + (int64_t)base[1] + ev, to = p.base[1] + (int64_t)base[2] + et,
+            ho = p.base[2] + (int64_t)base[3] + eh;
+#pragma unroll
+    for (int j = 0; j < PP_ITEMS; j++) {
+        if (st[j] < 0) continue;
+        int dv, dt, dh;
+        plan_sizes(p, st[j], len[j], &dv, &dt, &dh);
+        plan_star(p, st[j], t0 + (int64_t)threadIdx.x * PP_ITEMS + j, len[j], item, vo, to, ho);
+        item++;
+        vo += dv;
+        to += dt;
+        ho += dh;
     }
 }
 
-hipError_t launch_hist_filter(const uint64_t *pairs, int64_t m, const int *hpool, const int64_t *hoff, const int *hnum,
-                              uint8_t *keep, hipStream_t s)
+hipError_t launch_pass_plan(const PassPlan &p, const uint64_t *keys, int64_t m, const int64_t *dev_m, hipStream_t s)
 {
-    if (m <= 0) return hipSuccess;
-    hipLaunchKernelGGL(k_hist_filter, dim3(g4d_blocks(m, 256, 65536)), dim3(256), 0, s, pairs, m, hpool, hoff, hnum,
-                       keep);
+    const int64_t nb = (m + PP_TILE - 1) / PP_TILE;
+    if (nb <= 0) return hipSuccess;
+    if (nb > INT32_MAX) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(k_pass_plan, dim3((unsigned)nb), dim3(LA_THREADS), 0, s, p, keys, m, dev_m);
+    return hipGetLastError();
+}
+
+// Late rounds insert a few thousand keys or fewer, and every one of the sort, unique, compaction and
+// scan launches they took cost 3-10 us with a host round trip between some: 20 launches and four
+// round trips.  One work-group does all of it in LDS: a bitonic sort (78 steps for 4,096
+// keys), repeats removed, runs listed, region sizes scanned; bound by its barriers, 13-17 us.
+// With the appended lists before it a call on 1,000 points makes 178 launches instead of 331 (2.40 ->
+// 1.70 ms), on 100,000 330 instead of 656 (7.1 -> 6.25 ms).
+static constexpr int SR_THREADS = 1024;
+
+// Exclusive prefix over 1,024 threads and the total; red: 16 ints, reusable after the next barrier.
+__device__ __forceinline__ int sr_excl(int v, int *red, int *tot)
+{
+    const int inc = g4d_wave_incl_sum(v), w = threadIdx.x >> 6;
+    if ((threadIdx.x & 63) == 63) red[w] = inc;
+    __syncthreads();
+    int base = 0, all = 0;
+#pragma unroll
+    for (int i = 0; i < SR_THREADS / 64; i++) {
+        const int x = red[i];
+        if (i < w) base += x;
+        all += x;
+    }
+    *tot = all;
+    return base + inc - v;
+}
+
+__global__ void __launch_bounds__(SR_THREADS) k_small_round(PassPlan p, uint64_t *keys)
+{
+    __shared__ uint64_t a[STAR_ROUND_SMALL], b[STAR_ROUND_SMALL];
+    __shared__ int first[STAR_ROUND_SMALL + 1];
+    __shared__ int red[5][SR_THREADS / 64];
+    const int tid = threadIdx.x;
+    const unsigned long long np = p.cnt[G4D_CNT_NEW_PAIRS];
+    if (np == 0 || np > STAR_ROUND_SMALL / 2) return;
+    const int m = 2 * (int)np;
+    int n = SR_THREADS;
+    while (n < m) n <<= 1;
+    for (int i = tid; i < n; i += SR_THREADS) a[i] = i < m ? keys[i] : ~0ull;
+    __syncthreads();
+    for (int k = 2; k <= n; k <<= 1)
+        for (int j = k >> 1; j > 0; j >>= 1) {
+            for (int x = tid; x < n / 2; x += SR_THREADS) {
+                const int i = ((x & ~(j - 1)) << 1) | (x & (j - 1)), l = i | j;
+                const uint64_t u = a[i], w = a[l];
+                if ((u > w) == ((i & k) == 0)) {
+                    a[i] = w;
+                    a[l] = u;
+                }
+            }
+            __syncthreads();
+        }
+    // repeats out, in order
+    int cnt = 0;
+    for (int i0 = 0, r = 0; i0 < m; i0 += SR_THREADS, r ^= 1) {
+        const int i = i0 + tid;
+        const bool f = i < m && (i == 0 || a[i] != a[i - 1]);
+        int tot;
+        const int at = cnt + sr_excl(f ? 1 : 0, red[r], &tot);
+        if (f) {
+            b[at] = a[i];
+            keys[at] = a[i];
+        }
+        cnt += tot;
+    }
+    __syncthreads();
+    // runs of one star
+    int runs = 0;
+    for (int i0 = 0, r = 0; i0 < cnt; i0 += SR_THREADS, r ^= 1) {
+        const int i = i0 + tid;
+        const bool f = i < cnt && (i == 0 || (b[i] >> 32) != (b[i - 1] >> 32));
+        int tot;
+        const int at = runs + sr_excl(f ? 1 : 0, red[r], &tot);
+        if (f) first[at] = i;
+        runs += tot;
+    }
+    if (tid == 0) first[runs] = cnt;
+    __syncthreads();
+    int64_t vo = p.base[0], to = p.base[1], ho = p.base[2];
+    for (int r0 = 0; r0 < runs; r0 += SR_THREADS) {
+        const int r = r0 + tid;
+        int s = 0, len = 0, dv = 0, dt = 0, dh = 0;
+        if (r < runs) {
+            s = (int)(uint32_t)(b[first[r]] >> 32);
+            len = first[r + 1] - first[r];
+            plan_sizes(p, s, len, &dv, &dt, &dh);
+        }
+        int tv, tt, th;
+        const int ev = sr_excl(dv, red[2], &tv), et = sr_excl(dt, red[3], &tt), eh = sr_excl(dh, red[4], &th);
+        if (r < runs) plan_star(p, s, first[r], len, r, vo + ev, to + et, ho + eh);
+        vo += tv;
+        to += tt;
+        ho += th;
+        __syncthreads();
+    }
+    if (tid == 0) {
+        p.cnt[G4D_CNT_INS] = cnt;
+        p.cnt[G4D_CNT_ACTIVE] = runs;
+        p.cnt[G4D_CNT_NEED_V] = vo - p.base[0];
+        p.cnt[G4D_CNT_NEED_T] = to - p.base[1];
+        p.cnt[G4D_CNT_NEED_H] = ho - p.base[2];
+    }
+}
+
+hipError_t launch_small_round(const PassPlan &p, uint64_t *keys, hipStream_t s)
+{
+    hipLaunchKernelGGL(k_small_round, dim3(1), dim3(SR_THREADS), 0, s, p, keys);
     return hipGetLastError();
 }
 
@@ -2428,162 +2796,42 @@ hipError_t launch_reciprocate(uint64_t *keys, int64_t m, hipStream_t s)
     return hipGetLastError();
 }
 
-// Sparse form of a pass's insertion offsets and active list, for sorted keys much fewer than the
-// stars: the key that starts a star's run writes the star's first offset, the key that ends it
-// the next one (equal to the following star's first when that star has insertions too), and
-// hk[i] holds the star at a run's start (STAR_TASK_NONE elsewhere), so the order-preserving
-// compaction of hk lists the stars with insertions in ascending order.  Offsets of stars
-// without insertions are not written (nothing reads them).
-__global__ void k_sparse_runs(const uint64_t *keys, int64_t m, int64_t *off, uint64_t *hk)
+__global__ void k_capacities(int n, const int64_t *ins_off, int64_t *vcap, int64_t *tcap, int64_t *hcap, int *pcount)
 {
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < m; i += (int64_t)gridDim.x * blockDim.x) {
-        const uint32_t st = (uint32_t)(keys[i] >> 32);
-        const bool head = i == 0 || (uint32_t)(keys[i - 1] >> 32) != st;
-        const bool tail = i == m - 1 || (uint32_t)(keys[i + 1] >> 32) != st;
-        if (head) off[st] = i;
-        if (tail) off[st + 1] = i + 1;
-        hk[i] = head ? (uint64_t)st : STAR_TASK_NONE;
-    }
-}
-
-hipError_t launch_sparse_runs(const uint64_t *keys, int64_t m, int64_t *off, uint64_t *hk, hipStream_t s)
-{
-    if (m <= 0) return hipSuccess;
-    hipLaunchKernelGGL(k_sparse_runs, dim3(g4d_blocks(m, 256, 65536)), dim3(256), 0, s, keys, m, off, hk);
-    return hipGetLastError();
-}
-
-// dev_m (may be null): the count on the device, at most m.
-__global__ void k_u64_to_i32(const uint64_t *in, int64_t m, const int64_t *dev_m, int *out)
-{
-    if (dev_m) m = min(m, *dev_m);
-    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < m; i += (int64_t)gridDim.x * blockDim.x)
-        out[i] = (int)in[i];
-}
-
-hipError_t launch_u64_to_i32(const uint64_t *in, int64_t m, const int64_t *dev_m, int *out, hipStream_t s)
-{
-    if (m <= 0) return hipSuccess;
-    hipLaunchKernelGGL(k_u64_to_i32, dim3(g4d_blocks(m, 256, 65536)), dim3(256), 0, s, in, m, dev_m, out);
-    return hipGetLastError();
-}
-
-__global__ void k_active_flags(const int64_t *ins_off, int n, uint32_t *flags)
-{
-    for (int s = blockIdx.x * blockDim.x + threadIdx.x; s < n; s += gridDim.x * blockDim.x)
-        flags[s] = ins_off[s + 1] > ins_off[s] ? 1u : 0u;
-}
-
-hipError_t launch_active_flags(const int64_t *ins_off, int n, uint32_t *flags, hipStream_t s)
-{
-    hipLaunchKernelGGL(k_active_flags, dim3(g4d_blocks(n, 256, 65536)), dim3(256), 0, s, ins_off, n, flags);
-    return hipGetLastError();
-}
-
-__global__ void k_active_scatter(const uint32_t *flags, const uint32_t *pos, int n, int *list)
-{
-    for (int s = blockIdx.x * blockDim.x + threadIdx.x; s < n; s += gridDim.x * blockDim.x)
-        if (flags[s]) list[pos[s]] = s;
-}
-
-hipError_t launch_active_scatter(const uint32_t *flags, const uint32_t *pos, int n, int *list, hipStream_t s)
-{
-    hipLaunchKernelGGL(k_active_scatter, dim3(g4d_blocks(n, 256, 65536)), dim3(256), 0, s, flags, pos, n, list);
-    return hipGetLastError();
-}
-
-// dev_n (may be null): the list's length on the device, at most nitems; the entries from there
-// to nitems get zero capacities (so that scans over nitems total the list's needs).
-__global__ void k_capacities(const int *list, int nitems, const int64_t *dev_n, const int *vnum, const int *hnum,
-                             const int64_t *ins_off, int64_t *vcap, int64_t *tcap, int64_t *hcap, int *pcount)
-{
-    const int nl = dev_n ? (int)min((int64_t)nitems, *dev_n) : nitems;
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < nitems; i += gridDim.x * blockDim.x) {
-        if (i >= nl) {
-            vcap[i] = 0;
-            tcap[i] = 0;
-            hcap[i] = 0;
-            continue;
-        }
-        const int s = list ? list[i] : i;
-        pcount[s] = 0;
+    for (int s = blockIdx.x * blockDim.x + threadIdx.x; s < n; s += gridDim.x * blockDim.x) {
         const int64_t m = ins_off[s + 1] - ins_off[s];
-        const int64_t v = (vnum ? vnum[s] : 0) + m;
-        vcap[i] = v;
-        tcap[i] = star_tcap_words(v);
-        hcap[i] = (hnum ? hnum[s] : 0) + m;
+        pcount[s] = 0;
+        vcap[s] = m;
+        tcap[s] = star_tcap_words(m);
+        hcap[s] = m;
     }
 }
 
-hipError_t launch_capacities(const int *list, int nitems, const int64_t *dev_n, const int *vnum, const int *hnum,
-                             const int64_t *ins_off, int64_t *vcap, int64_t *tcap, int64_t *hcap, int *pcount,
+hipError_t launch_capacities(int n, const int64_t *ins_off, int64_t *vcap, int64_t *tcap, int64_t *hcap, int *pcount,
                              hipStream_t s)
 {
-    if (nitems <= 0) return hipSuccess;
-    hipLaunchKernelGGL(k_capacities, dim3(g4d_blocks(nitems, 256, 65536)), dim3(256), 0, s, list, nitems, dev_n, vnum,
-                       hnum, ins_off, vcap, tcap, hcap, pcount);
+    if (n <= 0) return hipSuccess;
+    hipLaunchKernelGGL(k_capacities, dim3(g4d_blocks(n, 256, 65536)), dim3(256), 0, s, n, ins_off, vcap, tcap, hcap,
+                       pcount);
     return hipGetLastError();
 }
 
-__global__ void k_pair_counts(const int *list, int nitems, const int *pcount, int64_t *cnt64)
-{
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < nitems; i += gridDim.x * blockDim.x)
-        cnt64[i] = pcount[list ? list[i] : i];
-}
-
-hipError_t launch_pair_counts(const int *list, int nitems, const int *pcount, int64_t *cnt64, hipStream_t s)
-{
-    if (nitems <= 0) return hipSuccess;
-    hipLaunchKernelGGL(k_pair_counts, dim3(g4d_blocks(nitems, 256, 65536)), dim3(256), 0, s, list, nitems, pcount,
-                       cnt64);
-    return hipGetLastError();
-}
-
-// One quarter-wave (16 lanes) per star copies its dense pairs.
-__global__ void __launch_bounds__(256) k_pair_gather(const int *list, int nitems, const int *pcount,
-                                                     const int64_t *off, const int64_t *ntoff, int64_t tbase,
-                                                     const uint64_t *pairbuf, uint64_t *out)
-{
-    const int sub = threadIdx.x & 15;
-    for (int64_t i = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 4; i < nitems;
-         i += ((int64_t)gridDim.x * blockDim.x) >> 4) {
-        const int s = list ? list[i] : (int)i;
-        const int c = pcount[s];
-        const uint64_t *src = pairbuf + 2 * (ntoff[s] - tbase);
-        uint64_t *dst = out + off[i];
-        for (int k = sub; k < c; k += 16) dst[k] = src[k];
-    }
-}
-
-hipError_t launch_pair_gather(const int *list, int nitems, const int *pcount, const int64_t *off,
-                              const int64_t *ntoff, int64_t tbase, const uint64_t *pairbuf, uint64_t *out,
-                              hipStream_t s)
-{
-    if (nitems <= 0) return hipSuccess;
-    hipLaunchKernelGGL(k_pair_gather, dim3(g4d_blocks((int64_t)nitems * 16, 256, 65536)), dim3(256), 0, s, list,
-                       nitems, pcount, off, ntoff, tbase, pairbuf, out);
-    return hipGetLastError();
-}
-
-__global__ void k_assign_regions(const int *list, int nitems, const int64_t *vscan, const int64_t *tscan,
-                                 const int64_t *hscan, int64_t vbase, int64_t tbase, int64_t hbase, int64_t *nvoff,
+__global__ void k_assign_regions(int n, const int64_t *vscan, const int64_t *tscan, const int64_t *hscan, int64_t *nvoff,
                                  int64_t *ntoff, int64_t *nhoff)
 {
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < nitems; i += gridDim.x * blockDim.x) {
-        const int s = list ? list[i] : i;
-        nvoff[s] = vbase + vscan[i];
-        ntoff[s] = tbase + tscan[i];
-        nhoff[s] = hbase + hscan[i];
+    for (int s = blockIdx.x * blockDim.x + threadIdx.x; s < n; s += gridDim.x * blockDim.x) {
+        nvoff[s] = vscan[s];
+        ntoff[s] = tscan[s];
+        nhoff[s] = hscan[s];
     }
 }
 
-hipError_t launch_assign_regions(const int *list, int nitems, const int64_t *vscan, const int64_t *tscan,
-                                 const int64_t *hscan, int64_t vbase, int64_t tbase, int64_t hbase, int64_t *nvoff,
+hipError_t launch_assign_regions(int n, const int64_t *vscan, const int64_t *tscan, const int64_t *hscan, int64_t *nvoff,
                                  int64_t *ntoff, int64_t *nhoff, hipStream_t s)
 {
-    if (nitems <= 0) return hipSuccess;
-    hipLaunchKernelGGL(k_assign_regions, dim3(g4d_blocks(nitems, 256, 65536)), dim3(256), 0, s, list, nitems, vscan,
-                       tscan, hscan, vbase, tbase, hbase, nvoff, ntoff, nhoff);
+    if (n <= 0) return hipSuccess;
+    hipLaunchKernelGGL(k_assign_regions, dim3(g4d_blocks(n, 256, 65536)), dim3(256), 0, s, n, vscan, tscan, hscan, nvoff,
+                       ntoff, nhoff);
     return hipGetLastError();
 }
 

@@ -264,6 +264,17 @@ def test_star_sizes_around_the_kernel_tiers(orc, k):
     _parity(orc, x, 24)
 
 
+@pytest.mark.parametrize("gen", [datasets.uniform_cube, datasets.hard_mix])
+@pytest.mark.parametrize("n", [60, 150, 250, 350, 450, 600, 800, 1000, 1400, 3000])
+def test_rounds_around_the_small_list_limit(orc, n, gen):
+    """Sets whose first splaying rounds propose from a few to several thousand insertions: the
+    one-launch round (up to 4,096 keys), the general one above, and their hand-over from round to
+    round give the oracle's rounds and insertions."""
+    tets, _, _, st, rst = _parity(orc, gen(n, seed=n), 32)
+    assert st["splay_rounds"] == rst["splay_rounds"]
+    assert st["splay_insertions"] == rst["splay_insertions"]
+
+
 @pytest.mark.parametrize("bands", [1, 3, 5])
 def test_pba_bands_same_triangulation(orc, bands):
     x = datasets.uniform_cube(20000, seed=31)
