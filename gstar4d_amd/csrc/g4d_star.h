@@ -141,6 +141,12 @@ hipError_t launch_drown_keys(const uint64_t *ins_keys, const uint8_t *dflag, int
 // Sorted drowned keys -> proof tasks (star<<32 | vertex), the mutual pairs left out; counter
 // G4D_CNT_TASKS.
 hipError_t launch_nonmutual(const uint64_t *keys, int64_t m, uint64_t *tasks, unsigned long long *cnt, hipStream_t s);
+// Both at once for at most DROWN_SMALL drowned (nd, as counted by the pass) of at most
+// DROWN_SMALL_INS insertions, which one work-group reads.
+static constexpr int DROWN_SMALL = 4096;
+static constexpr int64_t DROWN_SMALL_INS = 1 << 16;
+hipError_t launch_drown_small(const uint64_t *ins_keys, const uint8_t *dflag, int64_t m, int64_t nd, uint64_t *tasks,
+                              unsigned long long *cnt, hipStream_t s);
 // Both directed keys of every pair (a<<32 | b, a < b) with b not in the history of star a, of the
 // last pass's stars (list = nullptr: stars 0..nitems-1) and of the proofs (four per task, tasks
 // counted at G4D_CNT_TASKS, at most ntasks); counter G4D_CNT_NEW_PAIRS (pairs).

@@ -416,6 +416,7 @@ __device__ __forceinline__ void star_body(const StarParams &p, int nitems)
 #pragma unroll(REGC ? KPL : 1)
                 for (int k = 0; k < KPL; k++) {
                     const int slot = lane + 64 * k;
+                    if (REGC && 64 * k >= T) break; // wave-uniform: a small star in a large tier
                     if (slot < T) {
                         const uint32_t t = L.tv[slot];
                         if ((t & (TF_ALIVE | TF_VIS)) == TF_ALIVE) {
@@ -554,8 +555,10 @@ __device__ __forceinline__ void star_body(const StarParams &p, int nitems)
                 // barrier after them
                 unsigned fm = 0;
 #pragma unroll(REGC ? KPL : 1)
-                for (int k = 0; k < KPL; k++)
+                for (int k = 0; k < KPL; k++) {
+                    if (REGC && 64 * k >= T) break;
                     if (lane + 64 * k < T && (L.tv[lane + 64 * k] & TF_FRESH)) fm |= 1u << k;
+                }
                 cofactors(fm);
                 // No barrier before the next step: its filter reads and writes only this lane's
                 // own slots and cofactor columns and the listed coordinates, and its first barrier
@@ -2390,6 +2393,46 @@ __device__ __forceinline__ int la_excl(int v, int *red, int *tot)
     return base + inc - v;
 }
 
+// Key of drowned insertion k = star << 32 | vertex: the pair in order, then who inserted whom.
+__device__ __forceinline__ uint64_t drown_key(uint64_t k)
+{
+    const uint32_t st = (uint32_t)(k >> 32), v = (uint32_t)k;
+    const uint32_t mn = st < v ? st : v, mx = st < v ? v : st;
+    return ((uint64_t)mn << 33) | ((uint64_t)mx << 1) | (uint64_t)(st == mn ? 0 : 1);
+}
+
+// Proof task of the sorted drowned key k between its neighbours (all ones at the ends), or
+// STAR_PAIR_NONE when the drowning is mutual.
+__device__ __forceinline__ uint64_t drown_task(uint64_t k, uint64_t prev, uint64_t next)
+{
+    const uint64_t pair = k >> 1;
+    if ((prev >> 1) == pair || (next >> 1) == pair) return STAR_PAIR_NONE;
+    const uint32_t mn = (uint32_t)(k >> 33), mx = (uint32_t)(pair & 0xffffffffu);
+    return (k & 1) ? (((uint64_t)mx << 32) | mn) : (((uint64_t)mn << 32) | mx);
+}
+
+// Sorts n keys in LDS (n a power of two, at least 128) with NT threads.  A step's pairs are at most 64
+// apart within the 128 keys of a wave's 64 pairs, so the work-group meets only around the wider
+// steps (6 of 55 for 1,024 keys, 15 of 78 for 4,096).
+template <int NT>
+__device__ __forceinline__ void lds_bitonic(uint64_t *a, int n)
+{
+    for (int k = 2; k <= n; k <<= 1)
+        for (int j = k >> 1; j > 0; j >>= 1) {
+            for (int x = threadIdx.x; x < n / 2; x += NT) {
+                const int i = ((x & ~(j - 1)) << 1) | (x & (j - 1)), l = i | j;
+                const uint64_t u = a[i], w = a[l];
+                if ((u > w) == ((i & k) == 0)) {
+                    a[i] = w;
+                    a[l] = u;
+                }
+            }
+            if (j > 64 || (j == 1 && k > 64)) __syncthreads();
+            else wave_sync();
+        }
+    __syncthreads();
+}
+
 // A tile of 16 flags a thread; HBM bound (one byte an insertion, 16 more for a drowned one).
 __global__ void __launch_bounds__(LA_THREADS) k_drown_keys(const uint64_t *ins_keys, const uint8_t *dflag, int64_t m,
                                                            uint64_t *keys, unsigned long long *cnt)
@@ -2410,12 +2453,7 @@ __global__ void __launch_bounds__(LA_THREADS) k_drown_keys(const uint64_t *ins_k
     if (threadIdx.x == 0 && tot) base = atomicAdd(&cnt[G4D_CNT_DROWN_KEYS], (unsigned long long)tot);
     __syncthreads();
     uint64_t *out = keys + base + at;
-    for (; bits; bits &= bits - 1) {
-        const uint64_t k = ins_keys[i0 + __builtin_ctz(bits)];
-        const uint32_t st = (uint32_t)(k >> 32), v = (uint32_t)k;
-        const uint32_t mn = st < v ? st : v, mx = st < v ? v : st;
-        *out++ = ((uint64_t)mn << 33) | ((uint64_t)mx << 1) | (uint64_t)(st == mn ? 0 : 1);
-    }
+    for (; bits; bits &= bits - 1) *out++ = drown_key(ins_keys[i0 + __builtin_ctz(bits)]);
 }
 
 hipError_t launch_drown_keys(const uint64_t *ins_keys, const uint8_t *dflag, int64_t m, uint64_t *keys,
@@ -2442,12 +2480,8 @@ __global__ void __launch_bounds__(LA_THREADS) k_nonmutual(const uint64_t *keys, 
         const int64_t i = b0 + j * LA_THREADS;
         task[j] = STAR_PAIR_NONE;
         if (i >= m) continue;
-        const uint64_t ki = keys[i], k = ki >> 1;
-        const bool mutual = (i > 0 && (keys[i - 1] >> 1) == k) || (i + 1 < m && (keys[i + 1] >> 1) == k);
-        if (mutual) continue;
-        const uint32_t mn = (uint32_t)(ki >> 33), mx = (uint32_t)(k & 0xffffffffu);
-        task[j] = (ki & 1) ? (((uint64_t)mx << 32) | mn) : (((uint64_t)mn << 32) | mx);
-        c++;
+        task[j] = drown_task(keys[i], i > 0 ? keys[i - 1] : ~0ull, i + 1 < m ? keys[i + 1] : ~0ull);
+        c += task[j] != STAR_PAIR_NONE ? 1 : 0;
     }
     int tot;
     int at = la_excl(c, red, &tot);
@@ -2464,6 +2498,67 @@ hipError_t launch_nonmutual(const uint64_t *keys, int64_t m, uint64_t *tasks, un
     const int64_t nb = (m + LA_THREADS * NM_ITEMS - 1) / (LA_THREADS * NM_ITEMS);
     if (nb > INT32_MAX) return hipErrorInvalidValue;
     hipLaunchKernelGGL(k_nonmutual, dim3((unsigned)nb), dim3(LA_THREADS), 0, s, keys, m, tasks, cnt);
+    return hipGetLastError();
+}
+
+// The drowned insertions of a late round, at most DROWN_SMALL of them, to proof tasks in one launch:
+// the keys collected in LDS, a bitonic sort, and the tasks of the ones that are not mutual, in the
+// place of three launches and the gaps between them.  Bound by latency: 13-17 us for up to a thousand
+// drowned, 24 us for 1,700 of 4,600 insertions, as long as the three kernels alone took.
+__global__ void __launch_bounds__(1024) k_drown_small(const uint64_t *ins_keys, const uint8_t *dflag, int m, int nd,
+                                                      uint64_t *tasks, unsigned long long *cnt)
+{
+    __shared__ uint64_t a[DROWN_SMALL];
+    __shared__ int have, ntask;
+    const int tid = threadIdx.x, lane = __lane_id();
+    int n = 128;
+    while (n < nd) n <<= 1;
+    for (int i = tid; i < n; i += 1024) a[i] = ~0ull;
+    if (tid == 0) have = ntask = 0;
+    __syncthreads();
+    // four flags a thread: their keys' reads are the chain here
+    for (int i0 = tid * 4; i0 < m; i0 += 1024 * 4) {
+        const uint32_t f = *reinterpret_cast<const uint32_t *>(dflag + i0);
+        uint64_t k[4];
+        bool d[4];
+        int c = 0;
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            d[j] = i0 + j < m && ((f >> (8 * j)) & 1u);
+            k[j] = d[j] ? ins_keys[i0 + j] : 0ull;
+            c += d[j] ? 1 : 0;
+        }
+        int at = c ? atomicAdd(&have, c) : 0;
+#pragma unroll
+        for (int j = 0; j < 4; j++)
+            if (d[j]) {
+                if (at < DROWN_SMALL) a[at] = drown_key(k[j]);
+                at++;
+            }
+    }
+    __syncthreads();
+    lds_bitonic<1024>(a, n);
+    const int c = min(have, DROWN_SMALL);
+    for (int i0 = 0; i0 < c; i0 += 1024) {
+        const int i = i0 + tid;
+        uint64_t task = STAR_PAIR_NONE;
+        if (i < c) task = drown_task(a[i], i > 0 ? a[i - 1] : ~0ull, i + 1 < c ? a[i + 1] : ~0ull);
+        const uint64_t mk = __ballot(task != STAR_PAIR_NONE);
+        int at = 0;
+        if (lane == 0 && mk) at = atomicAdd(&ntask, __popcll(mk));
+        at = __builtin_amdgcn_readfirstlane(at) + __popcll(mk & ((1ull << lane) - 1ull));
+        if (task != STAR_PAIR_NONE) tasks[at] = task;
+    }
+    __syncthreads();
+    if (tid == 0) cnt[G4D_CNT_TASKS] = (unsigned long long)ntask;
+}
+
+hipError_t launch_drown_small(const uint64_t *ins_keys, const uint8_t *dflag, int64_t m, int64_t nd, uint64_t *tasks,
+                              unsigned long long *cnt, hipStream_t s)
+{
+    if (nd <= 0 || m <= 0) return hipSuccess;
+    if (nd > DROWN_SMALL || m > DROWN_SMALL_INS) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(k_drown_small, dim3(1), dim3(1024), 0, s, ins_keys, dflag, (int)m, (int)nd, tasks, cnt);
     return hipGetLastError();
 }
 
@@ -2707,22 +2802,11 @@ __global__ void __launch_bounds__(SR_THREADS) k_small_round(PassPlan p, uint64_t
     const unsigned long long np = p.cnt[G4D_CNT_NEW_PAIRS];
     if (np == 0 || np > STAR_ROUND_SMALL / 2) return;
     const int m = 2 * (int)np;
-    int n = SR_THREADS;
+    int n = 128;
     while (n < m) n <<= 1;
     for (int i = tid; i < n; i += SR_THREADS) a[i] = i < m ? keys[i] : ~0ull;
     __syncthreads();
-    for (int k = 2; k <= n; k <<= 1)
-        for (int j = k >> 1; j > 0; j >>= 1) {
-            for (int x = tid; x < n / 2; x += SR_THREADS) {
-                const int i = ((x & ~(j - 1)) << 1) | (x & (j - 1)), l = i | j;
-                const uint64_t u = a[i], w = a[l];
-                if ((u > w) == ((i & k) == 0)) {
-                    a[i] = w;
-                    a[l] = u;
-                }
-            }
-            __syncthreads();
-        }
+    lds_bitonic<SR_THREADS>(a, n);
     // repeats out, in order
     int cnt = 0;
     for (int i0 = 0, r = 0; i0 < m; i0 += SR_THREADS, r ^= 1) {
