@@ -101,7 +101,7 @@ struct g4d_ctx {
     DevBuf xyz_up, keys, pts, perm, vox, bounds, settab, ptset, grid, gtmp, idgrid, pbaspill, pbaenv, pbacnt, pcount, pairs,
         ws_off, cnt;
     Store store;
-    DevBuf settet, dflag, pairbuf, spcount, dkeys, tasks, cand, ins, ins_off, vcap, tcap, hcap, active, mid, big, huge, xstars,
+    DevBuf settet, dflag, pairbuf, spcount, dkeys, tasks, cand, ins, ins_off, active, mid, big, huge, xstars,
         xtasks, xtris, gwork, tetcnt, tetoff, tets, opp, table;
     // learned proposal: parameters, candidates, features, proposed pairs, capacity bins, labels
     DevBuf mlp_params, fkeys, ford, frank, pcand, pd2, pfeat, ppairs, pcap, plab, pvcap;
@@ -653,8 +653,10 @@ static int run_device(g4d_ctx *ctx, const double *d_xyz, int n, const SetSpec &s
     if (batched) HCK(g4d::launch_set_bounds(d_xyz, GS, dbounds, s));
     else HCK(g4d::launch_bounds(d_xyz, n, dbounds, s));
     {
-        std::vector<double> hb(2 * (size_t)S);
-        HCK(hipMemcpyAsync(hb.data(), dbounds, sizeof(double) * 2 * (size_t)S, hipMemcpyDeviceToHost, s));
+        std::vector<double> hv(2 * (size_t)S);
+        int64_t *slot = S == 1 ? hslot(ctx, 10, nullptr) : nullptr; // two slots
+        double *hb = slot ? reinterpret_cast<double *>(slot) : hv.data();
+        HCK(hipMemcpyAsync(hb, dbounds, sizeof(double) * 2 * (size_t)S, hipMemcpyDeviceToHost, s));
         HCK(hipStreamSynchronize(s));
         for (int k = 0; k < S; k++)
             if (!std::isfinite(hb[2 * k]) || !std::isfinite(hb[2 * k + 1]) || !(hb[2 * k + 1] > hb[2 * k]))
@@ -671,7 +673,12 @@ static int run_device(g4d_ctx *ctx, const double *d_xyz, int n, const SetSpec &s
     double *pts = buf<double>(ctx->pts);
     int *perm = buf<int>(ctx->perm);
     uint64_t *vox = buf<uint64_t>(ctx->vox);
-    HCK(g4d::launch_gather_sorted(d_xyz, keys, n, GS, pts, perm, vox, s));
+    Store &store = ctx->store;
+    HCK(store.vnum.ensure(sizeof(int) * (size_t)n));
+    HCK(store.tnum.ensure(sizeof(int) * (size_t)n));
+    HCK(store.hnum.ensure(sizeof(int) * (size_t)n));
+    const g4d::StarRecords rec = {buf<int>(store.vnum), buf<int>(store.tnum), buf<int>(store.hnum)};
+    HCK(g4d::launch_gather_sorted(d_xyz, keys, n, GS, pts, perm, vox, rec, s));
     HCK(g4d::launch_dup_check(pts, vox, n, GS, cnt, s));
     ev_record(ctx, EV_MORTON);
 
@@ -713,27 +720,26 @@ static int run_device(g4d_ctx *ctx, const double *d_xyz, int n, const SetSpec &s
     CK(guard_keys(ctx, 2 * (ngp + (int64_t)n), "grid pairs"));
     const int64_t ucap = ngp + n;
     const int64_t prop_room = ctx->prop_on ? 2 * (int64_t)g4d::PROP_SLOTS * n : 0;
-    HCK(ctx->pairs.ensure(sizeof(uint64_t) * (size_t)(2 * ucap + prop_room + 2 * (int64_t)n * min_ws + 64)));
-    uint64_t *pr = buf<uint64_t>(ctx->pairs);
-    HCK(g4d::launch_grid_pairs_dedup(idg, GS, ntiles, pcnt, pr + ucap, tcnt, ttot, s));
+    // the keys, both directions, and behind them the tiles' raw regions; after the sort the pumped
+    // and proposed keys in their place
+    HCK(ctx->pairs.ensure(sizeof(uint64_t) *
+                          (size_t)(2 * ucap + std::max<int64_t>(ngp, prop_room + 2 * (int64_t)n * min_ws + 64))));
+    uint64_t *pr = buf<uint64_t>(ctx->pairs), *raw = pr + 2 * ucap;
+    HCK(g4d::launch_grid_pairs_dedup(idg, GS, ntiles, pcnt, raw, tcnt, ttot, s));
     HCK(g4d::scan_excl_i64(P, ttot, ttot, ntiles, ttot + ntiles, s));
-    HCK(g4d::launch_gather_tiles(pr + ucap, pcnt, tcnt, ntiles, ttot, pr, s));
-    HCK(hipMemsetAsync(cnt + G4D_CNT_APPEND0, 0, 8, s));
-    HCK(g4d::launch_missing(vox, n, GS, idg, pr + ucap + ngp, cnt + G4D_CNT_APPEND0, n, s));
+    HCK(g4d::launch_gather_tiles(raw, pcnt, tcnt, ntiles, ttot, pr, s));
+    HCK(g4d::launch_missing(vox, n, GS, idg, ttot + ntiles, pr, cnt + G4D_CNT_MISSING, s));
     int64_t ngd_f = 0, *ngd_h = hslot(ctx, 1, &ngd_f);
     HCK(hipMemcpyAsync(ngd_h, ttot + ntiles, 8, hipMemcpyDeviceToHost, s));
     CK(read_counters(ctx, hc));
     const int64_t ngd = *ngd_h;
     CK(check_dev_error(ctx, hc[G4D_CNT_ERROR], "morton"));
-    const int64_t nmiss = (int64_t)hc[G4D_CNT_APPEND0];
-    if (nmiss > 0)
-        HCK(hipMemcpyAsync(pr + ngd, pr + ucap + ngp, sizeof(uint64_t) * (size_t)nmiss, hipMemcpyDeviceToDevice, s));
+    const int64_t nmiss = (int64_t)hc[G4D_CNT_MISSING];
     trace("n %d in %d set(s), grid %d: grid pairs %lld raw, %lld after tile dedup, missing %lld", n, S, gmax,
           (long long)ngp, (long long)ngd, (long long)nmiss);
     // Both directions of every pair, then one sort and one unique: each distinct pair leaves
     // exactly its two directed keys (a missing point appears in no grid pair).
     const int64_t u = ngd + nmiss;
-    HCK(g4d::launch_reciprocate(pr, u, s));
     int64_t m = 2 * u;
     HCK(sort_unique_pairs(P, pr, &m, nb, n, s));
     ctx->st.num_missing = nmiss;
@@ -750,10 +756,9 @@ static int run_device(g4d_ctx *ctx, const double *d_xyz, int n, const SetSpec &s
         HCK(g4d::launch_csr_offsets(pr, m, n, ws_off, s));
     }
     ev_record(ctx, EV_PROP1);
-    HCK(hipMemsetAsync(cnt + G4D_CNT_APPEND0, 0, 8, s));
-    HCK(g4d::launch_pump(pr, ws_off, n, GS, min_ws, pr + m, cnt + G4D_CNT_APPEND0, 2 * (int64_t)n * min_ws + 64, s));
+    HCK(g4d::launch_pump(pr, ws_off, n, GS, min_ws, pr + m, cnt + G4D_CNT_PUMPED, 2 * (int64_t)n * min_ws + 64, s));
     CK(read_counters(ctx, hc));
-    const int64_t npump = (int64_t)hc[G4D_CNT_APPEND0];
+    const int64_t npump = (int64_t)hc[G4D_CNT_PUMPED];
     if (npump > 0) {
         // A pumped candidate is not in the star's list, and the lists are symmetric, so no
         // pumped key is already present: sort and deduplicate the pumped keys alone (two stars
@@ -768,39 +773,26 @@ static int run_device(g4d_ctx *ctx, const double *d_xyz, int n, const SetSpec &s
         HCK(hipMemcpyAsync(pr, merged, sizeof(uint64_t) * (size_t)(m + np), hipMemcpyDeviceToDevice, s));
         ctx->st.num_pumped = np;
         m += np;
-        HCK(g4d::launch_csr_offsets(pr, m, n, ws_off, s));
     }
     ctx->st.num_workset = m;
     trace("worksets %lld keys (%lld pumped)", (long long)m, (long long)ctx->st.num_pumped);
     ev_record(ctx, EV_PAIRS);
 
     // ---- E: star creation (GD/GDelaunay/GDelHost.cu:543-743) ----
-    HCK(ctx->vcap.ensure(sizeof(int64_t) * (size_t)(n + 1)));
-    HCK(ctx->tcap.ensure(sizeof(int64_t) * (size_t)(n + 1)));
-    HCK(ctx->hcap.ensure(sizeof(int64_t) * (size_t)(n + 1)));
     HCK(ctx->mid.ensure(sizeof(int) * (size_t)n));
     HCK(ctx->big.ensure(sizeof(int) * (size_t)n));
     HCK(ctx->huge.ensure(sizeof(int) * (size_t)n));
     HCK(ctx->xstars.ensure(sizeof(int) * (size_t)n));
-    int64_t *vcap = buf<int64_t>(ctx->vcap), *tcap = buf<int64_t>(ctx->tcap), *hcap = buf<int64_t>(ctx->hcap);
     const int nblk_star = 5120; // 256 CUs x 20 resident waves of the 32-vertex tier (5 per SIMD)
     const int lds_limit = std::min(g4d::STAR_LDS_LIMIT, ctx->opt.lds_star_limit > 0 ? ctx->opt.lds_star_limit
                                                                                   : g4d::STAR_LDS_LIMIT);
 
-    Store &store = ctx->store;
-    HCK(store.vnum.ensure(sizeof(int) * (size_t)n));
-    HCK(store.tnum.ensure(sizeof(int) * (size_t)n));
-    HCK(store.hnum.ensure(sizeof(int) * (size_t)n));
     HCK(store.voff.ensure(sizeof(int64_t) * (size_t)n));
     HCK(store.toff.ensure(sizeof(int64_t) * (size_t)n));
     HCK(store.hoff.ensure(sizeof(int64_t) * (size_t)n));
     HCK(store.nvoff.ensure(sizeof(int64_t) * (size_t)n));
     HCK(store.ntoff.ensure(sizeof(int64_t) * (size_t)n));
     HCK(store.nhoff.ensure(sizeof(int64_t) * (size_t)n));
-    // empty records until a star is built (a star that fails is reported, never read)
-    HCK(hipMemsetAsync(store.vnum.ptr, 0, sizeof(int) * (size_t)n, s));
-    HCK(hipMemsetAsync(store.tnum.ptr, 0, sizeof(int) * (size_t)n, s));
-    HCK(hipMemsetAsync(store.hnum.ptr, 0, sizeof(int) * (size_t)n, s));
     store.top[0] = store.top[1] = store.top[2] = 0;
     store.repacks = 0;
 
@@ -809,7 +801,7 @@ static int run_device(g4d_ctx *ctx, const double *d_xyz, int n, const SetSpec &s
     HCK(ctx->active.ensure(sizeof(int) * (size_t)n));
     int *active = buf<int>(ctx->active);
     HCK(ctx->ins_off.ensure(sizeof(int64_t) * (size_t)(n + 1)));
-    // splaying: the next pass's plan (regions from the arenas' tops as they are when it is launched)
+    // the next pass's plan (regions from the arenas' tops as they are when it is launched)
     auto pass_plan = [&]() {
         g4d::PassPlan pl;
         for (int k = 0; k < 3; k++) pl.base[k] = store.top[k];
@@ -826,28 +818,19 @@ static int run_device(g4d_ctx *ctx, const double *d_xyz, int n, const SetSpec &s
     };
     int64_t tbase_last = 0;
 
-    // One pass over the stars with insertions (mode 0: every star, from its workset; mode 1: the
-    // nitems stars of the active list, whose regions of need[] elements are planned).  Each such
-    // star gets a fresh region at the arenas' tops; the others are not touched.  Returns the
-    // drowned insertions and the insertion pairs of the pass.
+    // One pass over the nitems stars of the active list (mode 0: every star, from its workset), whose
+    // regions of need[] elements are planned at the arenas' tops; the others are not touched.
+    // Returns the drowned insertions and the insertion pairs of the pass.
     auto star_pass = [&](int mode, const uint64_t *ins_keys, const int64_t *ins_off, int64_t nins, int nitems,
-                         int64_t *need, int64_t *drown_n, int64_t *tp_n) -> int {
-        const int *list = mode ? active : nullptr;
+                         const int64_t *need, int64_t *drown_n, int64_t *tp_n) -> int {
+        const int *list = active;
         if (mode == 0) {
-            HCK(g4d::launch_capacities(n, ins_off, vcap, tcap, hcap, spc, s));
-            int64_t *caps[3] = {vcap, tcap, hcap};
-            int64_t *need_h = hslot(ctx, 3, need); // three slots
-            for (int k = 0; k < 3; k++) {
-                HCK(g4d::scan_excl_i64(P, caps[k], caps[k], n, caps[k] + n, s));
-                HCK(hipMemcpyAsync(&need_h[k], caps[k] + n, 8, hipMemcpyDeviceToHost, s));
-            }
-            HCK(g4d::launch_assign_regions(n, vcap, tcap, hcap, buf<int64_t>(store.nvoff), buf<int64_t>(store.ntoff),
-                                           buf<int64_t>(store.nhoff), s));
-            HCK(hipStreamSynchronize(s));
-            for (int k = 0; k < 3; k++) need[k] = need_h[k];
-            // room for the splaying rounds: their regions come to about twice the creation's;
-            // with the proposal's predicted link sizes, room for that many rebuilt stars too
-            int64_t want[3] = {3 * need[0], 3 * need[1], 3 * need[2]};
+            // Room for the splaying rounds: their regions come to about twice the creation's (in a
+            // small set sometimes more, and there a repack costs as much as a round: 4 MB at
+            // 32,768 points); with the proposal's predicted link sizes, room for that many rebuilt
+            // stars too.
+            const int64_t times = n <= 32768 ? 4 : 3;
+            int64_t want[3] = {times * need[0], times * need[1], times * need[2]};
             if (pred_vertices > 0) {
                 want[0] = std::max(want[0], 3 * pred_vertices);
                 want[1] = std::max(want[1], 3 * (2 * pred_vertices - 4 * (int64_t)n));
@@ -1031,12 +1014,20 @@ static int run_device(g4d_ctx *ctx, const double *d_xyz, int n, const SetSpec &s
         return G4D_OK;
     };
 
-    int64_t nd = 0, ntp = 0, need[3] = {0, 0, 0};
-    const uint64_t *pass_keys = pr; // the last pass's insertions, and its stars
+    int64_t nd = 0, ntp = 0, need[3];
+    const uint64_t *pass_keys = pr; // the last pass's insertions, and the number of its stars
     int64_t pass_n = m;
-    const int *pass_list = nullptr;
     int pass_items = n;
-    CK(star_pass(0, pr, ws_off, m, n, need, &nd, &ntp));
+    auto read_needs = [&]() {
+        need[0] = (int64_t)hc[G4D_CNT_NEED_V];
+        need[1] = (int64_t)hc[G4D_CNT_NEED_T];
+        need[2] = (int64_t)hc[G4D_CNT_NEED_H];
+    };
+    HCK(g4d::launch_pass_plan(pass_plan(), pr, m, nullptr, s));
+    CK(read_counters(ctx, hc));
+    if ((int64_t)hc[G4D_CNT_ACTIVE] != n) return set_err(ctx, G4D_ERR_INTERNAL, "a star has no candidates");
+    read_needs();
+    CK(star_pass(0, pr, buf<int64_t>(ctx->ins_off), m, n, need, &nd, &ntp));
     ev_record(ctx, EV_STAR);
 
     // ---- F: splaying rounds (GD/GDelaunay/GDelHost.cu:1389-1470) ----
@@ -1096,7 +1087,7 @@ static int run_device(g4d_ctx *ctx, const double *d_xyz, int n, const SetSpec &s
             HCK(ctx->ins.ensure(sizeof(uint64_t) * (size_t)(2 * ncand + 2)));
             uint64_t *ins = buf<uint64_t>(ctx->ins);
             g4d::NewPairs np;
-            np.list = pass_list;
+            np.list = active;
             np.nitems = pass_items;
             np.pcount = spc;
             np.ntoff = buf<int64_t>(store.ntoff);
@@ -1139,11 +1130,8 @@ static int run_device(g4d_ctx *ctx, const double *d_xyz, int n, const SetSpec &s
         ctx->st.splay_insertions += nrec;
         pass_keys = buf<uint64_t>(ctx->ins);
         pass_n = nrec;
-        pass_list = active;
         pass_items = (int)hc[G4D_CNT_ACTIVE];
-        need[0] = (int64_t)hc[G4D_CNT_NEED_V];
-        need[1] = (int64_t)hc[G4D_CNT_NEED_T];
-        need[2] = (int64_t)hc[G4D_CNT_NEED_H];
+        read_needs();
         CK(star_pass(1, pass_keys, buf<int64_t>(ctx->ins_off), nrec, pass_items, need, &nd, &ntp));
     }
     if (!converged) return set_err(ctx, G4D_ERR_NOT_CONVERGED, "splaying did not converge in %d rounds", rounds);
@@ -1166,24 +1154,34 @@ static int run_device(g4d_ctx *ctx, const double *d_xyz, int n, const SetSpec &s
     op.star_tet_off = buf<int64_t>(ctx->tetoff);
     op.cnt = cnt;
     op.tets = nullptr;
-    // owner triangles the orient3d filter cannot decide: exact pass marks the ones to keep
+    op.perm = !batched && ctx->opt.index_space == G4D_INDEX_INPUT ? perm : nullptr;
+    // Owner triangles the orient3d filter cannot decide go to a list whose exact pass marks the ones to
+    // keep.  The counts are scanned and read along with the list's length, so that a set without
+    // such triangles waits once; with some, the exact pass and the scan follow.
+    int64_t *toffs = buf<int64_t>(ctx->tetoff);
+    int64_t nt_f = 0, *nt_h = hslot(ctx, 8, &nt_f);
+    auto scan_tets = [&]() -> int {
+        HCK(g4d::scan_excl_i64(P, buf<int64_t>(ctx->tetcnt), toffs, n, toffs + n, s));
+        HCK(hipMemcpyAsync(nt_h, toffs + n, 8, hipMemcpyDeviceToHost, s));
+        return G4D_OK;
+    };
     int64_t xcap = std::max<int64_t>(n / 16, 4096);
     for (int attempt = 0; attempt < 2; attempt++) {
         HCK(ctx->xtris.ensure(sizeof(uint64_t) * (size_t)xcap));
-        HCK(hipMemsetAsync(cnt + G4D_CNT_APPEND5, 0, 8, s));
+        if (attempt) HCK(g4d::launch_zero_counters(cnt, 1ull << G4D_CNT_OUT_EXACT, s));
         HCK(g4d::launch_out_flag(op, buf<uint64_t>(ctx->xtris), xcap, s));
+        CK(scan_tets());
         CK(read_counters(ctx, hc));
-        if ((int64_t)hc[G4D_CNT_APPEND5] <= xcap) break;
-        xcap = (int64_t)hc[G4D_CNT_APPEND5];
+        if ((int64_t)hc[G4D_CNT_OUT_EXACT] <= xcap) break;
+        xcap = (int64_t)hc[G4D_CNT_OUT_EXACT];
     }
-    const int64_t nxt = (int64_t)hc[G4D_CNT_APPEND5];
+    const int64_t nxt = (int64_t)hc[G4D_CNT_OUT_EXACT];
     if (nxt > xcap) return set_err(ctx, G4D_ERR_INTERNAL, "output exact list sizing failed");
-    HCK(g4d::launch_out_exact(op, buf<uint64_t>(ctx->xtris), nxt, s));
-    int64_t *toffs = buf<int64_t>(ctx->tetoff);
-    HCK(g4d::scan_excl_i64(P, buf<int64_t>(ctx->tetcnt), toffs, n, toffs + n, s));
-    int64_t nt_f = 0, *nt_h = hslot(ctx, 8, &nt_f);
-    HCK(hipMemcpyAsync(nt_h, toffs + n, 8, hipMemcpyDeviceToHost, s));
-    HCK(hipStreamSynchronize(s));
+    if (nxt > 0) {
+        HCK(g4d::launch_out_exact(op, buf<uint64_t>(ctx->xtris), nxt, s));
+        CK(scan_tets());
+        HCK(hipStreamSynchronize(s));
+    }
     const int64_t nt = *nt_h;
     CK(guard_tets(ctx, nt));
     HCK(ctx->tets.ensure(sizeof(int) * 4 * (size_t)std::max<int64_t>(nt, 1)));
@@ -1209,8 +1207,6 @@ static int run_device(g4d_ctx *ctx, const double *d_xyz, int n, const SetSpec &s
         HCK(hipMemcpyAsync(ctx->h_set_tet_off.data(), tet_off, sizeof(int64_t) * (size_t)(S + 1), hipMemcpyDeviceToHost,
                            s));
         ctx->h_set_grid = spec.g;
-    } else if (ctx->opt.index_space == G4D_INDEX_INPUT) {
-        HCK(g4d::launch_map_perm(buf<int>(ctx->tets), 4 * nt, perm, s));
     }
     ev_record(ctx, EV_ADJ);
     if (ctx->prop_export) {
@@ -1319,8 +1315,7 @@ void g4d_destroy(g4d_ctx *ctx)
     if (ctx->stream) (void)hipStreamSynchronize(ctx->stream);
     DevBuf *bufs[] = {&ctx->xyz_up, &ctx->keys, &ctx->pts, &ctx->perm, &ctx->vox, &ctx->bounds, &ctx->settab, &ctx->ptset, &ctx->grid,
                       &ctx->gtmp, &ctx->idgrid, &ctx->pbaspill, &ctx->pbaenv, &ctx->pbacnt, &ctx->pcount, &ctx->pairs, &ctx->ws_off, &ctx->cnt, &ctx->settet, &ctx->dflag, &ctx->pairbuf, &ctx->spcount, &ctx->dkeys,
-                      &ctx->tasks, &ctx->cand, &ctx->ins, &ctx->ins_off, &ctx->vcap, &ctx->tcap,
-                      &ctx->hcap, &ctx->active, &ctx->mid, &ctx->big, &ctx->huge, &ctx->xstars, &ctx->xtasks, &ctx->xtris, &ctx->gwork, &ctx->tetcnt, &ctx->tetoff, &ctx->tets, &ctx->opp, &ctx->table,
+                      &ctx->tasks, &ctx->cand, &ctx->ins, &ctx->ins_off, &ctx->active, &ctx->mid, &ctx->big, &ctx->huge, &ctx->xstars, &ctx->xtasks, &ctx->xtris, &ctx->gwork, &ctx->tetcnt, &ctx->tetoff, &ctx->tets, &ctx->opp, &ctx->table,
                       &ctx->mlp_params, &ctx->fkeys, &ctx->ford, &ctx->frank, &ctx->pcand, &ctx->pd2, &ctx->pfeat,
                       &ctx->ppairs, &ctx->pcap, &ctx->plab, &ctx->pvcap};
     destroy_graphs(ctx);
@@ -1854,7 +1849,7 @@ int g4d_diag_morton(g4d_ctx *ctx, const double *xyz, int32_t n, int32_t grid, in
     HCK(g4d::launch_morton_keys(d_xyz, n, GS, buf<uint64_t>(ctx->keys), s));
     HCK(g4d::radix_sort_u64(ctx->P, buf<uint64_t>(ctx->keys), n, GS.key_shift, 64, s));
     HCK(g4d::launch_gather_sorted(d_xyz, buf<uint64_t>(ctx->keys), n, GS, buf<double>(ctx->pts), buf<int>(ctx->perm),
-                                  buf<uint64_t>(ctx->vox), s));
+                                  buf<uint64_t>(ctx->vox), {}, s));
     std::vector<uint64_t> vs((size_t)n);
     HCK(hipMemcpyAsync(perm_out, ctx->perm.ptr, sizeof(int) * (size_t)n, hipMemcpyDeviceToHost, s));
     HCK(hipMemcpyAsync(vs.data(), ctx->vox.ptr, sizeof(uint64_t) * (size_t)n, hipMemcpyDeviceToHost, s));
@@ -2161,13 +2156,14 @@ int g4d_diag_grid_pairs(g4d_ctx *ctx, const int32_t *id_grid, int32_t grid, uint
     int64_t raw = 0, m = 0;
     HCK(hipMemcpyAsync(&raw, pcnt + ntiles, 8, hipMemcpyDeviceToHost, s));
     HCK(hipStreamSynchronize(s));
-    HCK(ctx->pairs.ensure(sizeof(uint64_t) * (size_t)std::max<int64_t>(2 * raw, 1)));
+    HCK(ctx->pairs.ensure(sizeof(uint64_t) * (size_t)std::max<int64_t>(3 * raw, 1)));
     uint64_t *pr = buf<uint64_t>(ctx->pairs);
-    HCK(g4d::launch_grid_pairs_dedup(buf<int>(ctx->gtmp), GS, ntiles, pcnt, pr + raw, tcnt, ttot, s));
+    HCK(g4d::launch_grid_pairs_dedup(buf<int>(ctx->gtmp), GS, ntiles, pcnt, pr + 2 * raw, tcnt, ttot, s));
     HCK(g4d::scan_excl_i64(ctx->P, ttot, ttot, ntiles, ttot + ntiles, s));
-    HCK(g4d::launch_gather_tiles(pr + raw, pcnt, tcnt, ntiles, ttot, pr, s));
+    HCK(g4d::launch_gather_tiles(pr + 2 * raw, pcnt, tcnt, ntiles, ttot, pr, s));
     HCK(hipMemcpyAsync(&m, ttot + ntiles, 8, hipMemcpyDeviceToHost, s));
     HCK(hipStreamSynchronize(s));
+    m *= 2;
     int maxid = 0;
     for (int64_t i = 0; i < G3; i++) maxid = std::max(maxid, id_grid[i]);
     const int nb = bits_for((int64_t)maxid + 1);
@@ -2177,6 +2173,7 @@ int g4d_diag_grid_pairs(g4d_ctx *ctx, const int32_t *id_grid, int32_t grid, uint
     HCK(hipStreamSynchronize(s));
     int64_t k = 0;
     for (int64_t i = 0; i < m; i++) {
+        if ((h[(size_t)i] >> 32) > (h[(size_t)i] & 0xffffffffull)) continue; // the pair's other direction
         if (out && k < cap) out[k] = h[(size_t)i];
         k++;
     }

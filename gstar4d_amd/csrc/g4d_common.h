@@ -71,7 +71,11 @@ enum g4d_counter : int {
     G4D_CNT_NEED_V = 31,
     G4D_CNT_NEED_T = 32,
     G4D_CNT_NEED_H = 33,
-    G4D_CNT_NUM = 34
+    // zero from the start of a call, used once in it
+    G4D_CNT_MISSING = 34,
+    G4D_CNT_PUMPED = 35,
+    G4D_CNT_OUT_EXACT = 36,
+    G4D_CNT_NUM = 37
 };
 
 #define HIP_CHECK_RET(expr)                                                                    \

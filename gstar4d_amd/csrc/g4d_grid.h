@@ -37,8 +37,12 @@ hipError_t launch_set_ids(const int64_t *pt_off, int nsets, int *pt_set, hipStre
 // key_shift..64); several sets: the batched layout (sort bits 24..64).
 int morton_key_shift(int g);
 hipError_t launch_morton_keys(const double *xyz, int n, const GridSets &S, uint64_t *keys, hipStream_t s);
+// rec (may be null pointers): star records to empty, n each.
+struct StarRecords {
+    int *vnum, *tnum, *hnum;
+};
 hipError_t launch_gather_sorted(const double *xyz, const uint64_t *keys, int n, const GridSets &S, double *pts,
-                                int *perm, uint64_t *vox, hipStream_t s);
+                                int *perm, uint64_t *vox, const StarRecords &rec, hipStream_t s);
 hipError_t launch_dup_check(const double *pts, const uint64_t *vox, int n, const GridSets &S, unsigned long long *cnt,
                             hipStream_t s);
 hipError_t launch_fill_i32(int *a, int64_t n, int v, hipStream_t s);
@@ -61,9 +65,10 @@ static constexpr int PBA_MAX_BANDS = 16;
 hipError_t pba_pass_banded(int axis, const GridSets &S, int64_t nblocks, int bands, const int *in, int *out,
                            const int *idgrid, int *spill, int *benv, int *bcnt, int *fcnt, const uint64_t *vox,
                            hipStream_t s);
-// Ordered pairs (min<<32 | max) of each non-leader point with its voxel's leader.
-hipError_t launch_missing(const uint64_t *vox, int n, const GridSets &S, const int *grid, uint64_t *out,
-                          unsigned long long *counter, int64_t cap, hipStream_t s);
+// Both directed keys of each non-leader point with its voxel's leader, behind the *first pairs (of
+// two keys) in out; the counter counts pairs.
+hipError_t launch_missing(const uint64_t *vox, int n, const GridSets &S, const int *grid, const int64_t *first,
+                          uint64_t *out, unsigned long long *counter, hipStream_t s);
 // Voronoi-neighbour pairs (min<<32 | max) by tiles of 256 threads, 16 x 16 columns by
 // grid_pair_chunk cubes (for the sets' grids g together); pair_thr[nsets] / 256 tiles in all.
 int grid_pair_chunk(const int *g, int nsets);
@@ -72,7 +77,8 @@ int64_t grid_pair_threads(int g, int zc);
 hipError_t launch_grid_pair_count(const int *grid, const GridSets &S, int64_t ntiles, int64_t *count, hipStream_t s);
 // Every tile's pairs, deduplicated on chip: tile b writes into its raw region [off[b], off[b + 1])
 // and reports (distinct, overflow) counts in cnt[b] and their sum in tot[b], whose exclusive scan
-// gives the dense offsets for launch_gather_tiles.
+// gives the dense offsets for launch_gather_tiles
+// (both directed keys of every pair, dst 16-byte aligned).
 hipError_t launch_grid_pairs_dedup(const int *grid, const GridSets &S, int64_t ntiles, const int64_t *off,
                                    uint64_t *out, uint2 *cnt, int64_t *tot, hipStream_t s);
 hipError_t launch_gather_tiles(const uint64_t *src, const int64_t *off, const uint2 *cnt, int64_t ntiles,

@@ -415,6 +415,39 @@ __global__ void __launch_bounds__(BK_THREADS) k_bk_count(const uint64_t *keys, i
         if (h[i]) atomicAdd(&count[i], h[i]);
 }
 
+// Bucket offsets (nbkt + 1 of them) and the scatter's cursors from the counts, in place of a scan's
+// two or three launches and a copy; nbkt <= BK_MAX_BUCKETS.
+__global__ void __launch_bounds__(BK_THREADS) k_bk_offsets(uint32_t *count, uint32_t *off, int nbkt)
+{
+    constexpr int R = BK_MAX_BUCKETS / BK_THREADS, W = BK_THREADS / 64;
+    __shared__ uint32_t wsum[W];
+    const int lane = __lane_id(), wid = threadIdx.x >> 6;
+    const int r = (nbkt + BK_THREADS - 1) / BK_THREADS, i0 = threadIdx.x * r;
+    uint32_t c[R], sum = 0;
+#pragma unroll
+    for (int j = 0; j < R; j++) {
+        c[j] = j < r && i0 + j < nbkt ? count[i0 + j] : 0u;
+        sum += c[j];
+    }
+    const uint32_t inc = wave_incl_scan_t<uint32_t>(sum);
+    if (lane == 63) wsum[wid] = inc;
+    __syncthreads();
+    uint32_t run = inc - sum, all = 0;
+#pragma unroll
+    for (int w = 0; w < W; w++) {
+        if (w < wid) run += wsum[w];
+        all += wsum[w];
+    }
+#pragma unroll
+    for (int j = 0; j < R; j++)
+        if (j < r && i0 + j < nbkt) {
+            off[i0 + j] = run;
+            count[i0 + j] = run;
+            run += c[j];
+        }
+    if (threadIdx.x == 0) off[nbkt] = all;
+}
+
 __global__ void __launch_bounds__(BK_THREADS) k_bk_scatter(const uint64_t *keys, int64_t m, int sh, int nbkt,
                                                            int tile, uint32_t *cursor, uint64_t *out)
 {
@@ -698,10 +731,11 @@ static hipError_t bucket_sort(Prims &P, uint64_t *keys, int64_t m, int ash, int 
 {
     const int nbkt = 1 << (na - sb);
     HIP_CHECK_RET(P.sort_tmp_keys.ensure(sizeof(uint64_t) * (size_t)m));
-    HIP_CHECK_RET(P.sort_hist.ensure(sizeof(uint32_t) * (size_t)(2 * nbkt + 2)));
+    HIP_CHECK_RET(P.sort_hist.ensure(sizeof(uint32_t) * (size_t)(2 * nbkt + 5)));
     uint64_t *tmp = P.sort_tmp_keys.as<uint64_t>();
-    uint32_t *count = P.sort_hist.as<uint32_t>(), *off = count + nbkt + 1;
-    HIP_CHECK_RET(hipMemsetAsync(count, 0, sizeof(uint32_t) * (size_t)(nbkt + 1), s));
+    uint32_t *count = P.sort_hist.as<uint32_t>(), *off = count + ((nbkt + 3) & ~3);
+    // a whole number of 16 bytes is one fill, an odd rest a second
+    HIP_CHECK_RET(hipMemsetAsync(count, 0, sizeof(uint32_t) * (size_t)((nbkt + 3) & ~3), s));
     // tiles of up to BK_TILE keys, at least ~512 of them
     const int64_t want = (m + 511) / 512;
     const int tile = (int)std::min<int64_t>(
@@ -710,8 +744,8 @@ static hipError_t bucket_sort(Prims &P, uint64_t *keys, int64_t m, int ash, int 
     const int sh = ash + sb;
     hipLaunchKernelGGL(k_bk_count, dim3((unsigned)nblk), dim3(BK_THREADS), 0, s, keys, m, sh, nbkt, tile, count);
     HIP_CHECK_RET(hipGetLastError());
-    HIP_CHECK_RET(scan_excl_u32(P, count, off, nbkt + 1, s)); // off[nbkt] = m
-    HIP_CHECK_RET(hipMemcpyAsync(count, off, sizeof(uint32_t) * (size_t)nbkt, hipMemcpyDeviceToDevice, s));
+    hipLaunchKernelGGL(k_bk_offsets, dim3(1), dim3(BK_THREADS), 0, s, count, off, nbkt); // off[nbkt] = m
+    HIP_CHECK_RET(hipGetLastError());
     hipLaunchKernelGGL(k_bk_scatter, dim3((unsigned)nblk), dim3(BK_THREADS), 0, s, keys, m, sh, nbkt, tile, count,
                        tmp);
     HIP_CHECK_RET(hipGetLastError());
@@ -730,6 +764,7 @@ static hipError_t bucket_sort(Prims &P, uint64_t *keys, int64_t m, int ash, int 
     }
     HIP_CHECK_RET(hipGetLastError());
     // buckets beyond LDS, if any (the others' work-groups leave at once)
+    if (m <= (int64_t)cap) return hipSuccess;
     hipLaunchKernelGGL(k_bk_sort_big<512>, dim3((unsigned)nbkt), dim3(512), 0, s, tmp, keys, off, ash, sb, nbb,
                        to_tmp ? 1 : 0, cap);
     return hipGetLastError();

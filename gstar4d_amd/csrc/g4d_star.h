@@ -190,13 +190,6 @@ static constexpr int STAR_ROUND_SMALL = 4096;
 hipError_t launch_small_round(const PassPlan &p, uint64_t *keys, hipStream_t s);
 // Reciprocate m ordered pairs in place into 2m directed keys.
 hipError_t launch_reciprocate(uint64_t *keys, int64_t m, hipStream_t s);
-// Star creation's regions: sizes per star (link vertices v = m, triangle words 2v - 4 (twice that
-// for stars that may need the wide format), history m), pcount[s] = 0; after scans, nvoff[s] =
-// vscan[s] (same for t, h).
-hipError_t launch_capacities(int n, const int64_t *ins_off, int64_t *vcap, int64_t *tcap, int64_t *hcap, int *pcount,
-                             hipStream_t s);
-hipError_t launch_assign_regions(int n, const int64_t *vscan, const int64_t *tscan, const int64_t *hscan, int64_t *nvoff,
-                                 int64_t *ntoff, int64_t *nhoff, hipStream_t s);
 // Live region sizes of every star (vertices, triangle words, history), for repacking.
 hipError_t launch_live_sizes(int n, const int *vnum, const int *tnum, const int *hnum, int64_t *vsz, int64_t *tsz,
                              int64_t *hsz, hipStream_t s);
@@ -220,11 +213,12 @@ struct OutParams {
     int64_t *star_tet_count; // per star
     const int64_t *star_tet_off;
     int *tets;               // 4 per tetra
+    const int *perm;         // null: Morton ranks; else the ids written
     unsigned long long *cnt;
 };
 // Decision pass over the owner triangles: filter-decided keeps get the keep bit in their word
 // and are counted in star_tet_count; inconclusive ones -> list (star<<32 | triangle), counter
-// G4D_CNT_APPEND5.  The exact pass keeps and counts those with exact orient3d < 0.  After the
+// G4D_CNT_OUT_EXACT.  The exact pass keeps and counts those with exact orient3d < 0.  After the
 // caller scans star_tet_count into star_tet_off, the write pass emits the kept triangles.
 hipError_t launch_out_flag(const OutParams &p, uint64_t *list, int64_t cap, hipStream_t s);
 hipError_t launch_out_exact(const OutParams &p, const uint64_t *list, int64_t m, hipStream_t s);
@@ -241,7 +235,6 @@ hipError_t launch_adjacency(const int *tets, int64_t nt, int *opp, uint32_t *tab
 // paired within tiles of 512 consecutive tetrahedra in LDS, the rest through `table`.
 hipError_t launch_adjacency_tiled(const int *tets, int64_t nt, int *opp, uint32_t *table, int64_t table_size,
                                   unsigned long long *cnt, hipStream_t s);
-hipError_t launch_map_perm(int *tets, int64_t m4, const int *perm, hipStream_t s);
 // out[i] = a[idx[i]] for i < m.
 hipError_t launch_gather_i64(const int64_t *a, const int64_t *idx, int64_t m, int64_t *out, hipStream_t s);
 // Batched output: vertex ids (sorted positions) -> input index within the set; opp (global

@@ -199,3 +199,27 @@ def test_stage_graph_replays_match_eager(orc):
                 assert np.array_equal(e1[0], ref1[0]), rep
     oracle, _, _ = orc.triangulate(single, 64)
     assert (g.canonical(ref1[0]) == oracle).all()
+
+
+@pytest.mark.parametrize("n", [5, 1365, 1366, 4097])
+def test_batch_bounds_see_every_coordinate(n):
+    """A set's bounds pass reads 4 x 1,024 coordinates at a time: the set's extremes, or a value that is
+    not finite, count wherever they lie (first, last, on both sides of a chunk's end)."""
+    rng = np.random.default_rng(n)
+    sets = [rng.random((40, 3)), rng.random((n, 3)), rng.random((60, 3))]
+    at = sorted({0, 3 * n - 1, min(4095, 3 * n - 1), min(4096, 3 * n - 1)})
+    with g.Triangulator(grid_size=64) as t:
+        off = np.cumsum([0, 40, n, 60]).astype(np.int64)
+        for i in at:
+            for bad in (np.nan, np.inf, -np.inf):
+                y = [s.copy() for s in sets]
+                y[1].reshape(-1)[i] = bad
+                with pytest.raises(g.G4DError) as e:
+                    t.triangulate_batch(np.concatenate(y), off, [16, 24, 16])
+                assert e.value.status == "INVALID_INPUT"
+            y = [s.copy() for s in sets]
+            y[1].reshape(-1)[i] = 9.5 if i % 2 else -9.5
+            tets, opp, toff, _ = t.triangulate_batch(np.concatenate(y), off, [16, 24, 16])
+            st, so = t.triangulate_batch(y[1], np.array([0, n]), [24])[:2]
+            assert np.array_equal(tets[toff[1]:toff[2]], st) and np.array_equal(opp[toff[1]:toff[2]], so)
+            assert t.check_mesh(y[1], st, so, full_empty_sphere=True)["empty_sphere_failures"] == 0
