@@ -89,9 +89,9 @@ enum {
     STAR_T0_DEFAULT = -1,
     STAR_T0_WAVE = 0,     // one star per wave (k_star32)
     STAR_T0_G16 = 1,      // four stars per wave, FP64 permanents, 3 waves per SIMD (k_star32g16)
-    STAR_T0_G16F = 2,     // four stars per wave, FP32 largest permanent, 3 waves per SIMD (k_star32g16f)
-    STAR_T0_G16F4 = 3,    // the same at 4 waves per SIMD (k_star32g16f4)
-    STAR_T0_G32F = 4,     // two stars per wave, FP32 largest permanent, 4 waves per SIMD (k_star32g32f)
+    STAR_T0_G16F = 2,     // four stars per wave, FP32 bound, 3 waves per SIMD (k_star32g16f)
+    STAR_T0_G16F4 = 3,    // the same at 4 waves per SIMD (k_star32g16f4), the default
+    STAR_T0_G32F = 4,     // two stars per wave, FP32 bound, 4 waves per SIMD (k_star32g32f)
     STAR_T0_NUM = 5
 };
 

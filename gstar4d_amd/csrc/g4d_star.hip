@@ -710,41 +710,44 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WPE, 8)
 // insertion of one star; here the chain is shared by 64 / GL stars.  Each lane owns KPL =
 // 64 / GL triangle slots (gl, gl + GL, ...) and keeps their cofactors and permanents in
 // registers (only the owning lane ever reads or writes them), so a star's LDS holds only its
-// link vertices, triangles and hole-boundary lists (about 3 KB).  Every barrier and ballot is
+// link vertices, triangles and hole-boundary lists (2 KB).  Every barrier and ballot is
 // reached by the whole wave in uniform control flow: the insertion loop runs to the largest
 // insertion count of the wave's stars, and a group with nothing to do in a step has its work
 // masked off.  Filters only (no multiprecision code): a star with an inconclusive orientation
 // goes to p.exact_list untouched, a star beyond the tier to p.defer_list, as in k_star32.
+//
+// Bound by vector instructions (two thirds of the issue slots at three waves per SIMD, of them a
+// fifth FP64), with the LDS pipe half busy.  At 4,194,304 uniform points (G = 512) all its passes took
+// 22.3 ms with 16-bit indices and the permanents of every triangle; 2 KB a star, which lets four waves
+// share a SIMD, one word per boundary edge, the cheap bound in place of the permanents (70 instructions
+// a triangle slot before, 43 now) and packed scans: 15.6 ms.
 // ------------------------------------------------------------------------------------
+
+static constexpr uint32_t GF_ALIVE = 1u << 31; // a triangle of the star as it stands (the sign of the word)
 
 struct StarGrpLds {
     static constexpr int VMAX = STAR_VMAX_T0;
     static constexpr int TMAX = 2 * VMAX;
     double vc[VMAX][4];
     int vid[VMAX];
-    int ins[VMAX];
     uint32_t tv[TMAX];
+    uint32_t to[TMAX]; // neighbours across the edges opposite vertices 0-2, a byte each
     union {
-        uint16_t to[TMAX][4]; // neighbours across the edges opposite vertices 0-2 (fourth unused)
-        uint64_t to64[TMAX];  // the same rows read as one word each
+        uint32_t be[TMAX]; // hole boundary: a, b, u | j << 6, then the edge's slot, a byte each
+        struct {           // finalisation
+            uint8_t present[VMAX], vremap[VMAX], remap[TMAX];
+        };
     };
-    int16_t vstart[VMAX];
-    int16_t vend[VMAX];
-    uint16_t freel[TMAX];
-    uint16_t be_a[TMAX], be_b[TMAX], be_u[TMAX], be_slot[TMAX];
-    uint8_t be_j[TMAX];
-    int16_t ins_local[VMAX];
+    uint8_t freel[TMAX];
+    uint8_t vstart[VMAX], vend[VMAX];
     uint8_t ord[VMAX]; // insertion order: list indices by distance to the star point
-    uint8_t present[VMAX];
-    uint16_t remap[TMAX];
-    uint16_t vremap[VMAX];
-    // The fields above take 3200 bytes.  Padded to 3264 (192 mod 256) the four groups' blocks
-    // start 48 banks apart (mod 64): group-parallel accesses (16 lanes of each group at the same
-    // offsets) do not all land on the same banks, as they would four ways at a multiple of 256.
-    uint8_t pad[64];
+    // 2,112 bytes: bytes for indices (all below 64), so that four waves fit each SIMD; at 64 mod 256
+    // the groups' blocks start 16 banks apart (mod 64), and accesses of the groups at the same
+    // offsets meet in no bank.
+    uint8_t pad[32];
 };
-static_assert(sizeof(StarGrpLds) % 256 == 192, "group blocks start 48 banks apart");
-static_assert(offsetof(StarGrpLds, to) % 8 == 0, "neighbour rows read as 64-bit words");
+static_assert(sizeof(StarGrpLds) % 256 == 64, "group blocks start 16 banks apart");
+static_assert(StarGrpLds::TMAX <= 64, "indices fit their bytes, slots the boundary word's six bits");
 
 // Ballot of this lane's group of GL lanes, shifted down to bit 0.
 template <int GL>
@@ -790,31 +793,83 @@ __device__ __forceinline__ int grp_excl(int v, int g, int gl, int *tot)
     return pre;
 }
 
-// Cofactors of a triangle slot, with either the four permanents in FP64 or only their largest,
-// rounded up to FP32.  The filter's error bound 32 u sum_j |v'_j| P_j is then replaced by
-// 32 u (sum_j |v'_j|) max_j P_j, which is no smaller, so a decided sign stays certain; an
-// overflow to +inf or a bound that vanishes only makes the filter inconclusive.
-__device__ __forceinline__ void grp_cofactors(const double *r0, const double *r1, const double *r2, double *C,
-                                              double (&P)[4])
+// Exclusive scans within the group, and totals, of NF flags (BITS = 1) or counts below 2^BITS each: in
+// groups of 16 lanes the fields travel packed through one scan.
+template <int GL, int BITS, int NF>
+__device__ __forceinline__ void grp_excl_n(const int (&v)[NF], int g, int gl, int (&pre)[NF], int (&tot)[NF])
 {
-    tri_cofactors(r0, r1, r2, C, P);
+    if constexpr (GL == 16) {
+        constexpr int W = 4 + BITS; // sums up to 16 (2^BITS - 1)
+        static_assert(NF * W <= 32, "packed sums fit a word");
+        uint32_t pk = 0u;
+#pragma unroll
+        for (int k = 0; k < NF; k++) pk |= (uint32_t)v[k] << (W * k);
+        int t;
+        const uint32_t x = (uint32_t)row16_scan((int)pk, &t) - pk;
+#pragma unroll
+        for (int k = 0; k < NF; k++) {
+            pre[k] = (int)((x >> (W * k)) & ((1u << W) - 1u));
+            tot[k] = (int)(((uint32_t)t >> (W * k)) & ((1u << W) - 1u));
+        }
+    } else {
+#pragma unroll
+        for (int k = 0; k < NF; k++) pre[k] = grp_excl<GL, BITS>(v[k], g, gl, &tot[k]);
+    }
 }
-__device__ __forceinline__ void grp_cofactors(const double *r0, const double *r1, const double *r2, double *C,
-                                              float &P)
+
+// A triangle slot's cofactors with the four permanents in FP64, or (PF) with tri_cofactors_m's bound on
+// them in FP32; rs2 = |x| + |y| + |z| + l of r2.
+template <bool PF> struct GrpBound {
+    double p[4];
+};
+template <> struct GrpBound<true> {
+    float m;
+};
+__device__ __forceinline__ void grp_cofactors(const double *r0, const double *r1, const double *r2, double, double,
+                                              double *C, GrpBound<false> &P)
 {
-    double Pd[4];
-    tri_cofactors(r0, r1, r2, C, Pd);
-    P = __double2float_ru(fmax(fmax(Pd[0], Pd[1]), fmax(Pd[2], Pd[3])));
+    tri_cofactors(r0, r1, r2, C, P.p);
 }
-// rs = |v'_x| + |v'_y| + |v'_z| + v'_l of the vertex being inserted (used with the FP32 form).
-__device__ __forceinline__ int grp_filter_sign(const double *r, double, const double *C, const double (&P)[4])
+__device__ __forceinline__ void grp_cofactors(const double *r0, const double *r1, const double *r2, double a2, double rs2,
+                                              double *C, GrpBound<true> &P)
 {
-    return cofactor_filter_sign(r, C, P);
+    P.m = (float)tri_cofactors_m(r0, r1, r2, a2, rs2, C);
 }
-__device__ __forceinline__ int grp_filter_sign(const double *r, double rs, const double *C, const float &P)
+// The vertex being inserted: its row's sums, and for PF the factors of the bound.  What decides whether a
+// star goes to the exact kernel (whose triangles come in another order) is 32 u rs max_j P_j with the
+// largest permanent rounded up to FP32; the bound m is no smaller than that, its roundings (2^-24 in FP32,
+// a dozen in FP64) within the 2^-20 and what the denormals lose within tiny.  A sign that it leaves open is
+// decided by the permanents themselves (grp_filter_tail).
+struct GrpRow {
+    double a, rs, as, tiny;
+};
+__device__ __forceinline__ GrpRow grp_row(const double *r)
+{
+    GrpRow w;
+    w.a = fabs(r[0]) + fabs(r[1]) + fabs(r[2]);
+    w.rs = w.a + r[3];
+    w.as = 32.0 * 1.1102230246251565e-16 * (1.0 + 0x1p-20) * w.rs;
+    w.tiny = fma(w.as, 3e-45, 1e-249);
+    return w;
+}
+__device__ __forceinline__ int grp_filter_sign(const double *r, const GrpRow &, const double *C, const GrpBound<false> &P)
+{
+    return cofactor_filter_sign(r, C, P.p);
+}
+__device__ __forceinline__ int grp_filter_sign(const double *r, const GrpRow &w, const double *C, const GrpBound<true> &P)
 {
     const double val = fma(r[3], C[3], fma(r[2], C[2], fma(r[1], C[1], r[0] * C[0])));
-    const double per = rs * (double)P;
+    const double bnd = fma(w.as, (double)P.m, w.tiny);
+    return val > bnd ? 1 : (-val > bnd ? -1 : 0);
+}
+__device__ __forceinline__ int grp_filter_tail(const double *r0, const double *r1, const double *r2,
+                                                         const double *r)
+{
+    double C[4], P[4];
+    tri_cofactors(r0, r1, r2, C, P);
+    const float p = __double2float_ru(fmax(fmax(P[0], P[1]), fmax(P[2], P[3])));
+    const double val = fma(r[3], C[3], fma(r[2], C[2], fma(r[1], C[1], r[0] * C[0])));
+    const double per = (fabs(r[0]) + fabs(r[1]) + fabs(r[2]) + r[3]) * (double)p;
     const double bnd = 32.0 * 1.1102230246251565e-16 * per;
     if (!(per > 1e-250)) return 0;
     return val > bnd ? 1 : (-val > bnd ? -1 : 0);
@@ -843,7 +898,8 @@ __device__ __forceinline__ void star_body_grp(const StarParams &p, int nitems)
     constexpr int KPL = TMAX / GL;
     __shared__ StarGrpLds Ls[NG];
     __shared__ int order[NG * STAR_CHUNK]; // the chunk's items by insertion count
-    const int lane = threadIdx.x, g = lane / GL, gl = lane % GL;
+    const int lane = threadIdx.x, g = lane / GL;
+    int gl = lane % GL;
     StarGrpLds &L = Ls[g];
     unsigned long long *cnt = p.cnt;
 
@@ -859,8 +915,6 @@ __device__ __forceinline__ void star_body_grp(const StarParams &p, int nitems)
     bool first = true;
     int nfilt = 0, ncof = 0;
     unsigned long long npairs = 0, ndrown = 0; // the wave's
-    double C[KPL][4];
-    typename std::conditional<PF, float, double[4]>::type P[KPL];
     for (;;) {
         int base = 0;
         if (one_each) {
@@ -894,6 +948,9 @@ __device__ __forceinline__ void star_body_grp(const StarParams &p, int nitems)
         }
 #pragma unroll 1
         for (int batch = base; batch < bend; batch++) {
+            // addresses made from gl are made again for each batch: kept across it they would cost
+            // more registers than four waves per SIMD leave
+            asm volatile("" : "+v"(gl));
             const int item = order[(batch - base) * NG + g];
             // ---- this group's star: checks, then its link and insertions into LDS ----
             bool act = item < nitems;
@@ -931,12 +988,12 @@ __device__ __forceinline__ void star_body_grp(const StarParams &p, int nitems)
             if (act) {
                 for (int q = gl; q < m; q += GL) {
                     const int gv = (int)(uint32_t)p.ins_keys[ib + q];
-                    L.ins[q] = gv;
-                    L.ins_local[q] = -1;
                     L.vid[vn + q] = gv;
                     rel_coords(p.pts, gv, sx, sy, sz, L.vc[vn + q]);
                 }
             }
+#pragma unroll
+            for (int k = 0; k < KPL; k++) L.tv[gl + GL * k] = 0u;
             wave_sync();
             // Insertion order: nearest to the star point first (ties by list index).  The star
             // that results does not depend on the order (the link is the unique convex hull of
@@ -973,10 +1030,8 @@ __device__ __forceinline__ void star_body_grp(const StarParams &p, int nitems)
                 }
                 for (int t = gl; t < tn; t += GL) {
                     const uint64_t h = p.tpool[ti + t];
-                    L.tv[t] = tpack(hvert(h, 0), hvert(h, 1), hvert(h, 2), TF_ALIVE | (hchecked(h) ? TF_CHECKED : 0u));
-                    L.to[t][0] = (uint16_t)hopp(h, 0);
-                    L.to[t][1] = (uint16_t)hopp(h, 1);
-                    L.to[t][2] = (uint16_t)hopp(h, 2);
+                    L.tv[t] = tpack(hvert(h, 0), hvert(h, 1), hvert(h, 2), GF_ALIVE | (hchecked(h) ? TF_CHECKED : 0u));
+                    L.to[t] = (uint32_t)hopp(h, 0) | ((uint32_t)hopp(h, 1) << 8) | ((uint32_t)hopp(h, 2) << 16);
                 }
                 T = tn;
             } else if (act) {
@@ -997,23 +1052,25 @@ __device__ __forceinline__ void star_body_grp(const StarParams &p, int nitems)
                     }
                     if (gl < 4) {
                         const int lt[4][3] = {{1, 2, 3}, {0, 3, 2}, {0, 1, 3}, {0, 2, 1}};
-                        L.tv[gl] = tpack(c[lt[gl][0]], c[lt[gl][1]], c[lt[gl][2]], TF_ALIVE);
-                        L.to[gl][0] = (uint16_t)lt[gl][0];
-                        L.to[gl][1] = (uint16_t)lt[gl][1];
-                        L.to[gl][2] = (uint16_t)lt[gl][2];
-                        L.ins_local[c[gl]] = (int16_t)c[gl];
+                        L.tv[gl] = tpack(c[lt[gl][0]], c[lt[gl][1]], c[lt[gl][2]], GF_ALIVE);
+                        L.to[gl] = (uint32_t)(lt[gl][0] | (lt[gl][1] << 8) | (lt[gl][2] << 16));
                     }
                     T = 4;
                 }
             }
             wave_sync();
             bool live = act && !unsure; // the group is building its star
+            // declared here, not before the loop over batches: their registers are free outside the insertions
+            double C[KPL][4];
+            GrpBound<PF> P[KPL];
 #pragma unroll
             for (int k = 0; k < KPL; k++) {
                 const int slot = gl + GL * k;
                 if (live && slot < T) {
                     const uint32_t t = L.tv[slot];
-                    grp_cofactors(L.vc[tvert(t, 0)], L.vc[tvert(t, 1)], L.vc[tvert(t, 2)], C[k], P[k]);
+                    const double *r2 = L.vc[tvert(t, 2)];
+                    const double a2 = fabs(r2[0]) + fabs(r2[1]) + fabs(r2[2]);
+                    grp_cofactors(L.vc[tvert(t, 0)], L.vc[tvert(t, 1)], r2, a2, a2 + r2[3], C[k], P[k]);
                     ncof++;
                 }
             }
@@ -1036,19 +1093,33 @@ __device__ __forceinline__ void star_body_grp(const StarParams &p, int nitems)
                     r[2] = L.vc[Vn][2];
                     r[3] = L.vc[Vn][3];
                 }
-                const double rs = fabs(r[0]) + fabs(r[1]) + fabs(r[2]) + r[3];
+                const GrpRow w = grp_row(r);
                 int nv = 0;
                 unsigned vm = 0; // bit k: slot gl + GL k sees the vertex
+                unsigned um = 0; // bit k: the sign is open
                 bool unc = false;
 #pragma unroll
                 for (int k = 0; k < KPL; k++) {
-                    const int slot = gl + GL * k;
-                    if (step && slot < T && (tk[k] & (TF_ALIVE | TF_VIS)) == TF_ALIVE) {
+                    if (step && (int)tk[k] < 0) {
                         nfilt++;
-                        const int sg = grp_filter_sign(r, rs, C[k], P[k]);
+                        const int sg = grp_filter_sign(r, w, C[k], P[k]);
+                        if (sg == 0) um |= 1u << k;
+                        if (sg < 0) {
+                            L.tv[gl + GL * k] = tk[k] & ~GF_ALIVE;
+                            vm |= 1u << k;
+                            nv++;
+                        }
+                    }
+                }
+                if constexpr (!PF) unc = um != 0;
+                else if (__builtin_expect(__ballot(um != 0) != 0ull, 0)) {
+                    for (; um; um &= um - 1) {
+                        const int k = __builtin_ctz(um), slot = gl + GL * k;
+                        const uint32_t t = L.tv[slot];
+                        const int sg = grp_filter_tail(L.vc[tvert(t, 0)], L.vc[tvert(t, 1)], L.vc[tvert(t, 2)], L.vc[Vn]);
                         if (sg == 0) unc = true;
                         if (sg < 0) {
-                            L.tv[slot] = tk[k] | TF_VIS;
+                            L.tv[slot] = t & ~GF_ALIVE;
                             vm |= 1u << k;
                             nv++;
                         }
@@ -1077,56 +1148,52 @@ __device__ __forceinline__ void star_body_grp(const StarParams &p, int nitems)
                     step = false;
                 }
                 if (nvis == 0) step = false; // drowned at insertion
-                if (step && gl == 0) L.ins_local[j] = (int16_t)Vn;
                 // the visible slots join the free list (positions nfree .. nfree + nvis - 1)
                 if (step) {
                     int fpos = nfree + vbase;
 #pragma unroll
                     for (int k = 0; k < KPL; k++)
-                        if ((vm >> k) & 1) L.freel[fpos++] = (uint16_t)(gl + GL * k);
+                        if ((vm >> k) & 1) L.freel[fpos++] = (uint8_t)(gl + GL * k);
                 }
                 wave_sync();
                 // Hole boundary: the edges of visible triangles whose neighbour is not visible, in
                 // the order of the visible list; its entry x is taken by lane x mod GL.  The edge's
-                // position in the neighbour u is that of u's vertex off the edge.
+                // position in the neighbour u is that of u's vertex off the edge (all triangles turn
+                // the same way round: the edge runs the other way in u).
                 int nbtot = 0;
                 for (int x0 = 0; __ballot(step && x0 < nvis) != 0ull; x0 += GL) {
                     const int x = x0 + gl;
                     const bool own = step && x < nvis;
-                    uint32_t t = 0u;
-                    uint64_t o = 0ull;
+                    uint32_t t = 0u, o = 0u;
                     if (own) {
                         const int slot = L.freel[nfree + x];
                         t = L.tv[slot];
-                        o = L.to64[slot];
+                        o = L.to[slot];
                     }
-                    uint32_t tu[3] = {TF_VIS, TF_VIS, TF_VIS};
+                    uint32_t tu[3] = {0u, 0u, 0u};
                     if (own)
 #pragma unroll
-                        for (int i = 0; i < 3; i++) tu[i] = L.tv[(int)(o >> (16 * i)) & (TMAX - 1)];
+                        for (int i = 0; i < 3; i++) tu[i] = L.tv[(o >> (8 * i)) & (TMAX - 1)];
                     int nb = 0;
 #pragma unroll
-                    for (int i = 0; i < 3; i++) nb += (tu[i] & TF_VIS) ? 0 : 1;
+                    for (int i = 0; i < 3; i++) nb += (int)(tu[i] >> 31);
                     int tot;
                     int e = nbtot + grp_excl<GL, 2>(nb, g, gl, &tot);
 #pragma unroll
                     for (int i = 0; i < 3; i++) {
-                        if (tu[i] & TF_VIS) continue;
+                        if ((int)tu[i] >= 0) continue;
                         const int a = tvert(t, (i + 1) % 3), b = tvert(t, (i + 2) % 3);
-                        const int u0 = tvert(tu[i], 0), u1 = tvert(tu[i], 1);
-                        if (e < TMAX) {
-                            L.be_a[e] = (uint16_t)a;
-                            L.be_b[e] = (uint16_t)b;
-                            L.be_u[e] = (uint16_t)(o >> (16 * i));
-                            L.be_j[e] = (uint8_t)((u0 != a && u0 != b) ? 0 : ((u1 != a && u1 != b) ? 1 : 2));
-                        }
+                        // u has the edge as b, a
+                        const int j = tvert(tu[i], 0) == b ? 2 : (tvert(tu[i], 1) == b ? 0 : 1);
+                        if (e < TMAX)
+                            L.be[e] = (uint32_t)(a | (b << 8) | (j << 22)) | (((o >> (8 * i)) & (TMAX - 1)) << 16);
                         e++;
                     }
                     nbtot += tot;
                 }
-                // The visible triangles keep their words, TF_VIS marking them dead, until a new
-                // triangle takes the slot: boundary edge k takes free slot nfree_tot - 1 - k (the
-                // visible ones first) or, past the free list, slot T + k - nfree_tot.
+                // The visible triangles keep their words, no longer alive, until a new triangle takes
+                // the slot: boundary edge k takes free slot nfree_tot - 1 - k (the visible ones first)
+                // or, past the free list, slot T + k - nfree_tot.
                 const int nfree_tot = nfree + nvis;
                 const int newT = T + (nbtot > nfree_tot ? nbtot - nfree_tot : 0);
                 if (step && (nbtot > TMAX || nbtot < 3 || newT > TMAX || Vn + 1 > VMAX)) {
@@ -1138,36 +1205,37 @@ __device__ __forceinline__ void star_body_grp(const StarParams &p, int nitems)
                 if (step)
                     for (int k = gl; k < nbtot; k += GL) {
                         const int slot = k < nfree_tot ? L.freel[nfree_tot - 1 - k] : T + (k - nfree_tot);
-                        const int a = L.be_a[k], b = L.be_b[k], u = L.be_u[k];
-                        L.be_slot[k] = (uint16_t)slot;
-                        L.tv[slot] = tpack(a, b, Vn, TF_ALIVE | TF_FRESH);
-                        L.to[slot][2] = (uint16_t)u;
-                        L.to[u][L.be_j[k]] = (uint16_t)slot;
-                        L.vstart[a] = (int16_t)slot;
-                        L.vend[b] = (int16_t)slot;
+                        const uint32_t e = L.be[k];
+                        const int a = (int)(e & 255u), b = (int)((e >> 8) & 255u), u = (int)((e >> 16) & 63u),
+                                  j = (int)((e >> 22) & 3u);
+                        L.be[k] = (e & 0x3fffffu) | ((uint32_t)slot << 24);
+                        L.tv[slot] = tpack(a, b, Vn, GF_ALIVE);
+                        reinterpret_cast<uint8_t *>(&L.to[u])[j] = (uint8_t)slot;
+                        L.vstart[a] = (uint8_t)slot;
+                        L.vend[b] = (uint8_t)slot;
                     }
                 wave_sync();
                 if (step) {
                     for (int k = gl; k < nbtot; k += GL) {
-                        const int slot = L.be_slot[k];
-                        L.to[slot][0] = (uint16_t)L.vstart[L.be_b[k]];
-                        L.to[slot][1] = (uint16_t)L.vend[L.be_a[k]];
+                        const uint32_t e = L.be[k];
+                        L.to[e >> 24] = (uint32_t)L.vstart[(e >> 8) & 255u] | ((uint32_t)L.vend[e & 255u] << 8) |
+                                        (e & 0x3f0000u);
                     }
                     nfree = nfree_tot - (nbtot < nfree_tot ? nbtot : nfree_tot);
                     T = newT;
                 }
                 // the link writes above touch only the new slots' neighbour rows: the cofactor
-                // pass below (triangle words and coordinates) needs no barrier after them
+                // pass below (triangle words and coordinates) needs no barrier after them.  The new
+                // triangles are those alive whose third vertex, here this lane's own r, is Vn.
 #pragma unroll
                 for (int k = 0; k < KPL; k++) tk[k] = L.tv[gl + GL * k];
+                const uint32_t fresh = step ? (uint32_t)Vn | (GF_ALIVE >> 18) : ~0u;
 #pragma unroll
                 for (int k = 0; k < KPL; k++) {
-                    const int slot = gl + GL * k;
-                    if (step && slot < T && (tk[k] & TF_FRESH)) {
-                        const uint32_t t = tk[k];
-                        grp_cofactors(L.vc[tvert(t, 0)], L.vc[tvert(t, 1)], L.vc[tvert(t, 2)], C[k], P[k]);
+                    const uint32_t t = tk[k];
+                    if ((t >> 18) == fresh) {
+                        grp_cofactors(L.vc[tvert(t, 0)], L.vc[tvert(t, 1)], r, w.a, w.rs, C[k], P[k]);
                         ncof++;
-                        L.tv[slot] = t & ~TF_FRESH;
                     }
                 }
                 // No barrier before the next step: its filter reads and writes only this lane's
@@ -1195,9 +1263,8 @@ __device__ __forceinline__ void star_body_grp(const StarParams &p, int nitems)
             uint32_t tf[KPL];
 #pragma unroll
             for (int k = 0; k < KPL; k++) {
-                const int slot = gl + GL * k;
-                const uint32_t t = L.tv[slot];
-                tf[k] = (fin && slot < T && (t & (TF_ALIVE | TF_VIS)) == TF_ALIVE) ? t : 0u;
+                const uint32_t t = L.tv[gl + GL * k];
+                tf[k] = fin && (int)t < 0 ? t : 0u;
             }
             wave_sync();
 #pragma unroll
@@ -1213,35 +1280,35 @@ __device__ __forceinline__ void star_body_grp(const StarParams &p, int nitems)
                 const int q = b0 + gl;
                 bool dr = false;
                 if (fin && q < m) {
-                    const int lv = L.ins_local[q];
-                    dr = lv < 0 || !L.present[lv];
+                    dr = !L.present[vn + q]; // a vertex that never entered is in no triangle
                     p.dflag[ib + q] = dr ? 1 : 0;
                 }
                 ndrown += __popcll(__ballot(dr));
             }
             const int64_t vo = fin ? p.nvoff[s] : 0, to = fin ? p.ntoff[s] : 0;
-            int vcount = 0;
+            // ranks of the link's vertices and of the live triangles, scanned together
+            constexpr int VPL = VMAX / GL;
+            int fl[VPL + KPL], rk[VPL + KPL], ct[VPL + KPL];
 #pragma unroll
-            for (int b0 = 0; b0 < VMAX; b0 += GL) {
-                const int v = b0 + gl;
-                const bool pr = fin && v < V && L.present[v];
-                int tot;
-                const int rk = grp_excl<GL, 1>(pr ? 1 : 0, g, gl, &tot);
-                if (pr) {
-                    L.vremap[v] = (uint16_t)(vcount + rk);
-                    p.vpool[vo + vcount + rk] = L.vid[v];
+            for (int i = 0; i < VPL; i++) fl[i] = fin && gl + GL * i < V && L.present[gl + GL * i] ? 1 : 0;
+#pragma unroll
+            for (int k = 0; k < KPL; k++) fl[VPL + k] = tf[k] ? 1 : 0;
+            grp_excl_n<GL, 1, VPL + KPL>(fl, g, gl, rk, ct);
+            int vcount = 0, tcount = 0;
+#pragma unroll
+            for (int i = 0; i < VPL; i++) {
+                const int v = gl + GL * i;
+                if (fl[i]) {
+                    L.vremap[v] = (uint8_t)(vcount + rk[i]);
+                    p.vpool[vo + vcount + rk[i]] = L.vid[v];
                 }
-                vcount += tot;
+                vcount += ct[i];
             }
-            int tcount = 0;
 #pragma unroll
-            for (int b0 = 0; b0 < TMAX; b0 += GL) {
-                const int t = b0 + gl;
-                const bool al = tf[b0 / GL] != 0u;
-                int tot;
-                const int rk = grp_excl<GL, 1>(al ? 1 : 0, g, gl, &tot);
-                if (al) L.remap[t] = (uint16_t)(tcount + rk);
-                tcount += tot;
+            for (int k = 0; k < KPL; k++) {
+                rk[VPL + k] += tcount;
+                if (tf[k]) L.remap[gl + GL * k] = (uint8_t)rk[VPL + k];
+                tcount += ct[VPL + k];
             }
             if (fin && (tcount > 2 * need - 4 || tcount != 2 * vcount - 4)) {
                 // not a triangulated 2-sphere: report instead of writing past the star's region
@@ -1263,24 +1330,24 @@ __device__ __forceinline__ void star_body_grp(const StarParams &p, int nitems)
                 prk[k] = TriPairs{STAR_PAIR_NONE, STAR_PAIR_NONE};
                 if (tt) {
                     const int a = tvert(tt, 0), b = tvert(tt, 1), c = tvert(tt, 2);
-                    const int d = L.remap[t];
-                    const uint64_t o = L.to64[t];
-                    p.tpool[to + d] = hpack(L.vremap[a], L.vremap[b], L.vremap[c], L.remap[(int)(o & 0xffff)],
-                                            L.remap[(int)((o >> 16) & 0xffff)], L.remap[(int)((o >> 32) & 0xffff)], true);
+                    const uint32_t o = L.to[t];
+                    p.tpool[to + rk[VPL + k]] = hpack(L.vremap[a], L.vremap[b], L.vremap[c], L.remap[o & 255u],
+                                                      L.remap[(o >> 8) & 255u], L.remap[(o >> 16) & 255u], true);
                     prk[k] = star_tri_pairs(L.vid[a], L.vid[b], L.vid[c], !(tt & TF_CHECKED));
                 }
             }
-            int npair = 0;
+            // the star's pairs, dense, in triangle order
+            int np[KPL], pat[KPL], ptot[KPL], npair = 0;
+#pragma unroll
+            for (int k = 0; k < KPL; k++)
+                np[k] = (prk[k].x != STAR_PAIR_NONE ? 1 : 0) + (prk[k].y != STAR_PAIR_NONE ? 1 : 0);
+            grp_excl_n<GL, 2, KPL>(np, g, gl, pat, ptot);
 #pragma unroll
             for (int k = 0; k < KPL; k++) {
-                const TriPairs pr = prk[k];
-                // the star's pairs, dense, in triangle order
-                const int np = (pr.x != STAR_PAIR_NONE ? 1 : 0) + (pr.y != STAR_PAIR_NONE ? 1 : 0);
-                int tot;
-                const int at = npair + grp_excl<GL, 2>(np, g, gl, &tot);
-                if (np > 0) p.pairbuf[pb + at] = pr.x;
-                if (np > 1) p.pairbuf[pb + at + 1] = pr.y;
-                npair += tot;
+                const int64_t at = pb + npair + pat[k];
+                if (np[k] > 0) p.pairbuf[at] = prk[k].x;
+                if (np[k] > 1) p.pairbuf[at + 1] = prk[k].y;
+                npair += ptot[k];
             }
             // groups not finalised count none
 #pragma unroll
@@ -1288,7 +1355,7 @@ __device__ __forceinline__ void star_body_grp(const StarParams &p, int nitems)
             int hn = 0;
             if (fin) {
                 if (gl == 0) p.pcount[s] = npair;
-                hn = star_history_merge(p, s, L.ins, m, gl, GL);
+                hn = star_history_merge(p, s, L.vid + vn, m, gl, GL);
             }
             wave_sync();
             if (fin && gl == 0) star_commit(p, s, vcount, vo, tcount, to, hn + m);
@@ -1325,9 +1392,9 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4, 8)))
 }
 
 // The 32-vertex filter-only kernel variant of a launch: the caller's choice, else the
-// G4D_STAR_T0 environment variable (measurement), else the measured best (four stars per wave
-// with the FP32 largest permanent: 73.4 ms per triangulation at 4,194,304 uniform points, G =
-// 512, against 89.1 for one star per wave).
+// G4D_STAR_T0 environment variable (measurement), else the measured best: four stars per wave with
+// the FP32 bound at four waves per SIMD, 15.6 ms of star kernel at 4,194,304 uniform points (G = 512)
+// against 18.3 at three (and 24 for two stars per wave).
 static int star_t0_variant(int requested)
 {
     if (requested >= 0 && requested < STAR_T0_NUM) return requested;
@@ -1337,7 +1404,7 @@ static int star_t0_variant(int requested)
         env = e ? atoi(e) : -1;
         if (env < 0 || env >= STAR_T0_NUM) env = -1;
     }
-    return env >= 0 ? env : STAR_T0_G16F;
+    return env >= 0 ? env : STAR_T0_G16F4;
 }
 
 static_assert(G4D_CNT_QUEUE0 + 7 <= G4D_CNT_PAIRS, "seven queue heads must fit the counter block");

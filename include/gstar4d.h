@@ -173,7 +173,7 @@ int g4d_triangulate_device_noalloc(g4d_ctx *ctx, const double *d_xyz, int32_t n,
 /* Tuning (no reference counterpart; gstar4d_amd/autotune.py measures the choices).
    g4d_set_star_kernel: variant of the 32-vertex star kernel, -1 for the built-in default,
    0 one star per wave, 1 four stars per wave (FP64 permanents), 2 four stars per wave (FP32
-   largest permanent), 3 the same at four waves per SIMD, 4 two stars per wave; the output never
+   bound), 3 the same at four waves per SIMD (the default), 4 two stars per wave; the output never
    depends on it.  g4d_set_grid_table: PBA grid of a batched set without an explicit grid =
    the smallest multiple of 8 in [32, 256] with at least voxels_per_point[k] voxels per point,
    k the first bucket with n <= max_points[k] (ascending; the last bucket takes every larger

@@ -275,6 +275,30 @@ def test_rounds_around_the_small_list_limit(orc, n, gen):
     assert st["splay_insertions"] == rst["splay_insertions"]
 
 
+@pytest.mark.parametrize("unit", [1e-12, 1e-6, 1.0, 1e5])
+@pytest.mark.parametrize("shape", ["uniform", "near_sphere", "flat", "lattice_pairs"])
+def test_star_filter_across_units(orc, shape, unit):
+    """The 32-vertex star kernel's sign bound is of another size in each unit of length (it adds
+    lengths to squared lengths) and for flat or near-degenerate triangles: what it leaves open the
+    permanents decide, then the exact kernel; every variant gives the oracle's triangulation."""
+    rng = np.random.default_rng(7)
+    x = rng.random((700, 3))
+    if shape == "near_sphere":
+        x -= 0.5
+        x = x / np.linalg.norm(x, axis=1, keepdims=True) * (1.0 + 1e-9 * rng.normal(size=(700, 1)))
+    elif shape == "flat":
+        x[:, 2] *= 1e-7
+    elif shape == "lattice_pairs":
+        x = np.unique(np.floor(x * 9), axis=0) + 1e-8 * rng.integers(0, 3, size=(1, 3))
+    x = x * unit
+    ref, _, _ = orc.triangulate(x, 24)
+    with g.Triangulator(grid_size=24) as t:
+        for v in (-1, 1, 2, 4):
+            t.set_star_kernel(v)
+            tets, _, _ = t.triangulate(x)
+            assert (g.canonical(tets) == ref).all(), v
+
+
 @pytest.mark.parametrize("bands", [1, 3, 5])
 def test_pba_bands_same_triangulation(orc, bands):
     x = datasets.uniform_cube(20000, seed=31)
