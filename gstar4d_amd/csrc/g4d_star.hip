@@ -2629,108 +2629,181 @@ hipError_t launch_drown_small(const uint64_t *ins_keys, const uint8_t *dflag, in
     return hipGetLastError();
 }
 
-// One pass from the stars' pair regions and the proofs' pairs to the appended keys: sixteen stars a
-// work-group step, 16 lanes each (a star of more than NP_WIDE pairs is left to the whole group),
-// then the proofs.  Surviving pairs are collected in LDS and leave a stage at a time, with one
-// atomic.  Bound by the latency of the histories' binary searches (dependent reads, some six for
-// a star of 40).  The gather of the pairs into one list, the filter over it and the compaction of
-// what it kept, three passes over 8 bytes a pair and six launches, took 4.3 ms on 4,194,304
-// uniform points (12 rounds); this takes 3.7.
-static constexpr int NP_STAGE = 2048, NP_WIDE = 128;
+// One pass from the stars' pair regions and the proofs' pairs to the appended keys.  An edge is in the
+// links of some five stars, which lie near each other in the list: a wave walks rows of consecutive
+// stars (16 lanes a star), drops the pairs that its work-group has lately seen, and queues the others,
+// so that the histories' binary searches (some six dependent reads each) run in full waves, two a lane.
+// What is new is staged and leaves with one atomic: all of them meet at one counter, and with a
+// stage of 160 instead of 672 the first pass below took 4.4 ms.  Bound by the searches' latency and
+// divergent lines.  4,194,304 uniform points, 12 rounds: 2.5 ms, of which the first pass 1.5; a search per
+// pair where it is read, with nothing dropped or queued, 3.75 and 2.1.
+static constexpr int NP_LANE = 2, NP_DRAIN = 64 * NP_LANE, NP_QUEUE = NP_DRAIN + 64, NP_STAGE = 672, NP_WIDE = 128,
+                     NP_SEEN = 1024, NP_ROW = 1024;
 
 __global__ void __launch_bounds__(LA_THREADS) k_new_pairs(NewPairs p)
 {
-    __shared__ uint64_t stage[NP_STAGE];
-    __shared__ int nst, nwide, wide[LA_THREADS / 16];
-    __shared__ unsigned long long base;
-    const int tid = threadIdx.x, sub = tid & 15, lane = __lane_id();
-    if (tid == 0) nst = 0;
+    constexpr int W = LA_THREADS / 64, G = LA_THREADS / 16;
+    __shared__ uint64_t queue_[W][NP_QUEUE], stage_[W][NP_STAGE], seen[NP_SEEN];
+    __shared__ int nwide;
+    __shared__ uint16_t wide[NP_ROW];
+    const int tid = threadIdx.x, sub = tid & 15, lane = tid & 63, wv = tid >> 6;
+    uint64_t *queue = queue_[wv], *stage = stage_[wv];
+    int nq = 0, ns = 0; // this wave's
+    for (int i = tid; i < NP_SEEN; i += LA_THREADS) seen[i] = STAR_PAIR_NONE;
+    if (tid == 0) nwide = 0;
     __syncthreads();
-    // Whether pair k is new (a < b and b not in a's history).
-    auto is_new = [&](uint64_t k) {
-        const uint32_t a = (uint32_t)(k >> 32), b = (uint32_t)k;
-        if (!(a < b)) return false;
-        const int *h = p.hpool + p.hoff[a];
-        const int hn = p.hnum[a];
-        int lo = 0, hi = hn;
-        while (lo < hi) {
-            const int mid = (lo + hi) >> 1;
-            if ((uint32_t)h[mid] < b) lo = mid + 1;
-            else hi = mid;
-        }
-        return !(lo < hn && (uint32_t)h[lo] == b);
+    // All of these are called by whole waves.
+    auto add = [&](int n) {
+        unsigned long long base = 0;
+        if (lane == 0) base = atomicAdd(&p.cnt[G4D_CNT_NEW_PAIRS], (unsigned long long)n);
+        return __shfl(base, 0, 64);
     };
-    auto emit = [&](unsigned long long at, uint64_t k) {
-        p.keys[2 * at] = k;
-        p.keys[2 * at + 1] = (k << 32) | (k >> 32);
+    auto flush = [&](int n, unsigned long long base) {
+        wave_sync();
+        for (int i = lane; i < n; i += 64) {
+            const uint64_t k = stage[i];
+            reinterpret_cast<ulonglong2 *>(p.keys)[base + i] = make_ulonglong2(k, (k << 32) | (k >> 32));
+        }
+        wave_sync();
+        ns = 0;
     };
-    // Called by whole waves; pairs that find the stage full are appended at once.
-    auto put = [&](bool keep, uint64_t k) {
-        const uint64_t mk = __ballot(keep);
-        if (!mk) return;
-        int at = 0;
-        if (lane == 0) at = atomicAdd(&nst, __popcll(mk));
-        at = __builtin_amdgcn_readfirstlane(at) + __popcll(mk & ((1ull << lane) - 1ull));
-        const bool full = keep && at >= NP_STAGE;
-        if (keep && !full) stage[at] = k;
-        if (__ballot(full)) {
-            const long long g = g4d_wave_append(full, &p.cnt[G4D_CNT_NEW_PAIRS]);
-            if (full) emit((unsigned long long)g, k);
+    // The last n <= NP_DRAIN pairs of the queue: new when b is not in a's history.
+    auto drain = [&](int n) {
+        wave_sync();
+        uint64_t k[NP_LANE];
+        int64_t h[NP_LANE];
+        int lo[NP_LANE], hi[NP_LANE];
+        nq -= n;
+#pragma unroll
+        for (int j = 0; j < NP_LANE; j++) {
+            const int i = j * 64 + lane;
+            k[j] = i < n ? queue[nq + i] : STAR_PAIR_NONE;
         }
-    };
-    // Called by the whole work-group: empties the stage when it holds more than `above`.
-    auto flush = [&](int above) {
-        __syncthreads();
-        const int have = min(nst, NP_STAGE);
-        __syncthreads();
-        if (have <= above) return;
-        if (tid == 0) {
-            base = atomicAdd(&p.cnt[G4D_CNT_NEW_PAIRS], (unsigned long long)have);
-            nst = 0;
+#pragma unroll
+        for (int j = 0; j < NP_LANE; j++) {
+            const bool v = k[j] != STAR_PAIR_NONE;
+            const uint32_t a = v ? (uint32_t)(k[j] >> 32) : 0u;
+            h[j] = p.hoff[a];
+            hi[j] = v ? p.hnum[a] : 0;
+            lo[j] = 0;
         }
-        __syncthreads();
-        for (int i = tid; i < have; i += LA_THREADS) emit(base + i, stage[i]);
-        __syncthreads();
-    };
-    for (int64_t i0 = (int64_t)blockIdx.x * (LA_THREADS / 16); i0 < p.nitems;
-         i0 += (int64_t)gridDim.x * (LA_THREADS / 16)) {
-        const int64_t i = i0 + (tid >> 4);
-        const int s = i < p.nitems ? (p.list ? p.list[i] : (int)i) : -1;
-        int c = s >= 0 ? p.pcount[s] : 0;
-        const uint64_t *src = s >= 0 ? p.pairbuf + 2 * (p.ntoff[s] - p.tbase) : p.pairbuf;
-        if (tid == 0) nwide = 0;
-        __syncthreads();
-        if (c > NP_WIDE) {
-            if (sub == 0) wide[atomicAdd(&nwide, 1)] = s;
-            c = 0;
-        }
-        const int cmax = g4d_wave_max(c);
-        for (int k0 = 0; k0 < cmax; k0 += 16) {
-            const int k = k0 + sub;
-            const uint64_t pr = k < c ? src[k] : 0ull;
-            put(k < c && is_new(pr), pr);
-        }
-        __syncthreads();
-        for (int w = 0; w < nwide; w++) {
-            const int sw = wide[w], cw = p.pcount[sw];
-            const uint64_t *srcw = p.pairbuf + 2 * (p.ntoff[sw] - p.tbase);
-            for (int k0 = 0; k0 < cw; k0 += LA_THREADS) {
-                const int k = k0 + tid;
-                const uint64_t pr = k < cw ? srcw[k] : 0ull;
-                put(k < cw && is_new(pr), pr);
+        for (;;) {
+            bool more = false;
+#pragma unroll
+            for (int j = 0; j < NP_LANE; j++) more = more || lo[j] < hi[j];
+            if (!__ballot(more)) break;
+            int mid[NP_LANE];
+            uint32_t x[NP_LANE];
+#pragma unroll
+            for (int j = 0; j < NP_LANE; j++) {
+                mid[j] = (lo[j] + hi[j]) >> 1;
+                // a search that is over reads the pool's first word, so that all reads leave together
+                x[j] = (uint32_t)p.hpool[lo[j] < hi[j] ? h[j] + mid[j] : 0];
+            }
+#pragma unroll
+            for (int j = 0; j < NP_LANE; j++) {
+                const bool in = lo[j] < hi[j], less = x[j] < (uint32_t)k[j], same = x[j] == (uint32_t)k[j];
+                if (in && less) lo[j] = mid[j] + 1;
+                if (in && !less) hi[j] = mid[j];
+                if (in && same) k[j] = STAR_PAIR_NONE, hi[j] = lo[j]; // found: not new
             }
         }
-        flush(NP_STAGE / 2);
+        wave_sync();
+#pragma unroll
+        for (int j = 0; j < NP_LANE; j++) {
+            const bool f = k[j] != STAR_PAIR_NONE;
+            const uint64_t mk = __ballot(f);
+            if (f) stage[ns + __popcll(mk & ((1ull << lane) - 1ull))] = k[j];
+            ns += __popcll(mk);
+        }
+        if (ns > NP_STAGE - NP_DRAIN) flush(ns, add(ns));
+    };
+    auto put = [&](bool have, uint64_t k) {
+        const uint32_t a = (uint32_t)(k >> 32), b = (uint32_t)k;
+        bool f = have && a < b;
+        if (f) {
+            // an entry is read and written whole (64-bit LDS accesses); one that another pair takes
+            // only means another look
+            uint64_t *e = &seen[(a * 0x9e3779b1u ^ b * 0x85ebca6bu) >> (32 - __builtin_ctz(NP_SEEN))];
+            f = __hip_atomic_load(e, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) != k;
+            if (f) __hip_atomic_store(e, k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        }
+        const uint64_t mk = __ballot(f);
+        if (f) queue[nq + __popcll(mk & ((1ull << lane) - 1ull))] = k;
+        nq += __popcll(mk);
+        if (nq >= NP_DRAIN) drain(NP_DRAIN);
+    };
+    const int row = max(G, min(NP_ROW, (p.nitems / (int)gridDim.x + G - 1) / G * G));
+    for (int64_t r0 = (int64_t)blockIdx.x * row; r0 < p.nitems; r0 += (int64_t)gridDim.x * row) {
+        // 16 stars of the row a step, four of them this wave's
+        const int nrow = (int)min((int64_t)row, p.nitems - r0);
+        // the reads of a step (list entry, then count and region, then the first pairs) are made one, two
+        // and three steps ahead: each waits for the one before
+        auto entry = [&](int i) { return i < nrow ? (p.list ? p.list[r0 + i] : (int)(r0 + i)) : -1; };
+        struct Region {
+            int c;
+            int64_t off;
+        };
+        auto region = [&](int s) { return s >= 0 ? Region{p.pcount[s], p.ntoff[s]} : Region{0, p.tbase}; };
+        auto pair = [&](const Region &g, int k) { return k < g.c ? p.pairbuf[2 * (g.off - p.tbase) + k] : 0ull; };
+        const int i1 = 4 * wv + (lane >> 4);
+        Region g0 = region(entry(i1)), g1 = region(entry(i1 + G));
+        int s2 = entry(i1 + 2 * G);
+        uint64_t pr0 = pair(g0, sub);
+        for (int i0 = 4 * wv; i0 < nrow; i0 += G) {
+            const int i = i0 + (lane >> 4);
+            const int s3 = entry(i + 3 * G);
+            const Region g2 = region(s2);
+            const uint64_t pr1 = pair(g1, sub);
+            int c = g0.c;
+            if (c > NP_WIDE) {
+                if (sub == 0) wide[atomicAdd(&nwide, 1)] = (uint16_t)i;
+                c = 0;
+            }
+            const int cmax = g4d_wave_max(c);
+            uint64_t pr = pr0;
+            for (int k0 = 0; k0 < cmax; k0 += 16) {
+                const int k = k0 + sub;
+                const uint64_t next = pair(g0, k + 16); // read ahead of this one's searches
+                put(k < c, pr);
+                pr = next;
+            }
+            g0 = g1;
+            g1 = g2;
+            s2 = s3;
+            pr0 = pr1;
+        }
+        __syncthreads();
+        // stars with many pairs: all waves together
+        const int nw = nwide;
+        __syncthreads();
+        if (nw == 0) continue;
+        if (tid == 0) nwide = 0;
+        for (int w = 0; w < nw; w++) {
+            const int64_t i = r0 + wide[w];
+            const int s = p.list ? p.list[i] : (int)i, c = p.pcount[s];
+            const uint64_t *src = p.pairbuf + 2 * (p.ntoff[s] - p.tbase);
+            for (int k0 = 64 * wv; k0 < c; k0 += LA_THREADS) put(k0 + lane < c, k0 + lane < c ? src[k0 + lane] : 0ull);
+        }
+        __syncthreads(); // wide[] and nwide are free again
     }
-    const int64_t nc = (int64_t)p.cnt[G4D_CNT_TASKS];
-    const int64_t np = 4 * min(nc, p.ntasks);
-    for (int64_t k0 = (int64_t)blockIdx.x * LA_THREADS; k0 < np; k0 += (int64_t)gridDim.x * LA_THREADS) {
-        const int64_t k = k0 + tid;
-        const uint64_t pr = k < np ? p.proofs[k] : 0ull;
-        put(k < np && is_new(pr), pr);
-        flush(NP_STAGE - LA_THREADS);
+    const int64_t np = 4 * min((int64_t)p.cnt[G4D_CNT_TASKS], p.ntasks);
+    for (int64_t k0 = ((int64_t)blockIdx.x * W + wv) * 64; k0 < np; k0 += (int64_t)gridDim.x * LA_THREADS)
+        put(k0 + lane < np, k0 + lane < np ? p.proofs[k0 + lane] : 0ull);
+    while (nq > 0) drain(min(nq, NP_DRAIN));
+    // what the waves have left, with one atomic
+    __shared__ int left[W];
+    __shared__ unsigned long long rest;
+    if (lane == 0) left[wv] = ns;
+    __syncthreads();
+    int before = 0, all = 0;
+    for (int w = 0; w < W; w++) {
+        if (w < wv) before += left[w];
+        all += left[w];
     }
-    flush(0);
+    if (tid == 0) rest = all ? atomicAdd(&p.cnt[G4D_CNT_NEW_PAIRS], (unsigned long long)all) : 0ull;
+    __syncthreads();
+    flush(ns, rest + before);
 }
 
 hipError_t launch_new_pairs(const NewPairs &p, hipStream_t s)
