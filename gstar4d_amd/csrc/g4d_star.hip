@@ -3073,22 +3073,33 @@ hipError_t launch_live_sizes(int n, const int *vnum, const int *tnum, const int 
     return hipGetLastError();
 }
 
-// One wave per star.
+// 16 lanes a star, whose regions hold some 16 to 30 elements; stars of more than 16 rounds are copied by
+// their whole wave afterwards.  Bound by the records' scattered reads and the copies; a wave per star
+// left most lanes idle: 4,000,000 stars of 1.5 GB 2.06 ms, this 1.08.
 __global__ void __launch_bounds__(256) k_repack(int n, const int *vnum, const int64_t *voff, const int *tnum,
                                                 const int64_t *toff, const int *hnum, const int64_t *hoff,
                                                 const int *vpool, const uint64_t *tpool, const int *hpool,
                                                 const int64_t *vdst, const int64_t *tdst, const int64_t *hdst,
                                                 int *vpool2, uint64_t *tpool2, int *hpool2)
 {
-    const int lane = threadIdx.x & 63;
-    const int w0 = (blockIdx.x * blockDim.x + threadIdx.x) >> 6, nw = (gridDim.x * blockDim.x) >> 6;
-    for (int s = w0; s < n; s += nw) {
+    const int lane = threadIdx.x & 63, sub = lane & 15;
+    const int64_t w0 = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6, nw = ((int64_t)gridDim.x * blockDim.x) >> 6;
+    auto copy = [&](int s, int at, int step, bool big) {
         const int v = vnum[s], h = hnum[s];
         const int64_t tw = v >= STAR_WIDE_MIN ? 2 * (int64_t)tnum[s] : tnum[s];
+        if (!big && max((int64_t)max(v, h), tw) > 256) return true;
         const int64_t vi = voff[s], ti = toff[s], hi = hoff[s], vo = vdst[s], to = tdst[s], ho = hdst[s];
-        for (int i = lane; i < v; i += 64) vpool2[vo + i] = vpool[vi + i];
-        for (int64_t i = lane; i < tw; i += 64) tpool2[to + i] = tpool[ti + i];
-        for (int i = lane; i < h; i += 64) hpool2[ho + i] = hpool[hi + i];
+        for (int i = at; i < v; i += step) vpool2[vo + i] = vpool[vi + i];
+        for (int64_t i = at; i < tw; i += step) tpool2[to + i] = tpool[ti + i];
+        for (int i = at; i < h; i += step) hpool2[ho + i] = hpool[hi + i];
+        return false;
+    };
+    for (int64_t s0 = 4 * w0; s0 < n; s0 += 4 * nw) {
+        const int64_t s = s0 + (lane >> 4);
+        const bool big = s < n && copy((int)s, sub, 16, false);
+        const uint64_t mk = __ballot(big);
+        for (int g = 0; g < 4; g++)
+            if ((mk >> (16 * g)) & 1) copy((int)(s0 + g), lane, 64, true);
     }
 }
 
@@ -3097,7 +3108,7 @@ hipError_t launch_repack(int n, const int *vnum, const int64_t *voff, const int 
                          const int *hpool, const int64_t *vdst, const int64_t *tdst, const int64_t *hdst, int *vpool2,
                          uint64_t *tpool2, int *hpool2, hipStream_t s)
 {
-    hipLaunchKernelGGL(k_repack, dim3(g4d_blocks(n, 4, 65536)), dim3(256), 0, s, n, vnum, voff, tnum, toff, hnum, hoff,
+    hipLaunchKernelGGL(k_repack, dim3(g4d_blocks(n, 16, 65536)), dim3(256), 0, s, n, vnum, voff, tnum, toff, hnum, hoff,
                        vpool, tpool, hpool, vdst, tdst, hdst, vpool2, tpool2, hpool2);
     return hipGetLastError();
 }

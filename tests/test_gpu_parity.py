@@ -299,6 +299,27 @@ def test_star_filter_across_units(orc, shape, unit):
             assert (g.canonical(tets) == ref).all(), v
 
 
+@pytest.mark.parametrize("hub", [0, 300, 700])
+def test_store_repacks_keep_the_stars(orc, hub):
+    """Dense clumps, rebuilt over many rounds, outgrow the star store, which is then repacked (stars of
+    more than 256 words, around hubs, by whole waves); a context that keeps its arenas gives a later
+    call, and one on another set in between, the oracle's triangulation too."""
+    rng = np.random.default_rng(100 + hub)
+    x = np.concatenate([c + 1e-3 * rng.normal(size=(1600, 3)) for c in rng.random((25, 3))])
+    if hub:
+        d = rng.normal(size=(hub, 3))
+        x = np.concatenate([x, 3.0 + 0.4 * d / np.linalg.norm(d, axis=1, keepdims=True), [[3.0, 3.0, 3.0]]])
+    ref, _, _ = orc.triangulate(x, 32)
+    y = datasets.uniform_cube(3000, seed=4)
+    refy, _, _ = orc.triangulate(y, 32)
+    with g.Triangulator(grid_size=32) as t:
+        for z, r in ((x, ref), (y, refy), (x, ref)):
+            tets, _, _ = t.triangulate(z)
+            if z is x:
+                assert t.stats()["store_repacks"] >= 1
+            assert (g.canonical(tets) == r).all()
+
+
 @pytest.mark.parametrize("bands", [1, 3, 5])
 def test_pba_bands_same_triangulation(orc, bands):
     x = datasets.uniform_cube(20000, seed=31)
