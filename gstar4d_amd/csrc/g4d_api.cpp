@@ -40,6 +40,11 @@ namespace {
 
 // Star storage: per-star records over three append-only arenas (link vertices as int,
 // triangle words as uint64, history vertices as int).  top[k] counts the elements in use.
+static constexpr int SIDE_STREAMS = 3;
+// Stars above 64 link vertices from which the 128- and 256-vertex tiers run beside the smaller ones: below
+// it the two events cost as much as the kernels' overlap gives.
+static constexpr int64_t FORK_STARS = 512;
+
 struct Store {
     static constexpr size_t esz[3] = {sizeof(int), sizeof(uint64_t), sizeof(int)};
     // Arenas that a repack has left are kept for the next one, or for the next call when they are the
@@ -105,7 +110,7 @@ struct g4d_ctx {
     DevBuf xyz_up, keys, pts, perm, vox, bounds, settab, ptset, grid, gtmp, idgrid, pbaspill, pbaenv, pbacnt, pcount, pairs,
         ws_off, cnt;
     Store store;
-    DevBuf settet, dflag, pairbuf, spcount, dkeys, tasks, cand, ins, ins_off, active, mid, big, huge, xstars,
+    DevBuf settet, dflag, pairbuf, spcount, dkeys, tasks, cand, ins, ins_off, active, mid, big, huge, xstars, wexact,
         xtasks, xtris, gwork, tetcnt, tetoff, tets, opp, table;
     // learned proposal: parameters, candidates, features, proposed pairs, capacity bins, labels
     DevBuf mlp_params, fkeys, ford, frank, pcand, pd2, pfeat, ppairs, pcap, plab, pvcap;
@@ -132,6 +137,10 @@ struct g4d_ctx {
     hipError_t noalloc_status = hipErrorNotInitialized; // lookup of the scratch array's address
     // tuning (g4d_set_star_kernel, g4d_set_grid_table)
     int star_t0_variant = -1;
+    // streams beside `stream` for the larger star tiers, made when a call first has such stars
+    hipStream_t side[SIDE_STREAMS] = {};
+    hipEvent_t ev_side[SIDE_STREAMS + 1] = {}; // one per side stream, and the fork's
+    bool side_ok = false, side_make = true;
     int pba_bands = 0; // bands of the y and x PBA passes (0: by grid size)
     int stage_graphs = -1; // grid-stage chain as a hipGraph: 1 always, 0 never, -1 batched calls only
     // captured grid-stage chains (site scatter and the PBA passes), keyed by everything the
@@ -335,12 +344,57 @@ static double ev_ms(g4d_ctx *ctx, int a, int b)
     return ms;
 }
 
-// Passes of at most this many stars run the filter tiers above 32 vertices as one launch: the waves
-// of the 256-vertex star kernel that are resident together (six a CU).
-static const int TIER_MERGE = 1536;
-// Counters of a pass's plan.
+// Side streams of one star pass.  use(i) makes side stream i wait for what the call's stream held at
+// open(); join() makes the call's stream wait for every one used, and is reached on every path that
+// launched on them.  Without side streams (not wanted, or none to be had) all work goes to the call's.
+struct SideStreams {
+    g4d_ctx *ctx;
+    bool on;
+    bool used[SIDE_STREAMS] = {};
+    hipStream_t main = nullptr;
+    SideStreams(g4d_ctx *c, bool want) : ctx(c), on(want)
+    {
+        if (on && !ctx->side_ok && ctx->side_make) {
+            ctx->side_make = false; // one attempt
+            bool ok = true;
+            for (int i = 0; i < SIDE_STREAMS; i++) ok = ok && hipStreamCreate(&ctx->side[i]) == hipSuccess;
+            for (int i = 0; i <= SIDE_STREAMS; i++)
+                ok = ok && hipEventCreateWithFlags(&ctx->ev_side[i], hipEventDisableTiming) == hipSuccess;
+            ctx->side_ok = ok;
+            if (!ok) (void)hipGetLastError();
+        }
+        on = on && ctx->side_ok;
+    }
+    hipError_t open(hipStream_t s)
+    {
+        main = s;
+        return on ? hipEventRecord(ctx->ev_side[SIDE_STREAMS], s) : hipSuccess;
+    }
+    hipStream_t use(int i)
+    {
+        if (!on) return main;
+        if (!used[i] && hipStreamWaitEvent(ctx->side[i], ctx->ev_side[SIDE_STREAMS], 0) != hipSuccess) return main;
+        used[i] = true;
+        return ctx->side[i];
+    }
+    hipError_t join(hipStream_t s)
+    {
+        hipError_t r = hipSuccess;
+        for (int i = 0; i < SIDE_STREAMS; i++) {
+            if (!used[i]) continue;
+            hipError_t e = hipEventRecord(ctx->ev_side[i], ctx->side[i]);
+            if (e == hipSuccess) e = hipStreamWaitEvent(s, ctx->ev_side[i], 0);
+            if (e != hipSuccess) {
+                (void)hipStreamSynchronize(ctx->side[i]);
+                r = e;
+            }
+        }
+        return r;
+    }
+};
+
 static const uint64_t PLAN_COUNTERS = (1ull << G4D_CNT_ACTIVE) | (1ull << G4D_CNT_NEED_V) | (1ull << G4D_CNT_NEED_T) |
-                                      (1ull << G4D_CNT_NEED_H);
+                                      (1ull << G4D_CNT_NEED_H) | (0xffull << G4D_CNT_TIER0);
 
 // The whole path on device-resident FP64 points.
 // Point sets of one call (host side): set k holds points [pt_off[k], pt_off[k+1]) with grid
@@ -822,9 +876,15 @@ static int run_device(g4d_ctx *ctx, const double *d_xyz, int n, const SetSpec &s
         pl.nhoff = buf<int64_t>(store.nhoff);
         pl.pcount = spc;
         pl.cnt = cnt;
+        pl.tier[0] = buf<int>(ctx->mid);
+        pl.tier[1] = buf<int>(ctx->big);
+        pl.tier[2] = buf<int>(ctx->huge);
+        pl.n = n;
+        pl.lds_limit = lds_limit;
         return pl;
     };
     int64_t tbase_last = 0;
+    int64_t tier_n[g4d::STAR_TIERS] = {}, nover64 = 0, need_max = 0; // as planned
 
     // One pass over the nitems stars of the active list (mode 0: every star, from its workset), whose
     // regions of need[] elements are planned at the arenas' tops; the others are not touched.
@@ -888,9 +948,8 @@ static int run_device(g4d_ctx *ctx, const double *d_xyz, int n, const SetSpec &s
         sp.pcount = spc;
         sp.cnt = cnt;
         sp.lds_limit = lds_limit;
-        sp.defer_list = buf<int>(ctx->mid);
+        sp.defer_list = nullptr; // larger stars are on the plan's lists
         sp.defer_cap = n;
-        sp.defer_counter = G4D_CNT_APPEND6;
         sp.exact_list = buf<int>(ctx->xstars);
         sp.exact_cap = n;
         sp.exact_counter = G4D_CNT_APPEND4;
@@ -898,66 +957,98 @@ static int run_device(g4d_ctx *ctx, const double *d_xyz, int n, const SetSpec &s
         // list counters, totals and work-queue heads of this pass, and the lists made after it
         {
             uint64_t zmask = PLAN_COUNTERS;
-            for (int c : {G4D_CNT_APPEND2, G4D_CNT_APPEND3, G4D_CNT_APPEND4, G4D_CNT_APPEND5, G4D_CNT_APPEND6, G4D_CNT_XMID,
+            for (int c : {G4D_CNT_APPEND3, G4D_CNT_APPEND4, G4D_CNT_APPEND5, G4D_CNT_XMID,
                           G4D_CNT_XBIG, G4D_CNT_XL, G4D_CNT_ORIENT4, G4D_CNT_COFACTOR, G4D_CNT_PAIRS, G4D_CNT_DROWNED,
                           G4D_CNT_DROWN_KEYS, G4D_CNT_TASKS, G4D_CNT_NEW_PAIRS, G4D_CNT_INS})
                 zmask |= 1ull << c;
             for (int q = 0; q < 7; q++) zmask |= 1ull << (G4D_CNT_QUEUE0 + q);
             HCK(g4d::launch_zero_counters(cnt, zmask, s));
         }
-        int queue = G4D_CNT_QUEUE0;
-        sp.work_counter = queue++;
+        sp.work_counter = G4D_CNT_QUEUE0;
         sp.star_list = list;
         sp.nlist = nitems;
         sp.nlist_dev = nullptr;
-        // Filter-only LDS kernels by size tier (32 -> 64 -> 128 -> 256 link vertices); each passes
-        // the stars it cannot hold to the next tier's list and the ones its filters cannot decide
-        // to the exact list.  Every later launch reads its list length on the device, so the chain
-        // runs without host round trips; lists and counters are reused in stream order.
-        if (ctx->ev_ok) (void)hipEventRecord(ctx->ev_t0[0], s);
-        HCK(g4d::launch_star_kernel(sp, g4d::STAR_VMAX_T0, false, nblk_star, s));
-        if (ctx->ev_ok) (void)hipEventRecord(ctx->ev_t0[1], s);
-        auto chain = [&](int *lst, int counter, int *defer, int defer_counter, int vmax, bool exact) -> int {
-            sp.star_list = lst;
-            sp.nlist = n;
-            sp.nlist_dev = cnt + counter;
-            sp.defer_list = defer;
-            sp.defer_counter = defer_counter;
-            sp.work_counter = queue++;
-            // a tier's list is a subset of the pass's stars: late rounds with a few thousand stars
-            // dispatch a few hundred work-groups instead of thousands that would leave at once; at
-            // most as many as the tier has resident waves
-            const int full = exact ? 1024 : vmax == g4d::STAR_VMAX_T1 ? 4096 : vmax == g4d::STAR_VMAX_TM ? 3072 : 1536;
-            const int nblk = nitems <= TIER_MERGE && !exact ? nitems : std::max(64, std::min(full, (nitems + 7) / 8));
-            HCK(g4d::launch_star_kernel(sp, vmax, exact, nblk, s));
-            return G4D_OK;
+        // Filter-only kernels by size tier over the plan's lists, each star in one of them: they need
+        // not wait for each other.  The many small stars run on the call's stream; those of the larger
+        // tiers, few at a time and each a long chain of insertions that one wave or work-group
+        // steps through, run beside them where there are enough to matter.
+        // 1,000,000 clustered points: tier after tier 76.4 ms a call, side by side 65.2.
+        const int *tl[g4d::STAR_TIERS];
+        for (int k = 0; k < g4d::STAR_TIERS; k++) {
+            const int *arr = k < 2 ? buf<int>(ctx->mid) : k < 4 ? buf<int>(ctx->big) : buf<int>(ctx->huge);
+            tl[k] = (k & 1) ? arr + n - tier_n[k] : arr;
+        }
+        const int64_t nwide = tier_n[3] + tier_n[4], nglobal = tier_n[5];
+        const bool fork128 = tier_n[1] + tier_n[2] >= FORK_STARS, forkw = nwide > 0, forkg = nglobal > 0;
+        const int64_t gstride = (g4d::star_global_bytes((int)need_max) + 4095) & ~(int64_t)4095;
+        // bounded workspace: at most 256 blocks and 1 GiB
+        auto global_blocks = [&](int64_t count, int64_t stride) {
+            return (int)std::max<int64_t>(1, std::min<int64_t>({count, 256, ((int64_t)1 << 30) / stride}));
         };
-        // filter tiers: mid list (A6) -> 64, big list (A2) -> 128, mid list again (XL) -> 256, beyond
-        // -> huge (A3)
-        // Late rounds: the 256-vertex tier's resident waves hold every star of the pass, so it takes the
-        // smaller ones too (the tiers number a star's slots alike) and the stars' chains of
-        // insertions run side by side, one star a wave, instead of tier after tier and eight stars a
-        // wave (100,000 uniform points, six late passes: 1.15 -> 0.30 ms).
-        if (nitems <= TIER_MERGE) {
-            CK(chain(buf<int>(ctx->mid), G4D_CNT_APPEND6, buf<int>(ctx->huge), G4D_CNT_APPEND3, g4d::STAR_VMAX_T2, false));
-        } else {
-            CK(chain(buf<int>(ctx->mid), G4D_CNT_APPEND6, buf<int>(ctx->big), G4D_CNT_APPEND2, g4d::STAR_VMAX_T1, false));
-            CK(chain(buf<int>(ctx->big), G4D_CNT_APPEND2, buf<int>(ctx->mid), G4D_CNT_XL, g4d::STAR_VMAX_TM, false));
-            CK(chain(buf<int>(ctx->mid), G4D_CNT_XL, buf<int>(ctx->huge), G4D_CNT_APPEND3, g4d::STAR_VMAX_T2, false));
+        if (nglobal > 0) HCK(ctx->gwork.ensure((size_t)(gstride * global_blocks(nglobal, gstride))));
+        if (nwide > 0) HCK(ctx->wexact.ensure(sizeof(int) * (size_t)n));
+        auto tier_launch = [&](int k, hipStream_t q) -> hipError_t {
+            if (tier_n[k] <= 0) return hipSuccess;
+            g4d::StarParams tp = sp;
+            tp.star_list = tl[k];
+            tp.nlist = (int)tier_n[k];
+            tp.work_counter = G4D_CNT_QUEUE0 + 1 + k;
+            if (k >= 3) {
+                tp.exact_list = buf<int>(ctx->wexact);
+                tp.exact_counter = G4D_CNT_XL;
+                return k == 5 ? g4d::launch_star_global(sp, tl[k], tp.nlist, buf<char>(ctx->gwork), gstride, (int)need_max,
+                                                        global_blocks(nglobal, gstride), q)
+                              : g4d::launch_star_wide(tp, k == 3 ? g4d::STAR_VMAX_W1 : g4d::STAR_VMAX_W2, q);
+            }
+            // at most as many work-groups as the tier has resident waves
+            const int vmax = k == 0 ? g4d::STAR_VMAX_T1 : k == 1 ? g4d::STAR_VMAX_TM : g4d::STAR_VMAX_T2;
+            const int full = k == 0 ? 4096 : k == 1 ? 3072 : 1536;
+            return g4d::launch_star_kernel(tp, vmax, false, std::min(full, tp.nlist), q);
+        };
+        {
+            SideStreams side(ctx, fork128 || forkw || forkg);
+            hipError_t e = side.open(s);
+            auto run = [&](int k, int lane) {
+                if (e == hipSuccess) e = tier_launch(k, side.use(lane));
+            };
+            if (forkg) run(5, 2);
+            if (forkw) run(4, 1), run(3, 1);
+            if (fork128) run(2, 0), run(1, 0);
+            if (ctx->ev_ok) (void)hipEventRecord(ctx->ev_t0[0], s);
+            if (e == hipSuccess) e = g4d::launch_star_kernel(sp, g4d::STAR_VMAX_T0, false, nblk_star, s);
+            if (ctx->ev_ok) (void)hipEventRecord(ctx->ev_t0[1], s);
+            if (e == hipSuccess) e = tier_launch(0, s);
+            if (!fork128) {
+                if (e == hipSuccess) e = tier_launch(1, s);
+                if (e == hipSuccess) e = tier_launch(2, s);
+            }
+            const hipError_t ej = side.join(s); // whatever was launched
+            HCK(e);
+            HCK(ej);
         }
         CK(read_counters(ctx, hc));
-        const int64_t nmid = (int64_t)hc[G4D_CNT_APPEND6], nbig = (int64_t)hc[G4D_CNT_APPEND2];
         const int64_t nexact = (int64_t)hc[G4D_CNT_APPEND4];
         if (nexact > 0) {
-            // The exact-capable kernels of tiers 32, 64 and 256 over the exact list.  They reuse the
-            // mid and big lists (the filter chain is done with them) under counters of their own, so
-            // the filter tiers' counts stay for the statistics.
-            CK(chain(buf<int>(ctx->xstars), G4D_CNT_APPEND4, buf<int>(ctx->mid), G4D_CNT_XMID, g4d::STAR_VMAX_T0, true));
-            CK(chain(buf<int>(ctx->mid), G4D_CNT_XMID, buf<int>(ctx->big), G4D_CNT_XBIG, g4d::STAR_VMAX_T1, true));
-            CK(chain(buf<int>(ctx->big), G4D_CNT_XBIG, buf<int>(ctx->huge), G4D_CNT_APPEND3, g4d::STAR_VMAX_T2, true));
+            // The exact-capable kernels of tiers 32, 64 and 256 over the exact list, each passing the
+            // stars it cannot hold to the next; they reuse the mid and big lists (the filter kernels
+            // are done with them) and read their lengths on the device.
+            auto chain = [&](int *lst, int counter, int *defer, int defer_counter, int vmax) -> int {
+                sp.star_list = lst;
+                sp.nlist = n;
+                sp.nlist_dev = cnt + counter;
+                sp.defer_list = defer;
+                sp.defer_counter = defer_counter;
+                sp.work_counter = G4D_CNT_QUEUE0 + 1 + (vmax == g4d::STAR_VMAX_T1 ? 1 : vmax == g4d::STAR_VMAX_T2 ? 2 : 0);
+                HCK(g4d::launch_star_kernel(sp, vmax, true, std::max(64, std::min(1024, (nitems + 7) / 8)), s));
+                return G4D_OK;
+            };
+            HCK(g4d::launch_zero_counters(cnt, 7ull << (G4D_CNT_QUEUE0 + 1), s));
+            CK(chain(buf<int>(ctx->xstars), G4D_CNT_APPEND4, buf<int>(ctx->mid), G4D_CNT_XMID, g4d::STAR_VMAX_T0));
+            CK(chain(buf<int>(ctx->mid), G4D_CNT_XMID, buf<int>(ctx->big), G4D_CNT_XBIG, g4d::STAR_VMAX_T1));
+            CK(chain(buf<int>(ctx->big), G4D_CNT_XBIG, buf<int>(ctx->huge), G4D_CNT_APPEND3, g4d::STAR_VMAX_T2));
             CK(read_counters(ctx, hc));
+            if (hc[G4D_CNT_APPEND3]) return set_err(ctx, G4D_ERR_INTERNAL, "exact star list holds a larger star");
         }
-        sp.nlist_dev = nullptr;
         {
             float ms = 0.f;
             if (ctx->ev_ok && hipEventElapsedTime(&ms, ctx->ev_t0[0], ctx->ev_t0[1]) == hipSuccess)
@@ -966,60 +1057,33 @@ static int run_device(g4d_ctx *ctx, const double *d_xyz, int n, const SetSpec &s
             ctx->st.star_t0_cofactors += (int64_t)hc[G4D_CNT_COFACTOR];
             ctx->st.star_t0_launches++;
         }
-        ctx->st.big_stars += (int32_t)nbig;
+        ctx->st.big_stars += (int32_t)nover64;
         ctx->st.exact_stars += nexact;
-        const int64_t nhuge = (int64_t)hc[G4D_CNT_APPEND3];
-        if (nhuge > 0) {
-            ctx->st.huge_stars += (int32_t)nhuge;
-            // Beyond the one-wave kernels: the wide LDS kernel's two tiers (huge list -> 512, big list
-            // -> 1024), then the global-memory kernel for larger stars and those that need exact
-            // predicates (mid list).  A lowered lds_star_limit sends every star to the latter.
-            int *glist = buf<int>(ctx->huge);
-            int64_t nglobal = nhuge;
-            if (lds_limit == g4d::STAR_LDS_LIMIT) {
-                const int q = G4D_CNT_QUEUE0;
-                HCK(g4d::launch_zero_counters(cnt, (1ull << G4D_CNT_XMID) | (1ull << G4D_CNT_XBIG) | (3ull << q), s));
-                glist = buf<int>(ctx->mid);
-                sp.exact_list = glist;
-                sp.exact_counter = G4D_CNT_XMID;
-                sp.nlist = n;
-                sp.star_list = buf<int>(ctx->huge);
-                sp.nlist_dev = cnt + G4D_CNT_APPEND3;
-                sp.defer_list = buf<int>(ctx->big);
-                sp.defer_counter = G4D_CNT_XBIG;
-                sp.work_counter = q;
-                HCK(g4d::launch_star_wide(sp, g4d::STAR_VMAX_W1, s));
-                sp.star_list = buf<int>(ctx->big);
-                sp.nlist_dev = cnt + G4D_CNT_XBIG;
-                sp.defer_list = glist;
-                sp.defer_counter = G4D_CNT_XMID;
-                sp.work_counter = q + 1;
-                HCK(g4d::launch_star_wide(sp, g4d::STAR_VMAX_W2, s));
-                sp.nlist_dev = nullptr;
-                CK(read_counters(ctx, hc));
-                nglobal = (int64_t)hc[G4D_CNT_XMID];
-            }
-            if (nglobal > 0) {
-                HCK(hipMemsetAsync(cnt + G4D_CNT_MISC, 0, 8, s));
-                HCK(g4d::launch_need_max(sp, glist, (int)nglobal, cnt + G4D_CNT_MISC, s));
-                CK(read_counters(ctx, hc));
-                const int vcap_g = (int)hc[G4D_CNT_MISC];
-                const int64_t stride = (g4d::star_global_bytes(vcap_g) + 4095) & ~(int64_t)4095;
-                // bounded workspace: at most 256 blocks and 1 GiB
-                const int nblk = (int)std::max<int64_t>(1, std::min<int64_t>({nglobal, 256, ((int64_t)1 << 30) / stride}));
-                HCK(ctx->gwork.ensure((size_t)(stride * nblk)));
-                HCK(g4d::launch_star_global(sp, glist, (int)nglobal, buf<char>(ctx->gwork), stride, vcap_g, nblk, s));
-                CK(read_counters(ctx, hc));
-                trace("global-memory star kernel: %lld stars, largest link plus insertions %d", (long long)nglobal, vcap_g);
-            }
+        ctx->st.huge_stars += (int32_t)(nwide + nglobal);
+        if (nglobal > 0)
+            trace("global-memory star kernel: %lld stars, largest link plus insertions %lld", (long long)nglobal,
+                  (long long)need_max);
+        if (nwide > 0 && hc[G4D_CNT_XL] > 0) {
+            // wide stars that need exact predicates: the global-memory kernel has them
+            const int64_t nx = (int64_t)hc[G4D_CNT_XL];
+            sp.nlist_dev = nullptr;
+            HCK(g4d::launch_zero_counters(cnt, 1ull << G4D_CNT_MISC, s));
+            HCK(g4d::launch_need_max(sp, buf<int>(ctx->wexact), (int)nx, cnt + G4D_CNT_MISC, s));
+            CK(read_counters(ctx, hc));
+            const int vcap_g = (int)hc[G4D_CNT_MISC];
+            const int64_t stride = (g4d::star_global_bytes(vcap_g) + 4095) & ~(int64_t)4095;
+            const int nblk = global_blocks(nx, stride);
+            HCK(ctx->gwork.ensure((size_t)(stride * nblk)));
+            HCK(g4d::launch_star_global(sp, buf<int>(ctx->wexact), (int)nx, buf<char>(ctx->gwork), stride, vcap_g, nblk, s));
+            CK(read_counters(ctx, hc));
         }
         CK(check_dev_error(ctx, hc[G4D_CNT_ERROR], mode ? "splaying" : "star creation"));
         *drown_n = (int64_t)hc[G4D_CNT_DROWNED];
         *tp_n = (int64_t)hc[G4D_CNT_PAIRS];
         if (*tp_n > npb) return set_err(ctx, G4D_ERR_INTERNAL, "star pairs exceed their regions");
-        trace("star pass mode %d: %lld insertions into %d stars, over 32: %lld, over 64: %lld, exact %lld, "
+        trace("star pass mode %d: %lld insertions into %d stars, over 64: %lld, exact %lld, "
               "beyond 256 %lld, drowned %lld, pairs %lld",
-              mode, (long long)nins, nitems, (long long)nmid, (long long)nbig, (long long)nexact, (long long)nhuge,
+              mode, (long long)nins, nitems, (long long)nover64, (long long)nexact, (long long)(nwide + nglobal),
               (long long)*drown_n, (long long)*tp_n);
         return G4D_OK;
     };
@@ -1032,6 +1096,9 @@ static int run_device(g4d_ctx *ctx, const double *d_xyz, int n, const SetSpec &s
         need[0] = (int64_t)hc[G4D_CNT_NEED_V];
         need[1] = (int64_t)hc[G4D_CNT_NEED_T];
         need[2] = (int64_t)hc[G4D_CNT_NEED_H];
+        for (int k = 0; k < g4d::STAR_TIERS; k++) tier_n[k] = (int64_t)hc[G4D_CNT_TIER0 + k];
+        nover64 = (int64_t)hc[G4D_CNT_OVER64];
+        need_max = (int64_t)hc[G4D_CNT_NEED_MAX];
     };
     HCK(g4d::launch_pass_plan(pass_plan(), pr, m, nullptr, s));
     CK(read_counters(ctx, hc));
@@ -1310,7 +1377,7 @@ int g4d_create(g4d_ctx **out, const g4d_options *opt)
     for (int i = 0; i < 2; i++)
         if (hipEventCreate(&ctx->ev_t0[i]) != hipSuccess) ctx->ev_ok = false;
     // staging of the small host reads; without it they go to pageable variables
-    if (ctx->hpin.ensure(sizeof(int64_t) * 64) == hipSuccess) {
+    if (ctx->hpin.ensure(sizeof(int64_t) * 96) == hipSuccess) {
         ctx->hstage = static_cast<int64_t *>(ctx->hpin.ptr);
         ctx->P.hstage = ctx->hstage + G4D_CNT_NUM + 16;
     }
@@ -1325,7 +1392,7 @@ void g4d_destroy(g4d_ctx *ctx)
     if (ctx->stream) (void)hipStreamSynchronize(ctx->stream);
     DevBuf *bufs[] = {&ctx->xyz_up, &ctx->keys, &ctx->pts, &ctx->perm, &ctx->vox, &ctx->bounds, &ctx->settab, &ctx->ptset, &ctx->grid,
                       &ctx->gtmp, &ctx->idgrid, &ctx->pbaspill, &ctx->pbaenv, &ctx->pbacnt, &ctx->pcount, &ctx->pairs, &ctx->ws_off, &ctx->cnt, &ctx->settet, &ctx->dflag, &ctx->pairbuf, &ctx->spcount, &ctx->dkeys,
-                      &ctx->tasks, &ctx->cand, &ctx->ins, &ctx->ins_off, &ctx->active, &ctx->mid, &ctx->big, &ctx->huge, &ctx->xstars, &ctx->xtasks, &ctx->xtris, &ctx->gwork, &ctx->tetcnt, &ctx->tetoff, &ctx->tets, &ctx->opp, &ctx->table,
+                      &ctx->tasks, &ctx->cand, &ctx->ins, &ctx->ins_off, &ctx->active, &ctx->mid, &ctx->big, &ctx->huge, &ctx->xstars, &ctx->wexact, &ctx->xtasks, &ctx->xtris, &ctx->gwork, &ctx->tetcnt, &ctx->tetoff, &ctx->tets, &ctx->opp, &ctx->table,
                       &ctx->mlp_params, &ctx->fkeys, &ctx->ford, &ctx->frank, &ctx->pcand, &ctx->pd2, &ctx->pfeat,
                       &ctx->ppairs, &ctx->pcap, &ctx->plab, &ctx->pvcap};
     destroy_graphs(ctx);
@@ -1341,6 +1408,10 @@ void g4d_destroy(g4d_ctx *ctx)
     if (ctx->ev_ok)
         for (int i = 0; i < 2; i++) (void)hipEventDestroy(ctx->ev_t0[i]);
     if (ctx->stream) (void)hipStreamDestroy(ctx->stream);
+    for (int i = 0; i < SIDE_STREAMS; i++)
+        if (ctx->side[i]) (void)hipStreamDestroy(ctx->side[i]);
+    for (int i = 0; i <= SIDE_STREAMS; i++)
+        if (ctx->ev_side[i]) (void)hipEventDestroy(ctx->ev_side[i]);
     delete ctx;
 }
 
@@ -1563,6 +1634,10 @@ int g4d_triangulate_device_noalloc(g4d_ctx *ctx, const double *d_xyz, int32_t n,
     tmp.pba_bands = ctx->pba_bands;
     tmp.stage_graphs = 0; // instantiating a graph allocates
     tmp.ev_ok = ctx->ev_ok;
+    tmp.side_ok = ctx->side_ok; // side streams if there are any: making them would allocate
+    for (int i = 0; i < SIDE_STREAMS; i++) tmp.side[i] = ctx->side[i], tmp.ev_side[i] = ctx->ev_side[i];
+    tmp.ev_side[SIDE_STREAMS] = ctx->ev_side[SIDE_STREAMS];
+    tmp.side_make = false;
     tmp.hstage = ctx->hstage; // the caller's page-locked staging (allocated at g4d_create)
     tmp.P.hstage = ctx->P.hstage;
     for (int i = 0; i < EV_NUM; i++) tmp.ev[i] = ctx->ev[i];

@@ -51,7 +51,7 @@ enum g4d_counter : int {
     G4D_CNT_SOS = 6,      // SoS resolutions
     G4D_CNT_ORIENT3 = 7,
     G4D_CNT_MISC = 8,
-    G4D_CNT_XL = 9,       // list length of the filter chain's 256-vertex tier
+    G4D_CNT_XL = 9,       // list length of the wide kernels' inconclusive stars
     G4D_CNT_APPEND3 = 10,
     G4D_CNT_APPEND4 = 11,
     G4D_CNT_APPEND5 = 12,
@@ -75,7 +75,12 @@ enum g4d_counter : int {
     G4D_CNT_MISSING = 34,
     G4D_CNT_PUMPED = 35,
     G4D_CNT_OUT_EXACT = 36,
-    G4D_CNT_NUM = 37
+    // made by a pass's plan: lengths of the lists of stars above 32 (64, 128, 256, 512, 1,024 vertices,
+    // and beyond), the number above 64, and the largest of the last list
+    G4D_CNT_TIER0 = 37,
+    G4D_CNT_OVER64 = 43,
+    G4D_CNT_NEED_MAX = 44,
+    G4D_CNT_NUM = 45
 };
 
 #define HIP_CHECK_RET(expr)                                                                    \

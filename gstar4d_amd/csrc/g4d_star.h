@@ -67,7 +67,8 @@ struct StarParams {
     uint64_t *pairbuf;    // per star, from 2 * (ntoff[s] - tbase): its insertion pairs (a<<32 | b,
     int64_t tbase;        // a < b) of unchecked triangles, dense, in triangle order
     int *pcount;          // per star: the number of those pairs
-    int *defer_list;      // stars that exceed this kernel's capacity, counter `defer_counter`
+    int *defer_list;      // stars that exceed this kernel's capacity, counter `defer_counter`; null in the
+                          // 32-vertex kernels: such stars are on a list of the plan and skipped
     int64_t defer_cap;
     int defer_counter;
     int *exact_list;      // stars whose filters were inconclusive (filter-only kernels),
@@ -102,8 +103,8 @@ enum {
 // Zeroes the counter words whose bits are set in mask (one launch instead of one fill per word).
 hipError_t launch_zero_counters(unsigned long long *cnt, uint64_t mask, hipStream_t s);
 hipError_t launch_star_kernel(const StarParams &p, int vmax, bool exact, int nblocks, hipStream_t s);
-// Wide LDS kernel, vmax = STAR_VMAX_W1 or W2, over the star_list whose length is at nlist_dev:
-// larger stars go to p.defer_list, inconclusive ones untouched to p.exact_list.
+// Wide LDS kernel, vmax = STAR_VMAX_W1 or W2, over the nlist stars of star_list, none larger;
+// inconclusive ones go untouched to p.exact_list.
 hipError_t launch_star_wide(const StarParams &p, int vmax, hipStream_t s);
 // Global-memory star kernel for the stars in `list` (any size up to vcap link vertices);
 // each block owns a workspace of star_global_bytes(vcap) bytes at ws + blockIdx * stride.
@@ -166,6 +167,7 @@ struct NewPairs {
     unsigned long long *cnt;
 };
 hipError_t launch_new_pairs(const NewPairs &p, hipStream_t s);
+static constexpr int STAR_TIERS = 6;
 // The next pass's work from its sorted distinct insertion keys: CSR offsets of the stars with
 // insertions, their list (G4D_CNT_ACTIVE), and fresh regions for them from the arenas' tops base[]
 // (sizes at G4D_CNT_NEED_V / _T / _H).  pcount[s] = 0 for these stars.
@@ -180,6 +182,12 @@ struct PassPlan {
     int64_t *nhoff;
     int *pcount;
     unsigned long long *cnt;
+    // Lists of the stars above 32 link vertices and insertions, two to an array of n (one from its
+    // front, one from its end): 64 and 128, 256 and 512, 1,024 and beyond (or above lds_limit);
+    // counters from G4D_CNT_TIER0.
+    int *tier[STAR_TIERS / 2];
+    int n;
+    int lds_limit;
 };
 // m keys, or *dev_m (at most m) when dev_m is given.
 hipError_t launch_pass_plan(const PassPlan &p, const uint64_t *keys, int64_t m, const int64_t *dev_m, hipStream_t s);

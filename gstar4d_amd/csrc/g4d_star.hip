@@ -291,7 +291,9 @@ __device__ __forceinline__ void star_body(const StarParams &p, int nitems)
             const int need = vn + m;
             const int lim = VMAX < p.lds_limit ? VMAX : p.lds_limit;
             if (need > lim) {
-                star_list_push(p.defer_list, p.defer_cap, &cnt[p.defer_counter], s, cnt);
+                if (p.defer_list) star_list_push(p.defer_list, p.defer_cap, &cnt[p.defer_counter], s, cnt);
+                else if (VMAX > STAR_VMAX_T0 && lane == 0) // not the list of this tier
+                    atomicOr(&cnt[G4D_CNT_ERROR], (unsigned long long)G4D_DEV_ERR_BUFFER);
                 continue;
             }
             if (p.mode == 0 && m < 4) {
@@ -714,7 +716,7 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WPE, 8)
 // reached by the whole wave in uniform control flow: the insertion loop runs to the largest
 // insertion count of the wave's stars, and a group with nothing to do in a step has its work
 // masked off.  Filters only (no multiprecision code): a star with an inconclusive orientation
-// goes to p.exact_list untouched, a star beyond the tier to p.defer_list, as in k_star32.
+// goes to p.exact_list untouched; a star beyond the tier is left to the plan's lists.
 //
 // Bound by vector instructions (two thirds of the issue slots at three waves per SIMD, of them a
 // fifth FP64), with the LDS pipe half busy.  At 4,194,304 uniform points (G = 512) all its passes took
@@ -960,14 +962,7 @@ __device__ __forceinline__ void star_body_grp(const StarParams &p, int nitems)
             const int vn = act && p.mode ? p.vnum[s] : 0;
             const int need = vn + m;
             const int lim = VMAX < p.lds_limit ? VMAX : p.lds_limit;
-            if (act && need > lim) {
-                if (gl == 0) {
-                    const unsigned long long k = atomicAdd(&cnt[p.defer_counter], 1ull);
-                    if ((int64_t)k < p.defer_cap) p.defer_list[k] = s;
-                    else atomicOr(&cnt[G4D_CNT_ERROR], (unsigned long long)G4D_DEV_ERR_BUFFER);
-                }
-                act = false;
-            }
+            if (act && need > lim) act = false; // on a list of the plan
             if (act && p.mode == 0 && m < 4) {
                 if (gl == 0) {
                     atomicOr(&cnt[G4D_CNT_ERROR], (unsigned long long)G4D_DEV_ERR_CONE);
@@ -1554,9 +1549,6 @@ __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(WPE, 8)
     const int tid = threadIdx.x;
     unsigned long long *cnt = p.cnt;
     double rc[KPL][4], rp[KPL][2];
-    const unsigned long long c = *p.nlist_dev;
-    nitems = c < (unsigned long long)nitems ? (int)c : nitems;
-    if ((int)blockIdx.x >= nitems) return;
     int ncof = 0, nfilt = 0;
     unsigned long long npairs = 0, ndrown = 0; // of the work-group, and of the wave
     for (;;) {
@@ -1570,10 +1562,8 @@ __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(WPE, 8)
         const int vn = p.mode ? p.vnum[s] : 0;
         const int need = vn + m;
         if (need > VMAX || (p.mode == 0 && m < 4)) {
-            if (need > VMAX) {
-                if (tid < 64) star_list_push(p.defer_list, p.defer_cap, &cnt[p.defer_counter], s, cnt);
-            } else if (tid == 0) {
-                atomicOr(&cnt[G4D_CNT_ERROR], (unsigned long long)G4D_DEV_ERR_CONE);
+            if (tid == 0) {
+                atomicOr(&cnt[G4D_CNT_ERROR], (unsigned long long)(need > VMAX ? G4D_DEV_ERR_BUFFER : G4D_DEV_ERR_CONE));
                 p.vnum[s] = 0;
                 p.tnum[s] = 0;
             }
@@ -1865,12 +1855,15 @@ __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(WPE, 8)
 
 hipError_t launch_star_wide(const StarParams &p, int vmax, hipStream_t s)
 {
-    if (!p.star_list || !p.nlist_dev || p.nlist <= 0) return hipErrorInvalidValue;
-    // one work-group per resident one: LDS takes 50 KB at 512 vertices, 100 KB at 1,024
+    if (p.nlist <= 0) return hipSuccess;
+    if (!p.star_list) return hipErrorInvalidValue;
+    // at most one work-group per resident one: LDS takes 50 KB at 512 vertices, 100 KB at 1,024
     if (vmax == STAR_VMAX_W1)
-        hipLaunchKernelGGL(HIP_KERNEL_NAME(k_star_wide<STAR_VMAX_W1, 256, 3>), dim3(768), dim3(256), 0, s, p, p.nlist);
+        hipLaunchKernelGGL(HIP_KERNEL_NAME(k_star_wide<STAR_VMAX_W1, 256, 3>), dim3(std::min(p.nlist, 768)), dim3(256), 0, s,
+                           p, p.nlist);
     else if (vmax == STAR_VMAX_W2)
-        hipLaunchKernelGGL(HIP_KERNEL_NAME(k_star_wide<STAR_VMAX_W2, 512, 2>), dim3(256), dim3(512), 0, s, p, p.nlist);
+        hipLaunchKernelGGL(HIP_KERNEL_NAME(k_star_wide<STAR_VMAX_W2, 512, 2>), dim3(std::min(p.nlist, 256)), dim3(512), 0, s,
+                           p, p.nlist);
     else
         return hipErrorInvalidValue;
     return hipGetLastError();
@@ -2052,7 +2045,7 @@ __global__ void __launch_bounds__(GSTAR_NT) k_star_global(StarParams p, const in
         for (int slot = tid; slot < T; slot += GSTAR_NT)
             tri_cofactors(L.vc + 4 * L.tva[3 * slot], L.vc + 4 * L.tva[3 * slot + 1], L.vc + 4 * L.tva[3 * slot + 2],
                           L.cof + 8 * slot, L.cof + 8 * slot + 4);
-        bool failed = false, unsure = false;
+        bool failed = false;
         for (int q = q0; q < m; q++) {
             const int gv = L.ins[q];
             const int Vn = vn + q;
@@ -2181,11 +2174,6 @@ __global__ void __launch_bounds__(GSTAR_NT) k_star_global(StarParams p, const in
                 }
             }
             __syncthreads();
-        }
-        if (unsure) {
-            star_list_push(p.exact_list, p.exact_cap, &cnt[p.exact_counter], s, cnt);
-            __syncthreads();
-            continue;
         }
         if (failed) {
             if (tid == 0) {
@@ -2834,6 +2822,23 @@ __device__ __forceinline__ void plan_star(const PassPlan &p, int s, int64_t firs
     p.pcount[s] = 0;
 }
 
+// Tier of a star above 32, -1 for one that the 32-vertex kernel takes.  A pass of few keys sends all of
+// tiers 64 to 256 to the 256-vertex kernel: its resident waves hold them all, the tiers number a star's
+// slots alike, and the stars' chains of insertions run side by side and not launch after launch
+// (100,000 uniform points, six late passes: 1.15 -> 0.30 ms; up to some 1,500 stars, four keys each).
+static constexpr int TIER_MERGE_KEYS = 6144;
+__device__ __forceinline__ int star_tier(int need, int lim, bool merge)
+{
+    if (need <= min(STAR_VMAX_T0, lim)) return -1;
+    if (need <= min(STAR_VMAX_T2, lim)) return merge || need > STAR_VMAX_TM ? 2 : (need > STAR_VMAX_T1 ? 1 : 0);
+    if (lim < STAR_LDS_LIMIT) return 5; // a lowered limit sends every larger star to the global-memory kernel
+    return need <= STAR_VMAX_W1 ? 3 : (need <= STAR_VMAX_W2 ? 4 : 5);
+}
+__device__ __forceinline__ void tier_put(const PassPlan &p, int tier, int k, int s)
+{
+    p.tier[tier >> 1][(tier & 1) ? p.n - 1 - k : k] = s;
+}
+
 // A tile of keys is read once, in order, into LDS (a thread that reads its own eight in a row loads
 // every line eight times); the keys that start a star's run are listed, and a thread plans a few
 // stars in a row.  Only the tile's last run has its end searched for, by doubling steps.  The tile's
@@ -2847,11 +2852,13 @@ __global__ void __launch_bounds__(LA_THREADS) k_pass_plan(PassPlan p, const uint
     __shared__ uint16_t first[PP_TILE + 1];
     __shared__ int red[5][LA_THREADS / 64];
     __shared__ unsigned long long base[4];
-    __shared__ int last_len;
+    __shared__ int last_len, tn[STAR_TIERS + 2]; // per tier, above 64, largest beyond the tiers
     if (dev_m) m = min(m, *dev_m);
     const int64_t t0 = (int64_t)blockIdx.x * PP_TILE;
     if (t0 >= m) return;
     const int nt = (int)min((int64_t)PP_TILE, m - t0), tid = threadIdx.x;
+    const bool merge = m <= TIER_MERGE_KEYS;
+    if (tid < STAR_TIERS + 2) tn[tid] = 0;
     {
         uint64_t k[PP_ITEMS];
 #pragma unroll
@@ -2911,6 +2918,12 @@ __global__ void __launch_bounds__(LA_THREADS) k_pass_plan(PassPlan p, const uint
         v += dv;
         t += dt;
         h += dh;
+        const int tier = star_tier(dv, p.lds_limit, merge);
+        if (tier >= 0) {
+            atomicAdd(&tn[tier], 1);
+            if (dv > min(STAR_VMAX_T1, p.lds_limit)) atomicAdd(&tn[STAR_TIERS], 1);
+            if (tier == STAR_TIERS - 1) atomicMax(&tn[STAR_TIERS + 1], dv);
+        }
     }
     int tv, tt, th;
     const int ev = la_excl(v, red[0], &tv), et = la_excl(t, red[1], &tt), eh = la_excl(h, red[2], &th);
@@ -2918,6 +2931,11 @@ __global__ void __launch_bounds__(LA_THREADS) k_pass_plan(PassPlan p, const uint
         const int add[4] = {runs, tv, tt, th};
         const int c[4] = {G4D_CNT_ACTIVE, G4D_CNT_NEED_V, G4D_CNT_NEED_T, G4D_CNT_NEED_H};
         base[tid] = atomicAdd(&p.cnt[c[tid]], (unsigned long long)add[tid]);
+    } else if (tid >= 64 && tid < 64 + STAR_TIERS + 2) {
+        const int i = tid - 64, c = tn[i];
+        if (c && i < STAR_TIERS) tn[i] = (int)atomicAdd(&p.cnt[G4D_CNT_TIER0 + i], (unsigned long long)c); // now a cursor
+        else if (c && i == STAR_TIERS) atomicAdd(&p.cnt[G4D_CNT_OVER64], (unsigned long long)c);
+        else if (c) atomicMax(&p.cnt[G4D_CNT_NEED_MAX], (unsigned long long)c);
     }
     __syncthreads();
     int64_t vo = p.base[0] + (int64_t)base[1] + ev, to = p.base[1] + (int64_t)base[2] + et,
@@ -2927,6 +2945,8 @@ __global__ void __launch_bounds__(LA_THREADS) k_pass_plan(PassPlan p, const uint
         int dv, dt, dh;
         plan_sizes(p, s, len, &dv, &dt, &dh);
         plan_star(p, s, t0 + first[r], len, base[0] + r, vo, to, ho);
+        const int tier = star_tier(dv, p.lds_limit, merge);
+        if (tier >= 0) tier_put(p, tier, atomicAdd(&tn[tier], 1), s);
         vo += dv;
         to += dt;
         ho += dh;
@@ -2972,6 +2992,7 @@ __global__ void __launch_bounds__(SR_THREADS) k_small_round(PassPlan p, uint64_t
     __shared__ uint64_t a[STAR_ROUND_SMALL], b[STAR_ROUND_SMALL];
     __shared__ int first[STAR_ROUND_SMALL + 1];
     __shared__ int red[5][SR_THREADS / 64];
+    __shared__ int tn[STAR_TIERS + 2];
     const int tid = threadIdx.x;
     const unsigned long long np = p.cnt[G4D_CNT_NEW_PAIRS];
     if (np == 0 || np > STAR_ROUND_SMALL / 2) return;
@@ -3008,6 +3029,8 @@ __global__ void __launch_bounds__(SR_THREADS) k_small_round(PassPlan p, uint64_t
     if (tid == 0) first[runs] = cnt;
     __syncthreads();
     int64_t vo = p.base[0], to = p.base[1], ho = p.base[2];
+    if (tid < STAR_TIERS + 2) tn[tid] = 0;
+    __syncthreads();
     for (int r0 = 0; r0 < runs; r0 += SR_THREADS) {
         const int r = r0 + tid;
         int s = 0, len = 0, dv = 0, dt = 0, dh = 0;
@@ -3018,7 +3041,15 @@ __global__ void __launch_bounds__(SR_THREADS) k_small_round(PassPlan p, uint64_t
         }
         int tv, tt, th;
         const int ev = sr_excl(dv, red[2], &tv), et = sr_excl(dt, red[3], &tt), eh = sr_excl(dh, red[4], &th);
-        if (r < runs) plan_star(p, s, first[r], len, r, vo + ev, to + et, ho + eh);
+        if (r < runs) {
+            plan_star(p, s, first[r], len, r, vo + ev, to + et, ho + eh);
+            const int tier = star_tier(dv, p.lds_limit, true); // at most STAR_ROUND_SMALL keys
+            if (tier >= 0) {
+                tier_put(p, tier, atomicAdd(&tn[tier], 1), s);
+                if (dv > min(STAR_VMAX_T1, p.lds_limit)) atomicAdd(&tn[STAR_TIERS], 1);
+                if (tier == STAR_TIERS - 1) atomicMax(&tn[STAR_TIERS + 1], dv);
+            }
+        }
         vo += tv;
         to += tt;
         ho += th;
@@ -3031,6 +3062,10 @@ __global__ void __launch_bounds__(SR_THREADS) k_small_round(PassPlan p, uint64_t
         p.cnt[G4D_CNT_NEED_T] = to - p.base[1];
         p.cnt[G4D_CNT_NEED_H] = ho - p.base[2];
     }
+    static_assert(G4D_CNT_OVER64 == G4D_CNT_TIER0 + STAR_TIERS && G4D_CNT_NEED_MAX == G4D_CNT_OVER64 + 1 &&
+                      STAR_ROUND_SMALL <= TIER_MERGE_KEYS,
+                  "one row of counters; small rounds merge the tiers");
+    if (tid < STAR_TIERS + 2) p.cnt[G4D_CNT_TIER0 + tid] = (unsigned long long)tn[tid];
 }
 
 hipError_t launch_small_round(const PassPlan &p, uint64_t *keys, hipStream_t s)
