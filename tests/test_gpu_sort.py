@@ -86,3 +86,19 @@ def test_sort_drowned_keys_matches_numpy():
     assert sh4 >= 0
     assert np.array_equal(got2, ref)
     assert np.array_equal(got4, ref)
+
+
+@pytest.mark.parametrize("big", [8191, 8192, 8193, 16385, 32767, 32768, 32769, 70000])
+def test_sort_one_full_bucket(big):
+    """One id with the given number of keys among evenly spread ones: its bucket ends at, below or above
+    what a work-group of 256 (8,192 keys) or 1,024 threads (32,768) sorts in LDS."""
+    rng = np.random.default_rng(big)
+    nb = 20
+    keys = np.concatenate([_keys(rng.integers(0, 1 << nb, 60_000), rng.integers(0, 1 << nb, 60_000)),
+                           _keys(np.full(big, 777_777), rng.integers(0, 1 << nb, big))])
+    keys = rng.permutation(keys)
+    with g.Triangulator(grid_size=16) as t:
+        for method in (0, 3):
+            got, _, shift = t.diag_sort_pairs(keys, nb, method=method)
+            assert shift >= 0
+            assert np.array_equal(got, np.sort(keys))
