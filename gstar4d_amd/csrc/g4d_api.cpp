@@ -393,6 +393,8 @@ struct SideStreams {
     }
 };
 
+// Passes of at most this many stars may run their two tiers in one launch.
+static constexpr int LATE_STARS = 6144;
 static const uint64_t PLAN_COUNTERS = (1ull << G4D_CNT_ACTIVE) | (1ull << G4D_CNT_NEED_V) | (1ull << G4D_CNT_NEED_T) |
                                       (1ull << G4D_CNT_NEED_H) | (0xffull << G4D_CNT_TIER0);
 
@@ -886,6 +888,63 @@ static int run_device(g4d_ctx *ctx, const double *d_xyz, int n, const SetSpec &s
     int64_t tbase_last = 0;
     int64_t tier_n[g4d::STAR_TIERS] = {}, nover64 = 0, need_max = 0; // as planned
 
+    // The round's work between two passes, from the drowned flags to the next pass's plan when that is
+    // small: mutual removal, proofs, new pairs.  nd drowned insertions, of which ntask may need a proof;
+    // nd < 0: launched right behind the pass, before the host has its counts.  A late round takes 100 to
+    // 200 us of short kernels, and the host's look in between added 20 to 30.
+    bool ahead = false;
+    auto launch_proofs = [&](int64_t ntask) -> int {
+        g4d::ProofParams pp;
+        pp.pts = pts;
+        pp.tasks = buf<uint64_t>(ctx->tasks);
+        pp.ntasks = ntask;
+        pp.vnum = buf<int>(store.vnum);
+        pp.voff = buf<int64_t>(store.voff);
+        pp.vpool = buf<int>(store.arena[0]);
+        pp.tnum = buf<int>(store.tnum);
+        pp.toff = buf<int64_t>(store.toff);
+        pp.tpool = buf<uint64_t>(store.arena[1]);
+        pp.out = buf<uint64_t>(ctx->cand);
+        pp.cnt = cnt;
+        pp.xlist = buf<int64_t>(ctx->xtasks);
+        pp.xcap = ntask;
+        HCK(g4d::launch_proofs(pp, false, s));
+        HCK(g4d::launch_proofs(pp, true, s)); // reads the filter pass's count on the device
+        return G4D_OK;
+    };
+    auto launch_pairs = [&](int nitems, int64_t ntask, bool is_ahead) -> int {
+        g4d::NewPairs np;
+        np.list = active;
+        np.nitems = nitems;
+        np.pcount = spc;
+        np.ntoff = buf<int64_t>(store.ntoff);
+        np.tbase = tbase_last;
+        np.pairbuf = buf<uint64_t>(ctx->pairbuf);
+        np.proofs = buf<uint64_t>(ctx->cand);
+        np.ntasks = ntask;
+        np.hpool = buf<int>(store.arena[2]);
+        np.hoff = buf<int64_t>(store.hoff);
+        np.hnum = buf<int>(store.hnum);
+        np.keys = buf<uint64_t>(ctx->ins);
+        np.cnt = cnt;
+        np.ahead = is_ahead;
+        HCK(g4d::launch_new_pairs(np, s));
+        HCK(g4d::launch_small_round(pass_plan(), buf<uint64_t>(ctx->ins), s));
+        return G4D_OK;
+    };
+    // Whether the buffers, as they are, hold whatever a pass of nins insertions and npb pair places makes.
+    auto round_fits = [&](int64_t nins, int64_t npb) {
+        return ctx->tasks.bytes >= sizeof(uint64_t) * (size_t)nins && ctx->xtasks.bytes >= sizeof(int64_t) * (size_t)nins &&
+               ctx->cand.bytes >= sizeof(uint64_t) * 4 * (size_t)nins &&
+               ctx->ins.bytes >= sizeof(uint64_t) * (size_t)(2 * (npb + 4 * nins) + 2);
+    };
+    auto launch_round = [&](const uint64_t *keys, int64_t nins, int nitems, int64_t nd, int64_t ntask) -> int {
+        HCK(g4d::launch_drown_small(keys, buf<uint8_t>(ctx->dflag), nins, nd, buf<uint64_t>(ctx->tasks), cnt, s));
+        CK(launch_proofs(ntask));
+        CK(launch_pairs(nitems, ntask, true));
+        return G4D_OK;
+    };
+
     // One pass over the nitems stars of the active list (mode 0: every star, from its workset), whose
     // regions of need[] elements are planned at the arenas' tops; the others are not touched.
     // Returns the drowned insertions and the insertion pairs of the pass.
@@ -1014,11 +1073,21 @@ static int run_device(g4d_ctx *ctx, const double *d_xyz, int n, const SetSpec &s
             if (forkg) run(5, 2);
             if (forkw) run(4, 1), run(3, 1);
             if (fork128) run(2, 0), run(1, 0);
+            const bool late = !fork128 && tier_n[0] == 0 && tier_n[1] == 0 && tier_n[2] > 0 && nitems <= LATE_STARS &&
+                              g4d::star_late_variant(sp.t0_variant);
             if (ctx->ev_ok) (void)hipEventRecord(ctx->ev_t0[0], s);
-            if (e == hipSuccess) e = g4d::launch_star_kernel(sp, g4d::STAR_VMAX_T0, false, nblk_star, s);
+            if (late) {
+                g4d::StarParams tp = sp;
+                tp.star_list = tl[2];
+                tp.nlist = (int)tier_n[2];
+                tp.work_counter = G4D_CNT_QUEUE0 + 3;
+                if (e == hipSuccess) e = g4d::launch_star_late(sp, tp, s);
+            } else if (e == hipSuccess) {
+                e = g4d::launch_star_kernel(sp, g4d::STAR_VMAX_T0, false, nblk_star, s);
+            }
             if (ctx->ev_ok) (void)hipEventRecord(ctx->ev_t0[1], s);
             if (e == hipSuccess) e = tier_launch(0, s);
-            if (!fork128) {
+            if (!fork128 && !late) {
                 if (e == hipSuccess) e = tier_launch(1, s);
                 if (e == hipSuccess) e = tier_launch(2, s);
             }
@@ -1026,8 +1095,11 @@ static int run_device(g4d_ctx *ctx, const double *d_xyz, int n, const SetSpec &s
             HCK(e);
             HCK(ej);
         }
+        ahead = mode == 1 && nins <= g4d::DROWN_SMALL && round_fits(nins, npb);
+        if (ahead) CK(launch_round(ins_keys, nins, nitems, -1, nins));
         CK(read_counters(ctx, hc));
         const int64_t nexact = (int64_t)hc[G4D_CNT_APPEND4];
+        if (nexact > 0 || hc[G4D_CNT_XL] > 0) ahead = false; // those launches did nothing
         if (nexact > 0) {
             // The exact-capable kernels of tiers 32, 64 and 256 over the exact list, each passing the
             // stars it cannot hold to the next; they reuse the mid and big lists (the filter kernels
@@ -1108,78 +1180,54 @@ static int run_device(g4d_ctx *ctx, const double *d_xyz, int n, const SetSpec &s
     ev_record(ctx, EV_STAR);
 
     // ---- F: splaying rounds (GD/GDelaunay/GDelHost.cu:1389-1470) ----
-    // Between two passes the host waits once where the round is small (k_small_round planned the next
-    // pass by then), twice where it sorts longer lists, and once more where the proofs' count
-    // sizes large buffers.
+    // The host waits once a pass where rounds are small (its kernels and the plan of the next one are
+    // launched together), twice where k_small_round plans a longer pass's, three times where it sorts
+    // longer lists, and once more where the proofs' count sizes large buffers.
     int rounds = 0;
     bool converged = false;
     for (int it = 0; it < ctx->opt.max_rounds; it++) {
-        // F1-F3: drowned insertions, mutual removal, containment proofs
-        int64_t ntask = 0; // bound
-        if (nd > 0) {
-            CK(guard_keys(ctx, nd, "drowned insertions"));
-            HCK(ctx->tasks.ensure(sizeof(uint64_t) * (size_t)nd));
-            if (nd <= g4d::DROWN_SMALL && pass_n <= g4d::DROWN_SMALL_INS) {
-                HCK(g4d::launch_drown_small(pass_keys, buf<uint8_t>(ctx->dflag), pass_n, nd, buf<uint64_t>(ctx->tasks),
-                                            cnt, s));
-            } else {
-                HCK(ctx->dkeys.ensure(sizeof(uint64_t) * (size_t)nd));
-                uint64_t *dk = buf<uint64_t>(ctx->dkeys);
-                HCK(g4d::launch_drown_keys(pass_keys, buf<uint8_t>(ctx->dflag), pass_n, dk, cnt, s));
-                HCK(g4d::sort_keys_ab(P, dk, nd, 33, nb, 1 + nb, n, false, s));
-                HCK(g4d::launch_nonmutual(dk, nd, buf<uint64_t>(ctx->tasks), cnt, s));
-            }
-            ntask = nd;
-            if (nd > (1 << 16)) { // the proofs' and the insertions' buffers by the count itself
-                CK(read_counters(ctx, hc));
-                ntask = (int64_t)hc[G4D_CNT_TASKS];
-            }
-            if (ntask > 0) {
-                HCK(ctx->xtasks.ensure(sizeof(int64_t) * (size_t)ntask));
-                HCK(ctx->cand.ensure(sizeof(uint64_t) * 4 * (size_t)ntask));
-                g4d::ProofParams pp;
-                pp.pts = pts;
-                pp.tasks = buf<uint64_t>(ctx->tasks);
-                pp.ntasks = ntask;
-                pp.vnum = buf<int>(store.vnum);
-                pp.voff = buf<int64_t>(store.voff);
-                pp.vpool = buf<int>(store.arena[0]);
-                pp.tnum = buf<int>(store.tnum);
-                pp.toff = buf<int64_t>(store.toff);
-                pp.tpool = buf<uint64_t>(store.arena[1]);
-                pp.out = buf<uint64_t>(ctx->cand);
-                pp.cnt = cnt;
-                pp.xlist = buf<int64_t>(ctx->xtasks);
-                pp.xcap = ntask;
-                HCK(g4d::launch_proofs(pp, false, s));
-                HCK(g4d::launch_proofs(pp, true, s)); // reads the filter pass's count on the device
-            }
-        }
-        // F4-F9: candidates = triangle pairs + proofs; those new to the histories, both directions,
-        // sorted without repeats; offsets, stars and regions of the next pass
-        const int64_t ncand = ntp + 4 * ntask;
+        // F1-F3: drowned insertions, mutual removal, containment proofs; F4-F9: candidates = triangle
+        // pairs + proofs; those new to the histories, both directions, sorted without repeats; offsets,
+        // stars and regions of the next pass.  A round launched ahead is done: hc holds its counts.
         int64_t nrec = 0;
-        if (ncand > 0) {
-            CK(guard_keys(ctx, 2 * ncand, "splaying candidates"));
-            HCK(ctx->ins.ensure(sizeof(uint64_t) * (size_t)(2 * ncand + 2)));
-            uint64_t *ins = buf<uint64_t>(ctx->ins);
-            g4d::NewPairs np;
-            np.list = active;
-            np.nitems = pass_items;
-            np.pcount = spc;
-            np.ntoff = buf<int64_t>(store.ntoff);
-            np.tbase = tbase_last;
-            np.pairbuf = buf<uint64_t>(ctx->pairbuf);
-            np.proofs = buf<uint64_t>(ctx->cand);
-            np.ntasks = ntask;
-            np.hpool = buf<int>(store.arena[2]);
-            np.hoff = buf<int64_t>(store.hoff);
-            np.hnum = buf<int>(store.hnum);
-            np.keys = ins;
-            np.cnt = cnt;
-            HCK(g4d::launch_new_pairs(np, s));
-            HCK(g4d::launch_small_round(pass_plan(), ins, s));
+        bool planned = ahead;
+        if (!ahead) {
+            int64_t ntask = 0; // bound
+            if (nd > 0) {
+                CK(guard_keys(ctx, nd, "drowned insertions"));
+                HCK(ctx->tasks.ensure(sizeof(uint64_t) * (size_t)nd));
+                if (nd <= g4d::DROWN_SMALL && pass_n <= g4d::DROWN_SMALL_INS) {
+                    HCK(g4d::launch_drown_small(pass_keys, buf<uint8_t>(ctx->dflag), pass_n, nd,
+                                                buf<uint64_t>(ctx->tasks), cnt, s));
+                } else {
+                    HCK(ctx->dkeys.ensure(sizeof(uint64_t) * (size_t)nd));
+                    uint64_t *dk = buf<uint64_t>(ctx->dkeys);
+                    HCK(g4d::launch_drown_keys(pass_keys, buf<uint8_t>(ctx->dflag), pass_n, dk, cnt, s));
+                    HCK(g4d::sort_keys_ab(P, dk, nd, 33, nb, 1 + nb, n, false, s));
+                    HCK(g4d::launch_nonmutual(dk, nd, buf<uint64_t>(ctx->tasks), cnt, s));
+                }
+                ntask = nd;
+                if (nd > (1 << 16)) { // the proofs' and the insertions' buffers by the count itself
+                    CK(read_counters(ctx, hc));
+                    ntask = (int64_t)hc[G4D_CNT_TASKS];
+                }
+                if (ntask > 0) {
+                    HCK(ctx->xtasks.ensure(sizeof(int64_t) * (size_t)ntask));
+                    HCK(ctx->cand.ensure(sizeof(uint64_t) * 4 * (size_t)ntask));
+                    CK(launch_proofs(ntask));
+                }
+            }
+            const int64_t ncand = ntp + 4 * ntask;
+            if (ncand > 0) {
+                CK(guard_keys(ctx, 2 * ncand, "splaying candidates"));
+                HCK(ctx->ins.ensure(sizeof(uint64_t) * (size_t)(2 * ncand + 2)));
+                CK(launch_pairs(pass_items, ntask, false));
+                planned = true;
+            }
             CK(read_counters(ctx, hc));
+        }
+        if (planned) {
+            uint64_t *ins = buf<uint64_t>(ctx->ins);
             const int64_t mk = 2 * (int64_t)hc[G4D_CNT_NEW_PAIRS];
             if (mk > g4d::STAR_ROUND_SMALL) {
                 int64_t nrec_f = 0, *nrec_h = hslot(ctx, 9, &nrec_f);
@@ -1191,8 +1239,6 @@ static int run_device(g4d_ctx *ctx, const double *d_xyz, int n, const SetSpec &s
             } else {
                 nrec = (int64_t)hc[G4D_CNT_INS];
             }
-        } else {
-            CK(read_counters(ctx, hc));
         }
         trace("round %d: %lld drowned, %lld proofs, %lld pairs, %lld new with repeats, %lld insertions", rounds + 1,
               (long long)nd, (long long)hc[G4D_CNT_TASKS], (long long)ntp, (long long)hc[G4D_CNT_NEW_PAIRS],

@@ -103,6 +103,9 @@ enum {
 // Zeroes the counter words whose bits are set in mask (one launch instead of one fill per word).
 hipError_t launch_zero_counters(unsigned long long *cnt, uint64_t mask, hipStream_t s);
 hipError_t launch_star_kernel(const StarParams &p, int vmax, bool exact, int nblocks, hipStream_t s);
+// The default 32-vertex kernel over p's list and the 256-vertex one over q's, side by side in one launch.
+hipError_t launch_star_late(const StarParams &p, const StarParams &q, hipStream_t s);
+bool star_late_variant(int requested); // whether the 32-vertex variant in use is that one
 // Wide LDS kernel, vmax = STAR_VMAX_W1 or W2, over the nlist stars of star_list, none larger;
 // inconclusive ones go untouched to p.exact_list.
 hipError_t launch_star_wide(const StarParams &p, int vmax, hipStream_t s);
@@ -143,7 +146,9 @@ hipError_t launch_drown_keys(const uint64_t *ins_keys, const uint8_t *dflag, int
 // G4D_CNT_TASKS.
 hipError_t launch_nonmutual(const uint64_t *keys, int64_t m, uint64_t *tasks, unsigned long long *cnt, hipStream_t s);
 // Both at once for at most DROWN_SMALL drowned (nd, as counted by the pass) of at most
-// DROWN_SMALL_INS insertions, which one work-group reads.
+// DROWN_SMALL_INS insertions, which one work-group reads.  nd < 0: launched before the host has looked at
+// the pass, of at most DROWN_SMALL insertions; the count is read on the device, and nothing is done
+// while the pass has exact stars left.
 static constexpr int DROWN_SMALL = 4096;
 static constexpr int64_t DROWN_SMALL_INS = 1 << 16;
 hipError_t launch_drown_small(const uint64_t *ins_keys, const uint8_t *dflag, int64_t m, int64_t nd, uint64_t *tasks,
@@ -165,6 +170,7 @@ struct NewPairs {
     const int *hnum;
     uint64_t *keys;
     unsigned long long *cnt;
+    bool ahead; // launched before the host has looked at the pass: nothing while exact stars are left
 };
 hipError_t launch_new_pairs(const NewPairs &p, hipStream_t s);
 static constexpr int STAR_TIERS = 6;

@@ -245,7 +245,7 @@ __device__ __forceinline__ void star_commit(const StarParams &p, int s, int vcou
 // lift's), which only that lane reads: without them in LDS a 256-vertex star takes 25 KB instead
 // of 57 and six waves share a CU instead of two.
 template <int VMAX, bool EXACT>
-__device__ __forceinline__ void star_body(const StarParams &p, int nitems)
+__device__ __forceinline__ void star_body(const StarParams &p, int nitems, int bid, int nblk)
 {
     constexpr bool REGC = !EXACT;
     using Lds = StarLds<VMAX, !REGC>;
@@ -266,15 +266,15 @@ __device__ __forceinline__ void star_body(const StarParams &p, int nitems)
     // atomic per STAR_CHUNK stars for the filter-only kernels (many small stars), per star for
     // the exact ones (uneven cost).
     constexpr int CHUNK = EXACT ? 1 : STAR_CHUNK;
-    const bool one_each = nitems <= (int)gridDim.x;
-    if ((int)blockIdx.x >= nitems) return;
+    const bool one_each = nitems <= nblk;
+    if (bid >= nitems) return;
     bool first = true;
     int nfilt = 0, ncof = 0; // this lane's cofactor-filter evaluations and cofactor computations
     unsigned long long npairs = 0, ndrown = 0; // the wave's
     for (;;) {
         int base = 0;
         if (one_each) {
-            base = first ? (int)blockIdx.x : nitems;
+            base = first ? bid : nitems;
             first = false;
         } else {
             if (lane == 0) base = (int)atomicAdd(&cnt[p.work_counter], (unsigned long long)CHUNK);
@@ -685,7 +685,7 @@ __device__ __forceinline__ void star_body(const StarParams &p, int nitems)
 // footprint instead.
 __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(5, 8))) k_star32(StarParams p, int nitems)
 {
-    star_body<STAR_VMAX_T0, false>(p, nitems);
+    star_body<STAR_VMAX_T0, false>(p, nitems, blockIdx.x, gridDim.x);
 }
 
 // The filter-only tiers above: the registers that each occupancy leaves, measured on 1,000,000
@@ -695,13 +695,13 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(5, 8)))
 template <int VMAX>
 __global__ void __launch_bounds__(64) k_star_exact(StarParams p, int nitems)
 {
-    star_body<VMAX, true>(p, nitems);
+    star_body<VMAX, true>(p, nitems, blockIdx.x, gridDim.x);
 }
 
 template <int VMAX, int WPE>
 __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WPE, 8))) k_star(StarParams p, int nitems)
 {
-    star_body<VMAX, false>(p, nitems);
+    star_body<VMAX, false>(p, nitems, blockIdx.x, gridDim.x);
 }
 
 // ------------------------------------------------------------------------------------
@@ -893,7 +893,7 @@ __device__ __forceinline__ int wave_max_i(int v)
 }
 
 template <int GL, bool PF>
-__device__ __forceinline__ void star_body_grp(const StarParams &p, int nitems)
+__device__ __forceinline__ void star_body_grp(const StarParams &p, int nitems, int bid, int nblk)
 {
     constexpr int NG = 64 / GL;
     constexpr int VMAX = StarGrpLds::VMAX, TMAX = StarGrpLds::TMAX;
@@ -912,15 +912,15 @@ __device__ __forceinline__ void star_body_grp(const StarParams &p, int nitems)
     // Work unit: a batch of NG consecutive list entries, one per group.  As many batches as
     // work-groups or fewer: one batch each, no queue; otherwise STAR_CHUNK batches per atomic.
     const int nbatch = (nitems + NG - 1) / NG;
-    const bool one_each = nbatch <= (int)gridDim.x;
-    if ((int)blockIdx.x >= nbatch) return;
+    const bool one_each = nbatch <= nblk;
+    if (bid >= nbatch) return;
     bool first = true;
     int nfilt = 0, ncof = 0;
     unsigned long long npairs = 0, ndrown = 0; // the wave's
     for (;;) {
         int base = 0;
         if (one_each) {
-            base = first ? (int)blockIdx.x : nbatch;
+            base = first ? bid : nbatch;
             first = false;
         } else {
             if (lane == 0) base = (int)atomicAdd(&cnt[p.work_counter], (unsigned long long)STAR_CHUNK);
@@ -1368,22 +1368,34 @@ __device__ __forceinline__ void star_body_grp(const StarParams &p, int nitems)
 
 __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3, 8))) k_star32g16(StarParams p, int nitems)
 {
-    star_body_grp<16, false>(p, nitems);
+    star_body_grp<16, false>(p, nitems, blockIdx.x, gridDim.x);
 }
 
 __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3, 8))) k_star32g16f(StarParams p, int nitems)
 {
-    star_body_grp<16, true>(p, nitems);
+    star_body_grp<16, true>(p, nitems, blockIdx.x, gridDim.x);
 }
 
 __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4, 8))) k_star32g16f4(StarParams p, int nitems)
 {
-    star_body_grp<16, true>(p, nitems);
+    star_body_grp<16, true>(p, nitems, blockIdx.x, gridDim.x);
 }
 
 __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4, 8))) k_star32g32f(StarParams p, int nitems)
 {
-    star_body_grp<32, true>(p, nitems);
+    star_body_grp<32, true>(p, nitems, blockIdx.x, gridDim.x);
+}
+
+// A late pass's two tiers (32 and, merged, 64 to 256 vertices) in one launch: work-groups below nb take
+// batches of p's list, the others stars of q's.  Both finish when their longest star does (some
+// 35 us each), which this pays once.  The registers and LDS of the larger tier cost the smaller one
+// nothing in a pass that does not fill the chip.  1,000 uniform points, five late rounds, with the
+// round's other kernels launched behind it at once: 1.40 -> 1.24 ms a call.
+__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 8))) k_star_late(StarParams p, int nb,
+                                                                                            StarParams q)
+{
+    if ((int)blockIdx.x < nb) star_body_grp<16, true>(p, p.nlist, blockIdx.x, nb);
+    else star_body<STAR_VMAX_T2, false>(q, q.nlist, blockIdx.x - nb, gridDim.x - nb);
 }
 
 // The 32-vertex filter-only kernel variant of a launch: the caller's choice, else the
@@ -1417,6 +1429,18 @@ hipError_t launch_zero_counters(unsigned long long *cnt, uint64_t mask, hipStrea
     hipLaunchKernelGGL(k_zero_counters, dim3(1), dim3(64), 0, s, cnt, mask);
     return hipGetLastError();
 }
+
+hipError_t launch_star_late(const StarParams &p, const StarParams &q, hipStream_t s)
+{
+    if (!p.star_list || p.nlist <= 0 || !q.star_list || q.nlist <= 0 || p.nlist_dev || q.nlist_dev ||
+        p.lds_limit > STAR_LDS_LIMIT)
+        return hipErrorInvalidValue;
+    const int nb = std::min(4096, (p.nlist + 3) / 4);
+    hipLaunchKernelGGL(k_star_late, dim3(nb + std::min(1536, q.nlist)), dim3(64), 0, s, p, nb, q);
+    return hipGetLastError();
+}
+
+bool star_late_variant(int requested) { return star_t0_variant(requested) == STAR_T0_G16F4; }
 
 hipError_t launch_star_kernel(const StarParams &p, int vmax, bool exact, int nblocks, hipStream_t s)
 {
@@ -2448,6 +2472,13 @@ __device__ __forceinline__ int la_excl(int v, int *red, int *tot)
     return base + inc - v;
 }
 
+// Whether a pass has stars left for the exact or the global-memory kernel, which the host launches when
+// it sees their counts: its lists are not complete yet.
+__device__ __forceinline__ bool pass_open(const unsigned long long *cnt)
+{
+    return cnt[G4D_CNT_APPEND4] != 0 || cnt[G4D_CNT_XL] != 0;
+}
+
 // Key of drowned insertion k = star << 32 | vertex: the pair in order, then who inserted whom.
 __device__ __forceinline__ uint64_t drown_key(uint64_t k)
 {
@@ -2566,6 +2597,11 @@ __global__ void __launch_bounds__(1024) k_drown_small(const uint64_t *ins_keys, 
     __shared__ uint64_t a[DROWN_SMALL];
     __shared__ int have, ntask;
     const int tid = threadIdx.x, lane = __lane_id();
+    if (nd < 0) { // launched ahead of the host's look at the pass
+        if (pass_open(cnt)) return;
+        nd = (int)min(cnt[G4D_CNT_DROWNED], (unsigned long long)DROWN_SMALL);
+        if (nd == 0) return;
+    }
     int n = 128;
     while (n < nd) n <<= 1;
     for (int i = tid; i < n; i += 1024) a[i] = ~0ull;
@@ -2611,8 +2647,8 @@ __global__ void __launch_bounds__(1024) k_drown_small(const uint64_t *ins_keys, 
 hipError_t launch_drown_small(const uint64_t *ins_keys, const uint8_t *dflag, int64_t m, int64_t nd, uint64_t *tasks,
                               unsigned long long *cnt, hipStream_t s)
 {
-    if (nd <= 0 || m <= 0) return hipSuccess;
-    if (nd > DROWN_SMALL || m > DROWN_SMALL_INS) return hipErrorInvalidValue;
+    if (nd == 0 || m <= 0) return hipSuccess;
+    if (nd > DROWN_SMALL || m > (nd < 0 ? DROWN_SMALL : DROWN_SMALL_INS)) return hipErrorInvalidValue;
     hipLaunchKernelGGL(k_drown_small, dim3(1), dim3(1024), 0, s, ins_keys, dflag, (int)m, (int)nd, tasks, cnt);
     return hipGetLastError();
 }
@@ -2637,6 +2673,7 @@ __global__ void __launch_bounds__(LA_THREADS) k_new_pairs(NewPairs p)
     const int tid = threadIdx.x, sub = tid & 15, lane = tid & 63, wv = tid >> 6;
     uint64_t *queue = queue_[wv], *stage = stage_[wv];
     int nq = 0, ns = 0; // this wave's
+    if (p.ahead && pass_open(p.cnt)) return;
     for (int i = tid; i < NP_SEEN; i += LA_THREADS) seen[i] = STAR_PAIR_NONE;
     if (tid == 0) nwide = 0;
     __syncthreads();
