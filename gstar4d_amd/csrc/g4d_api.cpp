@@ -792,7 +792,7 @@ static int run_device(g4d_ctx *ctx, const double *d_xyz, int n, const SetSpec &s
     HCK(g4d::launch_grid_pairs_dedup(idg, GS, ntiles, pcnt, raw, tcnt, ttot, s));
     HCK(g4d::scan_excl_i64(P, ttot, ttot, ntiles, ttot + ntiles, s));
     HCK(g4d::launch_gather_tiles(raw, pcnt, tcnt, ntiles, ttot, pr, s));
-    HCK(g4d::launch_missing(vox, n, GS, idg, ttot + ntiles, pr, cnt + G4D_CNT_MISSING, s));
+    HCK(g4d::launch_missing(vox, n, GS, ttot + ntiles, pr, cnt + G4D_CNT_MISSING, s));
     int64_t ngd_f = 0, *ngd_h = hslot(ctx, 1, &ngd_f);
     HCK(hipMemcpyAsync(ngd_h, ttot + ntiles, 8, hipMemcpyDeviceToHost, s));
     CK(read_counters(ctx, hc));
@@ -823,6 +823,7 @@ static int run_device(g4d_ctx *ctx, const double *d_xyz, int n, const SetSpec &s
     HCK(g4d::launch_pump(pr, ws_off, n, GS, min_ws, pr + m, cnt + G4D_CNT_PUMPED, 2 * (int64_t)n * min_ws + 64, s));
     CK(read_counters(ctx, hc));
     const int64_t npump = (int64_t)hc[G4D_CNT_PUMPED];
+    const uint64_t *worksets = pr;
     if (npump > 0) {
         // A pumped candidate is not in the star's list, and the lists are symmetric, so no
         // pumped key is already present: sort and deduplicate the pumped keys alone (two stars
@@ -834,7 +835,7 @@ static int run_device(g4d_ctx *ctx, const double *d_xyz, int n, const SetSpec &s
         HCK(P.sort_tmp_keys.ensure(sizeof(uint64_t) * (size_t)(m + np)));
         uint64_t *merged = P.sort_tmp_keys.as<uint64_t>();
         HCK(g4d::merge_u64(pr, m, pk, np, merged, s));
-        HCK(hipMemcpyAsync(pr, merged, sizeof(uint64_t) * (size_t)(m + np), hipMemcpyDeviceToDevice, s));
+        worksets = merged; // in the sort's buffer: the first sort after it, of the drowned keys, is behind their last use
         ctx->st.num_pumped = np;
         m += np;
     }
@@ -1161,7 +1162,7 @@ static int run_device(g4d_ctx *ctx, const double *d_xyz, int n, const SetSpec &s
     };
 
     int64_t nd = 0, ntp = 0, need[3];
-    const uint64_t *pass_keys = pr; // the last pass's insertions, and the number of its stars
+    const uint64_t *pass_keys = worksets; // the last pass's insertions, and the number of its stars
     int64_t pass_n = m;
     int pass_items = n;
     auto read_needs = [&]() {
@@ -1172,11 +1173,11 @@ static int run_device(g4d_ctx *ctx, const double *d_xyz, int n, const SetSpec &s
         nover64 = (int64_t)hc[G4D_CNT_OVER64];
         need_max = (int64_t)hc[G4D_CNT_NEED_MAX];
     };
-    HCK(g4d::launch_pass_plan(pass_plan(), pr, m, nullptr, s));
+    HCK(g4d::launch_pass_plan(pass_plan(), worksets, m, nullptr, s));
     CK(read_counters(ctx, hc));
     if ((int64_t)hc[G4D_CNT_ACTIVE] != n) return set_err(ctx, G4D_ERR_INTERNAL, "a star has no candidates");
     read_needs();
-    CK(star_pass(0, pr, buf<int64_t>(ctx->ins_off), m, n, need, &nd, &ntp));
+    CK(star_pass(0, worksets, buf<int64_t>(ctx->ins_off), m, n, need, &nd, &ntp));
     ev_record(ctx, EV_STAR);
 
     // ---- F: splaying rounds (GD/GDelaunay/GDelHost.cu:1389-1470) ----

@@ -67,8 +67,8 @@ hipError_t pba_pass_banded(int axis, const GridSets &S, int64_t nblocks, int ban
                            hipStream_t s);
 // Both directed keys of each non-leader point with its voxel's leader, behind the *first pairs (of
 // two keys) in out; the counter counts pairs.
-hipError_t launch_missing(const uint64_t *vox, int n, const GridSets &S, const int *grid, const int64_t *first,
-                          uint64_t *out, unsigned long long *counter, hipStream_t s);
+hipError_t launch_missing(const uint64_t *vox, int n, const GridSets &S, const int64_t *first, uint64_t *out,
+                          unsigned long long *counter, hipStream_t s);
 // Voronoi-neighbour pairs (min<<32 | max) by tiles of 256 threads, 16 x 16 columns by
 // grid_pair_chunk cubes (for the sets' grids g together); pair_thr[nsets] / 256 tiles in all.
 int grid_pair_chunk(const int *g, int nsets);

@@ -821,7 +821,7 @@ hipError_t sort_unique_pair_keys(Prims &P, uint64_t *keys, int64_t m, int nb, in
 
 // ------------------------------------------------------------------------------------
 // Merge of two sorted lists, for a long list `a` and a short one `b`.  Work-group w writes
-// outputs [w*MG_TILE, (w+1)*MG_TILE): its first thread finds where the two tile boundaries cross
+// outputs [w*MG_TILE, (w+1)*MG_TILE): two waves find where the tile's boundaries cross
 // the inputs (merge path, ties take `a` first), the tile's part of `b` is staged in LDS, and
 // every element goes straight to its output: an `a` element after the staged `b` elements
 // smaller than it, a `b` element after the tile's `a` elements not greater than it.
@@ -829,13 +829,21 @@ hipError_t sort_unique_pair_keys(Prims &P, uint64_t *keys, int64_t m, int nb, in
 
 static constexpr int MG_TILE = 4096;
 
+// Of the first d outputs, how many come from a.  A whole wave searches, 64 probes a step: one thread's
+// 20 to 26 dependent reads, twice, held up the tile for longer than its copies take (66 million keys with
+// 1 million: 0.55 ms; 0.34 so, with eight reads in flight a thread).
 __device__ __forceinline__ int64_t merge_split(const uint64_t *a, int64_t na, const uint64_t *b, int64_t nb, int64_t d)
 {
+    const int lane = threadIdx.x & 63;
     int64_t lo = d > nb ? d - nb : 0, hi = d < na ? d : na;
     while (lo < hi) {
-        const int64_t mid = (lo + hi) >> 1;
-        if (a[mid] <= b[d - mid - 1]) lo = mid + 1;
-        else hi = mid;
+        const int64_t span = hi - lo;
+        auto probe = [&](int l) { return lo + span * (l + 1) / 65; }; // below hi
+        const int64_t i = probe(lane);
+        const int c = __popcll(__ballot(a[i] <= b[d - i - 1])); // true up to the answer
+        const int64_t nlo = c > 0 ? probe(c - 1) + 1 : lo, nhi = c < 64 ? probe(c) : hi;
+        lo = nlo;
+        hi = nhi;
     }
     return lo;
 }
@@ -848,27 +856,33 @@ __global__ void __launch_bounds__(256) k_merge_u64(const uint64_t *a, int64_t na
     const int64_t total = na + nb;
     const int64_t o0 = (int64_t)blockIdx.x * MG_TILE;
     const int64_t o1 = o0 + MG_TILE < total ? o0 + MG_TILE : total;
-    if (threadIdx.x == 0) {
-        const int64_t i0 = merge_split(a, na, b, nb, o0), i1 = merge_split(a, na, b, nb, o1);
-        sp[0] = i0;
-        sp[1] = o0 - i0;
-        sp[2] = i1;
-        sp[3] = o1 - i1;
+    if (threadIdx.x < 128) { // a wave for each end of the tile
+        const int e = threadIdx.x >> 6;
+        const int64_t o = e ? o1 : o0, i = merge_split(a, na, b, nb, o);
+        sp[2 * e] = i;
+        sp[2 * e + 1] = o - i;
     }
     __syncthreads();
     const int64_t i0 = sp[0], j0 = sp[1], i1 = sp[2], j1 = sp[3];
     const int nbw = (int)(j1 - j0);
     for (int k = threadIdx.x; k < nbw; k += blockDim.x) bw[k] = b[j0 + k];
     __syncthreads();
-    for (int64_t i = i0 + threadIdx.x; i < i1; i += blockDim.x) {
-        const uint64_t v = a[i];
-        int lo = 0, hi = nbw; // staged b elements < v
-        while (lo < hi) {
-            const int mid = (lo + hi) >> 1;
-            if (bw[mid] < v) lo = mid + 1;
-            else hi = mid;
-        }
-        out[o0 + (i - i0) + lo] = v;
+    constexpr int R = 8; // reads in flight a thread
+    for (int64_t i = i0 + threadIdx.x; i < i1; i += R * 256) {
+        uint64_t v[R];
+#pragma unroll
+        for (int r = 0; r < R; r++) v[r] = a[min(i + r * 256, i1 - 1)];
+        int lo[R];
+#pragma unroll
+        for (int r = 0; r < R; r++) lo[r] = 0;
+        // staged b elements < v: the same halving for all, on a length that is padded by the bound
+        for (int w = nbw > 0 ? 1 << (31 - __builtin_clz(nbw)) : 0; w > 0; w >>= 1)
+#pragma unroll
+            for (int r = 0; r < R; r++)
+                if (lo[r] + w <= nbw && bw[lo[r] + w - 1] < v[r]) lo[r] += w;
+#pragma unroll
+        for (int r = 0; r < R; r++)
+            if (i + r * 256 < i1) out[o0 + (i + r * 256 - i0) + lo[r]] = v[r];
     }
     for (int k = threadIdx.x; k < nbw; k += blockDim.x) {
         const uint64_t v = bw[k];
