@@ -67,8 +67,8 @@ struct StarParams {
     uint64_t *pairbuf;    // per star, from 2 * (ntoff[s] - tbase): its insertion pairs (a<<32 | b,
     int64_t tbase;        // a < b) of unchecked triangles, dense, in triangle order
     int *pcount;          // per star: the number of those pairs
-    int *defer_list;      // stars that exceed this kernel's capacity, counter `defer_counter`; null in the
-                          // 32-vertex kernels: such stars are on a list of the plan and skipped
+    int *defer_list;      // stars that exceed this kernel's capacity, counter `defer_counter` (exact kernels;
+                          // the others have the plan's lists, and null)
     int64_t defer_cap;
     int defer_counter;
     int *exact_list;      // stars whose filters were inconclusive (filter-only kernels),
@@ -76,7 +76,7 @@ struct StarParams {
     int exact_counter;
     int work_counter; // counter word of this launch's work queue (zero at launch)
     int lds_limit;        // largest vn + m handled in LDS (<= STAR_LDS_LIMIT)
-    // work list (nullptr = all stars); with nlist_dev the list length is read on the device
+    // work list (nullptr = all stars; an entry below 0 is skipped); with nlist_dev the list length is read on the device
     // (the counter a previous kernel appended with), nlist being its capacity
     const int *star_list;
     int nlist;
@@ -154,7 +154,7 @@ static constexpr int64_t DROWN_SMALL_INS = 1 << 16;
 hipError_t launch_drown_small(const uint64_t *ins_keys, const uint8_t *dflag, int64_t m, int64_t nd, uint64_t *tasks,
                               unsigned long long *cnt, hipStream_t s);
 // Both directed keys of every pair (a<<32 | b, a < b) with b not in the history of star a, of the
-// last pass's stars (list = nullptr: stars 0..nitems-1) and of the proofs (four per task, tasks
+// last pass's stars (the plan's list) and of the proofs (four per task, tasks
 // counted at G4D_CNT_TASKS, at most ntasks); counter G4D_CNT_NEW_PAIRS (pairs).
 struct NewPairs {
     const int *list;

@@ -285,6 +285,7 @@ __device__ __forceinline__ void star_body(const StarParams &p, int nitems, int b
 #pragma unroll 1
         for (int item = base; item < bend; item++) {
             const int s = p.star_list ? p.star_list[item] : item;
+            if (s < 0) continue; // on another tier's list
             const int64_t ib = p.ins_off[s];
             const int m = (int)(p.ins_off[s + 1] - ib);
             const int vn = p.mode ? p.vnum[s] : 0;
@@ -292,7 +293,7 @@ __device__ __forceinline__ void star_body(const StarParams &p, int nitems, int b
             const int lim = VMAX < p.lds_limit ? VMAX : p.lds_limit;
             if (need > lim) {
                 if (p.defer_list) star_list_push(p.defer_list, p.defer_cap, &cnt[p.defer_counter], s, cnt);
-                else if (VMAX > STAR_VMAX_T0 && lane == 0) // not the list of this tier
+                else if (lane == 0) // not the list of this tier
                     atomicOr(&cnt[G4D_CNT_ERROR], (unsigned long long)G4D_DEV_ERR_BUFFER);
                 continue;
             }
@@ -937,7 +938,7 @@ __device__ __forceinline__ void star_body_grp(const StarParams &p, int nitems, i
             int key = INT_MAX;
             if (lane < nit && my < nitems) {
                 const int s = p.star_list ? p.star_list[my] : my;
-                key = (int)(p.ins_off[s + 1] - p.ins_off[s]);
+                key = s < 0 ? 0 : (int)(p.ins_off[s + 1] - p.ins_off[s]);
             }
             int rank = 0;
 #pragma unroll
@@ -955,14 +956,18 @@ __device__ __forceinline__ void star_body_grp(const StarParams &p, int nitems, i
             asm volatile("" : "+v"(gl));
             const int item = order[(batch - base) * NG + g];
             // ---- this group's star: checks, then its link and insertions into LDS ----
-            bool act = item < nitems;
-            const int s = act ? (p.star_list ? p.star_list[item] : item) : 0;
+            const int entry = item < nitems ? (p.star_list ? p.star_list[item] : item) : -1;
+            bool act = entry >= 0; // below: on another tier's list
+            const int s = act ? entry : 0;
             const int64_t ib = act ? p.ins_off[s] : 0;
             const int m = act ? (int)(p.ins_off[s + 1] - ib) : 0;
             const int vn = act && p.mode ? p.vnum[s] : 0;
             const int need = vn + m;
             const int lim = VMAX < p.lds_limit ? VMAX : p.lds_limit;
-            if (act && need > lim) act = false; // on a list of the plan
+            if (act && need > lim) { // not the list of this tier
+                if (gl == 0) atomicOr(&cnt[G4D_CNT_ERROR], (unsigned long long)G4D_DEV_ERR_BUFFER);
+                act = false;
+            }
             if (act && p.mode == 0 && m < 4) {
                 if (gl == 0) {
                     atomicOr(&cnt[G4D_CNT_ERROR], (unsigned long long)G4D_DEV_ERR_CONE);
@@ -2764,7 +2769,11 @@ __global__ void __launch_bounds__(LA_THREADS) k_new_pairs(NewPairs p)
         const int nrow = (int)min((int64_t)row, p.nitems - r0);
         // the reads of a step (list entry, then count and region, then the first pairs) are made one, two
         // and three steps ahead: each waits for the one before
-        auto entry = [&](int i) { return i < nrow ? (p.list ? p.list[r0 + i] : (int)(r0 + i)) : -1; };
+        auto star = [&](int64_t i) { // ~s: on a tier's list
+            const int s = p.list[i];
+            return s < 0 ? ~s : s;
+        };
+        auto entry = [&](int i) { return i < nrow ? star(r0 + i) : -1; };
         struct Region {
             int c;
             int64_t off;
@@ -2805,8 +2814,7 @@ __global__ void __launch_bounds__(LA_THREADS) k_new_pairs(NewPairs p)
         if (nw == 0) continue;
         if (tid == 0) nwide = 0;
         for (int w = 0; w < nw; w++) {
-            const int64_t i = r0 + wide[w];
-            const int s = p.list ? p.list[i] : (int)i, c = p.pcount[s];
+            const int s = star(r0 + wide[w]), c = p.pcount[s];
             const uint64_t *src = p.pairbuf + 2 * (p.ntoff[s] - p.tbase);
             for (int k0 = 64 * wv; k0 < c; k0 += LA_THREADS) put(k0 + lane < c, k0 + lane < c ? src[k0 + lane] : 0ull);
         }
@@ -2835,6 +2843,7 @@ hipError_t launch_new_pairs(const NewPairs &p, hipStream_t s)
 {
     const int64_t work = std::max<int64_t>(16 * (int64_t)p.nitems, 4 * p.ntasks);
     if (work <= 0) return hipSuccess;
+    if (!p.list && p.nitems > 0) return hipErrorInvalidValue;
     hipLaunchKernelGGL(k_new_pairs, dim3(g4d_blocks(work, LA_THREADS, 2048)), dim3(LA_THREADS), 0, s, p);
     return hipGetLastError();
 }
@@ -2847,12 +2856,14 @@ __device__ __forceinline__ void plan_sizes(const PassPlan &p, int s, int m, int 
     *h = p.hnum[s] + m;
 }
 
+// A star on a tier's list is marked on the pass's list (~s): the 32-vertex kernel must not look at its
+// record, which the other tier's kernel may have rebuilt already, to see that it is not its own.
 __device__ __forceinline__ void plan_star(const PassPlan &p, int s, int64_t first, int m, unsigned long long item,
-                                          int64_t v, int64_t t, int64_t h)
+                                          int64_t v, int64_t t, int64_t h, bool tiered)
 {
     p.ins_off[s] = first;
     p.ins_off[s + 1] = first + m; // the following star's first, when that has insertions too
-    p.list[item] = s;
+    p.list[item] = tiered ? ~s : s;
     p.nvoff[s] = v;
     p.ntoff[s] = t;
     p.nhoff[s] = h;
@@ -2981,8 +2992,8 @@ __global__ void __launch_bounds__(LA_THREADS) k_pass_plan(PassPlan p, const uint
         const int s = (int)sid[first[r]], len = r + 1 < runs ? first[r + 1] - first[r] : last_len;
         int dv, dt, dh;
         plan_sizes(p, s, len, &dv, &dt, &dh);
-        plan_star(p, s, t0 + first[r], len, base[0] + r, vo, to, ho);
         const int tier = star_tier(dv, p.lds_limit, merge);
+        plan_star(p, s, t0 + first[r], len, base[0] + r, vo, to, ho, tier >= 0);
         if (tier >= 0) tier_put(p, tier, atomicAdd(&tn[tier], 1), s);
         vo += dv;
         to += dt;
@@ -3079,8 +3090,8 @@ __global__ void __launch_bounds__(SR_THREADS) k_small_round(PassPlan p, uint64_t
         int tv, tt, th;
         const int ev = sr_excl(dv, red[2], &tv), et = sr_excl(dt, red[3], &tt), eh = sr_excl(dh, red[4], &th);
         if (r < runs) {
-            plan_star(p, s, first[r], len, r, vo + ev, to + et, ho + eh);
             const int tier = star_tier(dv, p.lds_limit, true); // at most STAR_ROUND_SMALL keys
+            plan_star(p, s, first[r], len, r, vo + ev, to + et, ho + eh, tier >= 0);
             if (tier >= 0) {
                 tier_put(p, tier, atomicAdd(&tn[tier], 1), s);
                 if (dv > min(STAR_VMAX_T1, p.lds_limit)) atomicAdd(&tn[STAR_TIERS], 1);

@@ -320,6 +320,24 @@ def test_store_repacks_keep_the_stars(orc, hub):
             assert (g.canonical(tets) == r).all()
 
 
+@pytest.mark.parametrize("kind", ["clumps", "uniform"])
+def test_tiers_side_by_side_leave_each_other_alone(kind):
+    """The kernels of a pass's tiers run beside each other, and a star of a larger tier that is rebuilt
+    before the 32-vertex kernel comes to its entry may by then have a link of less than 32: it must
+    not be built again.  Every run of a context gives the same bits."""
+    rng = np.random.default_rng(17)
+    if kind == "clumps":
+        x = np.concatenate([c + 1e-3 * rng.normal(size=(1200, 3)) for c in rng.random((20, 3))] + [rng.random((60000, 3))])
+    else:
+        x = rng.random((400000, 3))
+    with g.Triangulator(grid_size=64) as t:
+        first = t.triangulate(x)[:2]
+        for k in range(12):
+            again = t.triangulate(x)[:2]
+            assert np.array_equal(first[0], again[0]) and np.array_equal(first[1], again[1]), k
+        assert t.check()["adjacency_failures"] == 0
+
+
 @pytest.mark.parametrize("bands", [1, 3, 5])
 def test_pba_bands_same_triangulation(orc, bands):
     x = datasets.uniform_cube(20000, seed=31)
