@@ -338,6 +338,21 @@ def test_tiers_side_by_side_leave_each_other_alone(kind):
         assert t.check()["adjacency_failures"] == 0
 
 
+@pytest.mark.parametrize("n", [15, 17, 64, (1 << 17) - 1, 1 << 17, (1 << 17) + 13])
+def test_output_owner_triangles_by_wave_sizes(n):
+    """The output's decision pass takes 4 stars a wave, 16 from 2^17 stars on, and decides their own
+    triangles 64 at a time: whole and partial groups give a valid Delaunay mesh."""
+    rng = np.random.default_rng(n)
+    x = rng.random((n - n // 8, 3))
+    if n >= 64:  # and stars of more than 32 link vertices: a clump around each of some points
+        x = np.concatenate([x, x[:1] + 1e-4 * rng.normal(size=(n // 8, 3))])
+    with g.Triangulator(grid_size=96 if n > 1000 else 16) as t:
+        tets, _, _ = t.triangulate(x)
+        rep = t.check(full_empty_sphere=n < 1000)
+        assert rep["euler"] == 1 and rep["orientation_failures"] == 0 and rep["adjacency_failures"] == 0
+        assert rep["insphere_failures"] == 0 and rep["empty_sphere_failures"] == 0
+
+
 @pytest.mark.parametrize("bands", [1, 3, 5])
 def test_pba_bands_same_triangulation(orc, bands):
     x = datasets.uniform_cube(20000, seed=31)
