@@ -36,8 +36,8 @@ METRIC = "points/s to exact 3D DT on 1 MI355X: plain vs learned-proposal+batched
 HBM_PEAK_GBS = 8000.0
 FP64_PEAK_TFLOPS = 78.6
 FLOPS_PER_ORIENT4 = 111     # filtered orient4 (insphere filter, GD/GDelaunay/GDelShewchukDevice.h:1074-1136)
-FLOPS_FILTER_EXECUTED = 15  # cached-cofactor filter: 4-term dot product and error bound
-FLOPS_COFACTORS = 64        # cofactors and permanents of one link triangle
+FLOPS_FILTER_EXECUTED = 9   # cached-cofactor filter: 4-term dot product and error bound
+FLOPS_COFACTORS = 49        # cofactors of one link triangle and the bound on its permanents
 
 
 def log(msg):
