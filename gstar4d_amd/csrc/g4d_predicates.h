@@ -843,11 +843,12 @@ __device__ __forceinline__ int frexp_top(double x, int top)
     return x == 0.0 ? top : max(top, e);
 }
 
-// x 2^sh into *X; whether that is a whole number.
+// x 2^sh into *X; whether that is a whole number.  A scale that takes x below the smallest denormal
+// leaves zero, which is not x's value: such coordinates span far more than the 61 bits.
 __device__ __forceinline__ bool scaled_whole(double x, int sh, double *X)
 {
     *X = __builtin_ldexp(x, sh);
-    return __builtin_rint(*X) == *X;
+    return __builtin_rint(*X) == *X && (*X != 0.0 || x == 0.0);
 }
 
 // fl(a - b) into *w; whether nothing was rounded.
