@@ -2266,6 +2266,62 @@ int g4d_diag_sort_pairs(g4d_ctx *ctx, const uint64_t *keys, int64_t m, int32_t n
     return G4D_OK;
 }
 
+int g4d_diag_pass_plan(g4d_ctx *ctx, int32_t n, const int32_t *vnum, const int32_t *hnum, const uint64_t *keys,
+                       int64_t m, int32_t small, const int64_t *base, int64_t *off, int64_t *plan)
+{
+    if (!ctx || n <= 0 || !vnum || !hnum || !keys || m <= 0 || !base || !off || !plan) return G4D_ERR_INVALID_INPUT;
+    if (m > G4D_MAX_SORT_KEYS || (small && (m % 2 || m > g4d::STAR_ROUND_SMALL)))
+        return set_err(ctx, G4D_ERR_INVALID_INPUT, "%lld keys", (long long)m);
+    for (int64_t i = 0; i < m; i++)
+        if ((keys[i] >> 32) >= (uint64_t)n || (i && keys[i] <= keys[i - 1]))
+            return set_err(ctx, G4D_ERR_INVALID_INPUT, "keys must be distinct, in order and of stars below n");
+    for (int32_t i = 0; i < n; i++)
+        if (vnum[i] < 0 || hnum[i] < 0 || vnum[i] > (1 << 29) || hnum[i] > (1 << 29))
+            return set_err(ctx, G4D_ERR_INVALID_INPUT, "star %d out of range", i);
+    HCK(hipSetDevice(ctx->opt.device));
+    hipStream_t s = ctx->stream;
+    DevBuf dv, dh, dk, di, dl, dof, dp, dt;
+    HCK(ctx->cnt.ensure(sizeof(unsigned long long) * G4D_CNT_NUM));
+    HCK(dv.ensure(sizeof(int) * (size_t)n));
+    HCK(dh.ensure(sizeof(int) * (size_t)n));
+    HCK(dk.ensure(sizeof(uint64_t) * (size_t)m));
+    HCK(di.ensure(sizeof(int64_t) * (size_t)(n + 1)));
+    HCK(dl.ensure(sizeof(int) * (size_t)n));
+    HCK(dof.ensure(sizeof(int64_t) * 3 * (size_t)n));
+    HCK(dp.ensure(sizeof(int) * (size_t)n));
+    HCK(dt.ensure(sizeof(int) * 3 * (size_t)n));
+    unsigned long long hc[G4D_CNT_NUM] = {};
+    hc[G4D_CNT_NEW_PAIRS] = (unsigned long long)m / 2;
+    HCK(hipMemcpyAsync(ctx->cnt.ptr, hc, sizeof(hc), hipMemcpyHostToDevice, s));
+    HCK(hipMemcpyAsync(dv.ptr, vnum, sizeof(int) * (size_t)n, hipMemcpyHostToDevice, s));
+    HCK(hipMemcpyAsync(dh.ptr, hnum, sizeof(int) * (size_t)n, hipMemcpyHostToDevice, s));
+    HCK(hipMemcpyAsync(dk.ptr, keys, sizeof(uint64_t) * (size_t)m, hipMemcpyHostToDevice, s));
+    HCK(hipMemsetAsync(dof.ptr, 0xff, sizeof(int64_t) * 3 * (size_t)n, s));
+    g4d::PassPlan pl;
+    for (int k = 0; k < 3; k++) pl.base[k] = base[k];
+    pl.vnum = buf<int>(dv);
+    pl.hnum = buf<int>(dh);
+    pl.ins_off = buf<int64_t>(di);
+    pl.list = buf<int>(dl);
+    pl.nvoff = buf<int64_t>(dof);
+    pl.ntoff = buf<int64_t>(dof) + n;
+    pl.nhoff = buf<int64_t>(dof) + 2 * (int64_t)n;
+    pl.pcount = buf<int>(dp);
+    pl.cnt = buf<unsigned long long>(ctx->cnt);
+    for (int k = 0; k < g4d::STAR_TIERS / 2; k++) pl.tier[k] = buf<int>(dt) + (int64_t)k * n;
+    pl.n = n;
+    pl.lds_limit = g4d::STAR_LDS_LIMIT;
+    if (small) HCK(g4d::launch_small_round(pl, buf<uint64_t>(dk), s));
+    else HCK(g4d::launch_pass_plan(pl, buf<uint64_t>(dk), m, nullptr, s));
+    HCK(hipMemcpyAsync(off, dof.ptr, sizeof(int64_t) * 3 * (size_t)n, hipMemcpyDeviceToHost, s));
+    CK(read_counters(ctx, hc));
+    DevBuf *all[] = {&dv, &dh, &dk, &di, &dl, &dof, &dp, &dt};
+    for (DevBuf *b : all) b->release();
+    for (int k = 0; k < 4; k++) plan[k] = (int64_t)hc[G4D_CNT_ACTIVE + k];
+    for (int k = 0; k < g4d::STAR_TIERS + 2; k++) plan[4 + k] = (int64_t)hc[G4D_CNT_TIER0 + k];
+    return G4D_OK;
+}
+
 int g4d_diag_grid_pairs(g4d_ctx *ctx, const int32_t *id_grid, int32_t grid, uint64_t *out, int64_t cap, int64_t *count)
 {
     if (!ctx || !id_grid || !count || grid < 4 || grid > G4D_MAX_GRID) return G4D_ERR_INVALID_INPUT;

@@ -118,6 +118,13 @@ __device__ __forceinline__ int g4d_wave_incl_sum(int v)
     return x + (row >= 1 ? r0 : 0) + (row >= 2 ? r1 : 0) + (row >= 3 ? r2 : 0);
 }
 
+// The same of non-negative values below 2^49: sums of the low 24 bits and of the rest.
+__device__ __forceinline__ int64_t g4d_wave_incl_sum64(int64_t v)
+{
+    const int lo = g4d_wave_incl_sum((int)(v & 0xffffff)), hi = g4d_wave_incl_sum((int)(v >> 24));
+    return ((int64_t)hi << 24) + lo;
+}
+
 __device__ __forceinline__ int g4d_wave_sum(int v)
 {
 #pragma unroll

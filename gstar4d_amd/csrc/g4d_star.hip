@@ -2458,24 +2458,30 @@ hipError_t launch_proofs(const ProofParams &p, bool exact, hipStream_t s)
 // reciprocation, capacities
 // ------------------------------------------------------------------------------------
 
-// Exclusive prefix of v over the work-group's threads and the total (LA_THREADS threads); red holds
-// LA_THREADS / 64 ints and is free again when every thread has passed the next barrier.
-static constexpr int LA_THREADS = 256;
-__device__ __forceinline__ int la_excl(int v, int *red, int *tot)
+// Exclusive prefix of v over the work-group's threads (NT of them) and the total; red holds NT / 64 values
+// and is free again when every thread has passed the next barrier.  T is int, or int64_t where a tile's
+// sum can pass 2^31: 4,096 stars of 131,074 vertices (a set of two skew lines, some 135,000 points) take
+// 2^31 triangle words.
+template <int NT, typename T>
+__device__ __forceinline__ T list_excl(T v, T *red, T *tot)
 {
-    const int inc = g4d_wave_incl_sum(v), w = threadIdx.x >> 6;
+    T inc;
+    if constexpr (sizeof(T) == 8) inc = g4d_wave_incl_sum64(v);
+    else inc = g4d_wave_incl_sum(v);
+    const int w = threadIdx.x >> 6;
     if ((threadIdx.x & 63) == 63) red[w] = inc;
     __syncthreads();
-    int base = 0, all = 0;
+    T base = 0, all = 0;
 #pragma unroll
-    for (int i = 0; i < LA_THREADS / 64; i++) {
-        const int x = red[i];
+    for (int i = 0; i < NT / 64; i++) {
+        const T x = red[i];
         if (i < w) base += x;
         all += x;
     }
     *tot = all;
     return base + inc - v;
 }
+static constexpr int LA_THREADS = 256;
 
 // Whether a pass has stars left for the exact or the global-memory kernel, which the host launches when
 // it sees their counts: its lists are not complete yet.
@@ -2540,7 +2546,7 @@ __global__ void __launch_bounds__(LA_THREADS) k_drown_keys(const uint64_t *ins_k
         if (m - i0 < 16) bits &= (1u << (m - i0)) - 1u;
     }
     int tot;
-    const int at = la_excl(__popc(bits), red, &tot);
+    const int at = list_excl<LA_THREADS, int>(__popc(bits), red, &tot);
     if (threadIdx.x == 0 && tot) base = atomicAdd(&cnt[G4D_CNT_DROWN_KEYS], (unsigned long long)tot);
     __syncthreads();
     uint64_t *out = keys + base + at;
@@ -2575,7 +2581,7 @@ __global__ void __launch_bounds__(LA_THREADS) k_nonmutual(const uint64_t *keys, 
         c += task[j] != STAR_PAIR_NONE ? 1 : 0;
     }
     int tot;
-    int at = la_excl(c, red, &tot);
+    int at = list_excl<LA_THREADS>(c, red, &tot);
     if (threadIdx.x == 0 && tot) base = atomicAdd(&cnt[G4D_CNT_TASKS], (unsigned long long)tot);
     __syncthreads();
 #pragma unroll
@@ -2849,10 +2855,10 @@ hipError_t launch_new_pairs(const NewPairs &p, hipStream_t s)
 }
 
 // Region sizes of star s with m insertions.
-__device__ __forceinline__ void plan_sizes(const PassPlan &p, int s, int m, int *v, int *t, int *h)
+__device__ __forceinline__ void plan_sizes(const PassPlan &p, int s, int m, int *v, int64_t *t, int *h)
 {
     *v = p.vnum[s] + m;
-    *t = (int)star_tcap_words(*v);
+    *t = star_tcap_words(*v);
     *h = p.hnum[s] + m;
 }
 
@@ -2898,7 +2904,8 @@ __global__ void __launch_bounds__(LA_THREADS) k_pass_plan(PassPlan p, const uint
 {
     __shared__ uint32_t sid[PP_TILE];
     __shared__ uint16_t first[PP_TILE + 1];
-    __shared__ int red[5][LA_THREADS / 64];
+    __shared__ int runs_[LA_THREADS / 64];
+    __shared__ int64_t red[3][LA_THREADS / 64];
     __shared__ unsigned long long base[4];
     __shared__ int last_len, tn[STAR_TIERS + 2]; // per tier, above 64, largest beyond the tiers
     if (dev_m) m = min(m, *dev_m);
@@ -2928,12 +2935,12 @@ __global__ void __launch_bounds__(LA_THREADS) k_pass_plan(PassPlan p, const uint
         fl[j] = __ballot(f);
         mine += __popcll(fl[j]);
     }
-    if (lane == 0) red[4][wv] = mine;
+    if (lane == 0) runs_[wv] = mine;
     __syncthreads();
     int at = 0, runs = 0;
     for (int w = 0; w < LA_THREADS / 64; w++) {
-        if (w < wv) at += red[4][w];
-        runs += red[4][w];
+        if (w < wv) at += runs_[w];
+        runs += runs_[w];
     }
 #pragma unroll
     for (int j = 0; j < PER / 64; j++) {
@@ -2959,9 +2966,10 @@ __global__ void __launch_bounds__(LA_THREADS) k_pass_plan(PassPlan p, const uint
     }
     __syncthreads();
     const int R = (runs + LA_THREADS - 1) / LA_THREADS, r0 = min(tid * R, runs), r1 = min(r0 + R, runs);
-    int v = 0, t = 0, h = 0;
+    int64_t v = 0, t = 0, h = 0;
     for (int r = r0; r < r1; r++) {
-        int dv, dt, dh;
+        int dv, dh;
+        int64_t dt;
         plan_sizes(p, (int)sid[first[r]], r + 1 < runs ? first[r + 1] - first[r] : last_len, &dv, &dt, &dh);
         v += dv;
         t += dt;
@@ -2973,10 +2981,11 @@ __global__ void __launch_bounds__(LA_THREADS) k_pass_plan(PassPlan p, const uint
             if (tier == STAR_TIERS - 1) atomicMax(&tn[STAR_TIERS + 1], dv);
         }
     }
-    int tv, tt, th;
-    const int ev = la_excl(v, red[0], &tv), et = la_excl(t, red[1], &tt), eh = la_excl(h, red[2], &th);
+    int64_t tv, tt, th;
+    const int64_t ev = list_excl<LA_THREADS>(v, red[0], &tv), et = list_excl<LA_THREADS>(t, red[1], &tt),
+                  eh = list_excl<LA_THREADS>(h, red[2], &th);
     if (tid < 4) {
-        const int add[4] = {runs, tv, tt, th};
+        const int64_t add[4] = {runs, tv, tt, th};
         const int c[4] = {G4D_CNT_ACTIVE, G4D_CNT_NEED_V, G4D_CNT_NEED_T, G4D_CNT_NEED_H};
         base[tid] = atomicAdd(&p.cnt[c[tid]], (unsigned long long)add[tid]);
     } else if (tid >= 64 && tid < 64 + STAR_TIERS + 2) {
@@ -2990,7 +2999,8 @@ __global__ void __launch_bounds__(LA_THREADS) k_pass_plan(PassPlan p, const uint
             ho = p.base[2] + (int64_t)base[3] + eh;
     for (int r = r0; r < r1; r++) {
         const int s = (int)sid[first[r]], len = r + 1 < runs ? first[r + 1] - first[r] : last_len;
-        int dv, dt, dh;
+        int dv, dh;
+        int64_t dt;
         plan_sizes(p, s, len, &dv, &dt, &dh);
         const int tier = star_tier(dv, p.lds_limit, merge);
         plan_star(p, s, t0 + first[r], len, base[0] + r, vo, to, ho, tier >= 0);
@@ -3018,28 +3028,12 @@ hipError_t launch_pass_plan(const PassPlan &p, const uint64_t *keys, int64_t m, 
 // 1.70 ms), on 100,000 330 instead of 656 (7.1 -> 6.25 ms).
 static constexpr int SR_THREADS = 1024;
 
-// Exclusive prefix over 1,024 threads and the total; red: 16 ints, reusable after the next barrier.
-__device__ __forceinline__ int sr_excl(int v, int *red, int *tot)
-{
-    const int inc = g4d_wave_incl_sum(v), w = threadIdx.x >> 6;
-    if ((threadIdx.x & 63) == 63) red[w] = inc;
-    __syncthreads();
-    int base = 0, all = 0;
-#pragma unroll
-    for (int i = 0; i < SR_THREADS / 64; i++) {
-        const int x = red[i];
-        if (i < w) base += x;
-        all += x;
-    }
-    *tot = all;
-    return base + inc - v;
-}
-
 __global__ void __launch_bounds__(SR_THREADS) k_small_round(PassPlan p, uint64_t *keys)
 {
     __shared__ uint64_t a[STAR_ROUND_SMALL], b[STAR_ROUND_SMALL];
     __shared__ int first[STAR_ROUND_SMALL + 1];
-    __shared__ int red[5][SR_THREADS / 64];
+    __shared__ int red[2][SR_THREADS / 64];
+    __shared__ int64_t sum[3][SR_THREADS / 64];
     __shared__ int tn[STAR_TIERS + 2];
     const int tid = threadIdx.x;
     const unsigned long long np = p.cnt[G4D_CNT_NEW_PAIRS];
@@ -3056,7 +3050,7 @@ __global__ void __launch_bounds__(SR_THREADS) k_small_round(PassPlan p, uint64_t
         const int i = i0 + tid;
         const bool f = i < m && (i == 0 || a[i] != a[i - 1]);
         int tot;
-        const int at = cnt + sr_excl(f ? 1 : 0, red[r], &tot);
+        const int at = cnt + list_excl<SR_THREADS>(f ? 1 : 0, red[r], &tot);
         if (f) {
             b[at] = a[i];
             keys[at] = a[i];
@@ -3070,7 +3064,7 @@ __global__ void __launch_bounds__(SR_THREADS) k_small_round(PassPlan p, uint64_t
         const int i = i0 + tid;
         const bool f = i < cnt && (i == 0 || (b[i] >> 32) != (b[i - 1] >> 32));
         int tot;
-        const int at = runs + sr_excl(f ? 1 : 0, red[r], &tot);
+        const int at = runs + list_excl<SR_THREADS>(f ? 1 : 0, red[r], &tot);
         if (f) first[at] = i;
         runs += tot;
     }
@@ -3081,14 +3075,16 @@ __global__ void __launch_bounds__(SR_THREADS) k_small_round(PassPlan p, uint64_t
     __syncthreads();
     for (int r0 = 0; r0 < runs; r0 += SR_THREADS) {
         const int r = r0 + tid;
-        int s = 0, len = 0, dv = 0, dt = 0, dh = 0;
+        int s = 0, len = 0, dv = 0, dh = 0;
+        int64_t dt = 0;
         if (r < runs) {
             s = (int)(uint32_t)(b[first[r]] >> 32);
             len = first[r + 1] - first[r];
             plan_sizes(p, s, len, &dv, &dt, &dh);
         }
-        int tv, tt, th;
-        const int ev = sr_excl(dv, red[2], &tv), et = sr_excl(dt, red[3], &tt), eh = sr_excl(dh, red[4], &th);
+        int64_t tv, tt, th;
+        const int64_t ev = list_excl<SR_THREADS, int64_t>(dv, sum[0], &tv), et = list_excl<SR_THREADS>(dt, sum[1], &tt),
+                      eh = list_excl<SR_THREADS, int64_t>(dh, sum[2], &th);
         if (r < runs) {
             const int tier = star_tier(dv, p.lds_limit, true); // at most STAR_ROUND_SMALL keys
             plan_star(p, s, first[r], len, r, vo + ev, to + et, ho + eh, tier >= 0);

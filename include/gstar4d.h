@@ -333,6 +333,15 @@ int g4d_diag_set_link_vertex(g4d_ctx *ctx, int32_t star, int32_t local, int32_t 
    the LSD sort runs. */
 int g4d_diag_sort_pairs(g4d_ctx *ctx, const uint64_t *keys, int64_t m, int32_t nb, int32_t method, uint64_t *out,
                         double *ms, int32_t *shift);
+/* The plan of a splaying pass alone: stars 0..n-1 with vnum[s] link vertices and hnum[s] history entries,
+   and m sorted distinct insertion keys star<<32|vertex.  small: the one-launch form of late rounds (m
+   even, at most 4,096).  base[3]: the arenas' tops (vertices, triangle words, history); off[3 * n]
+   receives the regions' offsets, three runs of n, for the stars with keys (-1 for the others), and
+   plan[12] the number of those stars, the three sizes needed, the lengths of the six tier lists (64,
+   128, 256, 512, 1,024 vertices and beyond), the number of stars above 64, and the largest of the
+   last list. */
+int g4d_diag_pass_plan(g4d_ctx *ctx, int32_t n, const int32_t *vnum, const int32_t *hnum, const uint64_t *keys,
+                       int64_t m, int32_t small, const int64_t *base, int64_t *off, int64_t *plan);
 /* Sorted unique Voronoi-neighbour pairs (min<<32|max) from an id grid. */
 int g4d_diag_grid_pairs(g4d_ctx *ctx, const int32_t *id_grid, int32_t grid, uint64_t *out, int64_t cap,
                         int64_t *count);

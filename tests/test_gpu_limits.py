@@ -52,3 +52,49 @@ def test_triangulation_of_coordinates_that_underflow_is_refused():
     with g.Triangulator(grid_size=16) as t:
         with pytest.raises(g.G4DError, match="PREDICATE_RANGE"):
             t.triangulate(x)
+
+
+# ---------------------------------------------------------------- the plan of a splaying pass
+
+def _plan(vnum, hnum, keys):
+    """Stars with keys, and their sizes (vertices, triangle words, history), in whole numbers."""
+    star, count = np.unique(keys >> np.uint64(32), return_counts=True)
+    star = star.astype(np.int64)
+    v = vnum[star].astype(np.int64) + count
+    t = np.where(v >= 4, 2 * v - 4, 4)
+    return star, v, np.where(v >= 512, 2 * t, t), hnum[star].astype(np.int64) + count
+
+
+@pytest.mark.parametrize("stars,keys,small", [(1, 2, True), (1, 5000, False), (63, 130, True), (1025, 2050, True),
+                                              (4095, 4096, True), (4096, 4096, True), (4096, 4096, False),
+                                              (4097, 4100, False), (9000, 30000, False)])
+@pytest.mark.parametrize("links", [20, 131073, 1 << 27])
+def test_pass_plan_sizes(tri, stars, keys, small, links):
+    """Regions of a pass's stars are next to each other, in some order, from the arenas' tops on, also
+    where a tile's words pass 2^31 (4,096 stars of 131,074 vertices) and 2^41."""
+    rng = np.random.default_rng(stars + links)
+    n = stars + stars // 2 + 1
+    own = rng.permutation(n)[:stars]
+    k = np.concatenate([own, rng.choice(own, keys - stars)]).astype(np.uint64) << np.uint64(32)
+    k = np.sort(k) + np.arange(keys, dtype=np.uint64)
+    vnum = links + rng.integers(0, 20, n)
+    hnum = 3 * vnum
+    base = np.array([7, 1 << 33, 1 << 40])
+    off, plan = tri.diag_pass_plan(vnum, hnum, k, base, small)
+    star, v, t, h = _plan(vnum, hnum, k)
+    assert plan[0] == star.shape[0]
+    assert (plan[1:4] == [v.sum(), t.sum(), h.sum()]).all()
+    for a, size in enumerate((v, t, h)):
+        o = off[a][star]
+        order = np.argsort(o)
+        assert o[order[0]] == base[a]
+        assert (np.diff(o[order]) == size[order][:-1]).all()
+    rest = np.setdiff1d(np.arange(n), star)
+    assert (off[:, rest] == -1).all()
+    # a pass of at most 6,144 keys puts 64 and 128 vertices on the 256-vertex list
+    merged = keys <= 6144
+    tiers = [(32, 32), (32, 32), (32, 256)] if merged else [(32, 64), (64, 128), (128, 256)]
+    tiers += [(256, 512), (512, 1024), (1024, 1 << 62)]
+    assert list(plan[4:10]) == [int(((v > a) & (v <= b)).sum()) for a, b in tiers]
+    assert plan[10] == (v > 64).sum()
+    assert plan[11] == (v.max() if v.max() > 1024 else 0)
