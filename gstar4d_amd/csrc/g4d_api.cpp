@@ -34,6 +34,30 @@ ScratchArena *&scratch_arena_slot()
     static thread_local ScratchArena *arena = nullptr;
     return arena;
 }
+
+KeptScope *&kept_scope_slot()
+{
+    static thread_local KeptScope *scope = nullptr;
+    return scope;
+}
+
+hipError_t device_alloc(void **ptr, size_t bytes)
+{
+    KeptScope *k = kept_scope_slot();
+    const bool fail = k && k->fail_at && *k->fail_at > 0 && --*k->fail_at == 0;
+    hipError_t e = fail ? hipErrorOutOfMemory : hipMalloc(ptr, bytes);
+    if (e == hipErrorOutOfMemory && k) {
+        size_t held = 0;
+        for (int i = 0; i < k->count; i++) held += k->bufs[i].bytes;
+        if (held > 0) {
+            (void)hipDeviceSynchronize();
+            for (int i = 0; i < k->count; i++) k->bufs[i].release();
+            e = hipMalloc(ptr, bytes);
+            (void)hipGetLastError(); // the first try's: no later launch must report it
+        }
+    }
+    return e;
+}
 } // namespace g4d
 
 namespace {
@@ -49,7 +73,8 @@ struct Store {
     static constexpr size_t esz[3] = {sizeof(int), sizeof(uint64_t), sizeof(int)};
     // Arenas that a repack has left are kept for the next one, or for the next call when they are the
     // larger ones, up to this many bytes in all: freeing and allocating them took 1.1 ms a repack and
-    // 0.75 ms a call on 1,000,000 clustered points.
+    // 0.75 ms a call on 1,000,000 clustered points.  An allocation of this context that finds the
+    // memory full frees them first (ENTER).
     static constexpr size_t keep = (size_t)6 << 30;
     DevBuf vnum, voff, tnum, toff, hnum, hoff, nvoff, ntoff, nhoff;
     DevBuf arena[3], spare[3], live[3];
@@ -141,6 +166,7 @@ struct g4d_ctx {
     hipStream_t side[SIDE_STREAMS] = {};
     hipEvent_t ev_side[SIDE_STREAMS + 1] = {}; // one per side stream, and the fork's
     bool side_ok = false, side_make = true;
+    int64_t fail_alloc = 0; // g4d_diag_fail_alloc
     int pba_bands = 0; // bands of the y and x PBA passes (0: by grid size)
     int stage_graphs = -1; // grid-stage chain as a hipGraph: 1 always, 0 never, -1 batched calls only
     // captured grid-stage chains (site scatter and the PBA passes), keyed by everything the
@@ -203,6 +229,11 @@ static int hip_fail(g4d_ctx *c, hipError_t e, const char *what, int line)
         hipError_t e_ = (x);                                                                                           \
         if (e_ != hipSuccess) return hip_fail(ctx, e_, #x, __LINE__);                                                  \
     } while (0)
+
+// Start of an entry point that allocates: its device, and the context's kept arenas for the allocations.
+#define ENTER()                                                                                                        \
+    HCK(hipSetDevice(ctx->opt.device));                                                                                \
+    g4d::KeptScope kept_(ctx->store.spare, 3, &ctx->fail_alloc)
 
 static int bits_for(int64_t n)
 {
@@ -303,9 +334,23 @@ static int repack_store(g4d_ctx *ctx, int n, const int64_t need[3])
         HCK(hipMemcpyAsync(&live[k], sz[k] + n, 8, hipMemcpyDeviceToHost, s));
     }
     HCK(hipStreamSynchronize(s));
-    for (int k = 0; k < 3; k++) {
-        const int64_t cap = std::max<int64_t>((live[k] + need[k]) * 3 / 2, 1024);
-        HCK(st.spare[k].ensure(Store::esz[k] * (size_t)cap));
+    auto room = [&]() -> hipError_t {
+        for (int k = 0; k < 3; k++) {
+            const int64_t cap = std::max<int64_t>((live[k] + need[k]) * 3 / 2, 1024);
+            HIP_CHECK_RET(st.spare[k].ensure(Store::esz[k] * (size_t)cap));
+        }
+        return hipSuccess;
+    };
+    {
+        g4d::KeptScope none(nullptr, 0, &ctx->fail_alloc); // those given room must stay
+        hipError_t e = room();
+        if (e == hipErrorOutOfMemory) { // kept ones may be larger than needed
+            HCK(hipStreamSynchronize(s));
+            for (int k = 0; k < 3; k++) st.spare[k].release();
+            e = room();
+            (void)hipGetLastError(); // the first try's
+        }
+        HCK(e);
     }
     HCK(g4d::launch_repack(n, buf<int>(st.vnum), buf<int64_t>(st.voff), buf<int>(st.tnum), buf<int64_t>(st.toff),
                            buf<int>(st.hnum), buf<int64_t>(st.hoff), buf<int>(st.arena[0]), buf<uint64_t>(st.arena[1]),
@@ -669,6 +714,7 @@ static int grid_stage_graph(g4d_ctx *ctx, const g4d::GridSets &GS, const SetTota
 
 static int run_device(g4d_ctx *ctx, const double *d_xyz, int n, const SetSpec &spec)
 {
+    ENTER();
     ctx->last_xyz = d_xyz;
     ctx->last_nsets = spec.nsets;
     hipStream_t s = ctx->stream;
@@ -1478,7 +1524,7 @@ int g4d_set_options(g4d_ctx *ctx, const g4d_options *opt)
 int g4d_upload_points(g4d_ctx *ctx, const double *xyz, int32_t n, const double **d_xyz)
 {
     if (!ctx || !xyz || n <= 0 || !d_xyz) return G4D_ERR_INVALID_INPUT;
-    HCK(hipSetDevice(ctx->opt.device));
+    ENTER();
     HCK(ctx->xyz_up.ensure(sizeof(double) * 3 * (size_t)n));
     HCK(hipMemcpyAsync(ctx->xyz_up.ptr, xyz, sizeof(double) * 3 * (size_t)n, hipMemcpyHostToDevice, ctx->stream));
     HCK(hipStreamSynchronize(ctx->stream));
@@ -1489,7 +1535,7 @@ int g4d_upload_points(g4d_ctx *ctx, const double *xyz, int32_t n, const double *
 int g4d_triangulate_device(g4d_ctx *ctx, const double *d_xyz, int32_t n, int64_t *num_tets)
 {
     if (!ctx || !d_xyz) return G4D_ERR_INVALID_INPUT;
-    HCK(hipSetDevice(ctx->opt.device));
+    ENTER();
     const int r = run_device(ctx, d_xyz, n, single_set(n, ctx->opt.grid_size));
     if (r != G4D_OK) return r;
     if (num_tets) *num_tets = ctx->num_tets;
@@ -1545,7 +1591,7 @@ int g4d_set_stage_graphs(g4d_ctx *ctx, int32_t mode)
     if (!ctx || mode < -1 || mode > 1) return G4D_ERR_INVALID_INPUT;
     ctx->stage_graphs = mode;
     if (mode == 0) {
-        HCK(hipSetDevice(ctx->opt.device));
+        ENTER();
         HCK(hipStreamSynchronize(ctx->stream));
         destroy_graphs(ctx);
     }
@@ -1589,7 +1635,7 @@ int g4d_triangulate_batch_device(g4d_ctx *ctx, const double *d_xyz, const int64_
                                  const int32_t *grids, int64_t *num_tets)
 {
     if (!ctx || !d_xyz) return G4D_ERR_INVALID_INPUT;
-    HCK(hipSetDevice(ctx->opt.device));
+    ENTER();
     SetSpec spec;
     int64_t n = 0;
     CK(batch_spec(ctx, set_offsets, nsets, grids, &n, spec));
@@ -1666,7 +1712,7 @@ int g4d_triangulate_device_noalloc(g4d_ctx *ctx, const double *d_xyz, int32_t n,
     if (ctx->opt.grid_size > G4D_NOALLOC_MAX_GRID)
         return set_err(ctx, G4D_ERR_CAPACITY, "allocation-free call: grid %d, at most %d", ctx->opt.grid_size,
                        G4D_NOALLOC_MAX_GRID);
-    HCK(hipSetDevice(ctx->opt.device));
+    ENTER();
     void *base = g4d::noalloc_scratch(ctx->opt.device);
     if (ctx->noalloc_status != hipSuccess || !base)
         return set_err(ctx, G4D_ERR_DEVICE, "allocation-free call: scratch array unavailable (%s)",
@@ -1758,7 +1804,7 @@ int g4d_set_proposal(g4d_ctx *ctx, const float *params, int32_t nparams, float t
     if (!params || nparams != g4d::MLP_NPARAM)
         return set_err(ctx, G4D_ERR_INVALID_INPUT, "proposal needs %d parameters", g4d::MLP_NPARAM);
     if (!std::isfinite(threshold)) return set_err(ctx, G4D_ERR_INVALID_INPUT, "threshold must be finite");
-    HCK(hipSetDevice(ctx->opt.device));
+    ENTER();
     HCK(ctx->mlp_params.ensure(sizeof(float) * g4d::MLP_NPARAM));
     HCK(hipMemcpyAsync(ctx->mlp_params.ptr, params, sizeof(float) * g4d::MLP_NPARAM, hipMemcpyHostToDevice,
                        ctx->stream));
@@ -1780,7 +1826,7 @@ int g4d_get_samples(g4d_ctx *ctx, int64_t offset, int64_t stride, float *feature
 {
     if (!ctx || !features || !labels || !count || offset < 0 || stride < 1 || cap < 0) return G4D_ERR_INVALID_INPUT;
     if (!ctx->have_samples) return set_err(ctx, G4D_ERR_INVALID_INPUT, "no samples: enable export before the call");
-    HCK(hipSetDevice(ctx->opt.device));
+    ENTER();
     const int n = ctx->samples_n;
     std::vector<float> f((size_t)n * g4d::PROP_FEATS);
     std::vector<uint32_t> y((size_t)n);
@@ -1804,7 +1850,7 @@ int g4d_mlp_forward(g4d_ctx *ctx, const float *params, const float *features, in
 {
     if (!ctx || !params || !features || !logits || n < 0) return G4D_ERR_INVALID_INPUT;
     if (n == 0) return G4D_OK;
-    HCK(hipSetDevice(ctx->opt.device));
+    ENTER();
     hipStream_t s = ctx->stream;
     DevBuf dp, df, dl;
     HCK(dp.ensure(sizeof(float) * g4d::MLP_NPARAM));
@@ -1825,7 +1871,7 @@ int g4d_mlp_grad(g4d_ctx *ctx, const float *params, const float *features, const
                  float *grad, double *loss)
 {
     if (!ctx || !params || !features || !labels || !grad || !loss || n < 0) return G4D_ERR_INVALID_INPUT;
-    HCK(hipSetDevice(ctx->opt.device));
+    ENTER();
     hipStream_t s = ctx->stream;
     DevBuf dp, df, dy, dg, dloss;
     HCK(dp.ensure(sizeof(float) * g4d::MLP_NPARAM));
@@ -1859,7 +1905,7 @@ int g4d_mlp_train(g4d_ctx *ctx, float *params, const float *features, const uint
     if (!ctx || !params || !features || !labels || n <= 0 || epochs < 1 || batch < 32 || !(lr > 0.f))
         return G4D_ERR_INVALID_INPUT;
     if (n > INT32_MAX) return set_err(ctx, G4D_ERR_INVALID_INPUT, "at most 2^31 - 1 samples");
-    HCK(hipSetDevice(ctx->opt.device));
+    ENTER();
     hipStream_t s = ctx->stream;
     DevBuf dp, dm, dv, dg, dloss, df, dy, didx;
     const size_t np = g4d::MLP_NPARAM;
@@ -1924,7 +1970,7 @@ int g4d_diag_orient4(g4d_ctx *ctx, const double *pts5, const int32_t *idx5, int6
 {
     if (!ctx || !pts5 || !idx5 || !sign_out || T < 0) return G4D_ERR_INVALID_INPUT;
     if (T == 0) return G4D_OK;
-    HCK(hipSetDevice(ctx->opt.device));
+    ENTER();
     DevBuf dp, di, ds, dd;
     HCK(dp.ensure(sizeof(double) * 15 * (size_t)T));
     HCK(di.ensure(sizeof(int) * 5 * (size_t)T));
@@ -1948,7 +1994,7 @@ int g4d_diag_orient3d(g4d_ctx *ctx, const double *pts4, int64_t T, int32_t *sign
 {
     if (!ctx || !pts4 || !sign_out || T < 0) return G4D_ERR_INVALID_INPUT;
     if (T == 0) return G4D_OK;
-    HCK(hipSetDevice(ctx->opt.device));
+    ENTER();
     DevBuf dp, ds;
     HCK(dp.ensure(sizeof(double) * 12 * (size_t)T));
     HCK(ds.ensure(sizeof(int) * (size_t)T));
@@ -1966,7 +2012,7 @@ int g4d_diag_orient3d(g4d_ctx *ctx, const double *pts4, int64_t T, int32_t *sign
 int g4d_diag_morton(g4d_ctx *ctx, const double *xyz, int32_t n, int32_t grid, int32_t *perm_out, int32_t *vox_out)
 {
     if (!ctx || !xyz || n <= 0 || !perm_out || !vox_out || grid < 4 || grid > G4D_MAX_GRID) return G4D_ERR_INVALID_INPUT;
-    HCK(hipSetDevice(ctx->opt.device));
+    ENTER();
     hipStream_t s = ctx->stream;
     const double *d_xyz = nullptr;
     CK(g4d_upload_points(ctx, xyz, n, &d_xyz));
@@ -2003,7 +2049,7 @@ int g4d_diag_pba(g4d_ctx *ctx, const int32_t *vox_sorted, int32_t n, int32_t gri
     const bool id_mode = grid > G4D_CODE_GRID || codes == 2;
     if (grid > G4D_CODE_GRID && codes == 1)
         return set_err(ctx, G4D_ERR_INVALID_INPUT, "site codes exist only for grids up to %d", G4D_CODE_GRID);
-    HCK(hipSetDevice(ctx->opt.device));
+    ENTER();
     hipStream_t s = ctx->stream;
     std::vector<uint64_t> enc((size_t)n);
     for (int k = 0; k < n; k++) {
@@ -2141,7 +2187,7 @@ int g4d_check_result(g4d_ctx *ctx, int32_t full_empty_sphere, g4d_check_report *
     if (!ctx || !rep || !ctx->have_result) return G4D_ERR_INVALID_INPUT;
     if (ctx->last_nsets > 1)
         return set_err(ctx, G4D_ERR_INVALID_INPUT, "the last result is a batch; check each set with g4d_check_mesh");
-    HCK(hipSetDevice(ctx->opt.device));
+    ENTER();
     const double *pts = ctx->opt.index_space == G4D_INDEX_MORTON ? buf<double>(ctx->pts) : ctx->last_xyz;
     const int *opp = ctx->opt.compute_adjacency ? buf<int>(ctx->opp) : nullptr;
     return check_device(ctx, pts, ctx->last_n, buf<int>(ctx->tets), opp, ctx->num_tets, full_empty_sphere != 0, rep);
@@ -2151,7 +2197,7 @@ int g4d_check_mesh(g4d_ctx *ctx, const double *xyz, int32_t n, const int32_t *te
                    int64_t num_tets, int32_t full_empty_sphere, g4d_check_report *rep)
 {
     if (!ctx || !xyz || n <= 0 || !rep || num_tets < 0 || (num_tets > 0 && !tets)) return G4D_ERR_INVALID_INPUT;
-    HCK(hipSetDevice(ctx->opt.device));
+    ENTER();
     hipStream_t s = ctx->stream;
     DevBuf dp, dt, dop;
     HCK(dp.ensure(sizeof(double) * 3 * (size_t)n));
@@ -2192,7 +2238,7 @@ static g4d::OutParams star_params(g4d_ctx *ctx)
 int g4d_check_stars(g4d_ctx *ctx, int64_t *inconsistent, int64_t *triangles)
 {
     if (!ctx || !inconsistent || !ctx->have_result) return G4D_ERR_INVALID_INPUT;
-    HCK(hipSetDevice(ctx->opt.device));
+    ENTER();
     hipStream_t s = ctx->stream;
     const g4d::OutParams op = star_params(ctx);
     HCK(g4d::launch_zero_counters(op.cnt, (1u << G4D_CNT_APPEND4) | (1u << G4D_CNT_APPEND5), s));
@@ -2207,7 +2253,7 @@ int g4d_check_stars(g4d_ctx *ctx, int64_t *inconsistent, int64_t *triangles)
 int g4d_diag_set_link_vertex(g4d_ctx *ctx, int32_t star, int32_t local, int32_t v)
 {
     if (!ctx || !ctx->have_result || star < 0 || star >= ctx->last_n) return G4D_ERR_INVALID_INPUT;
-    HCK(hipSetDevice(ctx->opt.device));
+    ENTER();
     Store &store = ctx->store;
     int vn = 0;
     int64_t vo = 0;
@@ -2221,7 +2267,7 @@ int g4d_diag_set_link_vertex(g4d_ctx *ctx, int32_t star, int32_t local, int32_t 
 int g4d_diag_copy(g4d_ctx *ctx, int64_t bytes, double *ms)
 {
     if (!ctx || bytes < 16) return G4D_ERR_INVALID_INPUT;
-    HCK(hipSetDevice(ctx->opt.device));
+    ENTER();
     const int64_t n16 = bytes / 16;
     DevBuf a, b;
     HCK(a.ensure((size_t)n16 * 16));
@@ -2243,7 +2289,7 @@ int g4d_diag_sort_pairs(g4d_ctx *ctx, const uint64_t *keys, int64_t m, int32_t n
     if (!ctx || m < 0 || (m > 0 && (!keys || !out)) || nb < 1 || nb > 31 || method < 0 || method > 4)
         return G4D_ERR_INVALID_INPUT;
     if (m > G4D_MAX_SORT_KEYS) return set_err(ctx, G4D_ERR_CAPACITY, "%lld keys exceed the sort limit", (long long)m);
-    HCK(hipSetDevice(ctx->opt.device));
+    ENTER();
     hipStream_t s = ctx->stream;
     if (shift)
         *shift = method == 1 ? -1 : g4d::key_sort_shift(m, nb, (method == 2 || method == 4) ? nb + 1 : nb, 0, method >= 3);
@@ -2266,6 +2312,18 @@ int g4d_diag_sort_pairs(g4d_ctx *ctx, const uint64_t *keys, int64_t m, int32_t n
     return G4D_OK;
 }
 
+int g4d_diag_fail_alloc(g4d_ctx *ctx, int64_t at, int64_t *left, int64_t *kept)
+{
+    if (!ctx || at < 0) return G4D_ERR_INVALID_INPUT;
+    if (left) *left = ctx->fail_alloc;
+    ctx->fail_alloc = at;
+    if (kept) {
+        *kept = 0;
+        for (int k = 0; k < 3; k++) *kept += (int64_t)ctx->store.spare[k].bytes;
+    }
+    return G4D_OK;
+}
+
 int g4d_diag_pass_plan(g4d_ctx *ctx, int32_t n, const int32_t *vnum, const int32_t *hnum, const uint64_t *keys,
                        int64_t m, int32_t small, const int64_t *base, int64_t *off, int64_t *plan)
 {
@@ -2278,7 +2336,7 @@ int g4d_diag_pass_plan(g4d_ctx *ctx, int32_t n, const int32_t *vnum, const int32
     for (int32_t i = 0; i < n; i++)
         if (vnum[i] < 0 || hnum[i] < 0 || vnum[i] > (1 << 29) || hnum[i] > (1 << 29))
             return set_err(ctx, G4D_ERR_INVALID_INPUT, "star %d out of range", i);
-    HCK(hipSetDevice(ctx->opt.device));
+    ENTER();
     hipStream_t s = ctx->stream;
     DevBuf dv, dh, dk, di, dl, dof, dp, dt;
     HCK(ctx->cnt.ensure(sizeof(unsigned long long) * G4D_CNT_NUM));
@@ -2325,7 +2383,7 @@ int g4d_diag_pass_plan(g4d_ctx *ctx, int32_t n, const int32_t *vnum, const int32
 int g4d_diag_grid_pairs(g4d_ctx *ctx, const int32_t *id_grid, int32_t grid, uint64_t *out, int64_t cap, int64_t *count)
 {
     if (!ctx || !id_grid || !count || grid < 4 || grid > G4D_MAX_GRID) return G4D_ERR_INVALID_INPUT;
-    HCK(hipSetDevice(ctx->opt.device));
+    ENTER();
     hipStream_t s = ctx->stream;
     const int64_t G3 = (int64_t)grid * grid * grid;
     HCK(ctx->gtmp.ensure(sizeof(int) * (size_t)G3));

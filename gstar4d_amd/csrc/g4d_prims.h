@@ -24,6 +24,21 @@ struct ScratchScope {
     ~ScratchScope() { scratch_arena_slot() = prev; }
 };
 
+struct DevBuf;
+// Buffers that hold nothing any more and are kept for later: while a scope is installed on the calling
+// thread, an allocation that finds the device's memory full frees them and tries again.  fail_at (may
+// be null, tests): the allocation from now at which the first try is taken to have failed.
+struct KeptScope {
+    KeptScope *prev;
+    DevBuf *bufs;
+    int count;
+    int64_t *fail_at;
+    inline KeptScope(DevBuf *b, int n, int64_t *fail);
+    inline ~KeptScope();
+};
+KeptScope *&kept_scope_slot();
+hipError_t device_alloc(void **ptr, size_t bytes);
+
 // Growable device buffer owned by a context; never shrinks, reused across calls.
 struct DevBuf {
     void *ptr = nullptr;
@@ -56,7 +71,7 @@ struct DevBuf {
             bytes = 0;
         }
         size_t cap = need + need / 8 + 256;
-        hipError_t e = hipMalloc(&ptr, cap);
+        hipError_t e = device_alloc(&ptr, cap);
         if (e != hipSuccess) {
             ptr = nullptr;
             return e;
@@ -76,6 +91,12 @@ struct DevBuf {
         return reinterpret_cast<T *>(ptr);
     }
 };
+
+inline KeptScope::KeptScope(DevBuf *b, int n, int64_t *fail) : prev(kept_scope_slot()), bufs(b), count(n), fail_at(fail)
+{
+    kept_scope_slot() = this;
+}
+inline KeptScope::~KeptScope() { kept_scope_slot() = prev; }
 
 struct Prims {
     DevBuf scan_tmp[4];

@@ -333,6 +333,11 @@ int g4d_diag_set_link_vertex(g4d_ctx *ctx, int32_t star, int32_t local, int32_t 
    the LSD sort runs. */
 int g4d_diag_sort_pairs(g4d_ctx *ctx, const uint64_t *keys, int64_t m, int32_t nb, int32_t method, uint64_t *out,
                         double *ms, int32_t *shift);
+/* Takes the at-th device allocation from now (0: none) of this context to find the memory full on its
+   first try, as a full device would.  *left (may be NULL) receives what an earlier call has left to
+   count, *kept (may be NULL) the bytes of arenas that the context keeps unused, and would give back
+   then. */
+int g4d_diag_fail_alloc(g4d_ctx *ctx, int64_t at, int64_t *left, int64_t *kept);
 /* The plan of a splaying pass alone: stars 0..n-1 with vnum[s] link vertices and hnum[s] history entries,
    and m sorted distinct insertion keys star<<32|vertex.  small: the one-launch form of late rounds (m
    even, at most 4,096).  base[3]: the arenas' tops (vertices, triangle words, history); off[3 * n]

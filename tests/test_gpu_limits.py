@@ -98,3 +98,47 @@ def test_pass_plan_sizes(tri, stars, keys, small, links):
     assert list(plan[4:10]) == [int(((v > a) & (v <= b)).sum()) for a, b in tiers]
     assert plan[10] == (v > 64).sum()
     assert plan[11] == (v.max() if v.max() > 1024 else 0)
+
+
+# ---------------------------------------------------------------- a full device
+
+def _clumps(seed, count, each):
+    rng = np.random.default_rng(seed)
+    return np.concatenate([c + 1e-3 * rng.normal(size=(each, 3)) for c in rng.random((count, 3))])
+
+
+def _bigger(kind):
+    """A set after _clumps(5, 25, 1600) that needs larger buffers, with and without a repack."""
+    return _clumps(6, 25, 3200) if kind == "clumps" else np.random.default_rng(6).random((120000, 3))
+
+
+@pytest.mark.parametrize("kind", ["clumps", "uniform"])
+def test_kept_arenas_are_given_back_when_the_device_is_full(kind):
+    """After a repack a context keeps the arenas it has left.  An allocation that finds the memory full, at
+    any place of the next call, gives them back and goes on: the same tetrahedra as a new context."""
+    first, x = _clumps(5, 25, 1600), _bigger(kind)
+    with g.Triangulator(grid_size=64) as t:
+        want = t.triangulate(x)[:2]
+    for at in range(1, 200, 3):
+        with g.Triangulator(grid_size=64) as t:
+            t.triangulate(first)
+            assert t.stats()["store_repacks"] >= 1 and t.diag_fail_alloc(at)[1] > 0
+            got = t.triangulate(x)[:2]
+            left, _ = t.diag_fail_alloc(0)
+        assert np.array_equal(got[0], want[0]) and np.array_equal(got[1], want[1]), at
+        if left:
+            break  # the call allocates less often
+    assert left and at > 10
+
+
+def test_full_device_without_kept_arenas_is_an_error_once(orc):
+    x = np.random.default_rng(8).random((4000, 3))
+    ref, _, _ = orc.triangulate(x, 32)
+    with g.Triangulator(grid_size=32) as t:
+        for at in (1, 5, 20):
+            assert t.diag_fail_alloc(at)[1] == 0
+            with pytest.raises(g.G4DError) as e:
+                t.triangulate(x)
+            assert e.value.status == "OOM"
+        tets, _, _ = t.triangulate(x)
+        assert (g.canonical(tets) == ref).all()
