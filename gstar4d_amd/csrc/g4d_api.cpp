@@ -1111,6 +1111,9 @@ static int run_device(g4d_ctx *ctx, const double *d_xyz, int n, const SetSpec &s
             const int full = k == 0 ? 4096 : k == 1 ? 3072 : 1536;
             return g4d::launch_star_kernel(tp, vmax, false, std::min(full, tp.nlist), q);
         };
+        // A late pass's launch takes both tiers and is left out of the 32-vertex kernel's statistics.
+        const bool late = !fork128 && tier_n[0] == 0 && tier_n[1] == 0 && tier_n[2] > 0 && nitems <= LATE_STARS &&
+                          g4d::star_late_variant(sp.t0_variant);
         {
             SideStreams side(ctx, fork128 || forkw || forkg);
             hipError_t e = side.open(s);
@@ -1120,9 +1123,7 @@ static int run_device(g4d_ctx *ctx, const double *d_xyz, int n, const SetSpec &s
             if (forkg) run(5, 2);
             if (forkw) run(4, 1), run(3, 1);
             if (fork128) run(2, 0), run(1, 0);
-            const bool late = !fork128 && tier_n[0] == 0 && tier_n[1] == 0 && tier_n[2] > 0 && nitems <= LATE_STARS &&
-                              g4d::star_late_variant(sp.t0_variant);
-            if (ctx->ev_ok) (void)hipEventRecord(ctx->ev_t0[0], s);
+            if (!late && ctx->ev_ok) (void)hipEventRecord(ctx->ev_t0[0], s);
             if (late) {
                 g4d::StarParams tp = sp;
                 tp.star_list = tl[2];
@@ -1132,7 +1133,7 @@ static int run_device(g4d_ctx *ctx, const double *d_xyz, int n, const SetSpec &s
             } else if (e == hipSuccess) {
                 e = g4d::launch_star_kernel(sp, g4d::STAR_VMAX_T0, false, nblk_star, s);
             }
-            if (ctx->ev_ok) (void)hipEventRecord(ctx->ev_t0[1], s);
+            if (!late && ctx->ev_ok) (void)hipEventRecord(ctx->ev_t0[1], s);
             if (e == hipSuccess) e = tier_launch(0, s);
             if (!fork128 && !late) {
                 if (e == hipSuccess) e = tier_launch(1, s);
@@ -1168,7 +1169,7 @@ static int run_device(g4d_ctx *ctx, const double *d_xyz, int n, const SetSpec &s
             CK(read_counters(ctx, hc));
             if (hc[G4D_CNT_APPEND3]) return set_err(ctx, G4D_ERR_INTERNAL, "exact star list holds a larger star");
         }
-        {
+        if (!late) {
             float ms = 0.f;
             if (ctx->ev_ok && hipEventElapsedTime(&ms, ctx->ev_t0[0], ctx->ev_t0[1]) == hipSuccess)
                 ctx->st.t_star_t0_ms += ms;

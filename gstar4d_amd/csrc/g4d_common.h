@@ -46,7 +46,7 @@ enum g4d_counter : int {
     G4D_CNT_APPEND0 = 1,  // generic append counters
     G4D_CNT_APPEND1 = 2,
     G4D_CNT_APPEND2 = 3,
-    G4D_CNT_ORIENT4 = 4,  // cofactor-filter orient4 evaluations in the LDS star kernels
+    G4D_CNT_ORIENT4 = 4,  // cofactor-filter orient4 evaluations in the 32-vertex star kernel
     G4D_CNT_EXACT = 5,    // exact insphere evaluations
     G4D_CNT_SOS = 6,      // SoS resolutions
     G4D_CNT_ORIENT3 = 7,
@@ -56,7 +56,7 @@ enum g4d_counter : int {
     G4D_CNT_APPEND4 = 11,
     G4D_CNT_APPEND5 = 12,
     G4D_CNT_APPEND6 = 13,
-    G4D_CNT_COFACTOR = 14, // cached-cofactor computations in the LDS star kernels
+    G4D_CNT_COFACTOR = 14, // cached-cofactor computations in the 32-vertex star kernel
     G4D_CNT_XMID = 15,     // list lengths of the exact chain's 64- and 256-vertex tiers
     G4D_CNT_XBIG = 16,
     G4D_CNT_QUEUE0 = 17,   // work-queue heads of the star-kernel launches of one pass (17..23)

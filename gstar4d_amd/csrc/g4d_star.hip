@@ -248,6 +248,7 @@ template <int VMAX, bool EXACT>
 __device__ __forceinline__ void star_body(const StarParams &p, int nitems, int bid, int nblk)
 {
     constexpr bool REGC = !EXACT;
+    constexpr bool COUNT = !EXACT && VMAX == STAR_VMAX_T0; // the statistics are the 32-vertex kernel's
     using Lds = StarLds<VMAX, !REGC>;
     constexpr int TMAX = Lds::TMAX;
     constexpr int KPL = TMAX / 64;
@@ -382,7 +383,7 @@ __device__ __forceinline__ void star_body(const StarParams &p, int nitems, int b
                             const uint32_t t = L.tv[lane + 64 * k];
                             tri_cofactors(L.vc[tvert(t, 0)], L.vc[tvert(t, 1)], L.vc[tvert(t, 2)], C, P);
                             L.tv[lane + 64 * k] = t & ~TF_FRESH;
-                            ncof++;
+                            if (COUNT) ncof++;
                         }
 #pragma unroll
                         for (int i = 0; i < KPL; i++)
@@ -402,7 +403,7 @@ __device__ __forceinline__ void star_body(const StarParams &p, int nitems, int b
                             const uint32_t t = L.tv[slot];
                             lds_cofactors<TMAX>(L.vc[tvert(t, 0)], L.vc[tvert(t, 1)], L.vc[tvert(t, 2)], L.cof, slot);
                             L.tv[slot] = t & ~TF_FRESH;
-                            ncof++;
+                            if (COUNT) ncof++;
                         }
                 }
             };
@@ -423,7 +424,7 @@ __device__ __forceinline__ void star_body(const StarParams &p, int nitems, int b
                     if (slot < T) {
                         const uint32_t t = L.tv[slot];
                         if ((t & (TF_ALIVE | TF_VIS)) == TF_ALIVE) {
-                            nfilt++;
+                            if (COUNT) nfilt++;
                             int sg;
                             if constexpr (REGC) {
                                 sg = cofactor_filter_sign2(r, rsum, rc[k], rp[k][0], rp[k][1]);
@@ -671,10 +672,14 @@ __device__ __forceinline__ void star_body(const StarParams &p, int nitems, int b
             wave_sync();
         }
     }
-    const int wf = g4d_wave_sum(nfilt), wc = g4d_wave_sum(ncof);
+    if (COUNT) {
+        const int wf = g4d_wave_sum(nfilt), wc = g4d_wave_sum(ncof);
+        if (lane == 0) {
+            atomicAdd(&cnt[G4D_CNT_ORIENT4], (unsigned long long)wf);
+            atomicAdd(&cnt[G4D_CNT_COFACTOR], (unsigned long long)wc);
+        }
+    }
     if (lane == 0) {
-        atomicAdd(&cnt[G4D_CNT_ORIENT4], (unsigned long long)wf);
-        atomicAdd(&cnt[G4D_CNT_COFACTOR], (unsigned long long)wc);
         if (npairs) atomicAdd(&cnt[G4D_CNT_PAIRS], npairs);
         if (ndrown) atomicAdd(&cnt[G4D_CNT_DROWNED], ndrown);
     }
@@ -893,7 +898,7 @@ __device__ __forceinline__ int wave_max_i(int v)
     return max(max(r0, r1), max(r2, r3));
 }
 
-template <int GL, bool PF>
+template <int GL, bool PF, bool COUNT = true>
 __device__ __forceinline__ void star_body_grp(const StarParams &p, int nitems, int bid, int nblk)
 {
     constexpr int NG = 64 / GL;
@@ -1071,7 +1076,7 @@ __device__ __forceinline__ void star_body_grp(const StarParams &p, int nitems, i
                     const double *r2 = L.vc[tvert(t, 2)];
                     const double a2 = fabs(r2[0]) + fabs(r2[1]) + fabs(r2[2]);
                     grp_cofactors(L.vc[tvert(t, 0)], L.vc[tvert(t, 1)], r2, a2, a2 + r2[3], C[k], P[k]);
-                    ncof++;
+                    if (COUNT) ncof++;
                 }
             }
             // ---- insertions: every group steps through its list in lock-step ----
@@ -1101,7 +1106,7 @@ __device__ __forceinline__ void star_body_grp(const StarParams &p, int nitems, i
 #pragma unroll
                 for (int k = 0; k < KPL; k++) {
                     if (step && (int)tk[k] < 0) {
-                        nfilt++;
+                        if (COUNT) nfilt++;
                         const int sg = grp_filter_sign(r, w, C[k], P[k]);
                         if (sg == 0) um |= 1u << k;
                         if (sg < 0) {
@@ -1235,7 +1240,7 @@ __device__ __forceinline__ void star_body_grp(const StarParams &p, int nitems, i
                     const uint32_t t = tk[k];
                     if ((t >> 18) == fresh) {
                         grp_cofactors(L.vc[tvert(t, 0)], L.vc[tvert(t, 1)], r, w.a, w.rs, C[k], P[k]);
-                        ncof++;
+                        if (COUNT) ncof++;
                     }
                 }
                 // No barrier before the next step: its filter reads and writes only this lane's
@@ -1362,10 +1367,14 @@ __device__ __forceinline__ void star_body_grp(const StarParams &p, int nitems, i
             wave_sync();
         }
     }
-    const int wf = g4d_wave_sum(nfilt), wc = g4d_wave_sum(ncof);
+    if (COUNT) {
+        const int wf = g4d_wave_sum(nfilt), wc = g4d_wave_sum(ncof);
+        if (lane == 0) {
+            atomicAdd(&cnt[G4D_CNT_ORIENT4], (unsigned long long)wf);
+            atomicAdd(&cnt[G4D_CNT_COFACTOR], (unsigned long long)wc);
+        }
+    }
     if (lane == 0) {
-        atomicAdd(&cnt[G4D_CNT_ORIENT4], (unsigned long long)wf);
-        atomicAdd(&cnt[G4D_CNT_COFACTOR], (unsigned long long)wc);
         if (npairs) atomicAdd(&cnt[G4D_CNT_PAIRS], npairs);
         if (ndrown) atomicAdd(&cnt[G4D_CNT_DROWNED], ndrown);
     }
@@ -1399,7 +1408,7 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4, 8)))
 __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 8))) k_star_late(StarParams p, int nb,
                                                                                             StarParams q)
 {
-    if ((int)blockIdx.x < nb) star_body_grp<16, true>(p, p.nlist, blockIdx.x, nb);
+    if ((int)blockIdx.x < nb) star_body_grp<16, true, false>(p, p.nlist, blockIdx.x, nb);
     else star_body<STAR_VMAX_T2, false>(q, q.nlist, blockIdx.x - nb, gridDim.x - nb);
 }
 
@@ -1578,7 +1587,6 @@ __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(WPE, 8)
     const int tid = threadIdx.x;
     unsigned long long *cnt = p.cnt;
     double rc[KPL][4], rp[KPL][2];
-    int ncof = 0, nfilt = 0;
     unsigned long long npairs = 0, ndrown = 0; // of the work-group, and of the wave
     for (;;) {
         __syncthreads(); // the previous star is done with L
@@ -1663,7 +1671,6 @@ __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(WPE, 8)
                     const uint64_t t = L.tv64[tid + NT * k];
                     tri_cofactors(L.vc[wtv(t, 0)], L.vc[wtv(t, 1)], L.vc[wtv(t, 2)], C, P);
                     L.tv[tid + NT * k][3] = (uint16_t)(wfl(t) & ~TW_FRESH);
-                    ncof++;
                 }
 #pragma unroll
                 for (int i = 0; i < KPL; i++)
@@ -1690,7 +1697,6 @@ __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(WPE, 8)
                 if (slot < T) {
                     const uint32_t f = L.tv[slot][3];
                     if ((f & (TW_ALIVE | TW_VIS)) == TW_ALIVE) {
-                        nfilt++;
                         const int sg = cofactor_filter_sign2(r, rsum, rc[k], rp[k][0], rp[k][1]);
                         unc = unc || sg == 0;
                         if (sg < 0) {
@@ -1873,10 +1879,7 @@ __global__ void __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(WPE, 8)
         __syncthreads(); // every read of the old record and regions before the switch
         if (tid == 0) star_commit(p, s, vcount, vo, tcount, to, hn + m);
     }
-    const int wf = g4d_wave_sum(nfilt), wc = g4d_wave_sum(ncof);
     if ((tid & 63) == 0) {
-        atomicAdd(&cnt[G4D_CNT_ORIENT4], (unsigned long long)wf);
-        atomicAdd(&cnt[G4D_CNT_COFACTOR], (unsigned long long)wc);
         if (tid == 0 && npairs) atomicAdd(&cnt[G4D_CNT_PAIRS], npairs);
         if (ndrown) atomicAdd(&cnt[G4D_CNT_DROWNED], ndrown);
     }

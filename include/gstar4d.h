@@ -92,7 +92,9 @@ typedef struct {
     int32_t store_repacks;     /* times the star arenas were compacted into larger ones */
     int32_t star_passes;       /* star kernel passes: creation plus one per splaying round */
     /* The 32-vertex LDS star kernel (the dominant kernel): launches, summed time (hipEvents on
-       the context's stream), cofactor-filter orient4 evaluations and cofactor computations. */
+       the context's stream; the larger stars' kernels may run beside it), its cofactor-filter
+       orient4 evaluations and cofactor computations.  Late passes, whose one launch takes the
+       larger stars too, are left out. */
     int32_t star_t0_launches;
     int32_t pad1;
     double t_star_t0_ms;

@@ -142,3 +142,28 @@ def test_full_device_without_kept_arenas_is_an_error_once(orc):
             assert e.value.status == "OOM"
         tets, _, _ = t.triangulate(x)
         assert (g.canonical(tets) == ref).all()
+
+
+# ---------------------------------------------------------------- statistics
+
+def test_star_kernel_statistics_are_the_32_vertex_kernels():
+    """Evaluations and cofactors of the 32-vertex kernel are the same whether the larger stars run in the
+    LDS kernels or, by a lowered limit, in the global-memory kernel; the default variant leaves out
+    the late passes, which share a launch."""
+    x = np.concatenate([_clumps(9, 10, 800), np.random.default_rng(9).random((4000, 3))])
+    def run(variant, limit):
+        with g.Triangulator(grid_size=32, lds_star_limit=limit) as t:
+            t.set_star_kernel(variant)
+            t.triangulate(x)
+            return t.stats()
+    for variant in (0, 1, 2, 4):
+        a, b = run(variant, 0), run(variant, 32)
+        assert a["big_stars"] > 0 and b["huge_stars"] > a["huge_stars"]
+        assert a["star_t0_launches"] == a["star_passes"] == b["star_passes"] == b["star_t0_launches"]
+        assert a["star_t0_filter_evals"] == b["star_t0_filter_evals"] > 0
+        assert a["star_t0_cofactors"] == b["star_t0_cofactors"] > 0
+    c = run(-1, 0)
+    assert 0 < c["star_t0_launches"] < c["star_passes"] == a["star_passes"]
+    d = run(2, 0)
+    assert 0 < c["star_t0_filter_evals"] < d["star_t0_filter_evals"]
+    assert 0 < c["star_t0_cofactors"] < d["star_t0_cofactors"]
