@@ -145,7 +145,8 @@ struct g4d_ctx {
     PinnedBuf h_tets, h_opp, h_perm; // results of g4d_triangulate / g4d_triangulate_batch
     // Page-locked staging of the small reads back to the host (counters and counts): a pageable
     // destination makes the runtime stage every such read itself, about 8 us more per read.
-    // The counters first, then 16 scalars, then the primitives' two counts.
+    // The counters first, then the scalars, then the primitives' counts.
+    static constexpr int STAGE_SCALARS = 16, STAGE_COUNTS = 2;
     PinnedBuf hpin;
     int64_t *hstage = nullptr; // in hpin, or the calling context's for a temporary context
     std::vector<int32_t> h_set_grid;
@@ -293,10 +294,12 @@ static int read_counters(g4d_ctx *ctx, unsigned long long *h)
     return G4D_OK;
 }
 
-// Scalar slot k (0..15) of the page-locked staging, or the caller's fallback variable.
-static int64_t *hslot(g4d_ctx *ctx, int k, int64_t *fallback)
+// Scalar slots K .. K + N - 1 of the page-locked staging, or the caller's fallback variables.
+template <int K, int N = 1>
+static int64_t *hslot(g4d_ctx *ctx, int64_t *fallback)
 {
-    return ctx->hstage ? ctx->hstage + G4D_CNT_NUM + k : fallback;
+    static_assert(K >= 0 && K + N <= g4d_ctx::STAGE_SCALARS, "scalar slots of the staging");
+    return ctx->hstage ? ctx->hstage + G4D_CNT_NUM + K : fallback;
 }
 
 static int check_dev_error(g4d_ctx *ctx, unsigned long long flags, const char *stage)
@@ -764,7 +767,7 @@ static int run_device(g4d_ctx *ctx, const double *d_xyz, int n, const SetSpec &s
     else HCK(g4d::launch_bounds(d_xyz, n, dbounds, s));
     {
         std::vector<double> hv(2 * (size_t)S);
-        int64_t *slot = S == 1 ? hslot(ctx, 10, nullptr) : nullptr; // two slots
+        int64_t *slot = S == 1 ? hslot<10, 2>(ctx, nullptr) : nullptr;
         double *hb = slot ? reinterpret_cast<double *>(slot) : hv.data();
         HCK(hipMemcpyAsync(hb, dbounds, sizeof(double) * 2 * (size_t)S, hipMemcpyDeviceToHost, s));
         HCK(hipStreamSynchronize(s));
@@ -823,7 +826,7 @@ static int run_device(g4d_ctx *ctx, const double *d_xyz, int n, const SetSpec &s
     uint2 *tcnt = reinterpret_cast<uint2 *>(ttot + ntiles + 1);
     HCK(g4d::launch_grid_pair_count(idg, GS, ntiles, pcnt, s));
     HCK(g4d::scan_excl_i64(P, pcnt, pcnt, ntiles, pcnt + ntiles, s));
-    int64_t ngp_f = 0, *ngp_h = hslot(ctx, 0, &ngp_f);
+    int64_t ngp_f = 0, *ngp_h = hslot<0>(ctx, &ngp_f);
     HCK(hipMemcpyAsync(ngp_h, pcnt + ntiles, 8, hipMemcpyDeviceToHost, s));
     HCK(hipStreamSynchronize(s));
     const int64_t ngp = *ngp_h;
@@ -839,7 +842,7 @@ static int run_device(g4d_ctx *ctx, const double *d_xyz, int n, const SetSpec &s
     HCK(g4d::scan_excl_i64(P, ttot, ttot, ntiles, ttot + ntiles, s));
     HCK(g4d::launch_gather_tiles(raw, pcnt, tcnt, ntiles, ttot, pr, s));
     HCK(g4d::launch_missing(vox, n, GS, ttot + ntiles, pr, cnt + G4D_CNT_MISSING, s));
-    int64_t ngd_f = 0, *ngd_h = hslot(ctx, 1, &ngd_f);
+    int64_t ngd_f = 0, *ngd_h = hslot<1>(ctx, &ngd_f);
     HCK(hipMemcpyAsync(ngd_h, ttot + ntiles, 8, hipMemcpyDeviceToHost, s));
     CK(read_counters(ctx, hc));
     const int64_t ngd = *ngd_h;
@@ -1278,7 +1281,7 @@ static int run_device(g4d_ctx *ctx, const double *d_xyz, int n, const SetSpec &s
             uint64_t *ins = buf<uint64_t>(ctx->ins);
             const int64_t mk = 2 * (int64_t)hc[G4D_CNT_NEW_PAIRS];
             if (mk > g4d::STAR_ROUND_SMALL) {
-                int64_t nrec_f = 0, *nrec_h = hslot(ctx, 9, &nrec_f);
+                int64_t nrec_f = 0, *nrec_h = hslot<9>(ctx, &nrec_f);
                 const int64_t *dev_m = nullptr;
                 HCK(g4d::sort_unique_pair_keys_deferred(P, ins, mk, nb, n, nrec_h, &dev_m, s));
                 HCK(g4d::launch_pass_plan(pass_plan(), ins, dev_m ? mk : *nrec_h, dev_m, s));
@@ -1330,7 +1333,7 @@ static int run_device(g4d_ctx *ctx, const double *d_xyz, int n, const SetSpec &s
     // keep.  The counts are scanned and read along with the list's length, so that a set without
     // such triangles waits once; with some, the exact pass and the scan follow.
     int64_t *toffs = buf<int64_t>(ctx->tetoff);
-    int64_t nt_f = 0, *nt_h = hslot(ctx, 8, &nt_f);
+    int64_t nt_f = 0, *nt_h = hslot<8>(ctx, &nt_f);
     auto scan_tets = [&]() -> int {
         HCK(g4d::scan_excl_i64(P, buf<int64_t>(ctx->tetcnt), toffs, n, toffs + n, s));
         HCK(hipMemcpyAsync(nt_h, toffs + n, 8, hipMemcpyDeviceToHost, s));
@@ -1471,9 +1474,10 @@ int g4d_create(g4d_ctx **out, const g4d_options *opt)
     for (int i = 0; i < 2; i++)
         if (hipEventCreate(&ctx->ev_t0[i]) != hipSuccess) ctx->ev_ok = false;
     // staging of the small host reads; without it they go to pageable variables
-    if (ctx->hpin.ensure(sizeof(int64_t) * 96) == hipSuccess) {
+    constexpr int counts_at = G4D_CNT_NUM + g4d_ctx::STAGE_SCALARS;
+    if (ctx->hpin.ensure(sizeof(int64_t) * (counts_at + g4d_ctx::STAGE_COUNTS)) == hipSuccess) {
         ctx->hstage = static_cast<int64_t *>(ctx->hpin.ptr);
-        ctx->P.hstage = ctx->hstage + G4D_CNT_NUM + 16;
+        ctx->P.hstage = ctx->hstage + counts_at;
     }
     *out = ctx;
     return G4D_OK;
