@@ -256,13 +256,7 @@ static T *buf(DevBuf &b)
     return b.as<T>();
 }
 
-// Sort directed keys (a<<32 | b) with a, b < n < 2^nb.
-static hipError_t sort_pairs(g4d::Prims &P, uint64_t *k, int64_t m, int nb, int64_t n, hipStream_t s)
-{
-    return g4d::sort_pair_keys(P, k, m, nb, n, s);
-}
-
-// The same, then without duplicates; *m becomes the distinct count.
+// Sort directed keys (a<<32 | b) with a, b < n < 2^nb, without duplicates; *m becomes the distinct count.
 static hipError_t sort_unique_pairs(g4d::Prims &P, uint64_t *k, int64_t *m, int nb, int64_t n, hipStream_t s)
 {
     return g4d::sort_unique_pair_keys(P, k, *m, nb, n, m, s);
@@ -1057,7 +1051,6 @@ static int run_device(g4d_ctx *ctx, const double *d_xyz, int n, const SetSpec &s
         sp.pcount = spc;
         sp.cnt = cnt;
         sp.lds_limit = lds_limit;
-        sp.defer_list = nullptr; // larger stars are on the plan's lists
         sp.defer_cap = n;
         sp.exact_list = buf<int>(ctx->xstars);
         sp.exact_cap = n;
@@ -1076,7 +1069,6 @@ static int run_device(g4d_ctx *ctx, const double *d_xyz, int n, const SetSpec &s
         sp.work_counter = G4D_CNT_QUEUE0;
         sp.star_list = list;
         sp.nlist = nitems;
-        sp.nlist_dev = nullptr;
         // Filter-only kernels by size tier over the plan's lists, each star in one of them: they need
         // not wait for each other.  The many small stars run on the call's stream; those of the larger
         // tiers, few at a time and each a long chain of insertions that one wave or work-group
@@ -1189,7 +1181,6 @@ static int run_device(g4d_ctx *ctx, const double *d_xyz, int n, const SetSpec &s
         if (nwide > 0 && hc[G4D_CNT_XL] > 0) {
             // wide stars that need exact predicates: the global-memory kernel has them
             const int64_t nx = (int64_t)hc[G4D_CNT_XL];
-            sp.nlist_dev = nullptr;
             HCK(g4d::launch_zero_counters(cnt, 1ull << G4D_CNT_MISC, s));
             HCK(g4d::launch_need_max(sp, buf<int>(ctx->wexact), (int)nx, cnt + G4D_CNT_MISC, s));
             CK(read_counters(ctx, hc));
@@ -2393,8 +2384,6 @@ int g4d_diag_grid_pairs(g4d_ctx *ctx, const int32_t *id_grid, int32_t grid, uint
     const int64_t G3 = (int64_t)grid * grid * grid;
     HCK(ctx->gtmp.ensure(sizeof(int) * (size_t)G3));
     HCK(hipMemcpyAsync(ctx->gtmp.ptr, id_grid, sizeof(int) * (size_t)G3, hipMemcpyHostToDevice, s));
-    HCK(ctx->cnt.ensure(sizeof(unsigned long long) * G4D_CNT_NUM));
-    unsigned long long *cnt = buf<unsigned long long>(ctx->cnt);
     g4d::GridSets GS;
     SetTotals tot;
     CK(setup_sets(ctx, single_set(1, grid), 1, GS, tot));

@@ -43,44 +43,39 @@ enum g4d_dev_error : uint32_t {
 // Counter block layout (int64 words), device resident, read back once per stage.
 enum g4d_counter : int {
     G4D_CNT_ERROR = 0,
-    G4D_CNT_APPEND0 = 1,  // generic append counters
-    G4D_CNT_APPEND1 = 2,
-    G4D_CNT_APPEND2 = 3,
-    G4D_CNT_ORIENT4 = 4,  // cofactor-filter orient4 evaluations in the 32-vertex star kernel
-    G4D_CNT_EXACT = 5,    // exact insphere evaluations
-    G4D_CNT_SOS = 6,      // SoS resolutions
-    G4D_CNT_ORIENT3 = 7,
-    G4D_CNT_MISC = 8,
-    G4D_CNT_XL = 9,       // list length of the wide kernels' inconclusive stars
-    G4D_CNT_APPEND3 = 10,
-    G4D_CNT_APPEND4 = 11,
-    G4D_CNT_APPEND5 = 12,
-    G4D_CNT_APPEND6 = 13,
-    G4D_CNT_COFACTOR = 14, // cached-cofactor computations in the 32-vertex star kernel
-    G4D_CNT_XMID = 15,     // list lengths of the exact chain's 64- and 256-vertex tiers
-    G4D_CNT_XBIG = 16,
-    G4D_CNT_QUEUE0 = 17,   // work-queue heads of the star-kernel launches of one pass (17..23)
+    G4D_CNT_ORIENT4 = 1,  // cofactor-filter orient4 evaluations in the 32-vertex star kernel
+    G4D_CNT_COFACTOR = 2, // its cached-cofactor computations
+    G4D_CNT_EXACT = 3,    // exact insphere evaluations
+    G4D_CNT_SOS = 4,      // SoS resolutions
+    G4D_CNT_MISC = 5,
+    G4D_CNT_XL = 6,       // list length of the wide kernels' inconclusive stars
+    G4D_CNT_APPEND3 = 7,  // generic append counters
+    G4D_CNT_APPEND4 = 8,
+    G4D_CNT_APPEND5 = 9,
+    G4D_CNT_XMID = 10,    // list lengths of the exact chain's 64- and 256-vertex tiers
+    G4D_CNT_XBIG = 11,
+    G4D_CNT_QUEUE0 = 12,  // work-queue heads of the star-kernel launches of one pass (12..18)
     // a star pass's totals (added by its kernels) and the splaying lists made of them
-    G4D_CNT_PAIRS = 24,    // insertion pairs the pass wrote
-    G4D_CNT_DROWNED = 25,  // insertions it drowned
-    G4D_CNT_DROWN_KEYS = 26,
-    G4D_CNT_TASKS = 27,    // containment proofs to find
-    G4D_CNT_NEW_PAIRS = 28, // pairs the histories do not hold, with repeats
-    G4D_CNT_INS = 29,      // distinct insertions (two per pair)
-    G4D_CNT_ACTIVE = 30,   // stars with insertions, and the region sizes they need
-    G4D_CNT_NEED_V = 31,
-    G4D_CNT_NEED_T = 32,
-    G4D_CNT_NEED_H = 33,
+    G4D_CNT_PAIRS = 19,   // insertion pairs the pass wrote
+    G4D_CNT_DROWNED = 20, // insertions it drowned
+    G4D_CNT_DROWN_KEYS = 21,
+    G4D_CNT_TASKS = 22,   // containment proofs to find
+    G4D_CNT_NEW_PAIRS = 23, // pairs the histories do not hold, with repeats
+    G4D_CNT_INS = 24,     // distinct insertions (two per pair)
+    G4D_CNT_ACTIVE = 25,  // stars with insertions, and the region sizes they need
+    G4D_CNT_NEED_V = 26,
+    G4D_CNT_NEED_T = 27,
+    G4D_CNT_NEED_H = 28,
     // zero from the start of a call, used once in it
-    G4D_CNT_MISSING = 34,
-    G4D_CNT_PUMPED = 35,
-    G4D_CNT_OUT_EXACT = 36,
+    G4D_CNT_MISSING = 29,
+    G4D_CNT_PUMPED = 30,
+    G4D_CNT_OUT_EXACT = 31,
     // made by a pass's plan: lengths of the lists of stars above 32 (64, 128, 256, 512, 1,024 vertices,
     // and beyond), the number above 64, and the largest of the last list
-    G4D_CNT_TIER0 = 37,
-    G4D_CNT_OVER64 = 43,
-    G4D_CNT_NEED_MAX = 44,
-    G4D_CNT_NUM = 45
+    G4D_CNT_TIER0 = 32,
+    G4D_CNT_OVER64 = 38,
+    G4D_CNT_NEED_MAX = 39,
+    G4D_CNT_NUM = 40
 };
 
 #define HIP_CHECK_RET(expr)                                                                    \

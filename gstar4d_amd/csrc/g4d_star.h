@@ -67,8 +67,8 @@ struct StarParams {
     uint64_t *pairbuf;    // per star, from 2 * (ntoff[s] - tbase): its insertion pairs (a<<32 | b,
     int64_t tbase;        // a < b) of unchecked triangles, dense, in triangle order
     int *pcount;          // per star: the number of those pairs
-    int *defer_list;      // stars that exceed this kernel's capacity, counter `defer_counter` (exact kernels;
-                          // the others have the plan's lists, and null)
+    int *defer_list;      // exact kernels: stars that exceed this kernel's capacity, counter `defer_counter`
+                          // (the others have the plan's lists)
     int64_t defer_cap;
     int defer_counter;
     int *exact_list;      // stars whose filters were inconclusive (filter-only kernels),
@@ -76,8 +76,8 @@ struct StarParams {
     int exact_counter;
     int work_counter; // counter word of this launch's work queue (zero at launch)
     int lds_limit;        // largest vn + m handled in LDS (<= STAR_LDS_LIMIT)
-    // work list (nullptr = all stars; an entry below 0 is skipped); with nlist_dev the list length is read on the device
-    // (the counter a previous kernel appended with), nlist being its capacity
+    // work list (an entry below 0 is skipped); with nlist_dev (exact kernels) the list length is read on the
+    // device (the counter a previous kernel appended with), nlist being its capacity
     const int *star_list;
     int nlist;
     const unsigned long long *nlist_dev;

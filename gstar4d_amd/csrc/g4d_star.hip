@@ -251,13 +251,13 @@ __device__ __forceinline__ void star_body(const StarParams &p, int nitems, int b
     constexpr bool COUNT = !EXACT && VMAX == STAR_VMAX_T0; // the statistics are the 32-vertex kernel's
     using Lds = StarLds<VMAX, !REGC>;
     constexpr int TMAX = Lds::TMAX;
-    constexpr int KPL = TMAX / 64;
+    constexpr int KPL = TMAX / 64, UNROLL = REGC ? KPL : 1;
     __shared__ Lds L;
     double rc[REGC ? KPL : 1][4], rp[REGC ? KPL : 1][2];
     const int lane = threadIdx.x;
     unsigned long long *cnt = p.cnt;
 
-    if (p.nlist_dev) {
+    if (EXACT && p.nlist_dev) {
         const unsigned long long c = *p.nlist_dev;
         nitems = c < (unsigned long long)nitems ? (int)c : nitems;
     }
@@ -285,7 +285,7 @@ __device__ __forceinline__ void star_body(const StarParams &p, int nitems, int b
         const int bend = one_each ? base + 1 : (base + CHUNK < nitems ? base + CHUNK : nitems);
 #pragma unroll 1
         for (int item = base; item < bend; item++) {
-            const int s = p.star_list ? p.star_list[item] : item;
+            const int s = p.star_list[item];
             if (s < 0) continue; // on another tier's list
             const int64_t ib = p.ins_off[s];
             const int m = (int)(p.ins_off[s + 1] - ib);
@@ -293,7 +293,7 @@ __device__ __forceinline__ void star_body(const StarParams &p, int nitems, int b
             const int need = vn + m;
             const int lim = VMAX < p.lds_limit ? VMAX : p.lds_limit;
             if (need > lim) {
-                if (p.defer_list) star_list_push(p.defer_list, p.defer_cap, &cnt[p.defer_counter], s, cnt);
+                if (EXACT) star_list_push(p.defer_list, p.defer_cap, &cnt[p.defer_counter], s, cnt);
                 else if (lane == 0) // not the list of this tier
                     atomicOr(&cnt[G4D_CNT_ERROR], (unsigned long long)G4D_DEV_ERR_BUFFER);
                 continue;
@@ -417,7 +417,7 @@ __device__ __forceinline__ void star_body(const StarParams &p, int nitems, int b
                 unsigned vm = 0; // bit k: slot lane + 64 k sees the vertex
                 unsigned um = 0; // bit k: its filter is inconclusive
                 const double rsum = fabs(r[0]) + fabs(r[1]) + fabs(r[2]);
-#pragma unroll(REGC ? KPL : 1)
+#pragma unroll UNROLL
                 for (int k = 0; k < KPL; k++) {
                     const int slot = lane + 64 * k;
                     if (REGC && 64 * k >= T) break; // wave-uniform: a small star in a large tier
@@ -558,7 +558,7 @@ __device__ __forceinline__ void star_body(const StarParams &p, int nitems, int b
                 // pass below (triangle words, coordinates, this lane's cofactor columns) needs no
                 // barrier after them
                 unsigned fm = 0;
-#pragma unroll(REGC ? KPL : 1)
+#pragma unroll UNROLL
                 for (int k = 0; k < KPL; k++) {
                     if (REGC && 64 * k >= T) break;
                     if (lane + 64 * k < T && (L.tv[lane + 64 * k] & TF_FRESH)) fm |= 1u << k;
@@ -911,10 +911,6 @@ __device__ __forceinline__ void star_body_grp(const StarParams &p, int nitems, i
     StarGrpLds &L = Ls[g];
     unsigned long long *cnt = p.cnt;
 
-    if (p.nlist_dev) {
-        const unsigned long long c = *p.nlist_dev;
-        nitems = c < (unsigned long long)nitems ? (int)c : nitems;
-    }
     // Work unit: a batch of NG consecutive list entries, one per group.  As many batches as
     // work-groups or fewer: one batch each, no queue; otherwise STAR_CHUNK batches per atomic.
     const int nbatch = (nitems + NG - 1) / NG;
@@ -942,7 +938,7 @@ __device__ __forceinline__ void star_body_grp(const StarParams &p, int nitems, i
             const int my = base * NG + lane;
             int key = INT_MAX;
             if (lane < nit && my < nitems) {
-                const int s = p.star_list ? p.star_list[my] : my;
+                const int s = p.star_list[my];
                 key = s < 0 ? 0 : (int)(p.ins_off[s + 1] - p.ins_off[s]);
             }
             int rank = 0;
@@ -961,7 +957,7 @@ __device__ __forceinline__ void star_body_grp(const StarParams &p, int nitems, i
             asm volatile("" : "+v"(gl));
             const int item = order[(batch - base) * NG + g];
             // ---- this group's star: checks, then its link and insertions into LDS ----
-            const int entry = item < nitems ? (p.star_list ? p.star_list[item] : item) : -1;
+            const int entry = item < nitems ? p.star_list[item] : -1;
             bool act = entry >= 0; // below: on another tier's list
             const int s = act ? entry : 0;
             const int64_t ib = act ? p.ins_off[s] : 0;
@@ -1458,9 +1454,9 @@ bool star_late_variant(int requested) { return star_t0_variant(requested) == STA
 
 hipError_t launch_star_kernel(const StarParams &p, int vmax, bool exact, int nblocks, hipStream_t s)
 {
-    const int nitems = p.star_list ? p.nlist : p.n;
+    const int nitems = p.nlist;
     if (nitems <= 0) return hipSuccess;
-    if (p.nlist_dev && !p.star_list) return hipErrorInvalidValue;
+    if (!p.star_list || (exact ? !p.defer_list : p.nlist_dev != nullptr)) return hipErrorInvalidValue;
     if (p.lds_limit > STAR_LDS_LIMIT) return hipErrorInvalidValue; // local ids must fit 9 bits
     if (nblocks > nitems) nblocks = nitems;
     if (exact) {
@@ -1477,7 +1473,6 @@ hipError_t launch_star_kernel(const StarParams &p, int vmax, bool exact, int nbl
         if (v == STAR_T0_WAVE) {
             hipLaunchKernelGGL(k_star32, dim3(nblocks), dim3(64), 0, s, p, nitems);
         } else {
-            // one work-group per resident wave: 256 CUs x 4 SIMDs x the variant's occupancy
             // one work-group per resident wave (256 CUs x 4 SIMDs x the variant's occupancy), or
             // one per batch of stars when the list is shorter
             const int per_simd = v <= STAR_T0_G16F ? 3 : 4;
