@@ -118,8 +118,9 @@ EXPORTS = ["g4d_default_options", "g4d_create", "g4d_destroy", "g4d_last_error",
            "g4d_mlp_forward", "g4d_mlp_grad", "g4d_mlp_train", "g4d_check_stars", "g4d_diag_set_link_vertex",
            "g4d_triangulate_device_noalloc", "g4d_set_star_kernel", "g4d_set_grid_table", "g4d_grid_for_set",
            "g4d_set_pba_bands", "g4d_set_stage_graphs", "g4d_diag_sort_pairs", "g4d_diag_pass_plan",
-           "g4d_diag_fail_alloc"]
+           "g4d_diag_fail_alloc", "g4d_diag_star_tiers"]
 
+STAR_TIERS = ("32", "64", "128", "256", "512", "1024", "global", "exact", "wide_exact", "late_passes", "ahead_passes")
 MLP_PARAMS = 7312
 PROP_FEATURES = 12
 PROP_SLOTS = 8
@@ -155,6 +156,7 @@ def load_library(path=None):
     L.g4d_diag_grid_pairs.argtypes = [_vp, _ip, ctypes.c_int32, _up, ctypes.c_int64, _lp]
     L.g4d_diag_copy.argtypes = [_vp, ctypes.c_int64, _dp]
     L.g4d_diag_sort_pairs.argtypes = [_vp, _up, ctypes.c_int64, ctypes.c_int32, ctypes.c_int32, _up, _dp, _ip]
+    L.g4d_diag_star_tiers.argtypes = [_vp, _lp]
     L.g4d_diag_fail_alloc.argtypes = [_vp, ctypes.c_int64, _lp, _lp]
     L.g4d_diag_pass_plan.argtypes = [_vp, ctypes.c_int32, _ip, _ip, _up, ctypes.c_int64, ctypes.c_int32, _lp, _lp, _lp]
     L.g4d_check_result.argtypes = [_vp, ctypes.c_int32, ctypes.POINTER(CheckReport)]
@@ -545,6 +547,12 @@ class Triangulator:
         self._check(self._L.g4d_diag_sort_pairs(self._ctx, _ptr(k, _up), k.shape[0], int(nb), int(method),
                                                 _ptr(out, _up), ctypes.byref(ms), ctypes.byref(sh)))
         return out[:k.shape[0]], ms.value, sh.value
+
+    def diag_star_tiers(self):
+        """Stars of the last call by the kernel that built them (see g4d_diag_star_tiers)."""
+        c = (ctypes.c_int64 * len(STAR_TIERS))()
+        self._check(self._L.g4d_diag_star_tiers(self._ctx, c))
+        return dict(zip(STAR_TIERS, c))
 
     def diag_fail_alloc(self, at=0):
         """The at-th device allocation from now (0: none) finds the memory full on its first try.

@@ -168,6 +168,7 @@ struct g4d_ctx {
     hipEvent_t ev_side[SIDE_STREAMS + 1] = {}; // one per side stream, and the fork's
     bool side_ok = false, side_make = true;
     int64_t fail_alloc = 0; // g4d_diag_fail_alloc
+    int64_t tier_stars[G4D_STAR_TIER_COUNTS] = {}; // g4d_diag_star_tiers
     int pba_bands = 0; // bands of the y and x PBA passes (0: by grid size)
     int stage_graphs = -1; // grid-stage chain as a hipGraph: 1 always, 0 never, -1 batched calls only
     // captured grid-stage chains (site scatter and the PBA passes), keyed by everything the
@@ -738,6 +739,7 @@ static int run_device(g4d_ctx *ctx, const double *d_xyz, int n, const SetSpec &s
     if (min_ws < 4 || min_ws > 64) return set_err(ctx, G4D_ERR_INVALID_INPUT, "min_workset %d outside [4, 64]", min_ws);
     const int nb = bits_for(n);
     memset(&ctx->st, 0, sizeof(ctx->st));
+    memset(ctx->tier_stars, 0, sizeof(ctx->tier_stars));
     ctx->st.num_points = n;
     ctx->st.grid_size = gmax;
     ctx->have_result = false;
@@ -1171,6 +1173,19 @@ static int run_device(g4d_ctx *ctx, const double *d_xyz, int n, const SetSpec &s
             ctx->st.star_t0_filter_evals += (int64_t)hc[G4D_CNT_ORIENT4];
             ctx->st.star_t0_cofactors += (int64_t)hc[G4D_CNT_COFACTOR];
             ctx->st.star_t0_launches++;
+        }
+        {
+            int64_t *ts = ctx->tier_stars, above = 0;
+            for (int k = 0; k < g4d::STAR_TIERS; k++) {
+                ts[1 + k] += tier_n[k];
+                above += tier_n[k];
+            }
+            ts[0] += nitems - above;
+            ts[1 + g4d::STAR_TIERS] += nexact;
+            ts[2 + g4d::STAR_TIERS] += nwide > 0 ? (int64_t)hc[G4D_CNT_XL] : 0;
+            ts[3 + g4d::STAR_TIERS] += late ? 1 : 0;
+            ts[4 + g4d::STAR_TIERS] += ahead ? 1 : 0;
+            static_assert(5 + g4d::STAR_TIERS == G4D_STAR_TIER_COUNTS, "star tier counts");
         }
         ctx->st.big_stars += (int32_t)nover64;
         ctx->st.exact_stars += nexact;
@@ -1763,6 +1778,7 @@ int g4d_triangulate_device_noalloc(g4d_ctx *ctx, const double *d_xyz, int32_t n,
     }
     if (scratch_used) *scratch_used = (int64_t)arena.top;
     ctx->st = tmp.st;
+    memcpy(ctx->tier_stars, tmp.tier_stars, sizeof(ctx->tier_stars));
     if (r != G4D_OK) ctx->err = tmp.err;
     return r;
 }
@@ -2305,6 +2321,13 @@ int g4d_diag_sort_pairs(g4d_ctx *ctx, const uint64_t *keys, int64_t m, int32_t n
     HCK(hipStreamSynchronize(s));
     if (ms) *ms = ctx->ev_ok ? ev_ms(ctx, EV_START, EV_MORTON) : 0.0;
     d.release();
+    return G4D_OK;
+}
+
+int g4d_diag_star_tiers(g4d_ctx *ctx, int64_t *counts)
+{
+    if (!ctx || !counts) return G4D_ERR_INVALID_INPUT;
+    memcpy(counts, ctx->tier_stars, sizeof(ctx->tier_stars));
     return G4D_OK;
 }
 

@@ -335,6 +335,12 @@ int g4d_diag_set_link_vertex(g4d_ctx *ctx, int32_t star, int32_t local, int32_t 
    the LSD sort runs. */
 int g4d_diag_sort_pairs(g4d_ctx *ctx, const uint64_t *keys, int64_t m, int32_t nb, int32_t method, uint64_t *out,
                         double *ms, int32_t *shift);
+/* Stars built by the last call, over its passes, by kernel: 32, 64, 128, 256, 512 and 1,024 vertices, and
+   the global-memory kernel; of them handed on to the exact kernels, and from the 512 and 1,024 ones to
+   the global-memory kernel; passes that took all their stars in one launch, and passes whose round was
+   launched before the host had looked. */
+#define G4D_STAR_TIER_COUNTS 11
+int g4d_diag_star_tiers(g4d_ctx *ctx, int64_t *counts);
 /* Takes the at-th device allocation from now (0: none) of this context to find the memory full on its
    first try, as a full device would.  *left (may be NULL) receives what an earlier call has left to
    count, *kept (may be NULL) the bytes of arenas that the context keeps unused, and would give back

@@ -167,3 +167,61 @@ def test_star_kernel_statistics_are_the_32_vertex_kernels():
     d = run(2, 0)
     assert 0 < c["star_t0_filter_evals"] < d["star_t0_filter_evals"]
     assert 0 < c["star_t0_cofactors"] < d["star_t0_cofactors"]
+
+
+# ---------------------------------------------------------------- which kernel builds a star
+
+@pytest.mark.parametrize("k,tier", [(16, "32"), (48, "64"), (96, "128"), (190, "256"), (380, "512"), (760, "1024"),
+                                    (1500, "global")])
+def test_star_of_each_size_is_built_by_its_kernel(orc, k, tier):
+    """The centre of a shell of k points has most of them in its workset and the rest in its next passes:
+    link and insertions come to k in one of them, k lies inside the tier, and no star needs more.
+    Enough other points that the first pass does not merge its tiers."""
+    rng = np.random.default_rng(k)
+    shell = rng.normal(size=(k, 3))
+    shell *= (0.3 + 0.001 * rng.random((k, 1))) / np.linalg.norm(shell, axis=1)[:, None]
+    x = np.concatenate([[[0.5, 0.5, 0.5]], 0.5 + shell, rng.random((1500, 3)) * 0.15])
+    with g.Triangulator(grid_size=128) as t:
+        tets, _, _ = t.triangulate(x)
+        n = t.diag_star_tiers()
+        st = t.stats()
+    ref, _, _ = orc.triangulate(x, 128)
+    assert (g.canonical(tets) == ref).all()
+    assert n[tier] >= 1
+    wide = ("512", "1024", "global")
+    assert st["huge_stars"] == sum(n[c] for c in wide)
+    assert all(n[c] == 0 for c in wide[wide.index(tier) + 1 if tier in wide else 0:])
+
+
+@pytest.mark.parametrize("norm,points,tier", [(314, 312, "512"), (614, 408, "512"), (1361, 720, "1024")])
+def test_inconclusive_wide_star_is_handed_on(orc, norm, points, tier):
+    """Whole points at one distance from the origin, and the origin: its star has a link of all of them and
+    only zero determinants, so the wide kernel gives it to the global-memory one."""
+    r = int(norm ** 0.5)
+    a = np.arange(-r, r + 1)
+    x = np.stack(np.meshgrid(a, a, a, indexing="ij"), -1).reshape(-1, 3)
+    x = np.concatenate([x[(x * x).sum(1) == norm], [[0, 0, 0]]]).astype(np.float64)
+    assert x.shape[0] == points + 1
+    with g.Triangulator(grid_size=128) as t:
+        tets, _, _ = t.triangulate(x)
+        n = t.diag_star_tiers()
+    ref, _, _ = orc.triangulate(x, 128)
+    assert g.canonical(tets).shape == ref.shape and (g.canonical(tets) == ref).all()
+    assert n[tier] >= 1 and n["wide_exact"] >= 1
+
+
+def test_small_rounds_take_the_short_way(orc):
+    """Late passes of a general set take one launch and are followed without the host's look; a set
+    whose stars need exact predicates throughout never is."""
+    rng = np.random.default_rng(3)
+    with g.Triangulator(grid_size=32) as t:
+        x = rng.random((1000, 3))
+        tets, _, _ = t.triangulate(x)
+        n = t.diag_star_tiers()
+        assert (g.canonical(tets) == orc.triangulate(x, 32)[0]).all()
+        assert n["ahead_passes"] >= 1 and n["exact"] == n["wide_exact"] == n["global"] == 0
+        lattice = np.stack(np.meshgrid(*[np.arange(9.0)] * 3, indexing="ij"), -1).reshape(-1, 3)
+        tets, _, _ = t.triangulate(lattice)
+        n = t.diag_star_tiers()
+        assert (g.canonical(tets) == orc.triangulate(lattice, 32)[0]).all()
+        assert n["exact"] > 0
