@@ -436,7 +436,11 @@ struct SideStreams {
     }
 };
 
-// Passes of at most this many stars may run their two tiers in one launch.
+// Passes of at most this many stars may run their two tiers in one launch: as many as a pass has keys
+// whose plan merges the tiers above 32, so that it is no more of a limit there (some 1,300 stars), but
+// keeps a long list of small stars with a few of more than 128 vertices out of that launch, which
+// holds fewer waves.  With 1,024 in its place the calls of k_star_late's comment are the same within
+// their runs' noise.
 static constexpr int LATE_STARS = 6144;
 static const uint64_t PLAN_COUNTERS = (1ull << G4D_CNT_ACTIVE) | (1ull << G4D_CNT_NEED_V) | (1ull << G4D_CNT_NEED_T) |
                                       (1ull << G4D_CNT_NEED_H) | (0xffull << G4D_CNT_TIER0);
@@ -893,7 +897,7 @@ static int run_device(g4d_ctx *ctx, const double *d_xyz, int n, const SetSpec &s
     HCK(ctx->big.ensure(sizeof(int) * (size_t)n));
     HCK(ctx->huge.ensure(sizeof(int) * (size_t)n));
     HCK(ctx->xstars.ensure(sizeof(int) * (size_t)n));
-    const int nblk_star = 5120; // 256 CUs x 20 resident waves of the 32-vertex tier (5 per SIMD)
+    const int nblk_star = 5120; // 256 CUs x 20 resident waves of k_star32; the grouped variants take their own
     const int lds_limit = std::min(g4d::STAR_LDS_LIMIT, ctx->opt.lds_star_limit > 0 ? ctx->opt.lds_star_limit
                                                                                   : g4d::STAR_LDS_LIMIT);
 

@@ -678,7 +678,10 @@ __device__ __noinline__ int sos_orient4(const double *const *pin, const int *idx
 //
 // Bound by the latency of one wave's dependent FP64 operations (few lanes have work).  30,000
 // points, half of them on a sphere and a lattice (1.8 M evaluations, 1.5 M of them zero): the
-// exact star kernels 125 -> 32 ms, the exact proofs 9.1 -> 4.0 ms.
+// exact star kernels 125 -> 32 ms, the exact proofs 9.1 -> 4.0 ms.  The determinant and the SoS
+// minors use all 256 VGPRs and some AGPRs, and the general forms behind them 2,368 bytes of scratch:
+// their kernels hold one wave per SIMD, where the integer forms alone left two in the 32- and
+// 64-vertex exact kernels and the proofs (248 VGPRs).
 // ------------------------------------------------------------------------------------
 
 namespace lb {

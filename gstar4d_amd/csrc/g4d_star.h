@@ -61,7 +61,7 @@ struct StarParams {
     const int64_t *nvoff;
     const int64_t *ntoff;
     const int64_t *nhoff;
-    // outputs without atomics (compacted by the host code after the pass)
+    // outputs, each star's in its own places
     uint8_t *dflag;       // per insertion, indexed like ins_keys: 1 when the vertex drowned (total:
                           // G4D_CNT_DROWNED; the pairs' total: G4D_CNT_PAIRS)
     uint64_t *pairbuf;    // per star, from 2 * (ntoff[s] - tbase): its insertion pairs (a<<32 | b,
@@ -96,12 +96,12 @@ enum {
     STAR_T0_NUM = 5
 };
 
-// LDS star kernel for stars of up to vmax (STAR_VMAX_T0, T1, TM or T2) link vertices plus
-// insertions; larger ones go to p.defer_list.  exact = false: filters only (no multiprecision
-// code, no private scratch), a star with an inconclusive orientation goes to p.exact_list
-// untouched.  exact = true: exact predicates and SoS, for the stars of star_list.
 // Zeroes the counter words whose bits are set in mask (one launch instead of one fill per word).
 hipError_t launch_zero_counters(unsigned long long *cnt, uint64_t mask, hipStream_t s);
+// LDS star kernel for stars of up to vmax link vertices plus insertions.  exact = false (vmax
+// STAR_VMAX_T0, T1, TM or T2): filters only, over a list of the plan; a star with an inconclusive
+// orientation goes to p.exact_list untouched.  exact = true (T0, T1 or T2): exact predicates and SoS,
+// for the stars of star_list; larger ones go to p.defer_list.
 hipError_t launch_star_kernel(const StarParams &p, int vmax, bool exact, int nblocks, hipStream_t s);
 // The default 32-vertex kernel over p's list and the 256-vertex one over q's, side by side in one launch.
 hipError_t launch_star_late(const StarParams &p, const StarParams &q, hipStream_t s);

@@ -10,19 +10,20 @@
 //   history                  GD/GDelaunay/GDelKernels.cu:984-1068,1625-1677
 //   tetra output             GD/GDelaunay/GDelKernels.cu:1097-1191, GD/GDelaunay/GDelPredKernels.cu:628-692
 //
-// MI355X design.  One wave64 owns one star at a time (dynamic work queue).  The star's link
-// (a triangulated 2-sphere) lives in LDS: local vertex table with coordinates relative to the
-// star point, triangles with 9-bit local vertices and 16-bit adjacency.  Each lane owns the
-// triangle slots lane, lane+64, ...; for each slot LDS caches the four cofactors of the
-// lifted 4x4 determinant, so the beneath test of a new vertex v against triangle
-// (a,b,c) is one 4-term dot product:
+// MI355X design.  A pass's plan lists its stars by size.  A group of 16 lanes builds a star of up to 32
+// link vertices (four stars a wave), a wave one of up to 256, a work-group larger ones.  The star's
+// link (a triangulated 2-sphere) lives in LDS, beyond 1,024 vertices in HBM: local vertex table with
+// coordinates relative to the star point, triangles with local vertices and adjacency.  Each lane owns
+// triangle slots (lane, lane + lanes, ...) and keeps for each the four cofactors of the lifted 4x4
+// determinant, in registers (in LDS in the exact kernels, in HBM in the global-memory one), so the
+// beneath test of a new vertex v against triangle (a,b,c) is one 4-term dot product:
 //     orient4(a,b,c,s,v) = v'x*Mx - v'y*My + v'z*Mz - v'l*Ml      (primes: relative to s)
-// with a forward-error bound from the cofactor permanents; uncertain lanes fall back to the
-// exact integer predicate with SoS.  The hole boundary after freeing beneath triangles is
-// found in parallel (edges of freed triangles whose neighbour survives), slots are assigned
-// with a wave prefix sum over a free-slot stack, and the fan's adjacency is closed through
-// two per-vertex maps (boundary edge starting / ending at each vertex).  The whole insertion
-// list of a star runs inside one kernel, so there is no host loop per insertion index.
+// with a forward-error bound from the cofactor permanents.  A star with an uncertain sign goes, untouched,
+// to a kernel that has the exact predicate with SoS.  The hole boundary after freeing beneath
+// triangles is found in parallel (edges of freed triangles whose neighbour survives), slots are
+// assigned with a prefix sum over a free-slot stack, and the fan's adjacency is closed through two
+// per-vertex maps (boundary edge starting / ending at each vertex).  The whole insertion list of a star
+// runs inside one kernel, so there is no host loop per insertion index.
 #include "g4d_predicates.h"
 #include <algorithm>
 #include <climits>
@@ -240,10 +241,10 @@ __device__ __forceinline__ void star_commit(const StarParams &p, int s, int vcou
 
 // EXACT = false: filters only.  A star with an inconclusive orientation is handed to
 // p.exact_list untouched (its output is written only at the end), so the kernel carries no
-// multiprecision code and no private scratch.  Its registers then have room for the cofactors of
-// the lane's own slots, with two permanents each (the largest of the three coordinates', and the
-// lift's), which only that lane reads: without them in LDS a 256-vertex star takes 25 KB instead
-// of 57 and six waves share a CU instead of two.
+// multiprecision code.  Its registers then have room for the cofactors of the lane's own slots, with
+// two permanents each (the largest of the three coordinates', and the lift's), which only that lane
+// reads: without them in LDS a 256-vertex star takes 25 KB instead of 57 and six waves share a CU
+// instead of two.  At the occupancies below 50 to 150 bytes a lane of other values spill.
 template <int VMAX, bool EXACT>
 __device__ __forceinline__ void star_body(const StarParams &p, int nitems, int bid, int nblk)
 {
@@ -685,25 +686,26 @@ __device__ __forceinline__ void star_body(const StarParams &p, int nitems, int b
     }
 }
 
-// The 32-vertex tier (7 KB of LDS) is compiled for 5 waves per SIMD (96 VGPRs, a few spilled
-// to scratch): measured at 4,194,304 uniform points, 5 waves beat 3, 4, 6 and 7 (49.8 ms per
-// triangulation against 63.2, 54.2, 51.0 and 62.9).  The larger tiers are limited by their LDS
-// footprint instead.
+// The 32-vertex tier with one star a wave, selectable: 3.2 KB of LDS, five waves per SIMD (96 VGPRs, 148
+// bytes spilled).  At 4,194,304 uniform points 46.8 ms where the grouped kernel below takes 15.3.
 __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(5, 8))) k_star32(StarParams p, int nitems)
 {
     star_body<STAR_VMAX_T0, false>(p, nitems, blockIdx.x, gridDim.x);
 }
 
-// The filter-only tiers above: the registers that each occupancy leaves, measured on 1,000,000
-// clustered points (12 passes): 64 vertices at 3, 4, 5 waves per SIMD 11.0, 9.9, 10.5 ms; 128 at
-// 2, 3 waves 9.5, 8.3 ms; 256 at 2 waves 8.5 ms.  With cofactors in LDS and no 128-vertex tier
-// the 64-vertex stars took 11.7 ms and all larger ones 38.8.
+// The exact predicates' callee takes 256 VGPRs, 34 to 43 AGPRs and 2,368 bytes of scratch a lane (the
+// integer forms for wide coordinates): one wave per SIMD.  Bound by that callee's latency in the few
+// lanes whose signs are open.
 template <int VMAX>
 __global__ void __launch_bounds__(64) k_star_exact(StarParams p, int nitems)
 {
     star_body<VMAX, true>(p, nitems, blockIdx.x, gridDim.x);
 }
 
+// The filter-only tiers above 32: the registers that each occupancy leaves, measured on 1,000,000
+// clustered points (12 passes): 64 vertices at 3, 4, 5 waves per SIMD 11.0, 9.9, 10.5 ms; 128 at
+// 2, 3 waves 9.5, 8.3 ms; 256 at 2 waves 8.5 ms.  With cofactors in LDS and no 128-vertex tier
+// the 64-vertex stars took 11.7 ms and all larger ones 38.8.
 template <int VMAX, int WPE>
 __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WPE, 8))) k_star(StarParams p, int nitems)
 {
@@ -725,10 +727,10 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(WPE, 8)
 // goes to p.exact_list untouched; a star beyond the tier is left to the plan's lists.
 //
 // Bound by vector instructions (two thirds of the issue slots at three waves per SIMD, of them a
-// fifth FP64), with the LDS pipe half busy.  At 4,194,304 uniform points (G = 512) all its passes took
+// fifth FP64), with the LDS pipe half busy.  At 4,194,304 uniform points (G = 512) its passes took
 // 22.3 ms with 16-bit indices and the permanents of every triangle; 2 KB a star, which lets four waves
 // share a SIMD, one word per boundary edge, the cheap bound in place of the permanents (70 instructions
-// a triangle slot before, 43 now) and packed scans: 15.6 ms.
+// a triangle slot before, 43 now) and packed scans: 15.3 ms.
 // ------------------------------------------------------------------------------------
 
 static constexpr uint32_t GF_ALIVE = 1u << 31; // a triangle of the star as it stands (the sign of the word)
@@ -1398,9 +1400,11 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4, 8)))
 
 // A late pass's two tiers (32 and, merged, 64 to 256 vertices) in one launch: work-groups below nb take
 // batches of p's list, the others stars of q's.  Both finish when their longest star does (some
-// 35 us each), which this pays once.  The registers and LDS of the larger tier cost the smaller one
-// nothing in a pass that does not fill the chip.  1,000 uniform points, five late rounds, with the
-// round's other kernels launched behind it at once: 1.40 -> 1.24 ms a call.
+// 35 us each), which this pays once.  The larger tier's 256 registers and both LDS blocks (33.9 KB)
+// leave one wave per SIMD, 1,024 work-groups on the chip; such a pass has some four keys a star, so
+// 6,144 keys come to some 1,300 stars, 330 batches beside a few hundred larger stars.  One launch
+// against two: 1,000 uniform points (five late passes) 1.20 and 1.34 ms a call, 7,000 1.77 and 1.81,
+// 100,000 4.72 and 4.89, 300,000 6.36 and 6.54.
 __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 8))) k_star_late(StarParams p, int nb,
                                                                                             StarParams q)
 {
@@ -1410,8 +1414,8 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2, 8)))
 
 // The 32-vertex filter-only kernel variant of a launch: the caller's choice, else the
 // G4D_STAR_T0 environment variable (measurement), else the measured best: four stars per wave with
-// the FP32 bound at four waves per SIMD, 15.6 ms of star kernel at 4,194,304 uniform points (G = 512)
-// against 18.3 at three (and 24 for two stars per wave).
+// the FP32 bound at four waves per SIMD, 15.3 ms of star kernel at 4,194,304 uniform points (G = 512)
+// against 18.1 at three (18.4 with the FP64 permanents), 22.6 for two stars per wave and 46.8 for one.
 static int star_t0_variant(int requested)
 {
     if (requested >= 0 && requested < STAR_T0_NUM) return requested;
@@ -1897,10 +1901,11 @@ hipError_t launch_star_wide(const StarParams &p, int vmax, hipStream_t s)
 }
 
 // ------------------------------------------------------------------------------------
-// Global-memory star kernel: the same insertion / finalisation as k_star for stars whose
-// link exceeds the LDS kernels' capacity.  One wave per star; the star's working arrays
-// (32-bit local indices, cached cofactors per triangle slot) live in a per-block HBM
-// workspace sized for the largest such star of the pass.
+// Global-memory star kernel: the same insertion / finalisation as k_star for stars whose link exceeds
+// the LDS kernels' capacity, and with exact predicates for the wide ones' inconclusive stars.  A
+// work-group of 512 threads per star; the star's working arrays (32-bit local indices, cached
+// cofactors per triangle slot) live in a per-block HBM workspace sized for the largest such star of
+// the pass.
 // ------------------------------------------------------------------------------------
 
 static constexpr int GSTAR_NT = STAR_ORDER; // threads per star in the global-memory kernel
