@@ -2604,7 +2604,8 @@ hipError_t launch_nonmutual(const uint64_t *keys, int64_t m, uint64_t *tasks, un
 // The drowned insertions of a late round, at most DROWN_SMALL of them, to proof tasks in one launch:
 // the keys collected in LDS, a bitonic sort, and the tasks of the ones that are not mutual, in the
 // place of three launches and the gaps between them.  Bound by latency: 13-17 us for up to a thousand
-// drowned, 24 us for 1,700 of 4,600 insertions, as long as the three kernels alone took.
+// drowned, 24 us for 1,700 of 4,600 insertions, as long as the three kernels alone took; 39 us for lists
+// that the sort pads to 4,096.
 __global__ void __launch_bounds__(1024) k_drown_small(const uint64_t *ins_keys, const uint8_t *dflag, int m, int nd,
                                                       uint64_t *tasks, unsigned long long *cnt)
 {
@@ -3026,7 +3027,8 @@ hipError_t launch_pass_plan(const PassPlan &p, const uint64_t *keys, int64_t m, 
 // Late rounds insert a few thousand keys or fewer, and every one of the sort, unique, compaction and
 // scan launches they took cost 3-10 us with a host round trip between some: 20 launches and four
 // round trips.  One work-group does all of it in LDS: a bitonic sort (78 steps for 4,096
-// keys), repeats removed, runs listed, region sizes scanned; bound by its barriers, 13-17 us.
+// keys), repeats removed, runs listed, region sizes scanned; bound by its barriers and LDS latency: 11 us
+// for lists that the sort pads to 512 keys, 18 for 1,024, 40 to 44 for 4,096.
 // With the appended lists before it a call on 1,000 points makes 178 launches instead of 331 (2.40 ->
 // 1.70 ms), on 100,000 330 instead of 656 (7.1 -> 6.25 ms).
 static constexpr int SR_THREADS = 1024;
